@@ -145,6 +145,11 @@ __device__ __forceinline__ u32x4 load16_unaligned(const void* p) {
   __builtin_memcpy(&v, p, 16);
   return v;
 }
+// The streaming form for addresses on any 4-byte boundary.
+__device__ __forceinline__ u32x4 load16_stream_any(const void* p) {
+  typedef unsigned u32x4_on_4 __attribute__((ext_vector_type(4), aligned(4)));
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_on_4*>(p));
+}
 __device__ __forceinline__ void store16_unaligned(void* p, const u32x4& v) { __builtin_memcpy(p, &v, 16); }
 // Non-temporal stores: a bare copy kernel runs ~4 % faster with the default policy, but in the
 // loss kernels (sparse corrections follow the dense row) the non-temporal hint measured faster.

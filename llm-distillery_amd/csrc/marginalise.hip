@@ -75,8 +75,17 @@ __device__ __forceinline__ float plan_tile_value(const float* tile, unsigned byt
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(tile) + byte_offset);
 }
 
+// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows that start on any element and end inside a 16-byte
+// unit (an odd vocabulary: no pitch keeps its rows on the 16-byte grid), for the planned form only.  Such a row is
+// still moved 16 bytes at a time -- global memory takes unaligned 16-byte loads -- and the unit its last 1-3
+// elements fall into is loaded as the row's last 16 bytes and shifted into place on its way to LDS.  Measured: 7067 rows x
+// 151665 probabilities onto 10352 ids 6.39 -> 1.12 ms, 457 rows onto 32000 ids 478 -> 91 us (on the grid: 1.00 ms for
+// the former; the LDS-atomic form such rows fell back to runs at one
+// lane per three cycles).
+enum MargLoad : int { MARG_SCALAR = 0, MARG_VEC = 1, MARG_ANY = 2 };
+
 // Marginal of one teacher row into marg[0, Vs) (LDS, zeroed here) along a plan; `tile` is LDS
-// scratch of plan_tile floats.  fp32 probabilities, 16-byte aligned rows.
+// scratch of plan_tile floats.  fp32 probabilities; LOAD = MARG_VEC: 16-byte aligned rows of whole units.
 //
 // The hot loop is straight-line code: per entry a read of the tile, a read of the entry's slot, the
 // running sum of the run (restarted where the entry says so) and a store of slot + running sum.
@@ -130,6 +139,7 @@ __device__ __forceinline__ void plan_consume_packed(const u32x4& d, const float*
 // scheduling barriers pin.  (With the entries of the first tile issued ahead of its data, as the
 // compiler had it, every wait in the loop became a wait for all but one or none of the loads: one
 // tile in flight whatever the depth, and the entries' trip to L2 and back waited for in full.)
+template <int LOAD>
 __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p, const char* prow, float* marg,
                                                             float* tile) {
   const int tid = threadIdx.x, lane = tid & (WAVE - 1);
@@ -149,8 +159,25 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   // in flight and never has to drain the whole queue.  What a clamped load brings is never used: no
   // entry points behind the end of the row, and a select on the value here would make the thread
   // wait for the load right away instead of two tiles later.
+  const int rem = LOAD == MARG_ANY ? (int)(p.Vt & 3) : 0;               // elements of the row's last, partial unit
+  const int last_unit = (int)(n4 - (int64_t)(ntiles - 1) * q_tile);     // its number inside the last tile
   u32x4 tbuf[2][2];
   auto fetch_tile = [&](int k, u32x4 (&buf)[2]) {
+    if constexpr (LOAD == MARG_ANY) {
+      const bool in_row = k < ntiles;
+      const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
+      const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const int c = u * MARG_NT + tid;
+        int off = (c < q_tile && c < left) ? c * 16 : 0;
+        // a tile of fewer than four elements has no whole unit of its own: the row's first one stands in
+        if (in_row && left == 0) off = -(int)((int64_t)k * TS * 4);
+        if (rem && k == ntiles - 1 && c == left) off = (c * 4 + rem - 4) * 4;      // the row's last 16 bytes (Vt >= 4)
+        buf[u] = load16_stream_any(base + off);
+      }
+      return;
+    }
     const bool in_row = k < ntiles;
     const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
     const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;      // 16-byte units from the tile's start to the row's end
@@ -199,6 +226,14 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   float run = 0.f;
   auto do_tile = [&](int k, u32x4 (&buf)[2], PlanBatch& e, PlanBatch& e_next) {
     __syncthreads();                                 // previous tile fully consumed (first pass: marg zeroed)
+    if (LOAD == MARG_ANY && rem && k == ntiles - 1) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (u * MARG_NT + tid == last_unit) {
+          const u32x4 v = buf[u];
+          buf[u] = rem == 1 ? u32x4{v[3], 0u, 0u, 0u} : rem == 2 ? u32x4{v[2], v[3], 0u, 0u} : u32x4{v[1], v[2], v[3], 0u};
+        }
+    }
 #pragma unroll
     for (int u = 0; u < 2; ++u)
       if (u * MARG_NT + tid < q_tile) *reinterpret_cast<u32x4*>(tile + ((int64_t)u * MARG_NT + tid) * 4) = buf[u];
@@ -241,13 +276,13 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
 }
 
 // Accumulate the slice [s_lo, s_lo + s_n) of one row's marginal into `acc` (LDS, zeroed here).
-template <bool VEC>
+template <int LOAD>
 __device__ __forceinline__ void accumulate_marginal(const MargParams& p, const char* prow, float* acc, int s_lo,
                                                     int s_n) {
   const int tid = threadIdx.x;
   for (int j = tid; j < s_n; j += MARG_NT) acc[j] = 0.f;
   __syncthreads();
-  if (VEC) {       // fp32 probabilities, 16-byte aligned: four columns per load
+  if constexpr (LOAD == MARG_VEC) {       // fp32 probabilities, 16-byte aligned: four columns per load
     // Double-buffered batches of U 16-byte loads of the probabilities and of the id map per thread:
     // the next batch is in flight while the current one is scattered into LDS.
     constexpr int U = 4;
@@ -299,7 +334,7 @@ __device__ __forceinline__ void accumulate_marginal(const MargParams& p, const c
 }
 
 // marg (or log marg) to memory; student vocabularies wider than the LDS slice take several passes.
-template <bool VEC>
+template <int LOAD>
 __global__ __launch_bounds__(MARG_NT) void marginalise_map_kernel(const MargParams p) {
   extern __shared__ __align__(16) float acc[];
   const int64_t r = xcd_banded_row(blockIdx.x);
@@ -307,15 +342,15 @@ __global__ __launch_bounds__(MARG_NT) void marginalise_map_kernel(const MargPara
   const int pb = p.p_dtype == F32 ? 4 : 2;
   const char* prow = reinterpret_cast<const char*>(p.probs) + r * p.p_stride * pb;
   float* out = p.marg + r * p.marg_stride;
-  if (VEC && p.plan_ent) {
+  if (LOAD != MARG_SCALAR && p.plan_ent) {
     float* marg = acc + p.plan_tile + PLAN_ZERO_WORDS;      // the tile sits first: its addresses are then plain offsets
-    accumulate_marginal_planned(p, prow, marg, acc);
+    accumulate_marginal_planned<LOAD>(p, prow, marg, acc);
     for (int j = threadIdx.x; j < p.Vs; j += MARG_NT) out[j] = p.out_log ? logf(marg[j]) : marg[j];
     return;
   }
   for (int64_t s_lo = 0; s_lo < p.Vs; s_lo += MARG_MAX_VS) {
     const int s_n = (int)min((int64_t)MARG_MAX_VS, p.Vs - s_lo);
-    accumulate_marginal<VEC>(p, prow, acc, (int)s_lo, s_n);
+    accumulate_marginal<LOAD>(p, prow, acc, (int)s_lo, s_n);
     for (int j = threadIdx.x; j < s_n; j += MARG_NT) out[s_lo + j] = p.out_log ? logf(acc[j]) : acc[j];
     __syncthreads();
   }
@@ -745,7 +780,7 @@ __device__ __forceinline__ void expand_gradient_row(const float* marg, const uns
   }
 }
 
-template <class TagS, int NU, bool VEC>
+template <class TagS, int NU, int LOAD>
 __global__ __launch_bounds__(MARG_NT) void rkl_marginalised_kernel(const MargParams p) {
   extern __shared__ __align__(16) float acc[];
   __shared__ float red[64];
@@ -766,13 +801,13 @@ __global__ __launch_bounds__(MARG_NT) void rkl_marginalised_kernel(const MargPar
   const char* prow = reinterpret_cast<const char*>(p.probs) + trow * p.p_stride * pb;
   float* marg = acc;
   // the student row is in flight during the accumulation
-  if (VEC && p.plan_ent) {
+  if (LOAD != MARG_SCALAR && p.plan_ent) {
     marg = acc + p.plan_tile + PLAN_ZERO_WORDS;  // the tile sits first: its addresses are then plain offsets
     if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
-    accumulate_marginal_planned(p, prow, marg, acc);
+    accumulate_marginal_planned<LOAD>(p, prow, marg, acc);
   } else {
     if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
-    accumulate_marginal<VEC>(p, prow, acc, 0, (int)p.Vs);
+    accumulate_marginal<LOAD>(p, prow, acc, 0, (int)p.Vs);
   }
   if (rkl_against_marginal<TagS, NU>(rows.s, rows.nunits, marg, red, p, r, grow, srow)) {      // the same for every thread
     __syncthreads();                             // the gradient of every compact column is in LDS
@@ -796,23 +831,35 @@ static void allow_large_lds() {
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (done_for == dev) return;
-  allow_large_lds_for(&marginalise_map_kernel<true>);
-  allow_large_lds_for(&marginalise_map_kernel<false>);
-  allow_large_lds_for(&rkl_marginalised_kernel<TagF32, MARG_NU, true>);
-  allow_large_lds_for(&rkl_marginalised_kernel<TagF32, MARG_NU, false>);
-  allow_large_lds_for(&rkl_marginalised_kernel<TagBF16, MARG_NU, true>);
-  allow_large_lds_for(&rkl_marginalised_kernel<TagBF16, MARG_NU, false>);
-  allow_large_lds_for(&rkl_marginalised_kernel<TagF16, MARG_NU, true>);
-  allow_large_lds_for(&rkl_marginalised_kernel<TagF16, MARG_NU, false>);
+  allow_large_lds_for(&marginalise_map_kernel<MARG_SCALAR>);
+  allow_large_lds_for(&marginalise_map_kernel<MARG_VEC>);
+  allow_large_lds_for(&marginalise_map_kernel<MARG_ANY>);
+#define DL_LARGE_RKLM(TAG)                                                      \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR>);     \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_VEC>);        \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_ANY>)
+  DL_LARGE_RKLM(TagF32);
+  DL_LARGE_RKLM(TagBF16);
+  DL_LARGE_RKLM(TagF16);
+#undef DL_LARGE_RKLM
   done_for = dev;
 }
 
 }  // namespace dl
 
+// The way the teacher's rows can be read: 16 bytes at a time on the grid (either form of the sum), or off it (the
+// planned form only: MARG_ANY holds while a usable plan is attached).
+static int marg_load_of(const void* probs, int p_dtype, int64_t p_stride, int64_t Vt, const int32_t* t2s) {
+  using namespace dl;
+  if (p_dtype != DL_F32) return MARG_SCALAR;
+  if (Vt % 4 == 0 && ok16(probs, p_stride, 4) && ok16(t2s, 0, 4)) return MARG_VEC;
+  return Vt >= 4 && reinterpret_cast<uintptr_t>(probs) % 4 == 0 ? MARG_ANY : MARG_SCALAR;
+}
+
 // Fills the plan fields of `p` if a usable plan is given; returns the dynamic LDS bytes to request.
 static size_t attach_plan(dl::MargParams& p, const int32_t* plan_row_off, const uint32_t* plan_ent, int plan_tile,
-                          const int32_t* plan_fold, int plan_n_fold, int plan_n_extra, bool vec, size_t lds_without_plan) {
-  if (!plan_row_off || !plan_ent || !vec) return lds_without_plan;
+                          const int32_t* plan_fold, int plan_n_fold, int plan_n_extra, int load, size_t lds_without_plan) {
+  if (!plan_row_off || !plan_ent || load == dl::MARG_SCALAR) return lds_without_plan;
   if (plan_tile < 4096 || plan_tile > 8192 || plan_tile % 1024) return lds_without_plan;
   if (plan_n_fold < 0 || plan_n_extra < 0 || (plan_n_fold > 0 && !plan_fold)) return lds_without_plan;
   const size_t need = (size_t)dl::plan_slot_words(p.Vs, plan_n_extra) * 4 + (size_t)(plan_tile + dl::PLAN_ZERO_WORDS) * 4;
@@ -836,13 +883,16 @@ extern "C" int dl_marginalise_map(const void* probs, int p_dtype, int64_t p_stri
   MargParams p{};
   p.probs = probs; p.p_dtype = p_dtype; p.p_stride = p_stride; p.n_rows = n_rows; p.Vt = Vt; p.t2s = t2s; p.Vs = Vs;
   p.marg = marg; p.marg_stride = marg_stride; p.out_log = out_log;
-  const bool vec = p_dtype == DL_F32 && Vt % 4 == 0 && ok16(probs, p_stride, 4) && ok16(t2s, 0, 4);
-  const size_t lds = attach_plan(p, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold, plan_n_extra, vec,
+  int load = marg_load_of(probs, p_dtype, p_stride, Vt, t2s);
+  const size_t lds = attach_plan(p, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold, plan_n_extra, load,
                                  (size_t)(Vs < MARG_MAX_VS ? Vs : MARG_MAX_VS) * 4);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   allow_large_lds();
-  if (vec) hipLaunchKernelGGL((marginalise_map_kernel<true>), dim3(xcd_banded_grid(n_rows)), dim3(MARG_NT), lds, st, p);
-  else hipLaunchKernelGGL((marginalise_map_kernel<false>), dim3(xcd_banded_grid(n_rows)), dim3(MARG_NT), lds, st, p);
+  if (load == MARG_ANY && !p.plan_ent) load = MARG_SCALAR;
+  const dim3 grid(xcd_banded_grid(n_rows)), block(MARG_NT);
+  if (load == MARG_VEC) hipLaunchKernelGGL((marginalise_map_kernel<MARG_VEC>), grid, block, lds, st, p);
+  else if (load == MARG_ANY) hipLaunchKernelGGL((marginalise_map_kernel<MARG_ANY>), grid, block, lds, st, p);
+  else hipLaunchKernelGGL((marginalise_map_kernel<MARG_SCALAR>), grid, block, lds, st, p);
   return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
 }
 
@@ -896,15 +946,17 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
   p.Vs = Vs; p.logits = logits; p.s_dtype = logits_dtype; p.row_stride = row_stride; p.n_srows = n_rows;
   p.row_map = row_map; p.inv_T_s = inv_T_student; p.inv_T_t = inv_T_teacher; p.grad_scale = grad_scale;
   p.row_loss = row_loss; p.grad = grad; p.grad_stride = grad_stride;
-  const bool vec = p_dtype == DL_F32 && Vt % 4 == 0 && ok16(t_probs, p_stride, 4) && ok16(t2s, 0, 4);
-  const size_t lds = attach_plan(p, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold, plan_n_extra, vec, (size_t)Vs * 4);
+  int load = marg_load_of(t_probs, p_dtype, p_stride, Vt, t2s);
+  const size_t lds = attach_plan(p, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold, plan_n_extra, load, (size_t)Vs * 4);
+  if (load == MARG_ANY && !p.plan_ent) load = MARG_SCALAR;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid(xcd_banded_grid(n_rows)), block(MARG_NT);
   allow_large_lds();
 #define DL_LAUNCH_RKLM(TAG)                                                                                  \
   do {                                                                                                       \
-    if (vec) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, true>), grid, block, lds, st, p);           \
-    else hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, false>), grid, block, lds, st, p);              \
+    if (load == MARG_VEC) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_VEC>), grid, block, lds, st, p);        \
+    else if (load == MARG_ANY) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_ANY>), grid, block, lds, st, p);   \
+    else hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR>), grid, block, lds, st, p);                      \
   } while (0)
   if (logits_dtype == DL_F32) DL_LAUNCH_RKLM(TagF32);
   else if (logits_dtype == DL_BF16) DL_LAUNCH_RKLM(TagBF16);

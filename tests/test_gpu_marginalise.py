@@ -387,3 +387,36 @@ def test_a_plan_that_holds_the_compact_form_only(D, Vs, dtype):
     assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
     m = D.vocab_utils.marginalise(probs.to(DEV), plan=plan, n_student=Vs).cpu().numpy()
     np.testing.assert_allclose(m, marg.numpy(), rtol=2e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize("Vt", [5, 1023, 4097, 8193, 12290, 20483, 24577])
+@pytest.mark.parametrize("shift", [0, 3])
+def test_planned_forms_on_teacher_rows_off_the_16_byte_grid(D, Vt, shift):
+    """A teacher vocabulary that is not a multiple of four ids (and rows starting on any element): rows shorter than a
+    tile, rows that end 1-3 elements into a 16-byte unit, and a last tile that holds nothing but those.  The rows end
+    where the buffer ends."""
+    R, Vs = 5, 2048
+    rng = np.random.default_rng(Vt)
+    t2s = rng.integers(-1, 700, Vt).astype(np.int32)
+    t2s[-1] = 13                                     # the last element counts
+    probs = torch.softmax(torch.randn(R, Vt, generator=torch.Generator().manual_seed(Vt)) * 2, -1)
+    buf = torch.zeros(shift + R * Vt, device=DEV)
+    on_gpu = buf[shift:].view(R, Vt)
+    on_gpu.copy_(probs)
+    ref = O.marginalise_map(probs.numpy(), t2s, Vs)
+    logits = torch.randn(R, Vs, generator=torch.Generator().manual_seed(1)) * 2
+    with np.errstate(divide="ignore"):
+        t_logits = O.marginal_to_teacher_logits(torch.tensor(ref))
+    _, rows64, grad64 = O.mean_loss_and_grad("rkl", logits, 1.3, t_logits=t_logits, dtype=torch.float64)
+    for form in ("full", "auto"):
+        plan = _map_in_the_form(D, form, t2s, Vs)
+        got = D.vocab_utils.marginalise(on_gpu, plan=plan, n_student=Vs).cpu().numpy()
+        np.testing.assert_allclose(got, ref, rtol=2e-6, atol=1e-9)
+        assert np.array_equal(got == 0, ref == 0)
+        rl, grad = D.vocab_utils.rkl_marginalised(logits.to(DEV), on_gpu, plan, T=1.3, grad_scale=1.0 / R)
+        rl2, grad2 = D.vocab_utils.rkl_marginalised(logits.to(DEV), on_gpu, plan, T=1.3, grad_scale=1.0 / R)
+        assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
+        np.testing.assert_allclose(rl.cpu().double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+        bound = O.marginal_rkl_gradient_tolerance(grad64, logits, t_logits, rows64, 1.3, 1.3, 1.0 / R, torch.float32, 1e-4)
+        err = (grad.cpu().double() - grad64).abs()
+        assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
