@@ -164,9 +164,9 @@ int dl_div_topk_static(int kind,
  * is irrelevant), scaled by inv_T_teacher.  Other arguments as for dl_div_topk.
  * Rows on the 16-byte grid (student, teacher and gradient; V a multiple of 8) are read once as far as
  * a workgroup's registers hold the pair (65536 columns of 16-bit rows, 32768 with an fp32 row) and
- * streamed in 16-byte chunks beyond that; rows off the grid take the same register kernels through
- * unaligned 16-byte accesses when student and teacher share a dtype and the pair fits, and a
- * kernel that streams them element by element otherwise.
+ * streamed in 16-byte chunks beyond that; rows off the grid take the same register kernels (from the student
+ * row's first 16-byte boundary on), and a kernel that streams them element by element where the pair does not fit
+ * or has no register kernel (bf16 against fp16).
  * Pointers and strides must be whole elements (else DL_ERR_ALIGN).
  */
 int dl_div_dense(int kind,
@@ -188,7 +188,7 @@ int dl_div_dense(int kind,
  * workspace   at least dl_div_dense_workspace_bytes(...) bytes, 16-byte aligned, contents irrelevant on entry
  *             and on return; NULL or too small: exactly dl_div_dense.  Launches that may overlap in time must
  *             not share a workspace.  dl_div_dense_workspace_bytes returns 0 where rows are not cut (JSD,
- *             narrow or very wide rows, V not a multiple of 8, dtype pairs without a register kernel).
+ *             narrow or very wide rows, dtype pairs without a register kernel).
  * flags       DL_TOPK_NO_WAIT: the parts never wait for their partners; DL_TOPK_PARTS(1 / 2 / 3): parts of
  *             256 / 512 / 1024 threads wherever two or more come out (test and tuning hooks).
  */

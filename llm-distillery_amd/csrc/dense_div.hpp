@@ -49,30 +49,10 @@ template <class Tag> struct Unit {
       else *reinterpret_cast<u32x4*>(row + (u * NC + k) * 16) = Chunk<Tag>::pack(f + k * Chunk<Tag>::N);
     }
   }
-  // The same for rows of V columns that may start anywhere (element-aligned) and end inside a chunk:
-  // whole chunks by unaligned 16-byte accesses, a partly filled one element by element (-inf / not
-  // stored beyond the row), nothing for chunks wholly beyond it.
-  __device__ __forceinline__ void load_any(const char* row, int64_t u, int64_t V) {
-    constexpr int N = Chunk<Tag>::N;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      const int64_t ch = u * NC + k;
-      c[k] = (ch + 1) * N <= V ? load16_unaligned(row + ch * 16)
-             : ch * N < V      ? load_chunk_elementwise<Tag>(row, (int)ch, (int)V)
-                               : Chunk<Tag>::neg_inf();
-    }
-  }
-  __device__ static __forceinline__ void store_any(char* row, int64_t u, int64_t V, const float* f) {
-    constexpr int N = Chunk<Tag>::N;
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      const int64_t ch = u * NC + k;
-      const u32x4 v = Chunk<Tag>::pack(f + k * N);
-      if ((ch + 1) * N <= V) store16_unaligned(row + ch * 16, v);
-      else if (ch * N < V) store_chunk_elementwise<Tag>(row, (int)ch, (int)V, v);
-    }
-  }
 };
+
+// How many columns a call of a sweep's function is handed.
+template <int N> struct Columns { static constexpr int value = N; };
 
 // Per-row results of the statistic sweeps, log2 domain.
 struct DenseStats {
@@ -136,8 +116,9 @@ __device__ __forceinline__ float dense_grad_column(float lp, float lq, float c, 
 }
 
 // The sweeps over a row pair held in registers.  `Rows` provides
-//   template <class F> void sweep(F f)       calls f(u, s[8], t[8]) for every unit this thread owns
-// (values already unpacked to fp32, -inf beyond the row), and `red` is LDS scratch of 64 floats.
+//   template <class F> void sweep(F f)       calls f(u, s[8], t[8], Columns<8>{}) for every unit this thread owns
+// (values already unpacked to fp32, -inf beyond the row), possibly f(u, s[1], t[1], Columns<1>{}) for a single column
+// behind the last unit, and store(grow, u, g, Columns<N>{}), the counterpart for the gradient; `red` is LDS scratch of 64 floats.
 // KIND is a compile-time constant: the per-column code carries no branch on it.
 //
 // Forward and reverse KL need three sweeps, not four: with es = 2^(s a_s - bs), et = 2^(t a_t - bt)
@@ -178,17 +159,17 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
       ms = nms;
       mt = nmt;
     };
-    rows.sweep([&](int64_t, const float* s, const float* t) {
+    rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
       float ums = -INFINITY, umt = -INFINITY;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < decltype(n)::value; ++e) {
         umt = fmaxf(umt, t[e]);
         ums = fmaxf(ums, (KIND == DL_RKL && t[e] == -INFINITY) ? -INFINITY : s[e]);
       }
       if (ums > ms || umt > mt) carry(fmaxf(ms, ums), fmaxf(mt, umt));
       const float bs = ms == -INFINITY ? 0.f : ms * a_s, bt = mt == -INFINITY ? 0.f : mt * a_t;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < decltype(n)::value; ++e) {
         const float xs = fmaf(s[e], a_s, -bs), xt = fmaf(t[e], a_t, -bt);
         const float es = fast_exp2(xs), et = fast_exp2(xt);
         stt += et;
@@ -209,9 +190,9 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
     bool have = false;
     if constexpr (KIND != DL_RKL && Rows::RAW_MAXIMA) have = rows.raw_maxima(ms, mt, red);      // RKL: the student's maximum is over the support
     if (!have) {
-      rows.sweep([&](int64_t, const float* s, const float* t) {
+      rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < decltype(n)::value; ++e) {
           mt = fmaxf(mt, t[e]);
           ms = fmaxf(ms, (KIND == DL_RKL && t[e] == -INFINITY) ? -INFINITY : s[e]);
         }
@@ -219,9 +200,9 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
       block_max2<NT>(ms, mt, red);
     }
     const float bs = ms * a_s, bt = mt * a_t;
-    rows.sweep([&](int64_t, const float* s, const float* t) {
+    rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < decltype(n)::value; ++e) {
         const float xs = fmaf(s[e], a_s, -bs), xt = fmaf(t[e], a_t, -bt);
         const float es = fast_exp2(xs), et = fast_exp2(xt);
         stt += et;
@@ -251,9 +232,9 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
   }
   float x = 0.f, y = 0.f;
   if constexpr (STASH) {
-    rows.sweep_rewrite([&](int64_t, float* s, float* t) {
+    rows.sweep_rewrite([&](int64_t, float* s, float* t, auto n) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
+      for (int e = 0; e < decltype(n)::value; ++e) {
         const float lp = fmaf(s[e], a_s, -st.ls), lq = fmaf(t[e], a_t, -st.lt);
         const float pr = fast_exp2(lp), q = fast_exp2(lq);
         const float lm = fast_log2(0.5f * pr + 0.5f * q);
@@ -265,9 +246,9 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
       }
     });
   } else {
-    rows.sweep([&](int64_t, const float* s, const float* t) {
+    rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) jsd_term(fmaf(s[e], a_s, -st.ls), fmaf(t[e], a_t, -st.lt), x, y);
+      for (int e = 0; e < decltype(n)::value; ++e) jsd_term(fmaf(s[e], a_s, -st.ls), fmaf(t[e], a_t, -st.lt), x, y);
     });
   }
   block_sum2<NT>(x, y, red);
@@ -280,11 +261,11 @@ template <int KIND, class TagS, class Rows>
 __device__ __forceinline__ void dense_grad_sweep(Rows& rows, const DenseStats& st, float c, char* grow) {
   const float a_s = st.a_s, a_t = st.a_t, ls = st.ls, lt = st.lt;
   const float kb = (KIND == DL_JSD ? 0.5f : 1.f) * c * LN2, k0 = (KIND == DL_JSD ? -0.5f : -1.f) * c * st.aux;
-  rows.sweep([&](int64_t u, const float* s, const float* t) {
-    float g[8];
+  rows.sweep([&](int64_t u, const float* s, const float* t, auto n) {
+    float g[decltype(n)::value];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) g[e] = dense_grad_column<KIND>(fmaf(s[e], a_s, -ls), fmaf(t[e], a_t, -lt), c, kb, k0);
-    rows.store(grow, u, g);
+    for (int e = 0; e < decltype(n)::value; ++e) g[e] = dense_grad_column<KIND>(fmaf(s[e], a_s, -ls), fmaf(t[e], a_t, -lt), c, kb, k0);
+    rows.store(grow, u, g, n);
   });
 }
 
@@ -292,11 +273,11 @@ __device__ __forceinline__ void dense_grad_sweep(Rows& rows, const DenseStats& s
 template <class TagS, class Rows>
 __device__ __forceinline__ void dense_jsd_grad_from_stash(Rows& rows, const DenseStats& st, float c, char* grow) {
   const float kb = 0.5f * c * LN2, k0 = -0.5f * c * st.aux;
-  rows.sweep([&](int64_t u, const float* pr, const float* d) {
-    float g[8];
+  rows.sweep([&](int64_t u, const float* pr, const float* d, auto n) {
+    float g[decltype(n)::value];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) g[e] = pr[e] * fmaf(d[e], kb, k0);
-    rows.store(grow, u, g);
+    for (int e = 0; e < decltype(n)::value; ++e) g[e] = pr[e] * fmaf(d[e], kb, k0);
+    rows.store(grow, u, g, n);
   });
 }
 

@@ -145,12 +145,15 @@ __device__ __forceinline__ u32x4 load16_unaligned(const void* p) {
   __builtin_memcpy(&v, p, 16);
   return v;
 }
-// The streaming form for addresses on any 4-byte boundary.
-__device__ __forceinline__ u32x4 load16_stream_any(const void* p) {
-  typedef unsigned u32x4_on_4 __attribute__((ext_vector_type(4), aligned(4)));
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_on_4*>(p));
-}
 __device__ __forceinline__ void store16_unaligned(void* p, const u32x4& v) { __builtin_memcpy(p, &v, 16); }
+// The streaming forms for addresses on any element boundary.
+typedef unsigned u32x4_on_2 __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ u32x4 load16_stream_any(const void* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_on_2*>(p));
+}
+__device__ __forceinline__ void store16_stream_any(void* p, const u32x4& v) {
+  __builtin_nontemporal_store((u32x4_on_2)v, reinterpret_cast<u32x4_on_2*>(p));
+}
 // Non-temporal stores: a bare copy kernel runs ~4 % faster with the default policy, but in the
 // loss kernels (sparse corrections follow the dense row) the non-temporal hint measured faster.
 __device__ __forceinline__ void store16_stream(void* p, const u32x4& v) {
@@ -585,7 +588,6 @@ __device__ __forceinline__ u32x4 load_chunk_elementwise(const char* part, int ch
   }
   return v;
 }
-// The counterpart for stores: the elements of chunk `chunk` that lie before column n_cols.
 // The chunk with -inf in place of its elements n .. N-1 (the columns behind a row's end).
 template <class Tag>
 __device__ __forceinline__ u32x4 chunk_keep_first(u32x4 v, int n) {
@@ -602,6 +604,7 @@ __device__ __forceinline__ u32x4 chunk_keep_first(u32x4 v, int n) {
   return v;
 }
 
+// The counterpart for stores: the elements of chunk `chunk` that lie before column n_cols.
 template <class Tag>
 __device__ __forceinline__ void store_chunk_elementwise(char* part, int chunk, int n_cols, const u32x4& v) {
   const int col0 = chunk * Chunk<Tag>::N;
@@ -619,12 +622,29 @@ __device__ __forceinline__ void store_chunk_elementwise(char* part, int chunk, i
   }
 }
 
+// Elements of a row ahead of its first 16-byte boundary, at most n_cols.
+template <class Tag>
+__device__ __forceinline__ int elements_to_grid(const char* row, int64_t n_cols) {
+  const int e = (int)((16u - (unsigned)(reinterpret_cast<uintptr_t>(row) & 15)) & 15u) / Tag::bytes;
+  return (int)min((int64_t)e, n_cols);
+}
+
 // zero-fill one gradient row (masked / padded token positions)
 template <class Tag, int NT>
 __device__ __forceinline__ void zero_row(void* grad_row, int64_t nchunks) {
   const u32x4 z{0u, 0u, 0u, 0u};
   for (int64_t c = threadIdx.x; c < nchunks; c += NT)
     store16_stream(reinterpret_cast<char*>(grad_row) + c * 16, z);
+}
+// The same for n_cols columns that start on any element.
+template <class Tag, int NT>
+__device__ __forceinline__ void zero_row_any(char* grad_row, int64_t n_cols) {
+  constexpr int N = Chunk<Tag>::N;
+  const int head = elements_to_grid<Tag>(grad_row, n_cols);
+  const int64_t whole = (n_cols - head) / N;
+  zero_row<Tag, NT>(grad_row + head * Tag::bytes, whole);
+  const int tail = (int)(n_cols - head - whole * N), tid = threadIdx.x;
+  if (tid < head + tail) store_from_float(grad_row, Tag::id, tid < head ? (int64_t)tid : whole * N + tid, 0.f);
 }
 
 }  // namespace dl

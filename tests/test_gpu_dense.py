@@ -378,3 +378,46 @@ def test_dense_gradient_may_overwrite_the_logits(D, kind, V, dtype):
     rl2, g2 = D.div_dense(kind, y, t, T=1.3, grad_out=y)
     assert g2.data_ptr() == y.data_ptr() and torch.equal(rl, rl2) and torch.equal(grad, y)
 
+
+
+@pytest.mark.parametrize("kind", ["fkl", "rkl", "jsd"])
+@pytest.mark.parametrize("dtype,t_dtype,V,pitch", [(torch.float32, torch.bfloat16, 5, 5), (torch.bfloat16, torch.float32, 2047, 2047),
+                                                   (torch.float32, torch.float16, 8197, 8204), (torch.float16, torch.float32, 20003, 20003),
+                                                   (torch.float32, torch.bfloat16, 20001, 20001)])
+def test_dense_rows_off_the_grid_with_a_teacher_of_another_dtype(D, kind, dtype, t_dtype, V, pitch):
+    """Mixed dtypes off the 16-byte grid: the register kernels as for equal ones, the V % 8 columns behind the last unit
+    in the first threads; with masked rows and rows of a wider pitch."""
+    R = 7
+    s, t = _pair(R, V, dtype, 21, t_dtype)
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[3] = False
+    wide = torch.full((R, pitch), 1e4, dtype=dtype)          # what lies behind a row must not be read as part of it
+    wide[:, :V] = s
+    rm = torch.full((R,), -1, dtype=torch.int32)
+    rm[valid] = torch.arange(R - 1, dtype=torch.int32)
+    loss64, rows64, grad64 = O.mean_loss_and_grad(kind, s, 1.3, t_logits=t[valid], valid=valid, dtype=torch.float64)
+    rl, grad = D.div_dense(kind, wide.to(DEV)[:, :V], t[valid].to(DEV), row_map=rm.to(DEV), T=1.3, grad_scale=1.0 / (R - 1))
+    np.testing.assert_allclose(rl.cpu()[valid].double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+    assert rl[3].item() == 0 and torch.count_nonzero(grad[3]) == 0
+    sel = torch.nonzero(valid).squeeze(-1)
+    bound = O.storage_tolerance(grad64, dtype, RTOL[dtype])
+    bound[sel] = O.dense_gradient_tolerance(grad64[sel], s[sel], t[valid], rows64, 1.3, 1.3, 1.0 / (R - 1), dtype, RTOL[dtype], kind=kind)
+    err = (grad.cpu().double() - grad64).abs()
+    assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+
+
+@pytest.mark.parametrize("kind", ["fkl", "rkl"])
+@pytest.mark.parametrize("dtype,t_dtype,V,threads", [(torch.bfloat16, torch.bfloat16, 16385, 256), (torch.bfloat16, torch.bfloat16, 65543, 512),
+                                                     (torch.float16, torch.float16, 16391, 256), (torch.float32, torch.float32, 8193, 256),
+                                                     (torch.float32, torch.float32, 33001, 0), (torch.bfloat16, torch.float32, 49157, 0),
+                                                     (torch.float32, torch.float16, 65537, 512), (torch.float32, torch.bfloat16, 70001, 1024)])
+@pytest.mark.parametrize("no_wait", [False, True])
+def test_dense_rows_off_the_grid_in_column_parts(D, kind, dtype, t_dtype, V, threads, no_wait):
+    """Column parts of rows that are no whole number of 8-column units long and start anywhere: the columns behind the
+    last unit belong to the last part; also where every part goes through the retry list."""
+    R = 5
+    s, t = _pair(R, V, dtype, 23, t_dtype)
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[2] = False
+    s[0, V - 1] = 60.0                                       # a row whose maximum is its last column
+    _check(D, kind, s, t[valid], T=1.3, valid=valid, no_wait=no_wait, part_threads=threads)
