@@ -50,6 +50,7 @@ typedef enum {
 #define DL_TOPK_FINE_PARTS 4   /* rows of 1025-16384 16-byte chunks are cut into parts of 1024 chunks   */
                                /* (up to 16 per row) where the workspace holds 20 bytes per row and    */
                                /* part + 16; else ignored                                               */
+#define DL_TOPK_ANY_ROWS 8     /* dl_fkl_multi_teacher: rows off the 16-byte grid are taken too        */
 #define DL_TOPK_PARTS_SHIFT 8  /* bits 8-11: column parts a row of 65537-131072 two-byte (half as many */
 #define DL_TOPK_PARTS(n) ((n) << DL_TOPK_PARTS_SHIFT)   /* four-byte) entries is cut into: 1, 2 or 4    */
                                /* (4 only where four parts of 32768 two-byte entries all hold columns); */
@@ -94,18 +95,15 @@ const char* dl_status_string(int status);
  * K <= DL_MAX_TOPK.
  * Alignment: any V and any element-aligned pointers and row strides are taken (else DL_ERR_ALIGN).  Rows
  * on the 16-byte grid (16-byte aligned pointers, logits and gradient; row strides whole numbers of 16-byte
- * chunks) take the aligned register kernels whatever V is: a row that ends inside a chunk -- the crop
- * logits[:, :, :V] of a vocabulary padded to a multiple of 8 (4 for fp32) columns,
- * classes/student/model.py:408 -- moves like a whole one, one workgroup per row or cut into column parts,
- * and only its last chunk is stored element by element; nothing beyond column V is written.  The kernels
- * READ that chunk's 16 bytes whole: they begin inside the row and, aligned as they are, end inside the
- * row's stride or at least inside the memory page of the row's last column, so the read cannot fault; what
- * it brings in from beyond column V is discarded.  The same holds for dl_rowcoef_grad_topk and
- * dl_fkl_multi_teacher.  Other rows (an odd row stride, a column slice that starts off the grid) are still
- * moved 16 bytes at a time: forward-KL rows by unaligned accesses in the register kernels (one workgroup per
- * row of up to 4096 16-byte chunks, column parts beyond where a workspace came along -- which
- * dl_div_topk_workspace_bytes asks for from 4097 chunks on when V is not a whole number of chunks); wider ones
- * without a workspace, and dl_rowstats_topk / dl_rowcoef_grad_topk, by the aligned chunks inside
+ * chunks) that are a whole number of chunks long move by aligned 16-byte accesses.  Forward-KL rows that start or
+ * end elsewhere (an odd row stride, a column slice, the crop logits[:, :, :V] of a padded vocabulary,
+ * classes/student/model.py:408) take the same kernels: their chunks start at the first 16-byte boundary of a
+ * logits row (part), the up to 7 columns on either side move one by one; nothing beside the row is read or
+ * written.  dl_rowstats_topk / dl_rowcoef_grad_topk take rows on the grid that end inside a chunk the same way,
+ * except that they READ that last chunk's 16 bytes whole: they begin inside the row and, aligned as they are, end
+ * inside the row's stride or at least inside the memory page of the row's last column, so the read cannot fault;
+ * what it brings in from beyond column V is discarded.  Rows off the grid there, and forward-KL rows too wide for
+ * the register kernels, move by the aligned chunks inside
  * each row, provided that logits and gradient rows share their address modulo 16 (the same stride from
  * 16-byte aligned bases, or the gradient written over the logits; reverse KL: any gradient row), and
  * element by element otherwise.
@@ -368,7 +366,7 @@ int dl_merge_remap_topk(int n_teachers, const void* const* t_vals, const void* c
  * that may overlap in time need different workspaces.
  * Limits: n_teachers <= DL_MAX_TEACHERS, n_teachers * K <= DL_MAX_TOPK; logits and gradient rows on the
  * 16-byte grid (aligned pointers, strides whole numbers of chunks; V itself may end inside a chunk, see
- * dl_div_topk), else DL_ERR_ALIGN; V <= 262144 two-byte / 131072 four-byte columns, else
+ * dl_div_topk), or with DL_TOPK_ANY_ROWS among the flags on any element, else DL_ERR_ALIGN; V <= 262144 two-byte / 131072 four-byte columns, else
  * DL_ERR_LIMIT (dl_fkl_multi_teacher_workspace_bytes then returns 0).  In those cases nothing was
  * launched: call dl_merge_remap_topk + dl_div_topk.
  */

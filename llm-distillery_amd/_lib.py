@@ -22,6 +22,7 @@ DL_MAX_HOST_CONVOS = 64
 DL_TOPK_UNIQUE_IDS = 1
 DL_TOPK_NO_WAIT = 2
 DL_TOPK_FINE_PARTS = 4
+DL_TOPK_ANY_ROWS = 8
 DL_TOPK_PARTS_SHIFT = 8
 DL_STATIC_SCRATCH_BYTES = 4 << 20
 

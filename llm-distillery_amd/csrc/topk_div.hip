@@ -40,11 +40,11 @@ static int div_topk_checked(int kind, const void* logits, int logits_dtype, int6
                (reinterpret_cast<uintptr_t>(workspace) % 16 == 0) ? workspace : nullptr, 1,
                (flags & DL_TOPK_NO_WAIT) ? 0 : SPIN_LIMIT, flags};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (kind == DL_FKL && on_grid && !aligned) return launch_fkl_tail(logits_dtype, p, workspace_bytes, st);
+  if (kind == DL_FKL && !aligned) return launch_fkl_any(logits_dtype, p, workspace_bytes, st);
   if (kind == DL_FKL)
-    return logits_dtype == DL_F32 ? launch_fkl<TagF32, false>(p, aligned, workspace_bytes, st)
-           : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, false>(p, aligned, workspace_bytes, st)
-                                     : launch_fkl<TagF16, false>(p, aligned, workspace_bytes, st);
+    return logits_dtype == DL_F32 ? launch_fkl<TagF32, false>(p, workspace_bytes, st)
+           : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, false>(p, workspace_bytes, st)
+                                     : launch_fkl<TagF16, false>(p, workspace_bytes, st);
   const hipError_t e = logits_dtype == DL_F32 ? launch_rkl<TagF32>(p, aligned, st)
                        : logits_dtype == DL_BF16 ? launch_rkl<TagBF16>(p, aligned, st)
                                                  : launch_rkl<TagF16>(p, aligned, st);

@@ -16,8 +16,7 @@
 // Reverse KL (student renormalised over the K ids) touches only the K gathered logits; its
 // gradient row is a zero fill plus K sparse values.
 //
-// Rows that do not fit (or break the 16-byte alignment rules) take the streaming kernel, which
-// reads the row twice.
+// Rows that do not fit take the streaming kernel, which reads the row twice.
 // This header holds the kernels and their launchers; topk_div.hip instantiates them for one stored
 // teacher (dl_div_topk), topk_multi.hip for several unmerged teachers (dl_fkl_multi_teacher).
 #pragma once
@@ -62,6 +61,7 @@ struct TopkParams {
 
 constexpr int MAX_PARTS = 16;             // parts a row may be cut into (parts of 256 x 4 chunks)
 constexpr int MAX_COARSE_PARTS = 8;       // of 256 x 16 chunks
+constexpr int REST_HEADS = 16;            // a part has up to 7 columns ahead of its first 16-byte boundary and 7 behind its last
 
 // What one part of a split row tells the others: three floats and a tag that depends on all of
 // them.  The four words are written and read with relaxed device-scope accesses (they bypass the
@@ -123,7 +123,7 @@ struct TopkLds {
   int* next;         // Kp  next entry owned by the same thread, or -1
   int* head;         // CORRECTION_HEADS list heads: first entry of a chunk's list, or -1
   unsigned* own;     // one per thread: bit i set = chunk i of the thread holds an entry
-  u32x4* tail;       // ROWS_TAIL: the logits of the row's ragged chunk, kept for the gradient by the one thread that holds it
+  int* rest;         // REST_HEADS list heads: entries on the part's columns beside its 16-byte chunks (ROWS_ANY)
   int Kp;
   __device__ TopkLds(unsigned char* base, int K, int owners = 0) {
     Kp = (K + 15) & ~15;
@@ -137,11 +137,11 @@ struct TopkLds {
     next = reinterpret_cast<int*>(val + Kp);
     head = next + Kp;
     own = reinterpret_cast<unsigned*>(head + (owners ? CORRECTION_HEADS : 0));
-    tail = reinterpret_cast<u32x4*>(own + owners);
+    rest = reinterpret_cast<int*>(own + owners);
   }
   __host__ __device__ static size_t bytes(int K, int owners = 0) {
     const size_t Kp = (size_t)((K + 15) & ~15);
-    return 512 + Kp * 16 + (owners ? Kp * 8 + (size_t)CORRECTION_HEADS * 4 + (size_t)owners * 4 + 16 : 0);
+    return 512 + Kp * 16 + (owners ? Kp * 8 + (size_t)CORRECTION_HEADS * 4 + (size_t)owners * 4 + REST_HEADS * 4 : 0);
   }
 };
 
@@ -204,6 +204,25 @@ __device__ __forceinline__ void bucket_issue(const TopkParams& p, int64_t trow, 
   hd.more_at = 0;                         // where this bucket's overflow starts in the row's share of `more`
   for (int g = 0; g < h; ++g) hd.more_at += max(min(head[g], p.bk.E) - p.bk.cap0, 0);
   hd.more_at = min(hd.more_at, p.bk.E - max(hd.n - p.bk.cap0, 0));
+}
+
+// The columns [lo, hi) of a part: the ones of its 16-byte chunks are [lob, hib); a part of a row off the 16-byte grid
+// (ANY) has up to 7 columns ahead of them and 7 behind.  Entries are linked into the list of the chunk their column lies
+// in, or into the list of the one column beside the chunks.
+struct PartCols {
+  int lo, hi, lob, hib;
+  __device__ __forceinline__ bool beside(int id) const { return id < lob || id >= hib; }      // of an id inside [lo, hi)
+  __device__ __forceinline__ int rest_of(int id) const { return id < lob ? id - lo : (lob - lo) + (id - hib); }
+};
+template <class Tag, int NT, int NCH, bool ANY>
+__device__ __forceinline__ void link_entry(const TopkLds& s, const PartCols& pc, int k, int id) {
+  if (ANY && pc.beside(id)) s.next[k] = atomicExch(&s.rest[pc.rest_of(id)], k);
+  else correction_link<Tag, NT, NCH>(s.head, s.own, s.next, k, id - pc.lob);
+}
+template <class Tag, int NT, int NCH, bool ANY>
+__device__ __forceinline__ int first_entry(const TopkLds& s, const PartCols& pc, int id) {
+  if (ANY && pc.beside(id)) return s.rest[pc.rest_of(id)];
+  return s.head[correction_head_slot<Tag, NT, NCH>(id - pc.lob)];
 }
 
 // Registers -> LDS, then the teacher's log-sum-exp; same result layout as stage_teacher.
@@ -319,9 +338,10 @@ __device__ __forceinline__ float mass_on_column(const int* next, const int* col,
 // row crowd into one part) are fetched here, from the row's overflow share.
 // Leaves q in s.q, Q_id(k) in s.val[k], z in s.z[k]; returns the number of LDS entry slots in use
 // (a multiple of NT); B as fkl_partials.
-template <class Tag, int NT, int NCH, int J>
+template <class Tag, int NT, int NCH, int J, bool ANY>
 __device__ __forceinline__ int bucket_finish(const TopkParams& p, const TopkLds& s, const TeacherEntries<J>& te,
-                                             const BucketHead& hd, int64_t trow, const char* row, int lo, int hi, float& B) {
+                                             const BucketHead& hd, int64_t trow, const char* row, const PartCols& pc, float& B) {
+  const int lo = pc.lo, hi = pc.hi;
   const int nk = max(J * NT, (hd.n + NT - 1) / NT * NT);
 #pragma unroll
   for (int j = 0; j < J; ++j) {
@@ -348,14 +368,14 @@ __device__ __forceinline__ int bucket_finish(const TopkParams& p, const TopkLds&
   }
   for (int k = threadIdx.x; k < nk; k += NT) {
     const int id = s.idx[k];                               // this thread's own store
-    if (id >= 0) correction_link<Tag, NT, NCH>(s.head, s.own, s.next, k, id - lo);
+    if (id >= 0) link_entry<Tag, NT, NCH, ANY>(s, pc, k, id);
   }
   __syncthreads();
   B = 0.f;
   for (int k = threadIdx.x; k < nk; k += NT) {
     const int id = s.idx[k];
     if (id < 0) continue;
-    const int first = s.head[correction_head_slot<Tag, NT, NCH>(id - lo)];
+    const int first = first_entry<Tag, NT, NCH, ANY>(s, pc, id);
     int same = 0;
     float big = 0.f;
     for (int e = first; e >= 0; e = s.next[e]) {
@@ -409,13 +429,21 @@ __device__ __forceinline__ void fkl_sparse_fix(const TopkLds& s, void* grow, int
 // student probability at the entry's column in s.val and link the entry into its owner's list; the
 // owner subtracts the teacher mass -- of all entries of that column, should ids repeat, which it
 // sees from the chunk's list: no scan over the row's ids.
-template <class Tag, int NT, int NCH>
-__device__ __forceinline__ void fkl_link_corrections(const TopkLds& s, int lo, int hi, float a, float b) {
+template <class Tag, int NT, int NCH, bool ANY>
+__device__ __forceinline__ void fkl_link_corrections(const TopkLds& s, const PartCols& pc, float a, float b) {
   for (int k = threadIdx.x; k < s.Kp; k += NT) {
     const int id = s.idx[k];
-    if (id < lo || id >= hi) continue;
+    if (id < pc.lo || id >= pc.hi) continue;
     s.val[k] = fast_exp2(fmaf(s.z[k], a, -b));
-    correction_link<Tag, NT, NCH>(s.head, s.own, s.next, k, id - lo);
+    link_entry<Tag, NT, NCH, ANY>(s, pc, k, id);
+  }
+}
+// The entries beside the part's chunks only (kernels that write the others behind their dense stores).
+template <int NT>
+__device__ __forceinline__ void fkl_link_rest(const TopkLds& s, const PartCols& pc) {
+  for (int k = threadIdx.x; k < s.Kp; k += NT) {
+    const int id = s.idx[k];
+    if (id >= pc.lo && id < pc.hi && pc.beside(id)) s.next[k] = atomicExch(&s.rest[pc.rest_of(id)], k);
   }
 }
 
@@ -460,39 +488,16 @@ __device__ __forceinline__ void row_stats_streamed(const char* row, int64_t V, f
 
 // How the rows of a register kernel lie in memory (template parameter RAG):
 //   ROWS_WHOLE  on the 16-byte grid (base and pitch), a whole number of chunks long
-//   ROWS_ANY    anywhere (element-aligned), any length: whole chunks move by unaligned 16-byte accesses
-//   ROWS_TAIL   on the 16-byte grid, but V is not a whole number of chunks (a crop of a padded vocabulary,
-//               logits[:, :, :crop]): every chunk but the row's last moves like a ROWS_WHOLE one
-// In the last two the row's last, partly filled chunk moves element by element, with -inf in the columns
-// it lacks (they add nothing to any statistic and are not stored).
-constexpr int ROWS_WHOLE = 0, ROWS_ANY = 1, ROWS_TAIL = 2;
-
-// Chunk c of a part that starts at `part`; `ncols` = columns from the part's first to the row's end.
-template <class Tag, int RAG>
-__device__ __forceinline__ u32x4 load_part_chunk(const char* part, int64_t c, int64_t ncols) {
-  // cached, not streaming, loads: the gather of the logits at the teacher ids that follows then
-  // finds its lines in L2 instead of fetching them a second time (0.47 GB less per 32768 rows of K = 200)
-  if constexpr (RAG == ROWS_WHOLE) return *reinterpret_cast<const u32x4*>(part + c * 16);
-  else if ((c + 1) * Chunk<Tag>::N <= ncols) {
-    if constexpr (RAG == ROWS_ANY) return load16_unaligned(part + c * 16);
-    else return *reinterpret_cast<const u32x4*>(part + c * 16);
-  }
-  else return load_chunk_elementwise<Tag>(part, (int)c, (int)ncols);
-}
-template <class Tag, int RAG>
-__device__ __forceinline__ void store_part_chunk(char* part, int64_t c, int64_t ncols, const u32x4& v) {
-  if constexpr (RAG == ROWS_WHOLE) store16_stream(part + c * 16, v);
-  else if ((c + 1) * Chunk<Tag>::N <= ncols) {
-    if constexpr (RAG == ROWS_ANY) store16_unaligned(part + c * 16, v);
-    else store16_stream(part + c * 16, v);
-  }
-  else store_chunk_elementwise<Tag>(part, (int)c, (int)ncols, v);
-}
-template <class Tag, int NT, int RAG>
-__device__ __forceinline__ void zero_part(char* gpart, int64_t nch, int64_t ncols) {
-  if constexpr (RAG == ROWS_WHOLE) zero_row<Tag, NT>(gpart, nch);
-  else for (int64_t ch = threadIdx.x; ch < nch; ch += NT) store_part_chunk<Tag, RAG>(gpart, ch, ncols, u32x4{0u, 0u, 0u, 0u});
-}
+//   ROWS_ANY    anywhere (element-aligned), any length
+// The chunks of a ROWS_ANY part start at its first 16-byte boundary, so that its loads (and the stores of a gradient row
+// of the same phase: every row of contiguous tensors) are aligned; a gradient row of another phase takes the same stores
+// unaligned.  The up to 7 columns ahead of the chunks and 7 behind them sit one per thread in the first threads of the
+// workgroup (x_rest, -inf in the others: adds nothing to any statistic).  The sweeps are then those of whole rows: no
+// bound and no branch inside them, and every shape that serves whole rows serves these, in their time: 16384 x 20003
+// bf16, K = 100, 351 -> 271 us (20008 columns: 265 us), 8192 x 151665 1096 -> 955 us, 4093 x 50257 with a tenth of the
+// rows masked 227 -> 174 us (unaligned accesses from the row's first column and an element-wise last chunk inside the
+// sweeps, with fewer shapes to choose from, before).
+constexpr int ROWS_WHOLE = 0, ROWS_ANY = 1;
 
 // ---------------------------------------------------------------------------------------
 // Forward KL, (part of) a row resident in registers: NT threads x NCH 16-byte chunks per thread.
@@ -506,61 +511,60 @@ __device__ __forceinline__ void zero_part(char* gpart, int64_t nch, int64_t ncol
 // RETRY: second launch over the parts that gave up waiting in the first (see split_retry_list):
 // every record of the row is published by then, so nothing is waited for.
 // MULTI: the row's teachers arrive prepared in buckets (TopkParams::bk), J * NT = cap0 entries in registers.
-// RAG: how the rows lie in memory (ROWS_WHOLE / ROWS_ANY / ROWS_TAIL above).
+// RAG: how the rows lie in memory (ROWS_WHOLE / ROWS_ANY above).
 template <class Tag, int NT, int NCH, bool SPLIT, int J, bool RETRY, bool MULTI, int RAG = ROWS_WHOLE>
 __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds& s, int64_t r, int h) {
   static_assert(!MULTI || J > 0, "the head of a bucket travels in registers");
-  static_assert(RAG != ROWS_ANY || !MULTI, "rows off the 16-byte grid: one stored teacher");
+  constexpr bool ANY = RAG == ROWS_ANY;
   using C = Chunk<Tag>;
   const int tid = threadIdx.x;
   const int P = SPLIT ? p.parts : 1;
-  const int64_t c0 = (int64_t)h * NT * NCH;                       // first chunk of this part
-  const int64_t nch_row = RAG != ROWS_WHOLE ? (p.V + C::N - 1) / C::N : p.V / C::N;
-  const int64_t nch = min((int64_t)NT * NCH, nch_row - c0);       // chunks of this part
-  const int lo = (int)(c0 * C::N);                                // its column range
-  const int hi = RAG != ROWS_WHOLE ? (int)min(p.V, (int64_t)lo + nch * C::N) : lo + (int)(nch * C::N);
-  const int64_t ncols = p.V - lo;                                 // columns from the part's first to the row's end
+  const int64_t c0 = (int64_t)h * NT * NCH;                       // the part starts c0 chunks into the row
+  PartCols pc;
+  pc.lo = pc.lob = (int)(c0 * C::N);
+  pc.hi = (int)min(p.V, (int64_t)pc.lo + NT * NCH * C::N);
+  const int lo = pc.lo, hi = pc.hi;
   char* grow = p.grad ? reinterpret_cast<char*>(p.grad) + r * p.grad_stride * Tag::bytes : nullptr;
   char* gpart = grow ? grow + c0 * 16 : nullptr;
   const int64_t trow = teacher_row(p.row_map, r, p.n_trows);
+  const auto zero_part = [&]() {
+    if constexpr (ANY) zero_row_any<Tag, NT>(gpart, hi - lo);
+    else zero_row<Tag, NT>(gpart, (hi - lo) / C::N);
+  };
   if (trow < 0) {
-    if (gpart) zero_part<Tag, NT, RAG>(gpart, nch, ncols);
+    if (gpart) zero_part();
     if (tid == 0 && h == 0 && p.row_loss) p.row_loss[r] = 0.f;
     return;
   }
   const char* row = reinterpret_cast<const char*>(p.logits) + r * p.row_stride * Tag::bytes;
   const char* rpart = row + c0 * 16;
+  const int head = ANY ? elements_to_grid<Tag>(rpart, hi - lo) : 0;
+  const int nch = (hi - lo - head) / C::N;                        // chunks of this part
+  pc.lob = lo + head;
+  pc.hib = pc.lob + nch * C::N;
+  const int rest = ANY ? head + (hi - pc.hib) : 0;                // columns beside them
+  const int rest_col = tid < head ? lo + tid : pc.hib + (tid - head);
+  const char* rbody = rpart + head * Tag::bytes;
 
   correction_clear<NT>(s.head, s.own);      // lists of corrections, filled after the row statistics
+  if constexpr (ANY) {
+    if (tid < REST_HEADS) s.rest[tid] = -1;
+  }
   TeacherEntries<(J > 0 ? J : 1)> te;
   BucketHead hd{};
   if constexpr (MULTI) bucket_issue<NT, J>(p, trow, h, P, te, hd);
   else if constexpr (J > 0) teacher_issue<NT, J>(p, trow, te);
-  // ROWS_TAIL: the part that holds the row's ragged chunk (part-relative number tail_c, else -1) loads it like the
-  // others -- the 16 bytes start inside the row and, aligned as they are, end inside the row's pitch or at least
-  // inside the page the row's last column lies in -- and the one thread that holds it puts -inf in the columns
-  // beyond the row.  Which of a thread's registers that is, is the same for every thread (a scalar): the
-  // unrolled sweeps pay a scalar compare per chunk for it, no vector work and no registers.
-  const int64_t tail_c = (RAG == ROWS_TAIL && ncols < nch * C::N) ? nch - 1 : -1;
-  const int tail_reg = tail_c >= 0 ? ChunkMap<NT, NCH>::reg((int)tail_c) : -1;
-  const bool tail_mine = tail_c >= 0 && ChunkMap<NT, NCH>::owner((int)tail_c) == tid;
-  const int64_t nfull = tail_c >= 0 ? nch - 1 : nch;              // chunks of this part that are stored whole
+  float x_rest = -INFINITY;
+  if constexpr (ANY) {
+    if (tid < rest) x_rest = load_as_float(row, Tag::id, rest_col);
+  }
   u32x4 reg[NCH];
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     const int64_t c = ChunkMap<NT, NCH>::chunk(i, tid);
-    if constexpr (RAG == ROWS_TAIL) reg[i] = c < nch ? load_part_chunk<Tag, ROWS_WHOLE>(rpart, c, ncols) : C::neg_inf();
-    else reg[i] = c < nch ? load_part_chunk<Tag, RAG>(rpart, c, ncols) : C::neg_inf();
-  }
-  u32x4 tail_raw = C::neg_inf();
-  if constexpr (RAG == ROWS_TAIL) {
-    if (tail_c >= 0) {
-#pragma unroll
-      for (int i = 0; i < NCH; ++i)
-        if (i == tail_reg && tail_mine) reg[i] = chunk_keep_first<Tag>(reg[i], (int)(ncols - tail_c * C::N));
-    }
-    // a second copy of the ragged chunk for the gradient sweep (same line: no traffic), parked in LDS below
-    if (tail_mine) tail_raw = load_part_chunk<Tag, ROWS_WHOLE>(rpart, tail_c, ncols);
+    // cached, not streaming, loads: the gather of the logits at the teacher ids that follows then
+    // finds its lines in L2 instead of fetching them a second time (0.47 GB less per 32768 rows of K = 200)
+    reg[i] = c < nch ? *reinterpret_cast<const u32x4*>(rbody + c * 16) : C::neg_inf();
   }
 
   // teacher side while the row is in flight
@@ -568,7 +572,7 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
   int nk = s.Kp;                      // LDS entry slots in use
   if constexpr (MULTI) {
     teacher_gather<Tag, J>(row, lo, hi, te);
-    if (hd.total > 0) nk = bucket_finish<Tag, NT, NCH, J>(p, s, te, hd, trow, row, lo, hi, B);
+    if (hd.total > 0) nk = bucket_finish<Tag, NT, NCH, J, ANY>(p, s, te, hd, trow, row, pc, B);
     tlse = hd.total > 0 ? 0.f : -INFINITY;
     Q = hd.qsum;
   } else if constexpr (J > 0) {
@@ -578,17 +582,14 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
     tlse = stage_teacher<Tag, NT>(p, s, trow, row, lo, hi);
   }
   if (tlse == -INFINITY) {            // no usable teacher entry: the row contributes nothing
-    if (gpart) zero_part<Tag, NT, RAG>(gpart, nch, ncols);
+    if (gpart) zero_part();
     if (tid == 0 && h == 0 && p.row_loss) p.row_loss[r] = 0.f;
     return;
   }
   if constexpr (!MULTI) fkl_partials<NT>(p, s, lo, hi, B, Q);
 
-  if constexpr (RAG == ROWS_TAIL) {
-    if (tail_mine) *s.tail = chunk_keep_first<Tag>(tail_raw, (int)(ncols - tail_c * C::N));      // read back by this thread only
-  }
   const float a = p.inv_T_s * LOG2E;
-  float mx = -INFINITY;
+  float mx = x_rest;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     float f[C::N];
@@ -602,7 +603,7 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
   // that value times a row constant, so each element costs one exp2, not two.
   float mb = (mx == -INFINITY) ? 0.f : mx * a;      // a part that holds only -inf logits: every 2^(.) below is 0, not NaN
   const float mb_own = mb - C::stash_bias;
-  float sm = 0.f;
+  float sm = ANY ? fast_exp2(fmaf(x_rest, a, -mb_own)) : 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
     float f[C::N];
@@ -663,9 +664,13 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
       }
       __syncthreads();
     } else if (IN_REGISTERS) {
-      fkl_link_corrections<Tag, NT, NCH>(s, lo, hi, a, b);
+      fkl_link_corrections<Tag, NT, NCH, ANY>(s, pc, a, b);
+      __syncthreads();
+    } else if (ANY) {
+      fkl_link_rest<NT>(s, pc);
       __syncthreads();
     }
+    char* gbody = gpart + head * Tag::bytes;
     const unsigned mine = IN_REGISTERS ? s.own[tid] : 0u;
     const bool may_repeat = !MULTI && (p.flags & DL_TOPK_UNIQUE_IDS) == 0;
     const auto mass = [&](int k) { return MULTI ? 0.f : s.q[k]; };
@@ -674,45 +679,39 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       const int64_t ch = ChunkMap<NT, NCH>::chunk(i, tid);
-      if (ch < nfull) {
+      if (ch < nch) {
         float f[C::N];
         forget(reg[i]);
         C::unstash(reg[i], f);
 #pragma unroll
         for (int e = 0; e < C::N; ++e) f[e] *= kc;
         if (mine & (1u << i))
-          if (correction_apply<Tag, NT, NCH>(s.head, s.next, s.idx, lo, i, f, mass, value)) repeats |= 1u << i;
-        if constexpr (RAG == ROWS_TAIL) store16_stream(gpart + ch * 16, C::pack(f));
-        else store_part_chunk<Tag, RAG>(gpart, ch, ncols, C::pack(f));
+          if (correction_apply<Tag, NT, NCH>(s.head, s.next, s.idx, pc.lob, i, f, mass, value)) repeats |= 1u << i;
+        if constexpr (ANY) store16_stream_any(gbody + ch * 16, C::pack(f));
+        else store16_stream(gbody + ch * 16, C::pack(f));
       }
     }
-    if constexpr (RAG == ROWS_TAIL) {
-      // The ragged chunk, by the one thread that holds it, from the copy of its logits in LDS, stored element by
-      // element.  The sweep above covers the whole chunks
-      // only and is the sweep of whole rows, instruction for instruction: a second bound inside it, or
-      // registers that must outlive it, make the 512 x 16 shape spill.
-      if (tail_mine) {
-        float f[C::N];
-        C::unpack(*s.tail, f);
-#pragma unroll
-        for (int e = 0; e < C::N; ++e) f[e] = fast_exp2(fmaf(f[e], a, -b)) * c;
-        if (mine & (1u << tail_reg))
-          if (correction_apply<Tag, NT, NCH>(s.head, s.next, s.idx, lo, tail_reg, f, mass, value)) repeats |= 1u << tail_reg;
-        store_chunk_elementwise<Tag>(gpart, (int)tail_c, (int)ncols, C::pack(f));
+    if constexpr (ANY) {
+      // a column beside the chunks: its dense value less the mass of the entries on its list
+      if (tid < rest) {
+        const int first = s.rest[tid];
+        float g = fast_exp2(fmaf(x_rest, a, -b));
+        if (first >= 0) g = MULTI ? s.val[first] : g - correction_exact_sum(s.next, s.idx, first, rest_col, [&](int k) { return s.q[k]; });
+        store_from_float(grow, Tag::id, rest_col, g * c);
       }
     }
     if (may_repeat && repeats)
-      correction_repeats<Tag, NT, NCH>(s.head, s.next, s.idx, lo, repeats, NCH, mass, value,
+      correction_repeats<Tag, NT, NCH>(s.head, s.next, s.idx, pc.lob, repeats, NCH, mass, value,
                                   [&](int column, float v) { store_from_float(grow, Tag::id, column, v); });
     if (!IN_REGISTERS) {
       __syncthreads();      // dense stores are ordered before the sparse corrections
       if constexpr (MULTI) {
         for (int k = tid; k < nk; k += NT) {
           const int id = s.idx[k];
-          if (id >= lo && id < hi) store_from_float(grow, Tag::id, id, s.val[k] * c);      // entries of one column: the same value
+          if (id >= pc.lob && id < pc.hib) store_from_float(grow, Tag::id, id, s.val[k] * c);      // entries of one column: the same value
         }
       } else {
-        fkl_sparse_fix<Tag, NT>(s, grow, lo, hi, a, b, c, (p.flags & DL_TOPK_UNIQUE_IDS) != 0);
+        fkl_sparse_fix<Tag, NT>(s, grow, pc.lob, pc.hib, a, b, c, (p.flags & DL_TOPK_UNIQUE_IDS) != 0);
       }
     }
   }
@@ -972,17 +971,6 @@ static void launch_reg_j(const TopkParams& p, unsigned grid, hipStream_t st) {
 #undef DL_REG_KERNEL
 }
 
-// one workgroup per row, rows of any alignment and length (one stored teacher)
-template <class Tag, int NT, int NCH>
-static int launch_reg_any(const TopkParams& p, hipStream_t st) {
-  constexpr bool MULTI = false;
-  const unsigned grid = xcd_banded_grid(p.n_rows);
-#define DL_REG_ANY_KERNEL(J) fkl_topk_reg_kernel<Tag, NT, NCH, false, J, false, ROWS_ANY>
-  DL_LAUNCH_BY_SLOTS(DL_REG_ANY_KERNEL, grid)
-#undef DL_REG_ANY_KERNEL
-  return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
-}
-
 template <class Tag, int NT, int NCH, bool MULTI, int RAG>
 static void launch_retry_j(const TopkParams& p, unsigned grid, hipStream_t st) {
 #define DL_RETRY_KERNEL(J) fkl_topk_retry_kernel<Tag, NT, NCH, J, MULTI, RAG>
@@ -1063,19 +1051,17 @@ static FklShape fkl_shape(int64_t nch, int bytes, int forced_parts, bool split_o
 }
 
 // MULTI has no streaming form: the caller checks fkl_shape first.
-// RAG = ROWS_WHOLE: `aligned` tells whether the rows are whole chunks on the 16-byte grid (else: the unaligned
-// register kernels or the streaming kernel).  RAG = ROWS_TAIL: rows on the grid that end inside a chunk
-// (`aligned` is true); the same shapes as whole rows of ceil(V / chunk) chunks.
+// RAG = ROWS_ANY: the shapes of whole rows of ceil(V / chunk) chunks.
 template <class Tag, bool MULTI, int RAG = ROWS_WHOLE>
-static int launch_fkl(const TopkParams& p, bool aligned, int64_t ws_bytes, hipStream_t st, bool ws_cleared = false) {
-  const int64_t nch = RAG == ROWS_TAIL ? (p.V + Tag::epc - 1) / Tag::epc : p.V / Tag::epc;
+static int launch_fkl(const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared = false) {
+  const int64_t nch = (p.V + Tag::epc - 1) / Tag::epc;
   const int forced = (p.flags >> DL_TOPK_PARTS_SHIFT) & 15;
   const bool fine = !MULTI && (p.flags & DL_TOPK_FINE_PARTS) != 0 &&
                     ws_bytes >= RetryList::bytes(p.n_rows, split_parts(nch, forced, true));
   // the shape a workspace would allow; without room for that shape's records, the shape that needs none
-  const FklShape wish = aligned ? fkl_shape(nch, Tag::bytes, forced, true, fine, !MULTI) : FklShape{0, 0, 0};
+  const FklShape wish = fkl_shape(nch, Tag::bytes, forced, true, fine, !MULTI);
   const bool split_ok = p.workspace && ws_bytes >= RetryList::bytes(p.n_rows, wish.parts) && p.n_rows * wish.parts <= 0x7fffffffLL;
-  const FklShape sh = !aligned || wish.parts <= 1 || split_ok ? wish : fkl_shape(nch, Tag::bytes, forced, false, fine, !MULTI);
+  const FklShape sh = wish.parts <= 1 || split_ok ? wish : fkl_shape(nch, Tag::bytes, forced, false, fine, !MULTI);
   switch (sh.NT * 100 + sh.NCH) {
     case 256 * 100 + 4:
       if constexpr (!MULTI)
@@ -1106,59 +1092,26 @@ static int launch_fkl(const TopkParams& p, bool aligned, int64_t ws_bytes, hipSt
     case 1024 * 100 + 16: return launch_reg<Tag, 1024, 16, MULTI, RAG>(p, st);
     default: break;
   }
-  if (MULTI) return aligned ? DL_ERR_LIMIT : DL_ERR_ALIGN;
-  // rows off the 16-byte grid: the streaming kernel moves their chunks by aligned vector accesses if logits
-  // and gradient rows share their address modulo 16 (the same pitch from 16-byte aligned bases, or the
-  // gradient written over the logits)
-  const bool same_phase = !p.grad || (reinterpret_cast<uintptr_t>(p.logits) % 16 == reinterpret_cast<uintptr_t>(p.grad) % 16 &&
-                                      ((p.row_stride - p.grad_stride) * Tag::bytes) % 16 == 0);
-  if constexpr (!MULTI && RAG == ROWS_WHOLE) {
-    if (!aligned) {
-      // ... or, as far as one workgroup holds a row, the register kernels with unaligned accesses.  Measured
-      // (16384 x 32100 bf16: 0.47 ms against 0.75 ms streaming; 16384 x 50257: 1.27 against 0.92): up to
-      // 256 x 16 chunks they win; the 512 x 16 shape spills under the extra addressing and only beats the
-      // element-wise kernel, which rows on different phases would otherwise take.
-      // Beyond 256 x 16 chunks: column parts of that shape (parts of a row start a whole number of chunks behind the
-      // row's first element, wherever that lies), where a workspace for their exchange came along.
-      const int64_t nch_any = (p.V + Tag::epc - 1) / Tag::epc;
-      const int parts_any = (int)((nch_any + 256 * 16 - 1) / (256 * 16));
-      if (parts_any >= 2 && parts_any <= MAX_COARSE_PARTS && p.workspace && ws_bytes >= RetryList::bytes(p.n_rows, parts_any) &&
-          p.n_rows * parts_any <= 0x7fffffffLL)
-        return launch_split<Tag, 256, 16, false, ROWS_ANY>(p, parts_any, st, ws_cleared);
-      const FklShape any = fkl_shape(nch_any, Tag::bytes, 0, false);
-      if (any.parts == 1) switch (any.NT * 100 + any.NCH) {
-        case 256 * 100 + 4: return launch_reg_any<Tag, 256, 4>(p, st);
-        case 256 * 100 + 8: return launch_reg_any<Tag, 256, 8>(p, st);
-        case 512 * 100 + 8:
-          if constexpr (Tag::bytes == 4) return launch_reg_any<Tag, 512, 8>(p, st);
-          break;
-        case 256 * 100 + 16:
-          if constexpr (Tag::bytes != 4) return launch_reg_any<Tag, 256, 16>(p, st);
-          break;
-        case 512 * 100 + 16:
-          if (!same_phase) return launch_reg_any<Tag, 512, 16>(p, st);
-          break;
-        default: break;
-      }
-    }
-  }
-  if (aligned && RAG == ROWS_WHOLE) {
-    hipLaunchKernelGGL((fkl_topk_stream_kernel<Tag, 1024, 1>), dim3(xcd_banded_grid(p.n_rows)), dim3(1024),
-                       TopkLds::bytes(p.K), st, p);
-  } else if (same_phase) {
-    hipLaunchKernelGGL((fkl_topk_stream_kernel<Tag, 1024, 2>), dim3(xcd_banded_grid(p.n_rows)), dim3(1024),
-                       TopkLds::bytes(p.K), st, p);
+  if (MULTI) return DL_ERR_LIMIT;
+  // too wide for the register kernels.  Rows off the 16-byte grid: the streaming kernel moves their chunks by aligned
+  // vector accesses if logits and gradient rows share their address modulo 16 (the same pitch from 16-byte aligned
+  // bases, or the gradient written over the logits)
+  const dim3 grid(xcd_banded_grid(p.n_rows));
+  if constexpr (RAG == ROWS_WHOLE) {
+    hipLaunchKernelGGL((fkl_topk_stream_kernel<Tag, 1024, 1>), grid, dim3(1024), TopkLds::bytes(p.K), st, p);
   } else {
-    hipLaunchKernelGGL((fkl_topk_stream_kernel<Tag, 1024, 0>), dim3(xcd_banded_grid(p.n_rows)), dim3(1024),
-                       TopkLds::bytes(p.K), st, p);
+    const bool same_phase = !p.grad || (reinterpret_cast<uintptr_t>(p.logits) % 16 == reinterpret_cast<uintptr_t>(p.grad) % 16 &&
+                                        ((p.row_stride - p.grad_stride) * Tag::bytes) % 16 == 0);
+    if (same_phase) hipLaunchKernelGGL((fkl_topk_stream_kernel<Tag, 1024, 2>), grid, dim3(1024), TopkLds::bytes(p.K), st, p);
+    else hipLaunchKernelGGL((fkl_topk_stream_kernel<Tag, 1024, 0>), grid, dim3(1024), TopkLds::bytes(p.K), st, p);
   }
   return launch_status();
 }
 
-// The ROWS_TAIL instantiations of launch_fkl live in translation units of their own (topk_div_tail.hip,
-// topk_multi_tail.hip), so that they compile beside the others.
-int launch_fkl_tail(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st);
-int launch_fkl_tail_multi(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared);
+// The ROWS_ANY instantiations of launch_fkl live in translation units of their own (topk_div_any.hip,
+// topk_multi_any.hip), so that they compile beside the others.
+int launch_fkl_any(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st);
+int launch_fkl_any_multi(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared);
 
 template <class Tag>
 static hipError_t launch_rkl(const TopkParams& p, bool aligned, hipStream_t st) {

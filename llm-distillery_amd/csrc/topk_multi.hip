@@ -292,8 +292,9 @@ extern "C" int dl_fkl_multi_teacher(const void* logits, int logits_dtype, int64_
   const int eb = logits_dtype == DL_F32 ? 4 : 2;
   const bool on_grid = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && ((row_stride * eb) % 16 == 0) &&
                        (!grad || (reinterpret_cast<uintptr_t>(grad) % 16 == 0 && (grad_stride * eb) % 16 == 0));
-  if (!on_grid) return DL_ERR_ALIGN;
-  const bool whole = V % (16 / eb) == 0;      // else the rows end inside a chunk: the ROWS_TAIL kernels
+  if (!on_grid && (flags & DL_TOPK_ANY_ROWS) == 0) return DL_ERR_ALIGN;
+  if (reinterpret_cast<uintptr_t>(logits) % eb != 0 || (grad && reinterpret_cast<uintptr_t>(grad) % eb != 0)) return DL_ERR_ALIGN;
+  const bool whole = on_grid && V % (16 / eb) == 0;      // else the ROWS_ANY kernels
   MultiPlan plan;
   if (!multi_plan(logits_dtype, n_rows, V, E, n_teacher_rows, flags, plan)) return DL_ERR_LIMIT;
   if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 256 != 0 ||
@@ -351,8 +352,8 @@ extern "C" int dl_fkl_multi_teacher(const void* logits, int logits_dtype, int64_
       else launch_prep<40, false>(q, st);
     }
   }
-  if (!whole) return launch_fkl_tail_multi(logits_dtype, p, plan.exchange_bytes, st, ws_cleared);
-  return logits_dtype == DL_F32 ? launch_fkl<TagF32, true>(p, true, plan.exchange_bytes, st, ws_cleared)
-         : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, true>(p, true, plan.exchange_bytes, st, ws_cleared)
-                                   : launch_fkl<TagF16, true>(p, true, plan.exchange_bytes, st, ws_cleared);
+  if (!whole) return launch_fkl_any_multi(logits_dtype, p, plan.exchange_bytes, st, ws_cleared);
+  return logits_dtype == DL_F32 ? launch_fkl<TagF32, true>(p, plan.exchange_bytes, st, ws_cleared)
+         : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, true>(p, plan.exchange_bytes, st, ws_cleared)
+                                   : launch_fkl<TagF16, true>(p, plan.exchange_bytes, st, ws_cleared);
 }

@@ -3,6 +3,7 @@ losses fed by them.  Thin wrappers over the C ABI; all arithmetic runs in the HI
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Sequence
 
 import torch
@@ -114,13 +115,13 @@ def fkl_multi_teacher(logits: torch.Tensor, vals: Sequence[torch.Tensor], idxs: 
     launch maps, weighs and renormalises the entries and deals them, unsorted, into one bucket per
     column part of the loss kernel's rows; the loss kernel's workgroups each fetch only their own
     bucket and sum the entries that share a student id on their per-chunk lists.  Other temperatures
-    and unaligned or very wide rows take the sorting form: `merge_remap_topk` (ascending unique ids
+    and very wide rows take the sorting form: `merge_remap_topk` (ascending unique ids
     through memory) feeding `ops.div_topk`.  `fused=True` insists on the first form (raises where it
-    does not apply), `fused=False` on the second."""
+    does not apply, and on rows off the 16-byte grid), `fused=False` on the second."""
     tT = T if teacher_T is None else teacher_T
     if fused is None or fused:
-        got = _fkl_multi_fused(logits, vals, idxs, weights, id_map, row_map, T, grad_scale, want_grad, grad_out, no_wait) \
-            if tT == 1.0 else None
+        got = _fkl_multi_fused(logits, vals, idxs, weights, id_map, row_map, T, grad_scale, want_grad, grad_out, no_wait,
+                               any_rows=not fused) if tT == 1.0 else None
         if got is not None:
             return got
         if fused:
@@ -132,7 +133,7 @@ def fkl_multi_teacher(logits: torch.Tensor, vals: Sequence[torch.Tensor], idxs: 
                         grad_scale=grad_scale, want_grad=want_grad, grad_out=grad_out, unique_ids=True, no_wait=no_wait)
 
 
-def _fkl_multi_fused(logits, vals, idxs, weights, id_map, row_map, T, grad_scale, want_grad, grad_out, no_wait):
+def _fkl_multi_fused(logits, vals, idxs, weights, id_map, row_map, T, grad_scale, want_grad, grad_out, no_wait, any_rows):
     """dl_fkl_multi_teacher; None where the library says the one-pass form does not apply."""
     _dev(logits, "logits")
     x = ops._rows_2d(logits)
@@ -155,9 +156,11 @@ def _fkl_multi_fused(logits, vals, idxs, weights, id_map, row_map, T, grad_scale
     lib = _lib.load()
     n = len(vals)
     flags = _lib.DL_TOPK_NO_WAIT if no_wait else 0
+    w = (ctypes.c_float * n)(*[float(v) for v in weights])
+    if any_rows and all(0.0 <= v < math.inf for v in w):      # rows off the grid with other weights: the sorting form takes those
+        flags |= _lib.DL_TOPK_ANY_ROWS
     ws_bytes = lib.dl_fkl_multi_teacher_workspace_bytes(_DT[x.dtype], R, V, n, K, N, flags)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    w = (ctypes.c_float * n)(*[float(v) for v in weights])
     with torch.cuda.device(dev):
         st = lib.dl_fkl_multi_teacher(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, n, _ptr_array(vals),
                                       _ptr_array(idxs), _DT[vals[0].dtype], _IT[idxs[0].dtype], K, N, w, map_ptr,

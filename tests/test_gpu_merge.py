@@ -224,6 +224,54 @@ def test_bucketed_multi_teacher_on_a_crop_of_padded_rows(D, V, pitch, dtype):
     assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
 
 
+@pytest.mark.parametrize("V,dtype,offset", [(151665, torch.bfloat16, 0), (20003, torch.float16, 0), (40001, torch.float32, 0),
+                                             (65537, torch.bfloat16, 3), (1003, torch.float32, 1)])
+def test_bucketed_multi_teacher_on_rows_off_the_grid(D, V, dtype, offset):
+    """Rows that start on any element take the bucketed form too (unless it is insisted on): entries, several on one id, in the
+    columns beside the parts' chunks, masked rows, a gradient buffer of another phase, waiting or not; against the oracle and the
+    sorting form, which keeps weights that the bucketed one refuses."""
+    g = torch.Generator().manual_seed(V)
+    R, K, n, Vt = 9, 100, 3, V + 4000
+    logits = (torch.randn(R, V, generator=g) * 3).to(dtype)
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[4] = False
+    nv = int(valid.sum())
+    vals, idxs = _teachers(nv, K, Vt, n, V + 1)
+    weights = [0.5, 0.3, 0.2]
+    id_map = torch.randint(0, V, (Vt,), generator=g, dtype=torch.int32)
+    id_map[torch.rand(Vt, generator=g) < 0.05] = -1
+    for j, col in enumerate((V - 1, V - 2, 0, 3, min(V, 32768) - 1, 32769 % V)):
+        id_map[idxs[j % 3][:, j].long()] = col
+        id_map[idxs[(j + 1) % 3][:, j].long()] = col
+    rm = torch.full((R,), -1, dtype=torch.int32)
+    rm[valid] = torch.arange(nv, dtype=torch.int32)
+    x = torch.full((R, V + 2 * offset), 3.0, dtype=dtype, device=DEV)[:, offset:offset + V]
+    x.copy_(logits.to(DEV))
+    args = (x, [v.to(DEV) for v in vals], [i.to(DEV) for i in idxs], weights, id_map.to(DEV))
+    kw = dict(row_map=rm.to(DEV), T=1.2, teacher_T=1.0, grad_scale=1.0 / nv)
+    out = torch.full((R, V + 3), 5.0, dtype=dtype, device=DEV)
+    rl, grad = D.fkl_multi_teacher(*args, **kw, grad_out=out[:, 2:2 + V])
+    assert (out[:, :2] == 5.0).all() and (out[:, 2 + V:] == 5.0).all()
+    rows64, grad64, cnt, ids = _oracle_multi(logits, vals, idxs, weights, id_map, 1.2, valid)
+    np.testing.assert_allclose(rl.cpu()[valid].double().numpy(), rows64.numpy(), rtol=2e-5, atol=2e-6)
+    assert torch.count_nonzero(rl.cpu()[~valid]) == 0 and torch.count_nonzero(grad.cpu()[~valid]) == 0
+    grad64 = grad64 / nv
+    rtol = 1e-4 if dtype == torch.float32 else 2e-3
+    bound = O.storage_tolerance(grad64, dtype, rtol)
+    vrows = torch.nonzero(valid).squeeze(-1)
+    bound[vrows] = O.sparse_gradient_tolerance(grad64[vrows], logits[vrows], 1.2, ids, dtype, rtol, row_coef=1.0 / (nv * 1.2))
+    for got in (grad, D.fkl_multi_teacher(*args, **kw, fused=False)[1]):
+        err = (got.cpu().double() - grad64).abs()
+        assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+    for no_wait in (False, True):
+        rl2, grad2 = D.fkl_multi_teacher(*args, **kw, no_wait=no_wait)
+        assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
+    if V % 2:
+        with pytest.raises(RuntimeError):
+            D.fkl_multi_teacher(*args, **kw, fused=True)
+        D.fkl_multi_teacher(*args[:3], [0.5, -0.25, 0.75], args[4], **kw)
+
+
 def test_bucketed_multi_teacher_edge_rows(D):
     """Rows whose entries are all dropped (loss 0, zero gradient), a teacher of weight 0, ids outside
     the teacher vocabulary, int64 ids with fp32 values, no map at all."""

@@ -434,3 +434,38 @@ def test_rows_whose_ids_all_repeat(D, kind):
     a = _check(D, kind, logits, tv, ti.to(torch.int32), T=1.2)
     b = _check(D, kind, logits, tv, ti.to(torch.int32), T=1.2)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 98305),        # the fourth part of 256 x 16 chunks holds one column
+                                     (torch.float16, 53255),         # the 512-thread shape's last chunk, 7 columns behind it
+                                     (torch.bfloat16, 204801),       # seven parts of 15 chunks per thread
+                                     (torch.float32, 65537),         # three parts of four-byte chunks, one column more
+                                     (torch.bfloat16, 16391)])       # 256 x 16 chunks, seven columns more
+def test_columns_beside_the_chunks_of_a_part(D, dtype, V):
+    """Contiguous rows of odd length: every row starts elsewhere on the 16-byte grid, and every column part has columns
+    ahead of its first chunk and behind its last.  Entries (one id twice) on those columns on both sides of the parts'
+    borders, a -inf logit among them, masked rows; waiting or not the same bits."""
+    R, step = 9, 32768 if dtype != torch.float32 else 16384
+    g = torch.Generator().manual_seed(V)
+    logits = (torch.randn(R, V, generator=g) * 3).to(dtype)
+    logits[3, 1] = -float("inf")
+    edges = [c + d for c in range(0, V, step) for d in range(-7, 8) if 0 <= c + d < V and c + d != 1] + [V - 1, V - 2, V - 7]
+    ids = torch.tensor(sorted(set(edges)))
+    ids = torch.cat([ids, torch.tensor([0, V - 1]), torch.randperm(V - 40, generator=g)[:20] + 20])
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[[1, 8]] = False
+    nv = int(valid.sum())
+    ti = ids.expand(nv, -1).contiguous().int()
+    tv = torch.log_softmax(torch.randn(nv, ids.numel(), generator=g), -1).half()
+    rm = torch.full((R,), -1, dtype=torch.int32)
+    rm[valid] = torch.arange(nv, dtype=torch.int32)
+    _, rows64, grad64 = O.mean_loss_and_grad("fkl", logits, 1.3, t_vals=tv, t_idx=ti, valid=valid, dtype=torch.float64)
+    bound = O.topk_gradient_tolerance("fkl", grad64, logits, tv, ti, 1.3, None, 1.0 / nv, dtype, TOL[dtype], valid)
+    got = [D.div_topk("fkl", logits.to(DEV), tv.to(DEV), ti.to(DEV), row_map=rm.to(DEV), T=1.3, grad_scale=1.0 / nv, no_wait=w)
+           for w in (False, True)]
+    rl, grad = got[0]
+    np.testing.assert_allclose(rl.cpu()[valid].double().numpy(), rows64.numpy(), rtol=2e-5, atol=2e-6)
+    assert torch.count_nonzero(rl.cpu()[~valid]) == 0 and torch.count_nonzero(grad.cpu()[~valid]) == 0
+    err = (grad.cpu().double() - grad64).abs()
+    assert (err <= bound).all(), f"worst {(err / bound).max():.2f}"
+    assert torch.equal(rl, got[1][0]) and torch.equal(grad, got[1][1])
