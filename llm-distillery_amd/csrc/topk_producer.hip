@@ -69,12 +69,10 @@ __host__ __device__ inline int producer_merge_slots(int K, int parts) {
   while (n2 < parts * producer_record_cap(K, parts)) n2 <<= 1;
   return n2;
 }
-// Chunk groups per thread of the part kernel: 1024 groups per part for K <= 256, else one per chunk (4096).
-__host__ __device__ inline int producer_groups(int K) { return K <= 256 ? PROD_G_SMALL : PROD_G_LARGE; }
 // A (row, part) record: 16-byte header, then either the part's candidates (8 bytes each) or the largest key of
-// each of its chunk groups (key_bytes each).
-__host__ __device__ inline int64_t producer_part_stride(int K, int parts, int key_bytes) {
-  const int64_t cands = (int64_t)producer_record_cap(K, parts) * 8, maxima = (int64_t)producer_groups(K) * PROD_NT * key_bytes;
+// each of its chunk groups (G per thread, key_bytes each).
+__host__ __device__ inline int64_t producer_part_stride(int K, int parts, int key_bytes, int G) {
+  const int64_t cands = (int64_t)producer_record_cap(K, parts) * 8, maxima = (int64_t)G * PROD_NT * key_bytes;
   return 16 + (((cands > maxima ? cands : maxima) + 15) & ~15LL);
 }
 
@@ -279,20 +277,26 @@ __device__ __forceinline__ int64_t producer_row(const ProducerParams& p, int64_t
 }
 
 // Chunk c of a part that starts at rpart and holds n_elems columns in nch chunks (beyond them: -inf).  ALIGNED: rows
-// on the 16-byte grid that hold a whole number of chunks.  Otherwise only a last chunk that the row does not fill is put
-// together element by element; the others come by 16-byte loads, from rows off the grid (`on_grid` false) by unaligned
-// ones (which the device takes).
-template <class Tag, bool ALIGNED>
-__device__ __forceinline__ u32x4 producer_load_chunk(const char* rpart, int c, int nch, int n_elems, bool on_grid) {
-  using C = Chunk<Tag>;
-  if constexpr (ALIGNED) {
-    return c < nch ? load16_stream(rpart + (int64_t)c * 16) : C::neg_inf();
-  } else {
-    const bool whole = (c + 1) * C::N <= n_elems;
-    return c >= nch ? C::neg_inf()
-           : !whole ? load_chunk_elementwise<Tag>(rpart, c, n_elems)
-           : on_grid ? load16_stream(rpart + (int64_t)c * 16) : load16_unaligned(rpart + (int64_t)c * 16);
-  }
+// on the 16-byte grid that hold a whole number of chunks.  Otherwise rows of at least one chunk that may start on any
+// element and end inside a chunk: the same 16-byte loads, unaligned where the row is (which the device takes), except
+// that the chunk the row does not fill is loaded as the row's last 16 bytes; producer_settle_chunk moves them into place
+// once every load is on its way.  No branch between the loads (8192 rows x 128253 of 128256 bf16, K = 200: 458 us with
+// the last chunk put together element by element, 431 us).
+template <class Tag, bool ALIGNED, bool STREAM = true>
+__device__ __forceinline__ u32x4 producer_load_chunk(const char* rpart, int c, int nch, int n_elems) {
+  if (c >= nch) return Chunk<Tag>::neg_inf();
+  if constexpr (ALIGNED) return load16_stream(rpart + (int64_t)c * 16);
+  const char* at = rpart + (int64_t)min(c * 16, n_elems * Tag::bytes - 16);
+  if constexpr (STREAM) return load16_stream_any(at);
+  else return load16_unaligned(at);
+}
+template <class Tag>
+__device__ __forceinline__ void producer_settle_chunk(u32x4& v, int c, int n_elems) {
+  const int over = c * 16 + 16 - n_elems * Tag::bytes;              // bytes the chunk reaches beyond the row
+  if (over <= 0 || over >= 16) return;
+  typedef unsigned __int128 u128;
+  const u128 x = __builtin_bit_cast(u128, v), inf = __builtin_bit_cast(u128, Chunk<Tag>::neg_inf());
+  v = __builtin_bit_cast(u32x4, (x >> (8 * over)) | (inf << (128 - 8 * over)));
 }
 
 constexpr int PART_FULL = 0;    // threshold, candidates and record of the part: all the part kernel's stages
@@ -300,9 +304,9 @@ constexpr int PART_LIGHT = 1;   // statistics and chunk-group maxima only: the c
 constexpr int PART_REDO = 2;    // PART_FULL for the rows the row-level selection handed back
 
 // G = chunk groups per thread whose maxima feed the threshold search: 256 * G groups per part must
-// be a few times K for the candidate set to stay close to K (4 for K <= 256, else 16).
+// be a few times K for the candidate set to stay close to K (producer_shape).
 // ALIGNED: rows start on 16-byte boundaries and hold a whole number of chunks (16-byte loads);
-// otherwise the chunks are assembled element by element and the last one is padded with -inf,
+// otherwise they may start on any element and the last chunk is padded with -inf,
 // which the collection leaves out (a padding entry has the lowest key and the highest columns of
 // its part, so the threshold searches, which only count, need no such test).
 template <class Tag, int G, bool ALIGNED, int MODE>
@@ -334,9 +338,33 @@ __device__ __forceinline__ void topk_part(const ProducerParams& p, int64_t ro, i
   const int select_wave = (int)((blockIdx.x >> 3) & (NW - 1));
 
   u32x4 reg[NCH];
-  const bool on_grid = (reinterpret_cast<uintptr_t>(rpart) & 15) == 0;      // the same for the whole workgroup
+  if constexpr (ALIGNED) {
 #pragma unroll
-  for (int i = 0; i < NCH; ++i) reg[i] = producer_load_chunk<Tag, ALIGNED>(rpart, i * NT + tid, nch, n_elems, on_grid);
+    for (int i = 0; i < NCH; ++i) reg[i] = producer_load_chunk<Tag, true>(rpart, i * NT + tid, nch, n_elems);
+  } else if ((reinterpret_cast<uintptr_t>(rpart) & 15) == 0 && p.V >= C::N) {      // the same for the whole workgroup
+    u32x4 end = load16_unaligned(rpart + n_elems * Tag::bytes - 16);      // the row's last 16 bytes, ahead of the others
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) reg[i] = producer_load_chunk<Tag, false>(rpart, i * NT + tid, nch, n_elems);
+    // (the settled chunk is made once, by every thread, and put in place by a select: settled where it lies, in one of
+    // eight registers, it costs spills)
+    const int last = nch - 1;
+    producer_settle_chunk<Tag>(end, last, n_elems);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      if (i != last / NT) continue;                                  // the same for every thread
+#pragma unroll
+      for (int d = 0; d < 4; ++d) reg[i][d] = tid == last % NT ? end[d] : reg[i][d];
+    }
+  } else {
+    // off the grid, where neighbouring loads share lines: cached, not streamed (3594 x 50257 fp16 131 against 108 us), and
+    // the last chunk element by element (8192 x 50257 bf16 299 us settled as above, with every load waited for at once)
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = i * NT + tid;
+      reg[i] = c >= nch ? C::neg_inf() : (c + 1) * C::N > n_elems ? load_chunk_elementwise<Tag>(rpart, c, n_elems)
+                                                                  : load16_unaligned(rpart + (int64_t)c * 16);
+    }
+  }
   if (tid == 0) s_n = 0;
 
   if constexpr (MODE == PART_LIGHT) {
@@ -349,11 +377,17 @@ __device__ __forceinline__ void topk_part(const ProducerParams& p, int64_t ro, i
     typedef typename KY::Stored KS;
     KS* gout = reinterpret_cast<KS*>(rec + 16);
     const int mine = (nch - tid + NT - 1) / NT;                       // chunks i < mine are inside the part
+    // rounds that lie behind the part's last chunk are left out by whole waves (a part of 1670 chunks fills 3.3 of its
+    // eight, and their exponentials are what bounds this kernel: 10516 rows x 13355 fp16 74 -> 66 us)
+    const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~(WAVE - 1));
     unsigned tk = 0u;                                                 // largest key of the thread (0: none)
     unsigned gk[NCH];                                                 // group maxima; stored at the end: a store between the
                                                                       // loads' waits would make each of them a wait for everything
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
+      gk[i] = 0u;
+      forget(reg[i]);
+      if (i * NT + wave0 >= nch) continue;
       unsigned e[4];
 #pragma unroll
       for (int d = 0; d < 4; ++d) e[d] = KY::encode(reg[i][d]);
@@ -374,6 +408,7 @@ __device__ __forceinline__ void topk_part(const ProducerParams& p, int64_t ro, i
     for (int i = 0; i < NCH; ++i) {
       float f[C::N];
       forget(reg[i]);
+      if (i * NT + wave0 >= nch) continue;
       C::unpack(reg[i], f);
 #pragma unroll
       for (int e = 0; e < C::N; ++e) st += fast_exp2(fmaf(f[e], LOG2E, -mbt));
@@ -659,17 +694,16 @@ __device__ __forceinline__ void emit_sorted(const ProducerParams& p, int64_t ro,
   }
 }
 
-// The same for narrow words (16-bit keys that share their leading bits `prefix`): the complement of the key's low
-// TAIL bits above CB bits of column.
+// The same for narrow words (16-bit keys): the key's distance below `top` above CB bits of column.
 template <class Tag, int EPL>
 __device__ __forceinline__ void emit_sorted_narrow(const ProducerParams& p, int64_t ro, float lse, const unsigned (&c)[EPL],
-                                                   unsigned prefix, int tail, int cb) {
+                                                   unsigned top, int cb) {
   const int lane = threadIdx.x & (WAVE - 1);
 #pragma unroll
   for (int j = 0; j < EPL; ++j) {
     const int k = lane * EPL + j;
     if (k < p.K) {
-      const unsigned key = prefix | (~(c[j] >> cb) & ((1u << tail) - 1u));
+      const unsigned key = top - (c[j] >> cb);
       const float logp = Keys<Tag>::value(key) - lse;
       const int col = (int)(c[j] & ((1u << cb) - 1u));
       store_from_float(p.out_val, p.out_dtype, ro * p.K + k, logp);
@@ -867,8 +901,8 @@ __host__ __device__ inline int producer_select_cands(int K) {
 __host__ __device__ inline int producer_select_groups(int K) { return 2 * K > 512 ? 2 * K : 512; }
 // Dynamic LDS of topk_select_kernel: the group maxima of all parts, later the candidate words; the selected
 // words; the list of groups to open.
-__host__ __device__ inline size_t producer_select_lds(int K, int parts, int key_bytes) {
-  const size_t maxima = (size_t)parts * producer_groups(K) * PROD_NT * key_bytes, cands = (size_t)producer_select_cands(K) * 8;
+__host__ __device__ inline size_t producer_select_lds(int K, int parts, int key_bytes, int G) {
+  const size_t maxima = (size_t)parts * G * PROD_NT * key_bytes, cands = (size_t)producer_select_cands(K) * 8;
   return ((maxima > cands ? maxima : cands) + 15) / 16 * 16 + (size_t)producer_sel_cap(K) * 8 + (size_t)producer_select_groups(K) * 4;
 }
 
@@ -959,169 +993,114 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p
   hist[tid] = 0;
   __syncthreads();
 
-  // Candidate words of 32 bits where the keys have 16 and the bound comes from the histogram step: every candidate then
-  // shares the six leading bits of the largest maximum, so 10 key bits and 22 bits of column tell the words apart,
-  // and the wave that sorts them moves and compares half as many registers.
-  constexpr int TAIL_BITS = KY::BITS - 6, COL_BITS = 32 - TAIL_BITS;
+  // L: a lower bound of the K-th largest group maximum, as tight as one histogram makes it.  (Any bound at or below the
+  // K-th largest key of the row gives the same result; a looser one costs candidates.)  256 bins of a 32nd of an octave
+  // count the maxima by their distance below the largest, over eight octaves whatever the storage type -- bins by
+  // leading key bits took in a single octave of fp16, whose K-th largest logit rarely lies that close, and the
+  // bisection that then takes over costs a barrier per key bit (10516 rows x 13360 fp16, K = 68: 192 us for this kernel;
+  // 71 us with the distance).
+  // Candidate words of 32 bits where the keys have 16 and the bound comes from the histogram: the distance below the
+  // largest key and the column tell the words apart, and the wave that sorts them moves and compares half as many registers.
+  constexpr int BIN_SHIFT = Tag::id == F32 ? 18 : Tag::id == BF16 ? 2 : 5;      // mantissa bits - 5
+  constexpr int TAIL_BITS = KY::BITS == 16 ? BIN_SHIFT + 8 : 16, COL_BITS = 32 - TAIL_BITS;
   bool narrow = false;
-  unsigned key_prefix = 0u;
   unsigned L = 0;
+  unsigned top = 0u;
   if constexpr (MAXR > 0) {
-    // every thread's maxima: `visit(key, group)` for each of them
-    const auto for_keys = [&](auto visit) {
+    unsigned dm = 0u;
+#pragma unroll
+    for (int rr = 0; rr < MAXR; ++rr)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) dm = KY::dword_max(dm, mreg[rr][d]);
+    top = KY::top_key(dm);
+  } else {
+    for (int a = tid; a < n_g; a += 256) top = max(top, (unsigned)gmax[a]);
+  }
+  top = wave_max(top);
+  if (lane == 0) sh.best[w] = top;
+  __syncthreads();
+  top = max(max(sh.best[0], sh.best[1]), max(sh.best[2], sh.best[3]));
+  // from here on the maxima are only met as their distances below the largest, `visit(distance, group)`: in the
+  // registers they take the maxima's place
+  if constexpr (MAXR > 0) {
+#pragma unroll
+    for (int rr = 0; rr < MAXR; ++rr)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        if constexpr (DW == 2)
+          mreg[rr][d] = __builtin_bit_cast(unsigned, (u16x2)(__builtin_bit_cast(u16x2, top * 0x00010001u) - __builtin_bit_cast(u16x2, (unsigned)mreg[rr][d])));
+        else mreg[rr][d] = top - mreg[rr][d];
+      }
+  }
+  const auto for_distances = [&](auto visit) {
+    if constexpr (MAXR > 0) {
 #pragma unroll
       for (int rr = 0; rr < MAXR; ++rr)
 #pragma unroll
         for (int d = 0; d < 4; ++d)
 #pragma unroll
           for (int h = 0; h < DW; ++h) visit(KY::key(mreg[rr][d], h), (rr * 256 + tid) * KPL + d * DW + h);
-    };
-    int probe = 0;
-    const auto count_ge = [&](unsigned t) {
-      int c = 0;
-      for_keys([&](unsigned k, int) { c += k >= t ? 1 : 0; });
-      c = wave_sum(c);
-      int* sl = s_sum + (probe++ & 1) * 4;
-      if (lane == 0) sl[w] = c;
-      __syncthreads();
-      return sl[0] + sl[1] + sl[2] + sl[3];
-    };
-    unsigned dm = 0u;
-#pragma unroll
-    for (int rr = 0; rr < MAXR; ++rr)
-#pragma unroll
-      for (int d = 0; d < 4; ++d) dm = KY::dword_max(dm, mreg[rr][d]);
-    unsigned top = wave_max(KY::top_key(dm));
-    if (lane == 0) sh.best[w] = top;
-    __syncthreads();
-    top = max(max(sh.best[0], sh.best[1]), max(sh.best[2], sh.best[3]));
-    constexpr int TAIL = KY::BITS - 6;                                // bits below the prefix
-    const unsigned prefix = top & ~((1u << TAIL) - 1u);
-    // histogram of the next eight bits of the maxima that share the prefix (prefix 0: the padding keys would count);
-    // should fewer than K of them share it, no bin is found and the bisection below takes over
-    bool found = false;
-    if (prefix != 0u) {
-      constexpr int SH = TAIL - 8;
-      for_keys([&](unsigned k, int) { if (k >= prefix) atomicAdd(&hist[(k >> SH) & 255u], 1); });
-      __syncthreads();
-      if (w == 0) {
-        int c[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) c[j] = hist[lane * 4 + j];
-        const int mine = c[0] + c[1] + c[2] + c[3];
-        int incl = mine;
-#pragma unroll
-        for (int o = 1; o < WAVE; o <<= 1) {
-          const int t = __shfl_up(incl, o, WAVE);
-          incl += lane >= o ? t : 0;
-        }
-        const int sharing = __shfl(incl, WAVE - 1, WAVE);
-        const int above = sharing - incl;
-        int run = above, bin = -1;
-#pragma unroll
-        for (int j = 3; j >= 0; --j) {
-          if (bin < 0 && run + c[j] >= K && run < K) bin = lane * 4 + j;
-          run += c[j];
-        }
-        if (lane == 0 && sharing < K) s_sum[0] = -1;
-        if (bin >= 0) s_sum[0] = bin;                                 // exactly one lane finds it when K or more share the prefix
-      }
-      __syncthreads();
-      const int bin = s_sum[0];
-      __syncthreads();
-      if (bin >= 0) {
-        L = prefix | ((unsigned)bin << SH);
-        narrow = KY::BITS == 16 && p.V <= (1ll << COL_BITS);
-        key_prefix = prefix;
-        found = true;
-      }
-    }
-    if (!found) {
-#pragma unroll 1
-      for (int b = KY::BITS - 1; b >= 0; --b) {
-        const unsigned t = L | (1u << b);
-        if (count_ge(t) >= K) L = t;
-      }
-    }
-    if (L != 0u)
-      for_keys([&](unsigned k, int a) {
-        if (k >= L) {
-          const int slot = atomicAdd(&s_nq, 1);
-          if (slot < qcap) glist[slot] = a;
-        }
-      });
-  } else {
-    // L: a lower bound of the K-th largest group maximum, as tight as a few steps make it.  (Any bound at or below the
-    // K-th largest key of the row gives the same result; a looser one costs candidates.)
-    int probe = 0;
-    const auto count_ge = [&](unsigned t) {
-      int c = 0;
-      for (int a = tid; a < n_g; a += 256) c += (unsigned)gmax[a] >= t ? 1 : 0;
-      c = wave_sum(c);
-      int* sl = s_sum + (probe++ & 1) * 4;
-      if (lane == 0) sl[w] = c;
-      __syncthreads();
-      return sl[0] + sl[1] + sl[2] + sl[3];
-    };
-    // the answer nearly always shares the six leading bits of the largest maximum
-    unsigned top = 0u;
-    for (int a = tid; a < n_g; a += 256) top = max(top, (unsigned)gmax[a]);
-    top = wave_max(top);
-    if (lane == 0) sh.best[w] = top;
-    __syncthreads();
-    top = max(max(sh.best[0], sh.best[1]), max(sh.best[2], sh.best[3]));
-    constexpr int TAIL = KY::BITS - 6;                                // bits below the prefix
-    const unsigned prefix = top & ~((1u << TAIL) - 1u);
-    if (count_ge(prefix) >= K) {
-      // histogram of the next eight bits of the maxima that share the prefix; the bin that holds the K-th largest,
-      // counted from the top, gives eight more bits of L (its lowest key: at most the bins' width below the true one)
-      constexpr int SH = TAIL - 8;
-      for (int a = tid; a < n_g; a += 256) {
-        const unsigned v = (unsigned)gmax[a];
-        if (v >= prefix) atomicAdd(&hist[(v >> SH) & 255u], 1);
-      }
-      __syncthreads();
-      if (w == 0) {
-        // lane l holds bins 4l .. 4l + 3; suffix sums from the top bin down
-        int c[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) c[j] = hist[lane * 4 + j];
-        const int mine = c[0] + c[1] + c[2] + c[3];
-        int incl = mine;                                               // inclusive scan over the lanes
-#pragma unroll
-        for (int o = 1; o < WAVE; o <<= 1) {
-          const int t = __shfl_up(incl, o, WAVE);
-          incl += lane >= o ? t : 0;
-        }
-        const int above = __shfl(incl, WAVE - 1, WAVE) - incl;         // entries in the bins of the lanes above this one
-        int run = above, bin = -1;
-#pragma unroll
-        for (int j = 3; j >= 0; --j) {
-          if (bin < 0 && run + c[j] >= K && run < K) bin = lane * 4 + j;
-          run += c[j];
-        }
-        if (bin >= 0) s_sum[0] = bin;                                 // exactly one lane finds it
-      }
-      __syncthreads();
-      L = prefix | ((unsigned)s_sum[0] << SH);
-      narrow = KY::BITS == 16 && p.V <= (1ll << COL_BITS);
-      key_prefix = prefix;
-      __syncthreads();
     } else {
-#pragma unroll 1
-      for (int b = KY::BITS - 1; b >= 0; --b) {
-        const unsigned t = L | (1u << b);
-        if (count_ge(t) >= K) L = t;
-      }
+      for (int a = tid; a < n_g; a += 256) visit(top - (unsigned)gmax[a], a);
     }
-    // the groups to open
-    for (int a = tid; a < n_g; a += 256) {
-      if ((unsigned)gmax[a] >= L) {
+  };
+  constexpr unsigned REACH = 256u << BIN_SHIFT;
+  const bool binned = top >= REACH;                                 // else the padding keys (0, at distance `top`) would count
+  if (binned) for_distances([&](unsigned d, int) { if (d < REACH) atomicAdd(&hist[d >> BIN_SHIFT], 1); });
+  __syncthreads();
+  if (w == 0) {
+    // lane l holds bins 4 l .. 4 l + 3; the bin at which the count from the top reaches K
+    int c[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c[j] = hist[lane * 4 + j];
+    const int mine = c[0] + c[1] + c[2] + c[3];
+    int incl = mine;
+#pragma unroll
+    for (int o = 1; o < WAVE; o <<= 1) {
+      const int t = __shfl_up(incl, o, WAVE);
+      incl += lane >= o ? t : 0;
+    }
+    int run = incl - mine, bin = -1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (bin < 0 && run < K && run + c[j] >= K) bin = lane * 4 + j;
+      run += c[j];
+    }
+    if (lane == WAVE - 1 && incl < K) s_sum[0] = -1;                // fewer than K of them within eight octaves
+    if (bin >= 0) s_sum[0] = bin;                                   // else exactly one lane finds it
+  }
+  __syncthreads();
+  const int bin = s_sum[0];
+  __syncthreads();
+  if (bin >= 0) {
+    const unsigned below = ((unsigned)(bin + 1) << BIN_SHIFT) - 1u;  // the bin's largest distance, below `top`
+    L = top - below;
+    narrow = KY::BITS == 16 && p.V <= (1ll << COL_BITS);
+  } else {
+    int probe = 0;
+    const auto count_ge = [&](unsigned t) {      // t <= top
+      int c = 0;
+      for_distances([&](unsigned d, int) { c += d <= top - t ? 1 : 0; });
+      c = wave_sum(c);
+      int* sl = s_sum + (probe++ & 1) * 4;
+      if (lane == 0) sl[w] = c;
+      __syncthreads();
+      return sl[0] + sl[1] + sl[2] + sl[3];
+    };
+#pragma unroll 1
+    for (int b = KY::BITS - 1; b >= 0; --b) {
+      const unsigned t = L | (1u << b);
+      if (t <= top && count_ge(t) >= K) L = t;
+    }
+  }
+  // the groups to open
+  if (L != 0u)
+    for_distances([&](unsigned d, int a) {
+      if (d <= top - L) {
         const int slot = atomicAdd(&s_nq, 1);
         if (slot < qcap) glist[slot] = a;
       }
-    }
-  }
+    });
   __syncthreads();                                                  // the maxima are done with: their LDS takes the candidates
   const int n_q = s_nq;
   bool redo = n_q > qcap || L == 0;                                 // L == 0: fewer than K groups hold anything; the part kernel's own selection takes every entry then
@@ -1160,13 +1139,16 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p
           const int n_elems = (int)min((int64_t)NT * NCH * C::N, p.V - lo);
           const int nch = (n_elems + C::N - 1) / C::N;
           const char* rpart = row + c0 * 16;
-          v[u] = producer_load_chunk<Tag, ALIGNED>(rpart, c, nch, n_elems, (reinterpret_cast<uintptr_t>(rpart) & 15) == 0);
+          v[u] = producer_load_chunk<Tag, ALIGNED, false>(rpart, c, nch, n_elems);
           base[u] = lo + c * C::N;
           left[u] = n_elems - c * C::N;
         }
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
+        if constexpr (!ALIGNED) {
+          if (left[u] > 0 && left[u] < C::N) producer_settle_chunk<Tag>(v[u], 0, left[u]);
+        }
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
           const unsigned kd = KY::encode(v[u][d]);
@@ -1177,7 +1159,7 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p
             if (k >= L && (ALIGNED || e < left[u])) {
               const int slot = atomicAdd(&s_total, 1);
               if (slot < acap) {
-                if (narrow) all32[slot] = ((~k & ((1u << TAIL_BITS) - 1u)) << COL_BITS) | (unsigned)(base[u] + e);
+                if (narrow) all32[slot] = ((top - k) << COL_BITS) | (unsigned)(base[u] + e);
                 else all[slot] = ((u64)(KY::BITS == 32 ? ~k : (0xffff0000u | (~k & 0xffffu))) << 32) | (unsigned)(base[u] + e);
               }
             }
@@ -1202,13 +1184,13 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p
 #pragma unroll
           for (int j = 0; j < 4; ++j) c[j] = lane * 4 + j < total ? all32[lane * 4 + j] : ~0u;
           wave_sort<unsigned, 4>(c);
-          emit_sorted_narrow<Tag, 4>(p, ro, lse, c, key_prefix, TAIL_BITS, COL_BITS);
+          emit_sorted_narrow<Tag, 4>(p, ro, lse, c, top, COL_BITS);
         } else {
           unsigned c[8];
 #pragma unroll
           for (int j = 0; j < 8; ++j) c[j] = lane * 8 + j < total ? all32[lane * 8 + j] : ~0u;
           wave_sort<unsigned, 8>(c);
-          emit_sorted_narrow<Tag, 8>(p, ro, lse, c, key_prefix, TAIL_BITS, COL_BITS);
+          emit_sorted_narrow<Tag, 8>(p, ro, lse, c, top, COL_BITS);
         }
       }
       return;
@@ -1222,7 +1204,7 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p
 #pragma unroll
     for (int j = 0; j < PER; ++j)
       if (j * 256 + tid < total) {
-        const unsigned key = key_prefix | (~(wv[j] >> COL_BITS) & ((1u << TAIL_BITS) - 1u));
+        const unsigned key = top - (wv[j] >> COL_BITS);
         all[j * 256 + tid] = ((u64)(0xffff0000u | (~key & 0xffffu)) << 32) | (wv[j] & ((1u << COL_BITS) - 1u));
       }
     __syncthreads();
@@ -1236,15 +1218,26 @@ static int producer_parts(int64_t V, int logits_dtype) {
   return (int)((nch + PROD_NT * PROD_NCH - 1) / (PROD_NT * PROD_NCH));
 }
 
+// How the rows of a call are served.  The row-level selection wants at least 4 K chunk groups per row that hold
+// anything (fewer bound the K-th key too loosely, or not at all, for opening groups a second time to pay), and their
+// maxima within 64 KiB of LDS: groups of four chunks (1024 per part) where a row has enough of them, whatever K, else
+// groups of one chunk (4096); else thresholds per part.  Measured: 3243 x 50304 fp32, K = 319 (groups of one chunk do not
+// fit the LDS) 639 us with thresholds per part, 196 us with groups of four; 8192 x 128256
+// bf16, K = 400 (groups of one chunk) 802 -> 517 us; 8192 x 8192 bf16, K = 100 (thresholds per part) 119 -> 88 us with groups of one.
+struct ProducerShape { int G; bool select; };
+static ProducerShape producer_shape(int K, int64_t V, int parts, int key_bytes) {
+  const int64_t chunks = (V * key_bytes + 15) / 16;
+  for (int G : {PROD_G_SMALL, PROD_G_LARGE})
+    if ((chunks * G + PROD_NCH - 1) / PROD_NCH >= 4 * (int64_t)K && producer_select_lds(K, parts, key_bytes, G) <= 64 * 1024) return {G, true};
+  return {K <= 256 ? PROD_G_SMALL : PROD_G_LARGE, false};
+}
+
 template <class Tag, int G, bool ALIGNED>
-static void launch_producer_shape(const ProducerParams& p, hipStream_t st) {
+static void launch_producer_shape(const ProducerParams& p, bool select, hipStream_t st) {
   const dim3 grid((unsigned)((p.n_out + 7) / 8 * 8 * p.parts));
   const size_t lds_merge = (size_t)(producer_merge_slots(p.K, p.parts) + producer_sel_cap(p.K)) * 8;      // <= 48 KiB
-  const size_t lds_select = producer_select_lds(p.K, p.parts, Tag::bytes == 4 ? 4 : 2);
-  // chunk groups of a row that hold anything: with fewer than 4 K of them the group maxima bound the K-th key too
-  // loosely (or not at all) for opening groups a second time to pay
-  const int64_t chunks = (p.V + Chunk<Tag>::N - 1) / Chunk<Tag>::N, groups = (chunks + (PROD_NCH / G) - 1) / (PROD_NCH / G);
-  if (lds_select > 64 * 1024 || groups < 4 * (int64_t)p.K) {      // (or too many groups for the selection's LDS): thresholds per part
+  const size_t lds_select = producer_select_lds(p.K, p.parts, Tag::bytes == 4 ? 4 : 2, G);
+  if (!select) {
     hipLaunchKernelGGL((topk_part_kernel<Tag, G, ALIGNED, PART_FULL>), grid, dim3(PROD_NT), 0, st, p);
     hipLaunchKernelGGL((topk_merge_kernel<Tag>), dim3((unsigned)p.n_out), dim3(256), lds_merge, st, p);
     return;
@@ -1272,12 +1265,13 @@ static int launch_producer(const ProducerParams& p, bool aligned, hipStream_t st
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&topk_select_kernel<Tag, PROD_G_LARGE, false, 0>), hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
     lds_allowed = true;
   }
-  if (aligned) {
-    if (p.K <= 256) launch_producer_shape<Tag, PROD_G_SMALL, true>(p, st);
-    else launch_producer_shape<Tag, PROD_G_LARGE, true>(p, st);
+  const ProducerShape sh = producer_shape(p.K, p.V, p.parts, Tag::bytes);
+  if (sh.G == PROD_G_SMALL) {
+    if (aligned) launch_producer_shape<Tag, PROD_G_SMALL, true>(p, sh.select, st);
+    else launch_producer_shape<Tag, PROD_G_SMALL, false>(p, sh.select, st);
   } else {
-    if (p.K <= 256) launch_producer_shape<Tag, PROD_G_SMALL, false>(p, st);
-    else launch_producer_shape<Tag, PROD_G_LARGE, false>(p, st);
+    if (aligned) launch_producer_shape<Tag, PROD_G_LARGE, true>(p, sh.select, st);
+    else launch_producer_shape<Tag, PROD_G_LARGE, false>(p, sh.select, st);
   }
   return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
 }
@@ -1288,7 +1282,8 @@ extern "C" int64_t dl_teacher_topk_workspace_bytes(int logits_dtype, int64_t n_o
   if (n_out <= 0 || V <= 0 || K <= 0) return 0;
   const int parts = dl::producer_parts(V, logits_dtype);
   if (parts > dl::PROD_MAX_PARTS || K > dl::PROD_MAX_K || (int64_t)parts * K > 4096) return 0;
-  const int64_t records = n_out * parts * dl::producer_part_stride(K, parts, logits_dtype == DL_F32 ? 4 : 2);
+  const int kb = logits_dtype == DL_F32 ? 4 : 2;
+  const int64_t records = n_out * parts * dl::producer_part_stride(K, parts, kb, dl::producer_shape(K, V, parts, kb).G);
   return records + 16 + ((n_out * 4 + 15) & ~15LL);                 // then the counter and the list of rows handed back
 }
 
@@ -1313,7 +1308,7 @@ extern "C" int dl_teacher_topk(const void* logits, int logits_dtype, int64_t row
   if (!workspace) return DL_ERR_NULL;
   if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return DL_ERR_ALIGN;
   if (workspace_bytes < dl_teacher_topk_workspace_bytes(logits_dtype, n_out, V, K)) return DL_ERR_WORKSPACE;
-  const int64_t stride = producer_part_stride(K, parts, eb == 4 ? 4 : 2);
+  const int64_t stride = producer_part_stride(K, parts, eb, producer_shape(K, V, parts, eb).G);
   char* redo = reinterpret_cast<char*>(workspace) + n_out * parts * stride;
   ProducerParams p{logits, row_stride, n_rows, V, row_list, n_out, K, parts, reinterpret_cast<char*>(workspace),
                    stride, out_val, out_dtype, out_idx, out_itype, reinterpret_cast<unsigned*>(redo),

@@ -163,6 +163,38 @@ def test_any_vocabulary_size(D, dtype, V, K):
     np.testing.assert_allclose(val.cpu().double().numpy(), rv.numpy(), rtol=0, atol=2e-6 * max(1.0, float(rv[torch.isfinite(rv)].abs().max())))
 
 
+@pytest.mark.parametrize("dtype,V,pitch,K", [(torch.bfloat16, 32771, 32771, 100),     # the second part holds three columns, fewer than a chunk
+                                             (torch.float32, 16385, 16387, 200),      # one column
+                                             (torch.float16, 13355, 13355, 104),      # 418 groups of four chunks: just enough for K = 104,
+                                             (torch.float16, 13355, 13355, 105),      # and one too few: groups of one chunk
+                                             (torch.bfloat16, 8008, 8009, 250),       # 1001 chunks: just enough groups of one chunk,
+                                             (torch.bfloat16, 8008, 8009, 251),       # and too few: thresholds per part
+                                             (torch.float32, 50304, 50432, 319),      # groups of four chunks for more than 256 entries
+                                             (torch.float16, 100277, 100277, 700)])
+def test_borders_of_the_rules_for_groups_and_rows_off_the_grid(D, dtype, V, pitch, K):
+    """Ids bit for bit and values of the row's K largest, ties to the smaller id, on both sides of the rules that choose the
+    chunk groups, with winners, ties and -inf in the last, partly filled chunk and at the borders of parts; columns behind the
+    row are never read into it."""
+    g = torch.Generator().manual_seed(V + K)
+    R = 9
+    full = torch.full((R, pitch), 50.0, dtype=dtype)
+    x = full[:, :V]
+    x.copy_((torch.randn(R, V, generator=g) * 3).to(dtype))
+    x[1, V - 1] = 30.0
+    x[2, V - 9:] = 25.0
+    x[3, V - 3:] = -float("inf")
+    x[4, 0] = 28.0
+    part = 32768 if dtype != torch.float32 else 16384
+    if V > part:
+        x[5, part - 2:part + 2] = 27.0
+    x[6, V - V // 2:] = x[6, :V // 2].clone()                  # ties everywhere
+    x[7] = (x[7] * 0.5).round()                                # a handful of distinct values: plateaus
+    val, idx = D.teacher_topk(full.to(DEV)[:, :V], K, val_dtype=torch.float32, idx_dtype=torch.int64)
+    rv, ri = _ref(x, V, K)
+    assert torch.equal(idx.cpu(), ri)
+    np.testing.assert_allclose(val.cpu().double().numpy(), rv.numpy(), rtol=0, atol=2e-6 * max(1.0, float(rv[torch.isfinite(rv)].abs().max())))
+
+
 def test_odd_crop_of_a_wider_vocabulary_and_tied_tails(D):
     g = torch.Generator().manual_seed(12)
     B, S, Vm, crop, K = 2, 7, 32003, 31999, 120
