@@ -185,8 +185,8 @@ int dl_div_dense(int kind,
  * bit-reproducible from call to call.
  * workspace   at least dl_div_dense_workspace_bytes(...) bytes, 16-byte aligned, contents irrelevant on entry
  *             and on return; NULL or too small: exactly dl_div_dense.  Launches that may overlap in time must
- *             not share a workspace.  dl_div_dense_workspace_bytes returns 0 where rows are not cut (JSD,
- *             narrow or very wide rows, dtype pairs without a register kernel).
+ *             not share a workspace.  dl_div_dense_workspace_bytes returns 0 where rows are not cut
+ *             (narrow or very wide rows, dtype pairs without a register kernel).
  * flags       DL_TOPK_NO_WAIT: the parts never wait for their partners; DL_TOPK_PARTS(1 / 2 / 3): parts of
  *             256 / 512 / 1024 threads wherever two or more come out (test and tuning hooks).
  */

@@ -268,7 +268,8 @@ static int dense_split_units(int s_dtype, int t_dtype) {
 }
 // How a row of V columns is cut: threads per part and parts (parts == 0: not cut).  Measured (forward KL, 512 and
 // 8192 rows, 32000 to 262144 columns, fp32 pairs, 16-bit pairs and a 16-bit student against an fp32 teacher):
-//   * a row that half a workgroup's registers hold (512 threads) stays whole;
+//   * a row that half a workgroup's registers hold (512 threads) stays whole (4096 x 20000 bf16 against fp32, which take
+//     1024 threads whole: 167 us, two parts of 256: 126);
 //   * with a 16-bit student up to four parts of 256 threads beat half as many of 512 (more workgroups per CU to
 //     hide the exchange behind), beyond that the partners to wait for cost more than they bring: parts of 512
 //     threads, at most 8; fp32 students (a part of 256 threads holds 8192 columns only) take parts of 512 from the start;
@@ -276,11 +277,14 @@ static int dense_split_units(int s_dtype, int t_dtype) {
 //     columns of a 16-bit pair, one workgroup per row streams the row from the caches);
 //   * on fewer than 1024 rows the cut pays only from 256 KiB of row pair upwards (one workgroup per row keeps
 //     the CUs busy by itself below that, and has no partners to wait for).
+//   * JSD, whose parts meet twice and have one more launch behind them: a pair that 1024 threads hold stays whole below
+//     1536 rows of 16-bit pairs (1024 x 50304: 102 us whole, 103 cut; 2048: 200 and 184) and 3072 rows of others
+//     (2048 x 20000 fp32: 114 and 116; 4096 x 32000: 327 and 290); a pair that they do not hold is always cut.
 // `forced_nt` (256 / 512 / 1024, a tuning hook) fixes the thread count and cuts wherever two parts or more come out.
 struct DenseCut { int nt, parts; };
 static DenseCut dense_split_cut(int kind, int s_dtype, int t_dtype, int64_t n_rows, int64_t V, int forced_nt = 0) {
   const int nu = dense_split_units(s_dtype, t_dtype);
-  if (kind == DL_JSD || nu == 0 || V < 8) return {0, 0};
+  if (nu == 0 || V < 8) return {0, 0};
   const int64_t units = (V + 7) / 8;
   const auto parts_of = [&](int nt) { return (units + (int64_t)nt * nu - 1) / ((int64_t)nt * nu); };
   const auto cut_of = [&](int nt) {
@@ -288,9 +292,14 @@ static DenseCut dense_split_cut(int kind, int s_dtype, int t_dtype, int64_t n_ro
     return parts >= 2 && parts <= DENSE_MAX_PARTS && (nt != 1024 || t_dtype == F32 || s_dtype == F32) ? DenseCut{nt, (int)parts} : DenseCut{0, 0};
   };
   if (forced_nt) return cut_of(forced_nt);
-  if (parts_of(512) < 2) return {0, 0};
-  const int64_t pair_bytes = V * ((s_dtype == F32 ? 4 : 2) + (t_dtype == F32 ? 4 : 2));
-  if (n_rows < 1024 && pair_bytes < 256 * 1024) return {0, 0};
+  const int whole_nu = s_dtype == t_dtype && s_dtype != F32 ? 8 : 4;      // units per thread of the kernels that hold a row whole
+  if (units <= 512 * whole_nu) return {0, 0};
+  if (kind == DL_JSD) {
+    if (units <= 1024 * whole_nu && n_rows < (whole_nu == 8 ? 1536 : 3072)) return {0, 0};
+  } else {
+    const int64_t pair_bytes = V * ((s_dtype == F32 ? 4 : 2) + (t_dtype == F32 ? 4 : 2));
+    if (n_rows < 1024 && pair_bytes < 256 * 1024) return {0, 0};
+  }
   if (parts_of(256) <= 4 && s_dtype != F32) return cut_of(256);      // (fp32 students: 8192 columns per such part only)
   if (parts_of(512) <= DENSE_MAX_PARTS) return cut_of(512);
   return cut_of(1024);
@@ -303,7 +312,7 @@ extern "C" int64_t dl_div_dense_workspace_bytes(int kind, int logits_dtype, int 
   // enough for every cut the flags of dl_div_dense_ws may ask for
   int parts = 0;
   for (int nt : {0, 256, 512, 1024}) parts = std::max(parts, dl::dense_split_cut(kind, logits_dtype, t_dtype, n_rows, V, nt).parts);
-  return parts ? dl::DenseSplit::bytes(n_rows, parts) : 0;
+  return parts ? dl::DenseSplit::bytes(kind, n_rows, parts) : 0;
 }
 
 extern "C" int dl_div_dense(int kind, const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows,
@@ -345,8 +354,8 @@ extern "C" int dl_div_dense_ws(int kind, const void* logits, int logits_dtype, i
   const int hook = (flags >> DL_TOPK_PARTS_SHIFT) & 15;      // 1 / 2: parts of 256 / 512 threads wherever the row can be cut
   const DenseCut cut = dense_split_cut(kind, logits_dtype, t_dtype, n_rows, V, hook == 1 ? 256 : hook == 2 ? 512 : hook == 3 ? 1024 : 0);
   if (cut.parts && workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 &&
-      workspace_bytes >= DenseSplit::bytes(n_rows, cut.parts) && n_rows * cut.parts <= 0x7fffffffLL) {
-    const DenseSplit x(workspace, n_rows, cut.parts, (flags & DL_TOPK_NO_WAIT) ? 0 : DENSE_SPIN_LIMIT, (V + 7) / 8,
+      workspace_bytes >= DenseSplit::bytes(kind, n_rows, cut.parts) && n_rows * cut.parts <= 0x7fffffffLL) {
+    const DenseSplit x(kind, workspace, n_rows, cut.parts, (flags & DL_TOPK_NO_WAIT) ? 0 : DENSE_SPIN_LIMIT, (V + 7) / 8,
                        (int64_t)cut.nt * dense_split_units(logits_dtype, t_dtype));
     if (vec) launch_dense_split_pair<false>(p, x, cut.nt, st);
     else launch_dense_split_any(p, x, cut.nt, st);

@@ -115,6 +115,32 @@ __device__ __forceinline__ float dense_grad_column(float lp, float lq, float c, 
   return pr * fmaf(log_ratio_to_mixture(lp, fast_log2(0.5f * pr + 0.5f * fast_exp2(lq))), kb, k0);
 }
 
+// This thread's share of the JSD sums KL(P || M), KL(Q || M) (log2), given the row's normalisers; STASH as below.
+template <bool STASH, class Rows>
+__device__ __forceinline__ void dense_jsd_sums(Rows& rows, const DenseStats& st, float& x, float& y) {
+  const float a_s = st.a_s, a_t = st.a_t;
+  if constexpr (STASH) {
+    rows.sweep_rewrite([&](int64_t, float* s, float* t, auto n) {
+#pragma unroll
+      for (int e = 0; e < decltype(n)::value; ++e) {
+        const float lp = fmaf(s[e], a_s, -st.ls), lq = fmaf(t[e], a_t, -st.lt);
+        const float pr = fast_exp2(lp), q = fast_exp2(lq);
+        const float lm = fast_log2(0.5f * pr + 0.5f * q);
+        const float d = log_ratio_to_mixture(lp, lm);       // finite: pr = 0 then gives a gradient of 0
+        x = fmaf(pr, d, x);
+        y = fmaf(q, log_ratio_to_mixture(lq, lm), y);
+        s[e] = pr;
+        t[e] = d;
+      }
+    });
+  } else {
+    rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
+#pragma unroll
+      for (int e = 0; e < decltype(n)::value; ++e) jsd_term(fmaf(s[e], a_s, -st.ls), fmaf(t[e], a_t, -st.lt), x, y);
+    });
+  }
+}
+
 // The sweeps over a row pair held in registers.  `Rows` provides
 //   template <class F> void sweep(F f)       calls f(u, s[8], t[8], Columns<8>{}) for every unit this thread owns
 // (values already unpacked to fp32, -inf beyond the row), possibly f(u, s[1], t[1], Columns<1>{}) for a single column
@@ -231,26 +257,7 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
     return st;
   }
   float x = 0.f, y = 0.f;
-  if constexpr (STASH) {
-    rows.sweep_rewrite([&](int64_t, float* s, float* t, auto n) {
-#pragma unroll
-      for (int e = 0; e < decltype(n)::value; ++e) {
-        const float lp = fmaf(s[e], a_s, -st.ls), lq = fmaf(t[e], a_t, -st.lt);
-        const float pr = fast_exp2(lp), q = fast_exp2(lq);
-        const float lm = fast_log2(0.5f * pr + 0.5f * q);
-        const float d = log_ratio_to_mixture(lp, lm);       // finite: pr = 0 then gives a gradient of 0
-        x = fmaf(pr, d, x);
-        y = fmaf(q, log_ratio_to_mixture(lq, lm), y);
-        s[e] = pr;
-        t[e] = d;
-      }
-    });
-  } else {
-    rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
-#pragma unroll
-      for (int e = 0; e < decltype(n)::value; ++e) jsd_term(fmaf(s[e], a_s, -st.ls), fmaf(t[e], a_t, -st.lt), x, y);
-    });
-  }
+  dense_jsd_sums<STASH>(rows, st, x, y);
   block_sum2<NT>(x, y, red);
   st.loss = 0.5f * LN2 * (x + y);
   st.aux = x * LN2;

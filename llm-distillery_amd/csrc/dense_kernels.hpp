@@ -230,7 +230,7 @@ __global__ __launch_bounds__(NT) void dense_reg_kernel(const DenseParams p) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Forward / reverse KL on rows cut into column parts.  A workgroup that holds a whole pair of rows is
+// Rows cut into column parts.  A workgroup that holds a whole pair of rows is
 // 512 or 1024 threads wide, so one or two of them fill a CU and nothing overlaps their load,
 // arithmetic and store phases.  Here a row pair is cut into P <= 8 parts of 256 (or 512) threads x NU units
 // instead; four (two) parts of different rows share a CU and hide each other's phases, and each part still
@@ -240,8 +240,12 @@ __global__ __launch_bounds__(NT) void dense_reg_kernel(const DenseParams p) {
 // written nothing yet, also when the gradient goes over the logits -- puts itself on a list that a second
 // launch finishes from the then complete records.  Every part combines the records in part order: all parts
 // of a row arrive at the same bits, and so does the second launch.  Parts of a row sit 8 workgroup ids
-// apart, i.e. on one XCD back to back.  JSD is not cut: its divergence needs the row's normalisers inside a
-// logarithm, which would take a second exchange.
+// apart, i.e. on one XCD back to back.
+// JSD needs the row's normalisers inside a logarithm, and the divergence again in its gradient: its parts meet a second
+// time, over (KL(P || M), KL(Q || M)) of their columns, in a second record each.  A part that gave up at either meeting is
+// finished by two launches: the first makes the second records of all listed parts, the second finds every record complete.
+// Against streaming such rows from memory (four scalar passes off the 16-byte grid): 4013 x 98922 bf16 against fp32
+// 3600 -> 897 us, 327 x 125715 fp32 against bf16 428 -> 143 us, 4096 x 128256 bf16 1064 -> 916 us.
 // ---------------------------------------------------------------------------------------
 struct DenseRecord { unsigned ms, mt, ss, st, w, tag, pad0, pad1; };
 constexpr int DENSE_MAX_PARTS = 8;
@@ -249,19 +253,24 @@ constexpr int DENSE_SPIN_LIMIT = 20000;
 
 struct DenseSplit {
   DenseRecord* records;      // n_rows * parts
+  DenseRecord* second;       // JSD: n_rows * parts more, right behind
   unsigned* retry_count;     // then a counter (16 bytes) and n_rows * parts list slots
   unsigned* retry_list;
   int parts;
   int spin_limit;
   int64_t part_units;        // units of 8 columns per part (the last part takes what is left)
-  __host__ __device__ static int64_t bytes(int64_t n_rows, int parts) { return n_rows * parts * (int64_t)(sizeof(DenseRecord) + 4) + 16; }
+  static int64_t n_records(int kind, int64_t n_rows, int parts) { return n_rows * parts * (kind == DL_JSD ? 2 : 1); }
+  static int64_t bytes(int kind, int64_t n_rows, int parts) {
+    return n_records(kind, n_rows, parts) * (int64_t)sizeof(DenseRecord) + n_rows * parts * 4 + 16;
+  }
   // The row is cut evenly, in whole waves of units: a last part that holds a few columns would still take a
   // workgroup, and its partners would wait for it like for a full one.
-  __host__ DenseSplit(void* ws, int64_t n_rows, int parts_, int spin, int64_t units, int64_t most_units) {
+  DenseSplit(int kind, void* ws, int64_t n_rows, int parts_, int spin, int64_t units, int64_t most_units) {
     part_units = ((units + parts_ - 1) / parts_ + 63) / 64 * 64;
     if (part_units > most_units || (parts_ - 1) * part_units >= units) part_units = most_units;
     records = reinterpret_cast<DenseRecord*>(ws);
-    char* base = reinterpret_cast<char*>(ws) + n_rows * parts_ * (int64_t)sizeof(DenseRecord);
+    second = records + n_rows * parts_;
+    char* base = reinterpret_cast<char*>(ws) + n_records(kind, n_rows, parts_) * (int64_t)sizeof(DenseRecord);
     retry_count = reinterpret_cast<unsigned*>(base);
     retry_list = reinterpret_cast<unsigned*>(base + 16);
     parts = parts_;
@@ -301,10 +310,33 @@ __device__ __forceinline__ bool dense_record_collect(DenseRecord* w, int limit, 
   return false;
 }
 
-template <int KIND, class TagS, class TagT, int NT, int NU, bool RETRY, bool ANY>
+// Publishes this part's record `w` (fresh) and collects the others' into xch; false (for every thread alike): a partner did
+// not answer in time, the part has put itself on the list.
+__device__ __forceinline__ bool dense_exchange(const DenseSplit& x, DenseRecord* ws, int64_t r, int h, bool publish, int limit,
+                                               const float (&mine)[5], float (*xch)[DENSE_MAX_PARTS], int* xok) {
+  const int tid = threadIdx.x, P = x.parts;
+  if (tid == 0 && publish) dense_record_publish(ws + h, mine[0], mine[1], mine[2], mine[3], mine[4]);
+  if (tid < P) {
+    float rec[5] = {mine[0], mine[1], mine[2], mine[3], mine[4]};
+    const int ok = (tid == h) || dense_record_collect(ws + tid, limit, rec);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) xch[k][tid] = rec[k];
+    xok[tid] = ok;
+  }
+  __syncthreads();
+  bool all_ok = true;
+  for (int j = 0; j < P; ++j) all_ok = all_ok && (xok[j] != 0);
+  if (!all_ok && tid == 0) x.retry_list[atomicAdd(x.retry_count, 1u)] = (unsigned)(r * P + h);
+  return all_ok;
+}
+
+// RETRY: SPLIT_FIRST the launch over all parts; SPLIT_FINISH over the listed ones, every record complete; SPLIT_SECOND
+// (JSD) over the listed ones before that, up to their second record.
+constexpr int SPLIT_FIRST = 0, SPLIT_FINISH = 1, SPLIT_SECOND = 2;
+
+template <int KIND, class TagS, class TagT, int NT, int NU, int RETRY, bool ANY>
 __device__ __forceinline__ void dense_split_part(const DenseParams& p, const DenseSplit& x, int64_t r, int h, float* red,
                                                  float (*xch)[DENSE_MAX_PARTS], int* xok) {
-  static_assert(KIND == DL_FKL || KIND == DL_RKL, "JSD rows are not cut into parts");
   const int tid = threadIdx.x;
   const int P = x.parts;
   const int64_t u0 = (int64_t)h * x.part_units;                        // first unit of this part
@@ -358,28 +390,15 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
         w += (on && es > 0.f) ? es * (xs - xt) : 0.f;
       } else {
         ss += es;
-        w += et > 0.f ? et * (xt - xs) : 0.f;
+        if (KIND == DL_FKL) w += et > 0.f ? et * (xt - xs) : 0.f;
       }
     }
   });
-  block_sum3<NT>(ss, stt, w, red);
+  if constexpr (KIND == DL_JSD) block_sum2<NT>(ss, stt, red);
+  else block_sum3<NT>(ss, stt, w, red);
 
-  DenseRecord* ws = x.records + r * P;
-  if (tid == 0 && !RETRY) dense_record_publish(ws + h, ms, mt, ss, stt, w);
-  if (tid < P) {
-    float rec[5] = {ms, mt, ss, stt, w};
-    const int ok = (tid == h) || dense_record_collect(ws + tid, RETRY ? 0x7fffffff : x.spin_limit, rec);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) xch[k][tid] = rec[k];
-    xok[tid] = ok;
-  }
-  __syncthreads();
-  bool all_ok = true;
-  for (int j = 0; j < P; ++j) all_ok = all_ok && (xok[j] != 0);
-  if (!all_ok) {
-    if (tid == 0) x.retry_list[atomicAdd(x.retry_count, 1u)] = (unsigned)(r * P + h);
-    return;
-  }
+  const int limit = RETRY == SPLIT_FIRST ? x.spin_limit : 0x7fffffff;
+  if (!dense_exchange(x, x.records + r * P, r, h, RETRY == SPLIT_FIRST, limit, {ms, mt, ss, stt, w}, xch, xok)) return;
   // the row's statistics from the parts', in part order (the same bits in every part)
   float Ms = xch[0][0], Mt = xch[1][0];
   for (int j = 1; j < P; ++j) { Ms = fmaxf(Ms, xch[0][j]); Mt = fmaxf(Mt, xch[1][j]); }
@@ -390,7 +409,7 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
     const float ds = pms == -INFINITY ? 0.f : (Ms - pms) * a_s, dt = pmt == -INFINITY ? 0.f : (Mt - pmt) * a_t;
     const float fs = fast_exp2(-ds), ft = fast_exp2(-dt);
     if (KIND == DL_FKL) W += ft * (pw - (dt - ds) * pst);
-    else W += fs * (pw - (ds - dt) * pss);
+    if (KIND == DL_RKL) W += fs * (pw - (ds - dt) * pss);
     S += pss * fs;
     T += pst * ft;
   }
@@ -399,11 +418,31 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
   const float l2s = fast_log2(S), l2t = fast_log2(T);
   st.ls = (Ms == -INFINITY ? 0.f : Ms * a_s) + l2s;
   st.lt = (Mt == -INFINITY ? 0.f : Mt * a_t) + l2t;
-  st.loss = (KIND == DL_FKL ? W / T - l2t + l2s : W / S - l2s + l2t) * LN2;
-  st.aux = st.loss;
   st.tmax = Mt;
+  if constexpr (KIND == DL_JSD) {
+    float kp = 0.f, kq = 0.f;
+    dense_jsd_sums<Rows::EXACT_STASH>(rows, st, kp, kq);
+    block_sum2<NT>(kp, kq, red);
+    DenseRecord* ws2 = x.second + r * P;
+    if (RETRY == SPLIT_SECOND) {
+      if (tid == 0) dense_record_publish(ws2 + h, kp, kq, 0.f, 0.f, 0.f);
+      return;
+    }
+    __syncthreads();      // the first meeting's records have been read
+    if (!dense_exchange(x, ws2, r, h, RETRY == SPLIT_FIRST, limit, {kp, kq, 0.f, 0.f, 0.f}, xch, xok)) return;
+    float X = 0.f, Y = 0.f;
+    for (int j = 0; j < P; ++j) { X += xch[0][j]; Y += xch[1][j]; }
+    st.loss = 0.5f * LN2 * (X + Y);
+    st.aux = X * LN2;
+  } else {
+    st.loss = (KIND == DL_FKL ? W / T - l2t + l2s : W / S - l2s + l2t) * LN2;
+    st.aux = st.loss;
+  }
   if (tid == 0 && h == 0 && p.row_loss) p.row_loss[r] = st.loss;
-  if (grow) dense_grad_sweep<KIND, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+  if (grow) {
+    if constexpr (KIND == DL_JSD && Rows::EXACT_STASH) dense_jsd_grad_from_stash<TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+    else dense_grad_sweep<KIND, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+  }
 }
 
 template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY>
@@ -416,18 +455,18 @@ void dense_split_kernel(const DenseParams p, const DenseSplit x) {
   const unsigned grp = blockIdx.x / (8u * P), t_in = blockIdx.x % (8u * P);
   const int64_t r = (int64_t)grp * 8 + (t_in & 7u);
   if (r >= p.n_rows) return;
-  dense_split_part<KIND, TagS, TagT, NT, NU, false, ANY>(p, x, r, (int)(t_in >> 3), red, xch, xok);
+  dense_split_part<KIND, TagS, TagT, NT, NU, SPLIT_FIRST, ANY>(p, x, r, (int)(t_in >> 3), red, xch, xok);
 }
 
 // One listed part, as a real call: the loop around it then costs the body no registers.
-template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY>
+template <int KIND, class TagS, class TagT, int NT, int NU, int RETRY, bool ANY>
 __device__ __attribute__((noinline)) void dense_split_part_again(const DenseParams& p, const DenseSplit& x, unsigned at, float* red,
                                                                  float (*xch)[DENSE_MAX_PARTS], int* xok) {
-  dense_split_part<KIND, TagS, TagT, NT, NU, true, ANY>(p, x, (int64_t)(at / (unsigned)x.parts), (int)(at % (unsigned)x.parts), red, xch, xok);
+  dense_split_part<KIND, TagS, TagT, NT, NU, RETRY, ANY>(p, x, (int64_t)(at / (unsigned)x.parts), (int)(at % (unsigned)x.parts), red, xch, xok);
 }
 
 // The parts that gave up waiting, a fixed grid striding over their list (normally empty).
-template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY>
+template <int KIND, class TagS, class TagT, int NT, int NU, int RETRY, bool ANY>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void dense_split_retry_kernel(const DenseParams p, const DenseSplit x) {
   __shared__ float red[64];
@@ -436,7 +475,7 @@ void dense_split_retry_kernel(const DenseParams p, const DenseSplit x) {
   const unsigned n = *x.retry_count;
 #pragma unroll 1
   for (unsigned e = blockIdx.x; e < n; e += gridDim.x) {
-    dense_split_part_again<KIND, TagS, TagT, NT, NU, ANY>(p, x, x.retry_list[e], red, xch, xok);
+    dense_split_part_again<KIND, TagS, TagT, NT, NU, RETRY, ANY>(p, x, x.retry_list[e], red, xch, xok);
     __syncthreads();
   }
 }
@@ -449,28 +488,27 @@ __global__ __launch_bounds__(NT) void dense_clear_kernel(u32x4* ws, int64_t n16)
 
 template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY>
 static void launch_dense_split_kind(const DenseParams& p, const DenseSplit& x, hipStream_t st) {
-  const int64_t n16 = p.n_rows * x.parts * 2 + 1;      // records, then the retry counter
+  const int64_t n16 = DenseSplit::n_records(KIND, p.n_rows, x.parts) * 2 + 1;      // records, then the retry counter
   hipLaunchKernelGGL((dense_clear_kernel<256>), dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st,
                      reinterpret_cast<u32x4*>(x.records), n16);
   hipLaunchKernelGGL((dense_split_kernel<KIND, TagS, TagT, NT, NU, ANY>), dim3((unsigned)((p.n_rows + 7) / 8 * 8 * x.parts)),
                      dim3(NT), 0, st, p, x);
-  hipLaunchKernelGGL((dense_split_retry_kernel<KIND, TagS, TagT, NT, NU, ANY>),
-                     dim3((unsigned)std::min<int64_t>(p.n_rows * x.parts, 256)), dim3(NT), 0, st, p, x);
+  const dim3 again((unsigned)std::min<int64_t>(p.n_rows * x.parts, 256));
+  if constexpr (KIND == DL_JSD)
+    hipLaunchKernelGGL((dense_split_retry_kernel<KIND, TagS, TagT, NT, NU, SPLIT_SECOND, ANY>), again, dim3(NT), 0, st, p, x);
+  hipLaunchKernelGGL((dense_split_retry_kernel<KIND, TagS, TagT, NT, NU, SPLIT_FINISH, ANY>), again, dim3(NT), 0, st, p, x);
+}
+template <class TagS, class TagT, int NT, int NU, bool ANY>
+static void launch_dense_split_nt(const DenseParams& p, const DenseSplit& x, hipStream_t st) {
+  if (p.kind == DL_FKL) launch_dense_split_kind<DL_FKL, TagS, TagT, NT, NU, ANY>(p, x, st);
+  else if (p.kind == DL_RKL) launch_dense_split_kind<DL_RKL, TagS, TagT, NT, NU, ANY>(p, x, st);
+  else launch_dense_split_kind<DL_JSD, TagS, TagT, NT, NU, ANY>(p, x, st);
 }
 template <class TagS, class TagT, int NU, bool ANY>
 static void launch_dense_split(const DenseParams& p, const DenseSplit& x, int nt, hipStream_t st) {
-  if (nt == 256) {
-    if (p.kind == DL_FKL) launch_dense_split_kind<DL_FKL, TagS, TagT, 256, NU, ANY>(p, x, st);
-    else launch_dense_split_kind<DL_RKL, TagS, TagT, 256, NU, ANY>(p, x, st);
-  } else if (nt == 1024) {
-    if constexpr (TagT::bytes == 4 || TagS::bytes == 4) {      // 16-bit pairs reach 262144 columns with parts of 512 threads
-      if (p.kind == DL_FKL) launch_dense_split_kind<DL_FKL, TagS, TagT, 1024, NU, ANY>(p, x, st);
-      else launch_dense_split_kind<DL_RKL, TagS, TagT, 1024, NU, ANY>(p, x, st);
-    }
-  } else {
-    if (p.kind == DL_FKL) launch_dense_split_kind<DL_FKL, TagS, TagT, 512, NU, ANY>(p, x, st);
-    else launch_dense_split_kind<DL_RKL, TagS, TagT, 512, NU, ANY>(p, x, st);
-  }
+  if (nt == 256) launch_dense_split_nt<TagS, TagT, 256, NU, ANY>(p, x, st);
+  else if (nt == 512) launch_dense_split_nt<TagS, TagT, 512, NU, ANY>(p, x, st);
+  else if constexpr (TagT::bytes == 4 || TagS::bytes == 4) launch_dense_split_nt<TagS, TagT, 1024, NU, ANY>(p, x, st);      // 16-bit pairs reach 262144 columns with parts of 512 threads
 }
 template <bool ANY>
 static void launch_dense_split_pair(const DenseParams& p, const DenseSplit& x, int nt, hipStream_t st) {

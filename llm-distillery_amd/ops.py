@@ -187,7 +187,7 @@ def div_dense(kind: str, logits: torch.Tensor, t_logits: torch.Tensor, *, row_ma
               grad_out: torch.Tensor | None = None, split: bool = True, no_wait: bool = False, part_threads: int = 0):
     """Per-token "fkl", "rkl" or "jsd" against a dense teacher [N, V] and, in the same launch,
     d(sum of row losses)/d(logits) * grad_scale.  Returns (row_loss fp32 [rows], grad or None).
-    `split=False` withholds the workspace that lets wide forward / reverse-KL rows be cut into column parts
+    `split=False` withholds the workspace that lets wide rows be cut into column parts
     (dl_div_dense_ws); `no_wait` and `part_threads` (256 / 512 / 1024) are the library's test hooks for those parts
     (DL_TOPK_NO_WAIT, DL_TOPK_PARTS)."""
     if kind not in KINDS:

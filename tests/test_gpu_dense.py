@@ -421,3 +421,42 @@ def test_dense_rows_off_the_grid_in_column_parts(D, kind, dtype, t_dtype, V, thr
     valid[2] = False
     s[0, V - 1] = 60.0                                       # a row whose maximum is its last column
     _check(D, kind, s, t[valid], T=1.3, valid=valid, no_wait=no_wait, part_threads=threads)
+
+
+@pytest.mark.parametrize("dtype,t_dtype,V,threads", [
+    (torch.bfloat16, torch.float32, 98922, 0),       # off the grid, 3 columns behind the last unit
+    (torch.float32, torch.bfloat16, 40003, 256),
+    (torch.float16, torch.float32, 200064, 0),       # parts of 1024 threads
+    (torch.float32, torch.float32, 50257, 0),        # fp32 pairs keep the gradient's ingredients in the registers
+    (torch.float32, torch.float32, 65536, 512),
+    (torch.bfloat16, torch.bfloat16, 70001, 0),
+    (torch.float16, torch.float16, 32776, 256)])     # three parts, the last one shorter
+def test_jsd_rows_cut_into_column_parts(D, dtype, t_dtype, V, threads):
+    """JSD parts meet twice: against the oracle and against one workgroup per row, twice and with parts that wait at neither
+    meeting (two further launches finish them) the same bits, with masked rows, a part without any mass, and the gradient
+    written over the logits."""
+    R = 9
+    s, t = _pair(R, V, dtype, 35, t_dtype, noise=1.5, std=3.0)
+    s[2, V // 2:] = -float("inf")
+    t[2, V // 2:] = -float("inf")
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[[0, 6]] = False
+    _check(D, "jsd", s[valid][:1], t[valid][:1], 1.3, teacher_T=1.0, part_threads=threads)
+    rm = torch.full((R,), -1, dtype=torch.int32)
+    rm[valid] = torch.arange(R - 2, dtype=torch.int32)
+    xs, xt, rm = s.to(DEV), t[valid].to(DEV), rm.to(DEV)
+    kw = dict(row_map=rm, T=1.3, teacher_T=1.0, grad_scale=1.0 / (R - 2), part_threads=threads)
+    assert D._lib.load().dl_div_dense_workspace_bytes(D.ops.KINDS["jsd"], D.ops._DT[dtype], D.ops._DT[t_dtype], R, V) > 0
+    rl, g = D.div_dense("jsd", xs, xt, **kw)
+    rl2, g2 = D.div_dense("jsd", xs, xt, **kw)
+    rl3, g3 = D.div_dense("jsd", xs, xt, no_wait=True, **kw)
+    assert torch.equal(rl, rl2) and torch.equal(g, g2) and torch.equal(rl, rl3) and torch.equal(g, g3)
+    assert torch.isfinite(rl).all() and torch.isfinite(g).all() and torch.count_nonzero(g[2, V // 2:]) == 0
+    assert torch.count_nonzero(rl[~valid.to(DEV)]) == 0 and torch.count_nonzero(g[~valid.to(DEV)]) == 0
+    rl1, g1 = D.div_dense("jsd", xs, xt, split=False, row_map=rm, T=1.3, teacher_T=1.0, grad_scale=1.0 / (R - 2))
+    np.testing.assert_allclose(rl.cpu().numpy(), rl1.cpu().numpy(), rtol=2e-6, atol=1e-7)
+    assert torch.linalg.norm(g.double() - g1.double()) <= 3e-3 * torch.linalg.norm(g1.double())
+    for no_wait in (False, True):
+        y = xs.clone()
+        rl4, g4 = D.div_dense("jsd", y, xt, grad_out=y, no_wait=no_wait, **kw)
+        assert g4.data_ptr() == y.data_ptr() and torch.equal(rl, rl4) and torch.equal(g, y)
