@@ -82,7 +82,8 @@ class BatchIndex:
             row_map[b * S + r] = np.arange(base, base + r.size)
             base += r.size
         self.total = base
-        parts = [row_map] + rows + [c[0] for c in ce] + [c[1] for c in ce]
+        label_flat = [c[0].astype(np.int64) + b * S for b, c in enumerate(ce)]      # the same positions in the batch's tokens seen as one row
+        parts = [row_map] + rows + [c[0] for c in ce] + [c[1] for c in ce] + label_flat
         sizes = [p.size for p in parts]
         host = torch.from_numpy(np.concatenate(parts))
         dev = torch.device(device)
@@ -95,11 +96,17 @@ class BatchIndex:
         self.rows = pieces[1:1 + B]
         self.label_pos = pieces[1 + B:1 + 2 * B]
         self.avoid = pieces[1 + 2 * B:1 + 3 * B]
+        self._label_flat = flat[cuts[1 + 3 * B]:]
+        self._batch = B
         self.seq_len = S
 
     def labels(self, tokens: torch.Tensor) -> list[torch.Tensor]:
         """Cross-entropy labels per conversation from the batch's token ids [B, S]
         (classes/student/model.py:423: `batch_tokenized[i][CE_indices]`)."""
+        if isinstance(tokens, torch.Tensor) and tokens.shape == (self._batch, self.seq_len) and tokens.is_contiguous():
+            # one gather for the batch; the conversations' labels are views of it (a gather each costs more host time
+            # than the loss's own launches on short conversations)
+            return list(tokens.view(-1)[self._label_flat].split([pos.numel() for pos in self.label_pos]))
         return [tokens[b][pos] for b, pos in enumerate(self.label_pos)]
 
 

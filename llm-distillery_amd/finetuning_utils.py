@@ -67,19 +67,20 @@ def _assemble(s_sup: Tensor, t: Tensor, indices: Tensor, labels: Tensor, alpha, 
 
 
 def _packed_rows(tensors) -> Tensor:
-    """The row-wise concatenation of 2-D tensors; no copy when they already lie back to back in
+    """The row-wise concatenation of 2-D (or of 1-D) tensors; no copy when they already lie back to back in
     memory (consecutive slices of one packed tensor, as `teachers_from_outgoing_batch` returns)."""
     if len(tensors) == 1:
         return tensors[0].contiguous()
-    first = tensors[0]
+    live = [t for t in tensors if t.numel()]      # an empty view has no address
+    first = live[0] if live else tensors[0]
     at = first.data_ptr()
-    for t in tensors:
+    for t in live or tensors:
         if not t.is_contiguous() or t.dtype != first.dtype or t.data_ptr() != at or \
                 t.untyped_storage().data_ptr() != first.untyped_storage().data_ptr():
             return torch.cat(tensors, dim=0)
         at += t.numel() * t.element_size()
     rows = sum(t.shape[0] for t in tensors)
-    return torch.as_strided(first, (rows, first.shape[1]), (first.shape[1], 1))
+    return torch.as_strided(first, (rows, *first.shape[1:]), first.stride())
 
 
 def _fusable(counts, labels, alpha) -> bool:
@@ -105,9 +106,9 @@ def _fused_dicts(x: Tensor, row_map, inv_T: float, crop: int, counts, t_vals, t_
     else:
         offs = torch.tensor([[0] + list(_cumsum(counts)), [0] + list(_cumsum(n_lab)), [0] + list(_cumsum(n_avoid))],
                             dtype=torch.int32).to(dev)
-    lab_cat = (torch.cat([lab.to(torch.int64) for lab in labels]) if C > 1 else labels[0].to(torch.int64)).contiguous()
+    lab_cat = _packed_rows([lab.to(torch.int64) for lab in labels])
     if C > 1:
-        avoid_cat = torch.cat([a.to(torch.int64) for a in avoids])
+        avoid_cat = _packed_rows([a.to(torch.int64) for a in avoids])
     else:
         avoid_cat = avoids[0] if avoids[0].dtype in ops._IT else avoids[0].to(torch.int64)
     train, nine = ops.composite_loss(x, _packed_rows(t_vals), _packed_rows(t_idxs), lab_cat, avoid_cat.contiguous(), offs,
@@ -118,6 +119,7 @@ def _fused_dicts(x: Tensor, row_map, inv_T: float, crop: int, counts, t_vals, t_
         d = LossDict(zip(LOSS_KEYS, row.unbind(0)))
         d["train_loss"] = d["custom loss"] = train[c]      # one tensor under both keys, with its graph, as in the reference
         d.packed, d.keys_packed = row, LOSS_KEYS
+        d.batch = (train, nine, c, d["train_loss"], row)
         out.append(d)
     return out
 

@@ -9,9 +9,26 @@ class LossDict(dict):
     """The nine-key dict of one conversation, as `calculate_divergence` returns it, that also remembers
     the one fp32 [9] tensor its values are views of (`packed`, in key order; entry 0 mirrors
     `train_loss` without its graph).  `Losses` then accumulates a conversation with one addition
-    instead of one per key."""
+    instead of one per key.  `batch` = (the train losses [C] and the nine values [C, 9] of all conversations
+    that one call made together, this dict's number among them, its own entries of both)."""
     packed: torch.Tensor | None = None
     keys_packed: tuple = ()
+    batch: tuple | None = None
+
+
+def _whole_batch(dicts):
+    """(train losses [C], nine values [C, 9]) when `dicts` are all the conversations of one call, in order, their train losses
+    untouched: the same sums as from the stacked entries, without a stack of views whose backward fills and adds a [C] tensor
+    per conversation.  None where an entry was replaced, or carries a hook or keeps its gradient."""
+    first = getattr(dicts[0], "batch", None)
+    if first is None or first[1].shape[0] != len(dicts):
+        return None
+    for c, d in enumerate(dicts):
+        b = getattr(d, "batch", None)
+        if b is None or b[0] is not first[0] or b[2] != c or d.get("train_loss") is not b[3] or d.packed is not b[4] \
+                or b[3]._backward_hooks or b[3].retains_grad:
+            return None
+    return first[0], first[1]
 
 
 class Losses:
@@ -113,8 +130,14 @@ class Losses:
         self.num_steps_accumulated += len(batch_losses) - 1  # add_losses counts the last one
         if all(getattr(d, "packed", None) is not None for d in batch_losses):
             summed = LossDict()
-            summed.packed = torch.stack([d.packed for d in batch_losses]).sum(0)
             summed.keys_packed = batch_losses[0].keys_packed
+            whole = _whole_batch(batch_losses)
+            if whole is not None:
+                summed.packed = whole[1].sum(0)
+                summed["train_loss"] = whole[0].sum(0)
+                self.add_losses(summed)
+                return
+            summed.packed = torch.stack([d.packed for d in batch_losses]).sum(0)
             if "train_loss" in keys:
                 summed["train_loss"] = torch.stack([d["train_loss"] for d in batch_losses]).sum(0)
             else:
@@ -135,6 +158,11 @@ class Losses:
         if self.logger is None:
             return
         prefix = "Val Loss" if self.validation else "Loss"
+        if average and self._packed is not None:      # one division for all keys
+            shown = (self._packed / self.num_steps_accumulated).unbind(0)
+            for key, value in zip(self._packed_keys[1:], shown[1:]):
+                self.logger.log({f"{prefix}/{key}": value}, step=step)
+            return
         for key, value in self._view().items():
             if key == "train_loss":
                 continue

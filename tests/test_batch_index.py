@@ -96,3 +96,17 @@ def test_teachers_from_outgoing_batch_drops_the_zero_padding():
     assert np.array_equal(wide[1][0].numpy(), padded[1, :9])
     with pytest.raises(ValueError):
         BI.teachers_from_outgoing_batch(padded, ids, [5, 10, 1], "cpu")
+
+
+def test_labels_of_the_whole_batch_in_one_gather():
+    """The one gather over contiguous tokens and the gather per conversation (other strides or lengths) give the same labels."""
+    import torch
+    from llm_distillery_amd.batch_index import BatchIndex
+    ranges, lengths, S = [[(1, 6), (8, 15)], [(0, 3)], [(2, 20)]], [16, 4, 20], 20
+    index = BatchIndex(ranges, lengths, S, S, "cpu")
+    tokens = torch.arange(3 * S).view(3, S) * 7
+    one = index.labels(tokens)
+    each = index.labels(torch.cat([tokens, tokens], 1)[:, :S])
+    longer = index.labels(torch.cat([tokens, tokens], 1).contiguous())
+    assert len(one) == 3 and all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(one, each, longer))
+    assert all(torch.equal(a, tokens[b][p]) for b, (a, p) in enumerate(zip(one, index.label_pos)))

@@ -245,3 +245,55 @@ def test_product_code_never_imports_the_oracle():
             if f.endswith((".py", ".hip", ".hpp", ".cpp", ".h")):
                 text = open(os.path.join(dirpath, f)).read()
                 assert "oracle" not in text.lower() or f == "synthetic.py", f"{f} mentions the oracle"
+
+
+def test_losses_of_a_whole_batch_are_summed_without_their_views():
+    """Dicts that one call made together: the same totals, logged values and gradients as one by one, also where one of them was
+    scaled in place; a hook on an entry still runs, a replaced entry still counts, a part of the batch is summed as before."""
+    from llm_distillery_amd.losses import LossDict
+    keys = tuple(D.finetuning_utils.LOSS_KEYS) if hasattr(D, "finetuning_utils") else ("train_loss", "custom loss", "CE loss")
+
+    def make():
+        leaf = torch.arange(1.0, 5.0, requires_grad=True)
+        train = leaf * leaf
+        nine = torch.arange(4.0 * len(keys)).view(4, len(keys))
+        out = []
+        for c in range(4):
+            row = nine[c]
+            d = LossDict(zip(keys, row.unbind(0)))
+            d["train_loss"] = train[c]
+            d.packed, d.keys_packed, d.batch = row, keys, (train, nine, c, d["train_loss"], row)
+            out.append(d)
+        return leaf, out
+
+    def plain(mutate=lambda o: None, pick=slice(None)):
+        leaf, out = make()
+        mutate(out)
+        L = D.Losses(None)
+        for d in out[pick]:
+            L.add_losses(d)
+        view = {k: v.clone() for k, v in L._view().items()}
+        L.backward(2)
+        return leaf.grad, view
+
+    def batch(mutate=lambda o: None, pick=slice(None)):
+        leaf, out = make()
+        mutate(out)
+        L = D.Losses(None)
+        L.add_batch(out[pick])
+        view = {k: v.clone() for k, v in L._view().items()}
+        L.backward(2)
+        return leaf.grad, view
+
+    def scale(out):
+        out[1]["train_loss"].mul_(3.0)
+
+    def replace(out):
+        out[2]["train_loss"] = out[2]["train_loss"] * 5.0
+
+    seen = []
+    for mutate, pick in ((lambda o: None, slice(None)), (scale, slice(None)), (replace, slice(None)), (lambda o: None, slice(1, 4)),
+                         (lambda o: o[0]["train_loss"].register_hook(lambda g: seen.append(1) or g * 10.0), slice(None))):
+        (ga, va), (gb, vb) = plain(mutate, pick), batch(mutate, pick)
+        assert torch.equal(ga, gb) and set(va) == set(vb) and all(torch.allclose(va[k], vb[k]) for k in va)
+    assert len(seen) == 2
