@@ -75,13 +75,9 @@ __device__ __forceinline__ float plan_tile_value(const float* tile, unsigned byt
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(tile) + byte_offset);
 }
 
-// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows that start on any element and end inside a 16-byte
-// unit (an odd vocabulary: no pitch keeps its rows on the 16-byte grid), for the planned form only.  Such a row is
-// still moved 16 bytes at a time -- global memory takes unaligned 16-byte loads -- and the unit its last 1-3
-// elements fall into is loaded as the row's last 16 bytes and shifted into place on its way to LDS.  Measured: 7067 rows x
-// 151665 probabilities onto 10352 ids 6.39 -> 1.12 ms, 457 rows onto 32000 ids 478 -> 91 us (on the grid: 1.00 ms for
-// the former; the LDS-atomic form such rows fell back to runs at one
-// lane per three cycles).
+// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows of whole 16-byte units that start on any element, for the
+// planned form only: the same loads, unaligned.  Rows that end inside a unit take the scalar form: with the row's
+// last 16 bytes shifted into place on their way to LDS its last 1-3 elements came out wrong for some plans (16387 ids).
 enum MargLoad : int { MARG_SCALAR = 0, MARG_VEC = 1, MARG_ANY = 2 };
 
 // Marginal of one teacher row into marg[0, Vs) (LDS, zeroed here) along a plan; `tile` is LDS
@@ -159,25 +155,8 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   // in flight and never has to drain the whole queue.  What a clamped load brings is never used: no
   // entry points behind the end of the row, and a select on the value here would make the thread
   // wait for the load right away instead of two tiles later.
-  const int rem = LOAD == MARG_ANY ? (int)(p.Vt & 3) : 0;               // elements of the row's last, partial unit
-  const int last_unit = (int)(n4 - (int64_t)(ntiles - 1) * q_tile);     // its number inside the last tile
   u32x4 tbuf[2][2];
   auto fetch_tile = [&](int k, u32x4 (&buf)[2]) {
-    if constexpr (LOAD == MARG_ANY) {
-      const bool in_row = k < ntiles;
-      const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
-      const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int c = u * MARG_NT + tid;
-        int off = (c < q_tile && c < left) ? c * 16 : 0;
-        // a tile of fewer than four elements has no whole unit of its own: the row's first one stands in
-        if (in_row && left == 0) off = -(int)((int64_t)k * TS * 4);
-        if (rem && k == ntiles - 1 && c == left) off = (c * 4 + rem - 4) * 4;      // the row's last 16 bytes (Vt >= 4)
-        buf[u] = load16_stream_any(base + off);
-      }
-      return;
-    }
     const bool in_row = k < ntiles;
     const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
     const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;      // 16-byte units from the tile's start to the row's end
@@ -185,7 +164,8 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
     for (int u = 0; u < 2; ++u) {
       const int c = u * MARG_NT + tid;
       const unsigned off = (c < q_tile && c < left) ? (unsigned)c * 16u : 0u;
-      buf[u] = load16_stream(base + off);
+      if constexpr (LOAD == MARG_ANY) buf[u] = load16_stream_any(base + off);
+      else buf[u] = load16_stream(base + off);
     }
   };
   // the constant address space tells the compiler that nothing in this kernel writes the offsets:
@@ -226,14 +206,6 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   float run = 0.f;
   auto do_tile = [&](int k, u32x4 (&buf)[2], PlanBatch& e, PlanBatch& e_next) {
     __syncthreads();                                 // previous tile fully consumed (first pass: marg zeroed)
-    if (LOAD == MARG_ANY && rem && k == ntiles - 1) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u)
-        if (u * MARG_NT + tid == last_unit) {
-          const u32x4 v = buf[u];
-          buf[u] = rem == 1 ? u32x4{v[3], 0u, 0u, 0u} : rem == 2 ? u32x4{v[2], v[3], 0u, 0u} : u32x4{v[1], v[2], v[3], 0u};
-        }
-    }
 #pragma unroll
     for (int u = 0; u < 2; ++u)
       if (u * MARG_NT + tid < q_tile) *reinterpret_cast<u32x4*>(tile + ((int64_t)u * MARG_NT + tid) * 4) = buf[u];
@@ -853,7 +825,7 @@ static int marg_load_of(const void* probs, int p_dtype, int64_t p_stride, int64_
   using namespace dl;
   if (p_dtype != DL_F32) return MARG_SCALAR;
   if (Vt % 4 == 0 && ok16(probs, p_stride, 4) && ok16(t2s, 0, 4)) return MARG_VEC;
-  return Vt >= 4 && reinterpret_cast<uintptr_t>(probs) % 4 == 0 ? MARG_ANY : MARG_SCALAR;
+  return Vt % 4 == 0 && reinterpret_cast<uintptr_t>(probs) % 4 == 0 ? MARG_ANY : MARG_SCALAR;
 }
 
 // Fills the plan fields of `p` if a usable plan is given; returns the dynamic LDS bytes to request.
