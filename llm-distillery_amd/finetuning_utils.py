@@ -75,12 +75,13 @@ def _packed_rows(tensors) -> Tensor:
     first = live[0] if live else tensors[0]
     at = first.data_ptr()
     for t in live or tensors:
-        if not t.is_contiguous() or t.dtype != first.dtype or t.data_ptr() != at or \
+        if not t.is_contiguous() or t.dtype != first.dtype or t.shape[1:] != first.shape[1:] or t.data_ptr() != at or \
                 t.untyped_storage().data_ptr() != first.untyped_storage().data_ptr():
             return torch.cat(tensors, dim=0)
         at += t.numel() * t.element_size()
     rows = sum(t.shape[0] for t in tensors)
-    return torch.as_strided(first, (rows, *first.shape[1:]), first.stride())
+    # strides from the shape: a tensor of one row counts as contiguous whatever its own row stride is
+    return torch.as_strided(first, (rows, *first.shape[1:]), (first.shape[1], 1) if first.dim() == 2 else (1,))
 
 
 def _fusable(counts, labels, alpha) -> bool:

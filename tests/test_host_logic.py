@@ -297,3 +297,20 @@ def test_losses_of_a_whole_batch_are_summed_without_their_views():
         (ga, va), (gb, vb) = plain(mutate, pick), batch(mutate, pick)
         assert torch.equal(ga, gb) and set(va) == set(vb) and all(torch.allclose(va[k], vb[k]) for k in va)
     assert len(seen) == 2
+
+
+def test_packed_rows_of_one_row_slices():
+    """One-row slices of a wider tensor count as contiguous whatever their row stride is: the concatenation is torch.cat's, also
+    where the slices lie back to back, for 2-D rows (teachers) and 1-D entries (labels, ignore lists), with empty ones between."""
+    from llm_distillery_amd.finetuning_utils import _packed_rows
+    full = torch.arange(5 * 2 * 4).view(5, 2, 4)
+    tok = torch.arange(10).view(5, 2)
+    wide = torch.arange(12).view(1, 3, 4)
+    row = torch.arange(24).view(6, 4)
+    for parts in ([full[0:1, 0], full[0:1, 1]], [full[1:2, 0], full[1:2, 1], full[2:3, 0]], [wide[:, c] for c in range(3)],
+                  [tok[2:3, 0], tok[2:3, 1]], [tok[0:1, 1], tok[1:2, 0], tok[3:3, 0]], [tok[0:0, 0], tok[1:2, 0], tok[1:2, 1]],
+                  [row[0:2], row[2:3], row[3:6]], [row[0:2], row[3:4]], [full[0:2, 0], full[0:2, 1]]):
+        assert torch.equal(_packed_rows(parts), torch.cat(parts))
+    assert _packed_rows([row[0:2], row[2:6]]).data_ptr() == row.data_ptr()      # and no copy where none is needed
+    with pytest.raises(RuntimeError):
+        _packed_rows([row[0:1], row.view(-1)[4:10].view(2, 3)])                 # other widths are no rows of one tensor
