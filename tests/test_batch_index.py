@@ -110,3 +110,20 @@ def test_labels_of_the_whole_batch_in_one_gather():
     longer = index.labels(torch.cat([tokens, tokens], 1).contiguous())
     assert len(one) == 3 and all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(one, each, longer))
     assert all(torch.equal(a, tokens[b][p]) for b, (a, p) in enumerate(zip(one, index.label_pos)))
+
+
+def test_labels_behind_the_sequence_are_refused():
+    """A conversation cut at the sequence length whose announced length goes on has its last label behind the sequence: an
+    IndexError, for whichever conversation it is, not the next conversation's first token; tokens that hold it give it."""
+    import torch
+    from llm_distillery_amd.batch_index import BatchIndex
+    tokens, longer = torch.arange(16).view(2, 8), torch.arange(18).view(2, 9)
+    for ranges, lengths in (([[(2, 8)], [(1, 5)]], [12, 8]), ([[(1, 5)], [(2, 8)]], [8, 12]), ([[(0, 3), (4, 8)], [(1, 8)]], [9, 10])):
+        index = BatchIndex(ranges, lengths, 8, 8, "cpu")
+        with pytest.raises(IndexError):
+            index.labels(tokens)
+        with pytest.raises(IndexError):
+            index.labels(torch.cat([tokens, tokens], 1)[:, :8])      # the gather per conversation says the same
+        assert all(torch.equal(a, longer[b][p]) for b, (a, p) in enumerate(zip(index.labels(longer), index.label_pos)))
+    index = BatchIndex([[(2, 8)], [(1, 8)]], [8, 8], 8, 8, "cpu")        # cut where the conversation ends: the label is dropped
+    assert [a.tolist() for a in index.labels(tokens)] == [[3, 4, 5, 6, 7], [10, 11, 12, 13, 14, 15]]
