@@ -9,26 +9,23 @@ class LossDict(dict):
     """The nine-key dict of one conversation, as `calculate_divergence` returns it, that also remembers
     the one fp32 [9] tensor its values are views of (`packed`, in key order; entry 0 mirrors
     `train_loss` without its graph).  `Losses` then accumulates a conversation with one addition
-    instead of one per key.  `batch` = (the train losses [C] and the nine values [C, 9] of all conversations
-    that one call made together, this dict's number among them, its own entries of both)."""
+    instead of one per key."""
     packed: torch.Tensor | None = None
     keys_packed: tuple = ()
-    batch: tuple | None = None
 
 
-def _whole_batch(dicts):
-    """(train losses [C], nine values [C, 9]) when `dicts` are all the conversations of one call, in order, their train losses
-    untouched: the same sums as from the stacked entries, without a stack of views whose backward fills and adds a [C] tensor
-    per conversation.  None where an entry was replaced, or carries a hook or keeps its gradient."""
-    first = getattr(dicts[0], "batch", None)
-    if first is None or first[1].shape[0] != len(dicts):
+def _whole_table(dicts) -> torch.Tensor | None:
+    """The [C, 9] tensor whose rows, all of them and in order, are the `packed` values of `dicts` (the conversations of one
+    call): its sum over the rows needs no stack.  None where they are anything else."""
+    table = dicts[0].packed._base
+    if table is None or table.dim() != 2 or table.shape != (len(dicts), dicts[0].packed.numel()):
         return None
+    step, at = table.stride(0), table.storage_offset()
     for c, d in enumerate(dicts):
-        b = getattr(d, "batch", None)
-        if b is None or b[0] is not first[0] or b[2] != c or d.get("train_loss") is not b[3] or d.packed is not b[4] \
-                or b[3]._backward_hooks or b[3].retains_grad:
+        p = d.packed
+        if p._base is not table or p.dim() != 1 or p.storage_offset() != at + c * step or p.stride(0) != table.stride(1):
             return None
-    return first[0], first[1]
+    return table
 
 
 class Losses:
@@ -131,13 +128,8 @@ class Losses:
         if all(getattr(d, "packed", None) is not None for d in batch_losses):
             summed = LossDict()
             summed.keys_packed = batch_losses[0].keys_packed
-            whole = _whole_batch(batch_losses)
-            if whole is not None:
-                summed.packed = whole[1].sum(0)
-                summed["train_loss"] = whole[0].sum(0)
-                self.add_losses(summed)
-                return
-            summed.packed = torch.stack([d.packed for d in batch_losses]).sum(0)
+            table = _whole_table(batch_losses)
+            summed.packed = (table if table is not None else torch.stack([d.packed for d in batch_losses])).sum(0)
             if "train_loss" in keys:
                 summed["train_loss"] = torch.stack([d["train_loss"] for d in batch_losses]).sum(0)
             else:

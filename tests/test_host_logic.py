@@ -247,7 +247,7 @@ def test_product_code_never_imports_the_oracle():
                 assert "oracle" not in text.lower() or f == "synthetic.py", f"{f} mentions the oracle"
 
 
-def test_losses_of_a_whole_batch_are_summed_without_their_views():
+def test_losses_of_a_whole_batch_equal_one_by_one():
     """Dicts that one call made together: the same totals, logged values and gradients as one by one, also where one of them was
     scaled in place; a hook on an entry still runs, a replaced entry still counts, a part of the batch is summed as before."""
     from llm_distillery_amd.losses import LossDict
@@ -262,7 +262,7 @@ def test_losses_of_a_whole_batch_are_summed_without_their_views():
             row = nine[c]
             d = LossDict(zip(keys, row.unbind(0)))
             d["train_loss"] = train[c]
-            d.packed, d.keys_packed, d.batch = row, keys, (train, nine, c, d["train_loss"], row)
+            d.packed, d.keys_packed = row, keys
             out.append(d)
         return leaf, out
 
@@ -297,6 +297,45 @@ def test_losses_of_a_whole_batch_are_summed_without_their_views():
         (ga, va), (gb, vb) = plain(mutate, pick), batch(mutate, pick)
         assert torch.equal(ga, gb) and set(va) == set(vb) and all(torch.allclose(va[k], vb[k]) for k in va)
     assert len(seen) == 2
+
+
+def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(monkeypatch):
+    """Every conversation's train loss of one call stays in the graph of the batch's sum: a hook or retain_grad() on it works
+    whether it came before or after `add_batch`, an entry may be scaled in place, and the sum can be differentiated with
+    respect to it.  The logged values come from the table of which the dicts hold the rows.  (The launch is stood in for.)"""
+    from llm_distillery_amd import finetuning_utils as FU
+    from llm_distillery_amd.losses import _whole_table
+    nine = torch.arange(4.0 * 9).view(4, 9).clone()
+    monkeypatch.setattr(FU.ops, "composite_loss", lambda x, *_: (x * x, nine))
+    one, none = torch.zeros(1, 2), torch.zeros(0, dtype=torch.long)
+
+    def make(grad=True):
+        leaf = torch.arange(1.0, 5.0, requires_grad=grad)
+        return leaf, FU._fused_dicts(leaf, None, 1.0, 0, [1] * 4, [one] * 4, [one.int()] * 4, [none] * 4, [none] * 4, 1.0, 2.0)
+
+    for after in (False, True):
+        leaf, out = make()
+        assert all(d["train_loss"] is d["custom loss"] for d in out)
+        out[2]["train_loss"].mul_(3.0)
+        L, seen = D.Losses(None), []
+        if after:
+            L.add_batch(out)
+        out[0]["train_loss"].register_hook(lambda g: seen.append(g.item()) or g * 10.0)
+        out[1]["train_loss"].retain_grad()
+        if not after:
+            L.add_batch(out)
+        assert torch.equal(L._packed, nine.sum(0))
+        L.backward(2)
+        assert leaf.grad.tolist() == [10.0, 2.0, 9.0, 4.0] and out[1]["train_loss"].grad.item() == 0.5 and seen == [0.5]
+    _, out = make()
+    L = D.Losses(None)
+    L.add_batch(out)
+    assert torch.autograd.grad(L._train, out[3]["train_loss"])[0].item() == 1.0
+    assert [d["train_loss"].item() for d in make(False)[1]] == [1.0, 4.0, 9.0, 16.0]
+    assert _whole_table(out) is nine                                         # and nothing else is taken for it
+    assert _whole_table(out[:3]) is None and _whole_table(out[::-1]) is None and _whole_table(out[:1] * 4) is None
+    out[1].packed = out[1].packed.clone()
+    assert _whole_table(out) is None
 
 
 def test_packed_rows_of_one_row_slices():
