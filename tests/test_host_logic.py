@@ -316,17 +316,17 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
     for after in (False, True):
         leaf, out = make()
         assert all(d["train_loss"] is d["custom loss"] for d in out)
-        out[2]["train_loss"].mul_(3.0)
         L, seen = D.Losses(None), []
         if after:
             L.add_batch(out)
         out[0]["train_loss"].register_hook(lambda g: seen.append(g.item()) or g * 10.0)
         out[1]["train_loss"].retain_grad()
         if not after:
+            out[2]["train_loss"].mul_(3.0)
             L.add_batch(out)
         assert torch.equal(L._packed, nine.sum(0))
         L.backward(2)
-        assert leaf.grad.tolist() == [10.0, 2.0, 9.0, 4.0] and out[1]["train_loss"].grad.item() == 0.5 and seen == [0.5]
+        assert leaf.grad.tolist() == [10.0, 2.0, 3.0 if after else 9.0, 4.0] and out[1]["train_loss"].grad.item() == 0.5 and seen == [0.5]
     _, out = make()
     L = D.Losses(None)
     L.add_batch(out)
