@@ -366,6 +366,7 @@ __device__ __forceinline__ int bucket_finish(const TopkParams& p, const TopkLds&
       s.z[k] = ok ? load_as_float(row, Tag::id, id) : 0.f;
     }
   }
+  __syncthreads();                                         // every wave's share of the lists is cleared
   for (int k = threadIdx.x; k < nk; k += NT) {
     const int id = s.idx[k];                               // this thread's own store
     if (id >= 0) link_entry<Tag, NT, NCH, ANY>(s, pc, k, id);

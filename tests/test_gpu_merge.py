@@ -272,6 +272,32 @@ def test_bucketed_multi_teacher_on_rows_off_the_grid(D, V, dtype, offset):
         D.fkl_multi_teacher(*args[:3], [0.5, -0.25, 0.75], args[4], **kw)
 
 
+@pytest.mark.parametrize("V,dtype", [(20003, torch.bfloat16), (40003, torch.float32), (131079, torch.float16)])
+def test_prepared_entries_of_the_last_waves_beside_the_chunks(D, V, dtype):
+    """A part's lists are cleared by all of its waves (those of the columns beside its chunks by the first) before any wave
+    links an entry: every teacher's last entries, which the last waves hold, lie on the row's first and last columns and, all on
+    one id, in its first and last chunk."""
+    R, K, n, Vt = 40, 250, 3, 3000
+    g = torch.Generator().manual_seed(V)
+    logits = (torch.randn(R, V, generator=g) * 2).to(dtype)
+    vals, idxs = _teachers(R, K, Vt, n, V)
+    id_map = torch.randint(64, V - 64, (Vt,), generator=g, dtype=torch.int32)
+    idxs = [torch.stack([torch.randperm(Vt - 30, generator=g)[:K] + 30 for _ in range(R)]).int() for _ in range(n)]
+    edges = [0, V - 1, 1, V - 2, 2, V - 3, 3, V - 7, 12, V - 12]
+    for t in range(n):                                   # ids below 30 are every teacher's last ten entries
+        idxs[t][:, K - 10:] = torch.arange(10).int() + 10 * t
+        id_map[10 * t:10 * t + 10] = torch.tensor(edges, dtype=torch.int32)
+    weights = [0.5, 0.3, 0.2]
+    rl, grad = D.fkl_multi_teacher(logits.to(DEV), [v.to(DEV) for v in vals], [i.to(DEV) for i in idxs], weights, id_map.to(DEV),
+                                   grad_scale=1.0 / R)
+    rows64, grad64, _, ids = _oracle_multi(logits, vals, idxs, weights, id_map, 1.0)
+    np.testing.assert_allclose(rl.cpu().double().numpy(), rows64.numpy(), rtol=2e-5, atol=2e-6)
+    rtol = 1e-4 if dtype == torch.float32 else 2e-3
+    bound = O.sparse_gradient_tolerance(grad64 / R, logits, 1.0, ids, dtype, rtol, row_coef=1.0 / R)
+    err = (grad.cpu().double() - grad64 / R).abs()
+    assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+
+
 def test_bucketed_multi_teacher_edge_rows(D):
     """Rows whose entries are all dropped (loss 0, zero gradient), a teacher of weight 0, ids outside
     the teacher vocabulary, int64 ids with fp32 values, no map at all."""
