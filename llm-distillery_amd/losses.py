@@ -14,18 +14,24 @@ class LossDict(dict):
     keys_packed: tuple = ()
 
 
-def _whole_table(dicts) -> torch.Tensor | None:
-    """The [C, 9] tensor whose rows, all of them and in order, are the `packed` values of `dicts` (the conversations of one
-    call): its sum over the rows needs no stack.  None where they are anything else."""
-    table = dicts[0].packed._base
-    if table is None or table.dim() != 2 or table.shape != (len(dicts), dicts[0].packed.numel()):
+def _whole(parts) -> torch.Tensor | None:
+    """The tensor whose entries along its first dimension, all of them and in order, are the tensors `parts` (the values of the
+    conversations of one call): its sum needs no stack.  None where they are anything else."""
+    first = parts[0]
+    whole = first._base
+    if whole is None or whole.shape != (len(parts), *first.shape):
         return None
-    step, at = table.stride(0), table.storage_offset()
-    for c, d in enumerate(dicts):
-        p = d.packed
-        if p._base is not table or p.dim() != 1 or p.storage_offset() != at + c * step or p.stride(0) != table.stride(1):
+    step, at = whole.stride(0), whole.storage_offset()
+    for c, p in enumerate(parts):
+        if p._base is not whole or p.shape != first.shape or p.storage_offset() != at + c * step or p.stride() != whole.stride()[1:]:
             return None
-    return table
+    return whole
+
+
+def _sum(parts) -> torch.Tensor:
+    """Their sum; with a graph always that of the parts themselves, on which the caller may have placed or may yet place marks."""
+    whole = None if any(p.requires_grad for p in parts) else _whole(parts)
+    return (torch.stack(parts) if whole is None else whole).sum(0)
 
 
 class Losses:
@@ -128,10 +134,9 @@ class Losses:
         if all(getattr(d, "packed", None) is not None for d in batch_losses):
             summed = LossDict()
             summed.keys_packed = batch_losses[0].keys_packed
-            table = _whole_table(batch_losses)
-            summed.packed = (table if table is not None else torch.stack([d.packed for d in batch_losses])).sum(0)
+            summed.packed = _sum([d.packed for d in batch_losses])
             if "train_loss" in keys:
-                summed["train_loss"] = torch.stack([d["train_loss"] for d in batch_losses]).sum(0)
+                summed["train_loss"] = _sum([d["train_loss"] for d in batch_losses])
             else:
                 summed[keys[0]] = summed.packed[0]
             self.add_losses(summed)

@@ -304,7 +304,7 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
     whether it came before or after `add_batch`, an entry may be scaled in place, and the sum can be differentiated with
     respect to it.  The logged values come from the table of which the dicts hold the rows.  (The launch is stood in for.)"""
     from llm_distillery_amd import finetuning_utils as FU
-    from llm_distillery_amd.losses import _whole_table
+    from llm_distillery_amd.losses import _whole
     nine = torch.arange(4.0 * 9).view(4, 9).clone()
     monkeypatch.setattr(FU.ops, "composite_loss", lambda x, *_: (x * x, nine))
     one, none = torch.zeros(1, 2), torch.zeros(0, dtype=torch.long)
@@ -331,11 +331,17 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
     L = D.Losses(None)
     L.add_batch(out)
     assert torch.autograd.grad(L._train, out[3]["train_loss"])[0].item() == 1.0
-    assert [d["train_loss"].item() for d in make(False)[1]] == [1.0, 4.0, 9.0, 16.0]
-    assert _whole_table(out) is nine                                         # and nothing else is taken for it
-    assert _whole_table(out[:3]) is None and _whole_table(out[::-1]) is None and _whole_table(out[:1] * 4) is None
-    out[1].packed = out[1].packed.clone()
-    assert _whole_table(out) is None
+    _, plain = make(False)                                                   # a validation call: views of one tensor
+    assert [d["train_loss"].item() for d in plain] == [1.0, 4.0, 9.0, 16.0]
+    plain[1]["train_loss"].mul_(2.0)
+    L = D.Losses(None)
+    L.add_batch(plain)
+    assert L._train.item() == 34.0 and torch.equal(L._packed, nine.sum(0))
+    for parts in ([d.packed for d in out], [d["train_loss"] for d in plain]):
+        assert _whole(parts) is parts[0]._base                               # and nothing else is taken for the whole
+        assert _whole(parts[:3]) is None and _whole(parts[::-1]) is None and _whole(parts[:1] * 4) is None
+        assert _whole(parts[:1] + [parts[1].clone()] + parts[2:]) is None
+    assert _whole([d["train_loss"] for d in out]) is None
 
 
 def test_packed_rows_of_one_row_slices():
