@@ -114,14 +114,11 @@ def _fused_dicts(x: Tensor, row_map, inv_T: float, crop: int, counts, t_vals, t_
         avoid_cat = avoids[0] if avoids[0].dtype in ops._IT else avoids[0].to(torch.int64)
     train, nine = ops.composite_loss(x, _packed_rows(t_vals), _packed_rows(t_idxs), lab_cat, avoid_cat.contiguous(), offs,
                                      row_map, inv_T, inv_T_teacher, alpha, crop)
-    # Several conversations with a graph: the train losses are copied apart by one node, whose backward is one launch (a
-    # view each costs a fill, a copy and an addition per conversation there).
-    apart = torch.unbind_copy(train) if C > 1 and train.requires_grad else [train[c] for c in range(C)]
     out = []
     for c in range(C):
         row = nine[c]
         d = LossDict(zip(LOSS_KEYS, row.unbind(0)))
-        d["train_loss"] = d["custom loss"] = apart[c]      # one tensor under both keys, with its graph, as in the reference
+        d["train_loss"] = d["custom loss"] = train[c]      # one tensor under both keys, with its graph, as in the reference
         d.packed, d.keys_packed = row, LOSS_KEYS
         out.append(d)
     return out

@@ -301,8 +301,8 @@ def test_losses_of_a_whole_batch_equal_one_by_one():
 
 def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(monkeypatch):
     """Every conversation's train loss of one call stays in the graph of the batch's sum: a hook or retain_grad() on it works
-    whether it came before or after `add_batch`, an entry may be scaled in place, and the sum can be differentiated with
-    respect to it.  The logged values come from the table of which the dicts hold the rows.  (The launch is stood in for.)"""
+    whether it came before or after `add_batch`, and the sum can be differentiated with respect to it; scaled in place an
+    entry counts as scaled.  The logged values come from the table of which the dicts hold the rows.  (The launch is stood in for.)"""
     from llm_distillery_amd import finetuning_utils as FU
     from llm_distillery_amd.losses import _whole
     nine = torch.arange(4.0 * 9).view(4, 9).clone()
@@ -322,11 +322,16 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
         out[0]["train_loss"].register_hook(lambda g: seen.append(g.item()) or g * 10.0)
         out[1]["train_loss"].retain_grad()
         if not after:
-            out[2]["train_loss"].mul_(3.0)
             L.add_batch(out)
         assert torch.equal(L._packed, nine.sum(0))
         L.backward(2)
-        assert leaf.grad.tolist() == [10.0, 2.0, 3.0 if after else 9.0, 4.0] and out[1]["train_loss"].grad.item() == 0.5 and seen == [0.5]
+        assert leaf.grad.tolist() == [10.0, 2.0, 3.0, 4.0] and out[1]["train_loss"].grad.item() == 0.5 and seen == [0.5]
+    leaf, out = make()
+    out[2]["train_loss"].mul_(3.0)
+    L = D.Losses(None)
+    L.add_batch(out)
+    L.backward()
+    assert leaf.grad.tolist() == [2.0, 4.0, 18.0, 8.0]
     _, out = make()
     L = D.Losses(None)
     L.add_batch(out)
@@ -341,7 +346,6 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
         assert _whole(parts) is parts[0]._base                               # and nothing else is taken for the whole
         assert _whole(parts[:3]) is None and _whole(parts[::-1]) is None and _whole(parts[:1] * 4) is None
         assert _whole(parts[:1] + [parts[1].clone()] + parts[2:]) is None
-    assert _whole([d["train_loss"] for d in out]) is None
 
 
 def test_packed_rows_of_one_row_slices():
