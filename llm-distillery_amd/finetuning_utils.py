@@ -120,6 +120,7 @@ def _fused_dicts(x: Tensor, row_map, inv_T: float, crop: int, counts, t_vals, t_
         d = LossDict(zip(LOSS_KEYS, row.unbind(0)))
         d["train_loss"] = d["custom loss"] = train[c]      # one tensor under both keys, with its graph, as in the reference
         d.packed, d.keys_packed = row, LOSS_KEYS
+        d.batch = (train, nine, c, d["train_loss"], row)
         out.append(d)
     return out
 

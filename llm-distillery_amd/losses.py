@@ -9,29 +9,24 @@ class LossDict(dict):
     """The nine-key dict of one conversation, as `calculate_divergence` returns it, that also remembers
     the one fp32 [9] tensor its values are views of (`packed`, in key order; entry 0 mirrors
     `train_loss` without its graph).  `Losses` then accumulates a conversation with one addition
-    instead of one per key."""
+    instead of one per key.  `batch` = (the train losses [C] and the nine values [C, 9] of all conversations
+    that one call made together, this dict's number among them, its own entries of both)."""
     packed: torch.Tensor | None = None
     keys_packed: tuple = ()
+    batch: tuple | None = None
 
 
-def _whole(parts) -> torch.Tensor | None:
-    """The tensor whose entries along its first dimension, all of them and in order, are the tensors `parts` (the values of the
-    conversations of one call): its sum needs no stack.  None where they are anything else."""
-    first = parts[0]
-    whole = first._base
-    if whole is None or whole.shape != (len(parts), *first.shape):
+def _whole_batch(dicts):
+    """(train losses [C], nine values [C, 9]) when `dicts` are all the conversations of one call, in order, no entry replaced:
+    the same sums as from the stacked entries, without a stack.  Else None."""
+    first = getattr(dicts[0], "batch", None)
+    if first is None or first[1].shape[0] != len(dicts):
         return None
-    step, at = whole.stride(0), whole.storage_offset()
-    for c, p in enumerate(parts):
-        if p._base is not whole or p.shape != first.shape or p.storage_offset() != at + c * step or p.stride() != whole.stride()[1:]:
+    for c, d in enumerate(dicts):
+        b = getattr(d, "batch", None)
+        if b is None or b[0] is not first[0] or b[2] != c or d.get("train_loss") is not b[3] or d.packed is not b[4]:
             return None
-    return whole
-
-
-def _sum(parts) -> torch.Tensor:
-    """Their sum; with a graph always that of the parts themselves, on which the caller may have placed or may yet place marks."""
-    whole = None if any(p.requires_grad for p in parts) else _whole(parts)
-    return (torch.stack(parts) if whole is None else whole).sum(0)
+    return first[0], first[1]
 
 
 class Losses:
@@ -134,9 +129,14 @@ class Losses:
         if all(getattr(d, "packed", None) is not None for d in batch_losses):
             summed = LossDict()
             summed.keys_packed = batch_losses[0].keys_packed
-            summed.packed = _sum([d.packed for d in batch_losses])
-            if "train_loss" in keys:
-                summed["train_loss"] = _sum([d["train_loss"] for d in batch_losses])
+            whole = _whole_batch(batch_losses)
+            summed.packed = (whole[1] if whole is not None else torch.stack([d.packed for d in batch_losses])).sum(0)
+            if whole is not None and not any(d["train_loss"].requires_grad for d in batch_losses):
+                summed["train_loss"] = whole[0].sum(0)
+            elif "train_loss" in keys:
+                # with a graph the sum is that of the entries themselves: on each the caller may place a hook, retain its
+                # gradient or differentiate with respect to it, before this call or after
+                summed["train_loss"] = torch.stack([d["train_loss"] for d in batch_losses]).sum(0)
             else:
                 summed[keys[0]] = summed.packed[0]
             self.add_losses(summed)

@@ -247,7 +247,7 @@ def test_product_code_never_imports_the_oracle():
                 assert "oracle" not in text.lower() or f == "synthetic.py", f"{f} mentions the oracle"
 
 
-def test_losses_of_a_whole_batch_equal_one_by_one():
+def test_losses_of_a_whole_batch_are_summed_without_their_views():
     """Dicts that one call made together: the same totals, logged values and gradients as one by one, also where one of them was
     scaled in place; a hook on an entry still runs, a replaced entry still counts, a part of the batch is summed as before."""
     from llm_distillery_amd.losses import LossDict
@@ -262,7 +262,7 @@ def test_losses_of_a_whole_batch_equal_one_by_one():
             row = nine[c]
             d = LossDict(zip(keys, row.unbind(0)))
             d["train_loss"] = train[c]
-            d.packed, d.keys_packed = row, keys
+            d.packed, d.keys_packed, d.batch = row, keys, (train, nine, c, d["train_loss"], row)
             out.append(d)
         return leaf, out
 
@@ -304,7 +304,6 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
     whether it came before or after `add_batch`, and the sum can be differentiated with respect to it; scaled in place an
     entry counts as scaled.  The logged values come from the table of which the dicts hold the rows.  (The launch is stood in for.)"""
     from llm_distillery_amd import finetuning_utils as FU
-    from llm_distillery_amd.losses import _whole
     nine = torch.arange(4.0 * 9).view(4, 9).clone()
     monkeypatch.setattr(FU.ops, "composite_loss", lambda x, *_: (x * x, nine))
     one, none = torch.zeros(1, 2), torch.zeros(0, dtype=torch.long)
@@ -342,10 +341,12 @@ def test_marks_on_the_train_losses_of_a_batch_work_before_and_after_adding_it(mo
     L = D.Losses(None)
     L.add_batch(plain)
     assert L._train.item() == 34.0 and torch.equal(L._packed, nine.sum(0))
-    for parts in ([d.packed for d in out], [d["train_loss"] for d in plain]):
-        assert _whole(parts) is parts[0]._base                               # and nothing else is taken for the whole
-        assert _whole(parts[:3]) is None and _whole(parts[::-1]) is None and _whole(parts[:1] * 4) is None
-        assert _whole(parts[:1] + [parts[1].clone()] + parts[2:]) is None
+    _, plain = make(False)
+    plain[0]["train_loss"].requires_grad_()
+    L = D.Losses(None)
+    L.add_batch(plain)
+    L.backward()
+    assert plain[0]["train_loss"].grad.item() == 1.0
 
 
 def test_packed_rows_of_one_row_slices():
