@@ -107,6 +107,11 @@ const char* dl_status_string(int status);
  * each row, provided that logits and gradient rows share their address modulo 16 (the same stride from
  * 16-byte aligned bases, or the gradient written over the logits; reverse KL: any gradient row), and
  * element by element otherwise.
+ * Precision: losses and sums are fp32.  Gradients of two-byte forward-KL rows held in registers are made from
+ * probabilities kept as pre-scaled fp16 (11 significant bits down to 2^-29 of the row part's largest, none below
+ * 2^-39), rounded once more to the gradient's type.  Wider rows (streamed) are not, nor are rows off the 16-byte grid of
+ * 4097 chunks or more that one workgroup holds, where V is a whole number of chunks or no workspace came along for
+ * more than 8192 chunks: those are made in fp32.
  * grad may be the logits buffer itself (same pointer and stride): every kernel holds, or has
  * consumed, what it still needs of a row before it writes there.  The same holds for dl_div_dense
  * and dl_rkl_marginalised, not for dl_rowcoef_grad_topk.

@@ -40,7 +40,7 @@ static int div_topk_checked(int kind, const void* logits, int logits_dtype, int6
                (reinterpret_cast<uintptr_t>(workspace) % 16 == 0) ? workspace : nullptr, 1,
                (flags & DL_TOPK_NO_WAIT) ? 0 : SPIN_LIMIT, flags};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (kind == DL_FKL && !aligned) return launch_fkl_any(logits_dtype, p, workspace_bytes, st);
+  if (kind == DL_FKL && !aligned) return launch_fkl_any(logits_dtype, p, workspace_bytes, st, !on_grid);
   if (kind == DL_FKL)
     return logits_dtype == DL_F32 ? launch_fkl<TagF32, false>(p, workspace_bytes, st)
            : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, false>(p, workspace_bytes, st)

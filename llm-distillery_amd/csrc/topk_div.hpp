@@ -498,7 +498,14 @@ __device__ __forceinline__ void row_stats_streamed(const char* row, int64_t V, f
 // bf16, K = 100, 351 -> 271 us (20008 columns: 265 us), 8192 x 151665 1096 -> 955 us, 4093 x 50257 with a tenth of the
 // rows masked 227 -> 174 us (unaligned accesses from the row's first column and an element-wise last chunk inside the
 // sweeps, with fewer shapes to choose from, before).
-constexpr int ROWS_WHOLE = 0, ROWS_ANY = 1;
+//   ROWS_EXACT  ROWS_ANY that keeps the logits in the registers (KEEP_LOGITS) where the other two leave 16-bit
+//               probabilities there: a second exponential per element, one rounding less, and no probability is lost for being
+//               2^-39 of the row's largest.  For the two-byte rows off the 16-byte grid (base or pitch) that had no other
+//               kernel than the streaming one, which makes every probability in fp32, where now one workgroup of 512 threads or
+//               more holds the row: a whole number of chunks long, or wider than 512 x 16 chunks without a workspace (8192 x
+//               50304 bf16, K = 100, pitch 50307: 386 us streamed, 344 us so, 327 us from 16 bits).  Rows that end inside
+//               a chunk have always had their probabilities held in 16 bits, in two column parts or on the grid.
+constexpr int ROWS_WHOLE = 0, ROWS_ANY = 1, ROWS_EXACT = 2;
 
 // ---------------------------------------------------------------------------------------
 // Forward KL, (part of) a row resident in registers: NT threads x NCH 16-byte chunks per thread.
@@ -512,11 +519,11 @@ constexpr int ROWS_WHOLE = 0, ROWS_ANY = 1;
 // RETRY: second launch over the parts that gave up waiting in the first (see split_retry_list):
 // every record of the row is published by then, so nothing is waited for.
 // MULTI: the row's teachers arrive prepared in buckets (TopkParams::bk), J * NT = cap0 entries in registers.
-// RAG: how the rows lie in memory (ROWS_WHOLE / ROWS_ANY above).
+// RAG: how the rows lie in memory (ROWS_WHOLE / ROWS_ANY / ROWS_EXACT above).
 template <class Tag, int NT, int NCH, bool SPLIT, int J, bool RETRY, bool MULTI, int RAG = ROWS_WHOLE>
 __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds& s, int64_t r, int h) {
   static_assert(!MULTI || J > 0, "the head of a bucket travels in registers");
-  constexpr bool ANY = RAG == ROWS_ANY;
+  constexpr bool ANY = RAG != ROWS_WHOLE, KEEP_LOGITS = RAG == ROWS_EXACT;
   using C = Chunk<Tag>;
   const int tid = threadIdx.x;
   const int P = SPLIT ? p.parts : 1;
@@ -601,9 +608,10 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
   }
   mx = block_max<NT>(mx, s.red);
   // Second sweep: 2^(x a - max a + bias) takes the place of x in the registers; the gradient is
-  // that value times a row constant, so each element costs one exp2, not two.
+  // that value times a row constant, so each element costs one exp2, not two.  (Not with KEEP_LOGITS, see above.)
+  constexpr float BIAS = KEEP_LOGITS ? 0.f : C::stash_bias;
   float mb = (mx == -INFINITY) ? 0.f : mx * a;      // a part that holds only -inf logits: every 2^(.) below is 0, not NaN
-  const float mb_own = mb - C::stash_bias;
+  const float mb_own = mb - BIAS;
   float sm = ANY ? fast_exp2(fmaf(x_rest, a, -mb_own)) : 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
@@ -615,10 +623,10 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
       f[e] = fast_exp2(fmaf(f[e], a, -mb_own));
       sm += f[e];
     }
-    reg[i] = C::stash(f);
+    if constexpr (!KEEP_LOGITS) reg[i] = C::stash(f);
     forget(reg[i]);         // pins the schedule chunk by chunk: no pile-up of unpacked values
   }
-  sm = block_sum<NT>(sm * __builtin_exp2f(-C::stash_bias), s.red);      // exact: a power of two
+  sm = block_sum<NT>(sm * __builtin_exp2f(-BIAS), s.red);      // exact: a power of two
 
   if (SPLIT) {
     // publish this part's statistics, collect the others'
@@ -683,9 +691,15 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
       if (ch < nch) {
         float f[C::N];
         forget(reg[i]);
-        C::unstash(reg[i], f);
+        if constexpr (KEEP_LOGITS) {
+          C::unpack(reg[i], f);
 #pragma unroll
-        for (int e = 0; e < C::N; ++e) f[e] *= kc;
+          for (int e = 0; e < C::N; ++e) f[e] = fast_exp2(fmaf(f[e], a, -b)) * c;
+        } else {
+          C::unstash(reg[i], f);
+#pragma unroll
+          for (int e = 0; e < C::N; ++e) f[e] *= kc;
+        }
         if (mine & (1u << i))
           if (correction_apply<Tag, NT, NCH>(s.head, s.next, s.idx, pc.lob, i, f, mass, value)) repeats |= 1u << i;
         if constexpr (ANY) store16_stream_any(gbody + ch * 16, C::pack(f));
@@ -1052,9 +1066,9 @@ static FklShape fkl_shape(int64_t nch, int bytes, int forced_parts, bool split_o
 }
 
 // MULTI has no streaming form: the caller checks fkl_shape first.
-// RAG = ROWS_ANY: the shapes of whole rows of ceil(V / chunk) chunks.
+// RAG = ROWS_ANY: the shapes of whole rows of ceil(V / chunk) chunks; off_grid: not on the 16-byte grid (ROWS_EXACT).
 template <class Tag, bool MULTI, int RAG = ROWS_WHOLE>
-static int launch_fkl(const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared = false) {
+static int launch_fkl(const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared = false, bool off_grid = false) {
   const int64_t nch = (p.V + Tag::epc - 1) / Tag::epc;
   const int forced = (p.flags >> DL_TOPK_PARTS_SHIFT) & 15;
   const bool fine = !MULTI && (p.flags & DL_TOPK_FINE_PARTS) != 0 &&
@@ -1063,6 +1077,14 @@ static int launch_fkl(const TopkParams& p, int64_t ws_bytes, hipStream_t st, boo
   const FklShape wish = fkl_shape(nch, Tag::bytes, forced, true, fine, !MULTI);
   const bool split_ok = p.workspace && ws_bytes >= RetryList::bytes(p.n_rows, wish.parts) && p.n_rows * wish.parts <= 0x7fffffffLL;
   const FklShape sh = wish.parts <= 1 || split_ok ? wish : fkl_shape(nch, Tag::bytes, forced, false, fine, !MULTI);
+  if constexpr (RAG == ROWS_ANY && Tag::bytes == 2) {
+    if (off_grid && sh.parts == 1 && (p.V % Tag::epc == 0 || sh.NT == 1024)) {
+      if constexpr (!MULTI)
+        if (sh.NT == 512 && sh.NCH == 13) return launch_reg<Tag, 512, 13, MULTI, ROWS_EXACT>(p, st);
+      if (sh.NT == 512 && sh.NCH == 16) return launch_reg<Tag, 512, 16, MULTI, ROWS_EXACT>(p, st);
+      if (sh.NT == 1024) return launch_reg<Tag, 1024, 16, MULTI, ROWS_EXACT>(p, st);
+    }
+  }
   switch (sh.NT * 100 + sh.NCH) {
     case 256 * 100 + 4:
       if constexpr (!MULTI)
@@ -1111,8 +1133,8 @@ static int launch_fkl(const TopkParams& p, int64_t ws_bytes, hipStream_t st, boo
 
 // The ROWS_ANY instantiations of launch_fkl live in translation units of their own (topk_div_any.hip,
 // topk_multi_any.hip), so that they compile beside the others.
-int launch_fkl_any(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st);
-int launch_fkl_any_multi(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared);
+int launch_fkl_any(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool off_grid);
+int launch_fkl_any_multi(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared, bool off_grid);
 
 template <class Tag>
 static hipError_t launch_rkl(const TopkParams& p, bool aligned, hipStream_t st) {

@@ -352,7 +352,7 @@ extern "C" int dl_fkl_multi_teacher(const void* logits, int logits_dtype, int64_
       else launch_prep<40, false>(q, st);
     }
   }
-  if (!whole) return launch_fkl_any_multi(logits_dtype, p, plan.exchange_bytes, st, ws_cleared);
+  if (!whole) return launch_fkl_any_multi(logits_dtype, p, plan.exchange_bytes, st, ws_cleared, !on_grid);
   return logits_dtype == DL_F32 ? launch_fkl<TagF32, true>(p, plan.exchange_bytes, st, ws_cleared)
          : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, true>(p, plan.exchange_bytes, st, ws_cleared)
                                    : launch_fkl<TagF16, true>(p, plan.exchange_bytes, st, ws_cleared);

@@ -469,3 +469,38 @@ def test_columns_beside_the_chunks_of_a_part(D, dtype, V):
     err = (grad.cpu().double() - grad64).abs()
     assert (err <= bound).all(), f"worst {(err / bound).max():.2f}"
     assert torch.equal(rl, got[1][0]) and torch.equal(grad, got[1][1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,pitch,offset", [(50304, 50312, 1),      # 512 x 13: whole chunks of columns, off the grid
+                                            (65536, 65537, 0),      # 512 x 16
+                                            (80008, 80013, 0), (100277, 100277, 0)])      # 1024 x 16: without a workspace
+@pytest.mark.parametrize("teachers", [1, 3])
+def test_probabilities_of_wide_rows_off_the_grid_are_rounded_once(D, monkeypatch, dtype, V, pitch, offset, teachers):
+    """Gradients of 16-bit rows that lie off the 16-byte grid and that one workgroup of 512 threads or more holds (whole chunks
+    of columns; without a workspace also wider rows of any length) are made from the logits, not from 16-bit probabilities: one rounding to the gradient's type (half a unit in the last place, and the 1e-5
+    that exponents of up to 64 leave of an fp32 exponential), also for probabilities of 2^-50 of the row's largest."""
+    R, K = 5, 16
+    g = torch.Generator().manual_seed(V + pitch)
+    x = torch.zeros(R, pitch + 8, dtype=dtype, device=DEV)[:, offset:offset + V] if pitch != V else torch.zeros(R, V, dtype=dtype, device=DEV)
+    logits = (torch.randn(R, V, generator=g) * 2).to(dtype)
+    logits[1] = (torch.rand(R, V, generator=g)[1] * -40).to(dtype)
+    logits[1, 70] = 1.0
+    x.copy_(logits.to(DEV))
+    ti = torch.stack([torch.randperm(V, generator=g)[:K] for _ in range(R)]).int()
+    tv = torch.log_softmax(torch.randn(R, K, generator=g), -1).half()
+    scale = float(V) if dtype == torch.float16 else 1.0      # entries of the first row among fp16's normal numbers
+    if teachers == 1:
+        monkeypatch.setattr(D._lib.load(), "dl_div_topk_workspace_bytes", lambda *a: 0)
+        _, grad = D.div_topk("fkl", x, tv.to(DEV), ti.to(DEV), grad_scale=scale)
+    elif V > 65536:
+        pytest.skip("prepared teachers always bring their workspace: column parts")
+    else:
+        _, grad = D.fkl_multi_teacher(x, [tv.to(DEV)] * 3, [ti.to(DEV)] * 3, [0.5, 0.25, 0.25], None, grad_scale=scale)
+    ref = torch.softmax(logits.double(), -1) * scale
+    smallest, bits = (2.0 ** -14, 10) if dtype == torch.float16 else (2.0 ** -126, 7)
+    ulp = torch.exp2(torch.floor(torch.log2(ref)) - bits)
+    dense = torch.ones(R, V, dtype=torch.bool).scatter_(1, ti.long(), False) & (ref > 2 * smallest)
+    assert dense[0].sum() > V // 2 and (dtype == torch.float16 or (dense[1] & (ref[1] < 2.0 ** -50)).any())
+    err = (grad.cpu().double() - ref).abs()
+    assert (err <= 0.5 * ulp + 1e-5 * ref)[dense].all(), (err / ulp)[dense].max()
