@@ -364,3 +364,15 @@ def test_packed_rows_of_one_row_slices():
     assert _packed_rows([row[0:2], row[2:6]]).data_ptr() == row.data_ptr()      # and no copy where none is needed
     with pytest.raises(RuntimeError):
         _packed_rows([row[0:1], row.view(-1)[4:10].view(2, 3)])                 # other widths are no rows of one tensor
+
+
+def test_rows_that_one_workgroup_holds_need_no_workspace():
+    """dl_div_topk_workspace_bytes asks for records where a row is cut into column parts, and only there: not below 8193 chunks of
+    16 bytes, whole or not, however many rows (dl_div_topk_static refuses by this size)."""
+    lib = D._lib.load()
+    size = lambda dtype, rows, V, kind=D.ops.KINDS["fkl"]: lib.dl_div_topk_workspace_bytes(kind, D.ops._DT[dtype], rows, V)
+    for rows in (1, 110000, 1 << 30):
+        assert all(size(torch.bfloat16, rows, V) == 0 for V in (5, 32768, 32769, 50257, 50304, 65535, 65536))
+        assert all(size(torch.float32, rows, V) == 0 for V in (5, 16385, 32767, 32768)) and size(torch.bfloat16, rows, 128256, 1) == 0
+        assert all(size(dt, rows, V) > 16 * rows for dt, V in ((torch.bfloat16, 65537), (torch.bfloat16, 262144), (torch.float32, 32769)))
+    assert size(torch.bfloat16, 1 << 20, 262145) == 0      # too wide to be cut
