@@ -375,7 +375,11 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
     });
     block_max2<NT>(ms, mt, red);
   }
-  // a part that holds no finite logit (a masked stretch of the vocabulary): bias 0 keeps 2^(-inf - bias) = 0
+  // A part that holds no finite logit (a masked stretch of the vocabulary): bias 0 keeps 2^(-inf - bias) = 0.  One masked
+  // with the lowest value of its type or nearly so counts as such: its bias would be infinite or, from 2^31 on, rounded by
+  // more than an exponential can hold.
+  if (ms * a_s < MASKED_BELOW) ms = -INFINITY;
+  if (mt * a_t < MASKED_BELOW) mt = -INFINITY;
   const float bs = ms == -INFINITY ? 0.f : ms * a_s, bt = mt == -INFINITY ? 0.f : mt * a_t;
   float ss = 0.f, stt = 0.f, w = 0.f;
   rows.sweep([&](int64_t, const float* s, const float* t, auto n) {
@@ -405,11 +409,13 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
   float S = 0.f, T = 0.f, W = 0.f;
   for (int j = 0; j < P; ++j) {
     const float pms = xch[0][j], pmt = xch[1][j], pss = xch[2][j], pst = xch[3][j], pw = xch[4][j];
-    // shifts of the part's biases to the row's (log2 domain, >= 0); a part without a finite maximum summed nothing on that side
-    const float ds = pms == -INFINITY ? 0.f : (Ms - pms) * a_s, dt = pmt == -INFINITY ? 0.f : (Mt - pmt) * a_t;
-    const float fs = fast_exp2(-ds), ft = fast_exp2(-dt);
-    if (KIND == DL_FKL) W += ft * (pw - (dt - ds) * pst);
-    if (KIND == DL_RKL) W += fs * (pw - (ds - dt) * pss);
+    // shifts of the part's biases to the row's (log2 domain; >= 0 but for a part without a finite maximum, whose bias is 0 and
+    // which summed nothing on that side)
+    const float ds = pms == -INFINITY ? Ms * a_s : (Ms - pms) * a_s, dt = pmt == -INFINITY ? Mt * a_t : (Mt - pmt) * a_t;
+    const float fs = pms == -INFINITY ? 0.f : fast_exp2(-ds), ft = pmt == -INFINITY ? 0.f : fast_exp2(-dt);
+    // (a part whose mass is nothing to the row's adds nothing, whatever the other side's logits are there)
+    if (KIND == DL_FKL && ft > 0.f) W += ft * (pw - (dt - ds) * pst);
+    if (KIND == DL_RKL && fs > 0.f) W += fs * (pw - (ds - dt) * pss);
     S += pss * fs;
     T += pst * ft;
   }

@@ -460,3 +460,41 @@ def test_jsd_rows_cut_into_column_parts(D, dtype, t_dtype, V, threads):
         y = xs.clone()
         rl4, g4 = D.div_dense("jsd", y, xt, grad_out=y, no_wait=no_wait, **kw)
         assert g4.data_ptr() == y.data_ptr() and torch.equal(rl, rl4) and torch.equal(g, y)
+
+
+@pytest.mark.parametrize("kind", ["fkl", "rkl", "jsd"])
+@pytest.mark.parametrize("dtype,t_dtype,V,threads", [(torch.bfloat16, torch.bfloat16, 40000, 256), (torch.bfloat16, torch.bfloat16, 40003, 256),
+                                                     (torch.float32, torch.float32, 33000, 256), (torch.float32, torch.float32, 33001, 256),
+                                                     (torch.float16, torch.float16, 49155, 256), (torch.bfloat16, torch.float32, 49157, 0),
+                                                     (torch.float32, torch.bfloat16, 49160, 512)])
+@pytest.mark.parametrize("T", [1.0, 2.0])
+def test_a_column_part_masked_with_low_finite_values(D, kind, dtype, t_dtype, V, threads, T):
+    """A stretch of the vocabulary wider than a column part, masked with the lowest value of the type or other finite ones
+    instead of -inf, in both rows, in the teacher's alone (forward KL, JSD) or in the student's alone (JSD): what -inf
+    gives there, which is held against the oracle.  (The value times 1 / T overflows at T = 1 and does not at T = 2.)"""
+    values = [v for v in (-3.38e38, -1e30, -2e9, -1e9, -6e4) if dtype != torch.float16 or v == -6e4] + [torch.finfo(dtype).min]
+    sides = {"fkl": ("both", "teacher"), "rkl": ("both",), "jsd": ("both", "teacher", "student")}[kind]
+    rows = [(side, v) for side in sides for v in values]
+    R = len(rows)
+    s, t = _pair(R, V, dtype, V, t_dtype, noise=1.5, std=3.0)
+    s0, t0 = s.clone(), t.clone()
+    a, b = int(0.24 * V), int(0.76 * V)
+    for r, (side, v) in enumerate(rows):
+        if side != "teacher":
+            s[r, a:b], s0[r, a:b] = v, -float("inf")
+        if side != "student":
+            t[r, a:b], t0[r, a:b] = max(v, torch.finfo(t_dtype).min), -float("inf")
+    assert D._lib.load().dl_div_dense_workspace_bytes(D.ops.KINDS[kind], D.ops._DT[dtype], D.ops._DT[t_dtype], R, V) > 0
+    rl0, g0 = D.div_dense(kind, s0.to(DEV), t0.to(DEV), T=T, part_threads=threads)
+    if kind != "jsd":
+        _check(D, kind, s0, t0, T, part_threads=threads)
+    else:                                                # (autograd's gradient of the oracle is NaN where a probability is 0)
+        rows64 = O.DENSE_ROWS[kind](s0.double() / T, t0.double() / T)
+        np.testing.assert_allclose(rl0.cpu().double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+        g1 = D.div_dense(kind, s0.to(DEV), t0.to(DEV), T=T, split=False)[1]
+        assert torch.linalg.norm(g0.double() - g1.double()) <= 3e-3 * torch.linalg.norm(g1.double())
+    for no_wait in (False, True):
+        rl, g = D.div_dense(kind, s.to(DEV), t.to(DEV), T=T, part_threads=threads, no_wait=no_wait)
+        # the parts' sums are those of the -inf masks; a part above the line where it counts as masked adds terms of 2^-80000
+        np.testing.assert_allclose(rl.cpu().numpy(), rl0.cpu().numpy(), rtol=1e-6, err_msg=str(rows))
+        assert torch.isfinite(g).all() and torch.allclose(g.float(), g0.float(), rtol=1e-2 if dtype != torch.float32 else 1e-5, atol=1e-9)
