@@ -610,7 +610,9 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
   // Second sweep: 2^(x a - max a + bias) takes the place of x in the registers; the gradient is
   // that value times a row constant, so each element costs one exp2, not two.  (Not with KEEP_LOGITS, see above.)
   constexpr float BIAS = KEEP_LOGITS ? 0.f : C::stash_bias;
-  float mb = (mx == -INFINITY) ? 0.f : mx * a;      // a part that holds only -inf logits: every 2^(.) below is 0, not NaN
+  // A part that holds only -inf logits, or only masked ones (MASKED_BELOW): every 2^(.) below is 0, not NaN.
+  if (SPLIT && mx * a < MASKED_BELOW) mx = -INFINITY;
+  float mb = (mx == -INFINITY) ? 0.f : mx * a;
   const float mb_own = mb - BIAS;
   float sm = ANY ? fast_exp2(fmaf(x_rest, a, -mb_own)) : 0.f;
 #pragma unroll
@@ -660,7 +662,7 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
 
   if (gpart) {
     const float c = p.inv_T_s * p.grad_scale;
-    const float kc = fast_exp2(mb_own - b) * c;       // stashed value -> gradient
+    const float kc = SPLIT && mx == -INFINITY ? 0.f : fast_exp2(mb_own - b) * c;       // stashed value -> gradient (a masked part's: 0)
     // 16 chunks of 4-byte logits leave no registers for placing the corrections during the sweep
     // (it spills): those shapes write them behind the dense stores instead.
     constexpr bool IN_REGISTERS = !(Tag::bytes == 4 && NCH == 16);

@@ -504,3 +504,29 @@ def test_probabilities_of_wide_rows_off_the_grid_are_rounded_once(D, monkeypatch
     assert dense[0].sum() > V // 2 and (dtype == torch.float16 or (dense[1] & (ref[1] < 2.0 ** -50)).any())
     err = (grad.cpu().double() - ref).abs()
     assert (err <= 0.5 * ulp + 1e-5 * ref)[dense].all(), (err / ulp)[dense].max()
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 128256), (torch.bfloat16, 128251), (torch.float32, 65536), (torch.float32, 65533)])
+@pytest.mark.parametrize("T", [1.0, 2.0])
+@pytest.mark.parametrize("level", [0.0, -300.0])
+def test_a_column_part_masked_with_low_finite_values(D, dtype, V, T, level):
+    """A stretch of the vocabulary wider than a column part masked with the lowest value of the type or other finite ones
+    instead of -inf: the row's loss and gradient are those of the -inf mask, which is held against the oracle; also where the
+    row's other logits lie so low that 2^-(their log-sum-exp) is out of fp32's range."""
+    g = torch.Generator().manual_seed(V)
+    values = [torch.finfo(dtype).min, -3.38e38, -1e30, -2e9, -1e9, -6e4]
+    R, K = len(values), 64
+    logits = (torch.randn(R, V, generator=g) * 3 + level).to(dtype)
+    a, b = int(0.24 * V), int(0.76 * V)
+    logits[:, a:b] = -float("inf")
+    tv, ti = torch.topk(torch.log_softmax(logits.float() + torch.randn(R, V, generator=g), -1), K)
+    tv, ti = tv.half(), ti.int()
+    if level == 0.0:      # (300 apart, loss and log-sum-exp cancel by more than the oracle's tolerance allows)
+        _check(D, "fkl", logits, tv, ti, T=T)
+    rl0, g0 = D.div_topk("fkl", logits.to(DEV), tv.to(DEV), ti.to(DEV), T=T)
+    for r, v in enumerate(values):
+        logits[r, a:b] = v
+    for no_wait in (False, True):
+        rl, grad = D.div_topk("fkl", logits.to(DEV), tv.to(DEV), ti.to(DEV), T=T, no_wait=no_wait)
+        np.testing.assert_allclose(rl.cpu().numpy(), rl0.cpu().numpy(), rtol=1e-6)
+        assert torch.isfinite(grad).all() and torch.equal(grad, g0)
