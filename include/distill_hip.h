@@ -453,9 +453,9 @@ int dl_marginal_plan_build(const int32_t* t2s, int64_t n_teacher, int64_t n_stud
  * p_dtype, marg fp32 [n_rows, Vs]; out_log != 0 stores log(marg) instead).  With a plan
  * (plan_row_off / plan_ent / plan_fold device copies of dl_marginal_plan_build's arrays, plan_tile,
  * plan_n_fold and plan_n_extra its tile, fold count and replica count;
- * fp32 probabilities, 16-byte aligned rows) every sum is added in a fixed order: bit-reproducible.
- * Without (NULL, NULL, 0) it accumulates with LDS floating-point atomics: sums then agree to fp32
- * rounding, not bit for bit.
+ * fp32 probabilities, Vt a multiple of 4) every sum is added in a fixed order: bit-reproducible.
+ * Without (NULL, NULL, 0), and for other probabilities or Vt, it accumulates with LDS floating-point
+ * atomics: sums then agree to fp32 rounding, not bit for bit.
  */
 int dl_marginalise_map(const void* probs, int p_dtype, int64_t p_stride, int64_t n_rows, int64_t Vt,
                        const int32_t* t2s, int64_t Vs,

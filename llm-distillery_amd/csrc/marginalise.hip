@@ -75,9 +75,12 @@ __device__ __forceinline__ float plan_tile_value(const float* tile, unsigned byt
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(tile) + byte_offset);
 }
 
-// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows of whole 16-byte units that start on any element, for the
-// planned form only: the same loads, unaligned.  Rows that end inside a unit take the scalar form: with the row's
-// last 16 bytes shifted into place on their way to LDS its last 1-3 elements came out wrong for some plans (16387 ids).
+// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows of whole 16-byte units that start on any element (a column
+// slice, an odd pitch), for the planned form only: the same loads, unaligned.  Measured, 4000 rows x 152064
+// probabilities onto 32000 ids: 3.71 ms with LDS atomics, which run at one lane per three cycles, 0.62 ms so, as on the
+// grid; 457 x 151664 465 -> 87 us.  Rows that end inside a unit take the scalar form, plan or not (4000 x 151665: 3.70 ms):
+// with the row's last 16 bytes shifted into place on their way to LDS the last 1-3 elements came out wrong for a plan
+// of 16387 ids onto 8192, for a reason that is not known.
 enum MargLoad : int { MARG_SCALAR = 0, MARG_VEC = 1, MARG_ANY = 2 };
 
 // Marginal of one teacher row into marg[0, Vs) (LDS, zeroed here) along a plan; `tile` is LDS

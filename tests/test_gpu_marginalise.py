@@ -419,3 +419,34 @@ def test_planned_forms_on_teacher_rows_off_the_16_byte_grid(D, Vt, shift):
         bound = O.marginal_rkl_gradient_tolerance(grad64, logits, t_logits, rows64, 1.3, 1.3, 1.0 / R, torch.float32, 1e-4)
         err = (grad.cpu().double() - grad64).abs()
         assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+
+
+@pytest.mark.parametrize("Vt,Vs", [(5, 2048), (1023, 2048), (4097, 2048), (8193, 2048), (12290, 2048), (16387, 8192), (20483, 2048),
+                                   (24577, 2048)])
+@pytest.mark.parametrize("shift", [0, 3])
+def test_a_plan_with_teacher_rows_that_end_inside_a_unit(D, Vt, Vs, shift):
+    """Teacher vocabularies that are no multiple of four ids: the last 1-3 probabilities of every row count, also where the last
+    tile of the attached plan holds nothing but those.  The rows end where the buffer ends."""
+    R = 5
+    rng = np.random.default_rng(Vt)
+    t2s = rng.integers(-1, 700, Vt).astype(np.int32)
+    t2s[-3:] = (13, 700, Vs - 1)                     # the last two ids of their own
+    probs = torch.softmax(torch.randn(R, Vt, generator=torch.Generator().manual_seed(Vt)) * 2, -1)
+    buf = torch.zeros(shift + R * Vt, device=DEV)
+    on_gpu = buf[shift:].view(R, Vt)
+    on_gpu.copy_(probs)
+    ref = O.marginalise_map(probs.numpy(), t2s, Vs)
+    logits = torch.randn(R, Vs, generator=torch.Generator().manual_seed(1)) * 2
+    with np.errstate(divide="ignore"):
+        t_logits = O.marginal_to_teacher_logits(torch.tensor(ref))
+    _, rows64, grad64 = O.mean_loss_and_grad("rkl", logits, 1.3, t_logits=t_logits, dtype=torch.float64)
+    for form in ("full", "auto"):
+        plan = _map_in_the_form(D, form, t2s, Vs)
+        got = D.vocab_utils.marginalise(on_gpu, plan=plan, n_student=Vs).cpu().numpy()
+        np.testing.assert_allclose(got, ref, rtol=2e-6, atol=1e-9)
+        assert np.array_equal(got == 0, ref == 0)
+        rl, grad = D.vocab_utils.rkl_marginalised(logits.to(DEV), on_gpu, plan, T=1.3, grad_scale=1.0 / R)
+        np.testing.assert_allclose(rl.cpu().double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+        bound = O.marginal_rkl_gradient_tolerance(grad64, logits, t_logits, rows64, 1.3, 1.3, 1.0 / R, torch.float32, 1e-4)
+        err = (grad.cpu().double() - grad64).abs()
+        assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
