@@ -278,8 +278,12 @@ static int dense_split_units(int s_dtype, int t_dtype) {
 //   * on fewer than 1024 rows the cut pays only from 256 KiB of row pair upwards (one workgroup per row keeps
 //     the CUs busy by itself below that, and has no partners to wait for).
 //   * JSD, whose parts meet twice and have one more launch behind them: a pair that 1024 threads hold stays whole below
-//     1536 rows of 16-bit pairs (1024 x 50304: 102 us whole, 103 cut; 2048: 200 and 184) and 3072 rows of others
-//     (2048 x 20000 fp32: 114 and 116; 4096 x 32000: 327 and 290); a pair that they do not hold is always cut.
+//     1536 rows of 16-bit pairs and 3072 rows of others; a pair that they do not hold is always cut.  At the lines, whole
+//     and cut: 16-bit pairs, 1536 rows of 33000 / 40960 / 50257 / 65536 columns 110 / 126 / 157 / 205 and 106 / 117 / 146 /
+//     169 us (1024 rows: 78 / 85 / 104 / 133 and 80 / 86 / 104 / 119); 3072 rows of 16392 / 24000 / 32768 columns, bf16
+//     against fp32 130 / 175 / 222 and 114 / 143 / 212, fp32 149 / 193 / 245 and 152 / 187 / 225, fp32 against bf16 154 /
+//     200 / 261 and 146 / 180 / 227.  (Mixed pairs gain up to 19 % from 2048 rows on, fp32 pairs up to 7 %, but not at every
+//     width: 2048 x 28000 bf16 against fp32 129 and 132.)
 // `forced_nt` (256 / 512 / 1024, a tuning hook) fixes the thread count and cuts wherever two parts or more come out.
 struct DenseCut { int nt, parts; };
 static DenseCut dense_split_cut(int kind, int s_dtype, int t_dtype, int64_t n_rows, int64_t V, int forced_nt = 0) {
