@@ -36,6 +36,7 @@ struct DenseParams {
 template <class TagS, class TagT, int NT, int NU, bool ANY = false>
 struct RegRows {
   static constexpr bool ONLINE = false;      // sweeps cost no memory traffic: maxima first, then sums
+  static constexpr bool CENTRED = ANY;       // reverse KL: gradient about the mean of the log ratios as they are rounded
   static constexpr bool BLOCKED = TagS::bytes == 4 && TagT::bytes == 4;
   Unit<TagS> s[NU];
   Unit<TagT> t[NU];
@@ -408,14 +409,22 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
   for (int j = 1; j < P; ++j) { Ms = fmaxf(Ms, xch[0][j]); Mt = fmaxf(Mt, xch[1][j]); }
   float S = 0.f, T = 0.f, W = 0.f;
   for (int j = 0; j < P; ++j) {
-    const float pms = xch[0][j], pmt = xch[1][j], pss = xch[2][j], pst = xch[3][j], pw = xch[4][j];
-    // shifts of the part's biases to the row's (log2 domain; >= 0 but for a part without a finite maximum, whose bias is 0 and
-    // which summed nothing on that side)
-    const float ds = pms == -INFINITY ? Ms * a_s : (Ms - pms) * a_s, dt = pmt == -INFINITY ? Mt * a_t : (Mt - pmt) * a_t;
-    const float fs = pms == -INFINITY ? 0.f : fast_exp2(-ds), ft = pmt == -INFINITY ? 0.f : fast_exp2(-dt);
-    // (a part whose mass is nothing to the row's adds nothing, whatever the other side's logits are there)
-    if (KIND == DL_FKL && ft > 0.f) W += ft * (pw - (dt - ds) * pst);
-    if (KIND == DL_RKL && fs > 0.f) W += fs * (pw - (ds - dt) * pss);
+    const float pms = xch[0][j], pmt = xch[1][j], pss = xch[2][j], pst = xch[3][j];
+    // shifts of the part's biases to the row's (log2 domain, >= 0); a part without a finite maximum summed nothing on that
+    // side (and where the other side has mass there, its terms are those of logits below MASKED_BELOW: their bias is nothing to them)
+    float ds, dt;
+    if constexpr (KIND == DL_RKL && Rows::CENTRED) {
+      ds = pms == -INFINITY ? 0.f : Ms * a_s - pms * a_s;
+      dt = pmt == -INFINITY ? 0.f : Mt * a_t - pmt * a_t;
+    } else {
+      ds = pms == -INFINITY ? 0.f : (Ms - pms) * a_s;
+      dt = pmt == -INFINITY ? 0.f : (Mt - pmt) * a_t;
+    }
+    const float fs = fast_exp2(-ds), ft = fast_exp2(-dt);
+    // a part whose mass is nothing to the row's adds nothing, whatever the other side's logits are there
+    const float pw = (KIND == DL_FKL ? ft : fs) > 0.f ? xch[4][j] : 0.f;
+    if (KIND == DL_FKL) W += ft * (pw - (dt - ds) * pst);
+    if (KIND == DL_RKL) W += fs * (pw - (ds - dt) * pss);
     S += pss * fs;
     T += pst * ft;
   }
@@ -442,7 +451,7 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
     st.aux = X * LN2;
   } else {
     st.loss = (KIND == DL_FKL ? W / T - l2t + l2s : W / S - l2s + l2t) * LN2;
-    st.aux = st.loss;
+    st.aux = KIND == DL_RKL && Rows::CENTRED ? rkl_centre(W / S, st, Ms * a_s, Mt * a_t) : st.loss;
   }
   if (tid == 0 && h == 0 && p.row_loss) p.row_loss[r] = st.loss;
   if (grow) {

@@ -498,3 +498,19 @@ def test_a_column_part_masked_with_low_finite_values(D, kind, dtype, t_dtype, V,
         # the parts' sums are those of the -inf masks; a part above the line where it counts as masked adds terms of 2^-80000
         np.testing.assert_allclose(rl.cpu().numpy(), rl0.cpu().numpy(), rtol=1e-6, err_msg=str(rows))
         assert torch.isfinite(g).all() and torch.allclose(g.float(), g0.float(), rtol=1e-2 if dtype != torch.float32 else 1e-5, atol=1e-9)
+
+
+@pytest.mark.parametrize("dtype,t_dtype,V", [(torch.float32, torch.float32, 50257), (torch.float32, torch.float32, 20003),
+                                             (torch.float32, torch.bfloat16, 100277), (torch.float32, torch.float16, 1003)])
+@pytest.mark.parametrize("T", [1.0, 1.5])
+def test_reverse_kl_gradient_rows_off_the_grid_sum_to_nothing(D, dtype, t_dtype, V, T):
+    """sum_j r_j (log ratio_j - mean) is 0 about the mean of the ratios as they are rounded: what is left is the rounding of the
+    mean itself, a sum of a few units in fp32 (2^-22 of it, taken as the root mean square over the rows); about the row's loss it
+    is the rounding of the two normalisers, half a unit in the last place of values of 8 to 32: 2^-20."""
+    R = 64
+    s, t = _pair(R, V, dtype, V, t_dtype)
+    rl, g = D.div_dense("rkl", s.to(DEV), t.to(DEV), T=T)
+    assert (g.double().sum(-1) * T).square().mean().sqrt().item() <= 2.0 ** -22
+    _, rows64, grad64 = O.mean_loss_and_grad("rkl", s, T, t_logits=t, dtype=torch.float64)
+    np.testing.assert_allclose(rl.cpu().double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+    assert torch.linalg.norm(g.cpu().double() - grad64 * R) <= 1e-6 * torch.linalg.norm(grad64 * R)
