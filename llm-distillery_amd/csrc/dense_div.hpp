@@ -186,8 +186,9 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
     const auto carry = [&](float nms, float nmt) {
       const float ds = ms == -INFINITY ? 0.f : (nms - ms) * a_s, dt = mt == -INFINITY ? 0.f : (nmt - mt) * a_t;
       const float fs = fast_exp2(-ds), ft = fast_exp2(-dt);
-      if (KIND == DL_FKL) w = ft * (w - (dt - ds) * stt);
-      if (KIND == DL_RKL) w = fs * (w - (ds - dt) * ss);
+      // (what is nothing on the new bias adds nothing, whatever the other side's logits were there)
+      if (KIND == DL_FKL) w = ft > 0.f ? ft * (w - (dt - ds) * stt) : 0.f;
+      if (KIND == DL_RKL) w = fs > 0.f ? fs * (w - (ds - dt) * ss) : 0.f;
       ss *= fs;
       stt *= ft;
       ms = nms;
@@ -200,6 +201,8 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
         umt = fmaxf(umt, t[e]);
         ums = fmaxf(ums, (KIND == DL_RKL && t[e] == -INFINITY) ? -INFINITY : s[e]);
       }
+      if (ums * a_s < MASKED_BELOW) ums = -INFINITY;      // columns masked with low finite values are no bias to sum on
+      if (umt * a_t < MASKED_BELOW) umt = -INFINITY;
       if (ums > ms || umt > mt) carry(fmaxf(ms, ums), fmaxf(mt, umt));
       const float bs = ms == -INFINITY ? 0.f : ms * a_s, bt = mt == -INFINITY ? 0.f : mt * a_t;
 #pragma unroll

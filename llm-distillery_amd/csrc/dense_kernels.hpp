@@ -377,8 +377,7 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
     block_max2<NT>(ms, mt, red);
   }
   // A part that holds no finite logit (a masked stretch of the vocabulary): bias 0 keeps 2^(-inf - bias) = 0.  One masked
-  // with the lowest value of its type or nearly so counts as such: its bias would be infinite or, from 2^31 on, rounded by
-  // more than an exponential can hold.
+  // with the lowest value of its type or nearly so counts as such (MASKED_BELOW).
   if (ms * a_s < MASKED_BELOW) ms = -INFINITY;
   if (mt * a_t < MASKED_BELOW) mt = -INFINITY;
   const float bs = ms == -INFINITY ? 0.f : ms * a_s, bt = mt == -INFINITY ? 0.f : mt * a_t;

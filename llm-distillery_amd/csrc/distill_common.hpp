@@ -32,10 +32,10 @@ struct TagF16 { static constexpr int id = F16; static constexpr int bytes = 2; s
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float fast_log2(float x) { return __builtin_amdgcn_logf(x); }
 
-// Logits (times inv_T log2 e) below this are taken for masked where a bias is chosen for part of a row only: 2^(x - bias) is
-// then 0 on any bias that the row's other logits give, while on a bias as low as these the rounding of x - bias (2^-24 of
-// it) would reach past the exponents of fp32.
-constexpr float MASKED_BELOW = -0x1p30f;
+// Logits (times inv_T log2 e) below this are taken for masked where a bias is chosen for part of a row only (a column part, a
+// thread's columns so far): 2^(x - bias) is then 0 on any bias that the row's other logits give.  On a bias as low as
+// these the rounding of x - bias, 2^-25 of it, would reach past the exponents of fp32, or the bias be infinite.
+constexpr float MASKED_BELOW = -0x1p31f;
 
 // ---- 16-byte chunk <-> floats -------------------------------------------------
 template <class Tag> struct Chunk;

@@ -56,7 +56,7 @@ __device__ __forceinline__ void rowstats_row(const StatsParams& p, const Composi
   float m = -INFINITY, sm = 0.f;
   const auto one = [&](float f) {
     if (f > m) { sm *= fast_exp2((m - f) * a); m = f; }
-    if (f > -INFINITY) sm += fast_exp2(fmaf(f, a, -m * a));
+    if (f * a > MASKED_BELOW) sm += fast_exp2(fmaf(f, a, -m * a));
   };
   unsigned traw[RECORD ? E : 1];      // the teacher's values as stored, converted behind the sweep: all loads in flight together
   if constexpr (RECORD) {
@@ -157,7 +157,7 @@ __device__ __forceinline__ void rowstats_row(const StatsParams& p, const Composi
       }
       if (cm > m) { sm *= fast_exp2((m - cm) * a); m = cm; }
       const float mb = m * a;
-      if (m > -INFINITY) {
+      if (mb > MASKED_BELOW) {      // nothing but masked columns so far: no bias to sum on
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll

@@ -460,7 +460,7 @@ __device__ __forceinline__ void row_stats_streamed(const char* row, int64_t V, f
   sm = 0.f;
   const auto one = [&](float f) {
     if (f > m) { sm *= fast_exp2((m - f) * a); m = f; }
-    if (f > -INFINITY) sm += fast_exp2(fmaf(f, a, -m * a));
+    if (f * a > MASKED_BELOW) sm += fast_exp2(fmaf(f, a, -m * a));
   };
   if (MODE != 0) {
     const RowSplit<Tag> sp(row, V, MODE == 2);
@@ -473,7 +473,7 @@ __device__ __forceinline__ void row_stats_streamed(const char* row, int64_t V, f
       for (int e = 1; e < C::N; ++e) cm = fmaxf(cm, f[e]);
       if (cm > m) { sm *= fast_exp2((m - cm) * a); m = cm; }
       const float mb = m * a;
-      if (m > -INFINITY) {
+      if (mb > MASKED_BELOW) {
 #pragma unroll
         for (int e = 0; e < C::N; ++e) sm += fast_exp2(fmaf(f[e], a, -mb));
       }
@@ -610,10 +610,19 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
   // Second sweep: 2^(x a - max a + bias) takes the place of x in the registers; the gradient is
   // that value times a row constant, so each element costs one exp2, not two.  (Not with KEEP_LOGITS, see above.)
   constexpr float BIAS = KEEP_LOGITS ? 0.f : C::stash_bias;
-  // A part that holds only -inf logits, or only masked ones (MASKED_BELOW): every 2^(.) below is 0, not NaN.
-  if (SPLIT && mx * a < MASKED_BELOW) mx = -INFINITY;
+  // A part that holds only -inf logits, or only masked ones (MASKED_BELOW; sooner where values are stashed in 16 bits, see
+  // below): every 2^(.) below is 0, not NaN.
+  if (SPLIT && mx * a < (Tag::bytes == 2 ? -0x1p27f : MASKED_BELOW)) mx = -INFINITY;
   float mb = (mx == -INFINITY) ? 0.f : mx * a;
-  const float mb_own = mb - BIAS;
+  float mb_own = mb - BIAS, lift = 0.f;
+  if constexpr (SPLIT && Tag::bytes == 2) {
+    // Where the bias of a part (masked with -1e7, say) is rounded by an exponent or more, up to 2^3 of them, the stashed values
+    // keep clear of fp16's infinity by as much: the part's factor kc of 0 then makes them 0.
+    if (mb < -0x1p20f) {
+      lift = mb * -0x1p-23f;
+      mb_own = mb + lift - BIAS;
+    }
+  }
   float sm = ANY ? fast_exp2(fmaf(x_rest, a, -mb_own)) : 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
@@ -629,6 +638,7 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
     forget(reg[i]);         // pins the schedule chunk by chunk: no pile-up of unpacked values
   }
   sm = block_sum<NT>(sm * __builtin_exp2f(-BIAS), s.red);      // exact: a power of two
+  if constexpr (SPLIT && Tag::bytes == 2) sm *= fast_exp2(lift);
 
   if (SPLIT) {
     // publish this part's statistics, collect the others'

@@ -577,3 +577,30 @@ def test_records_made_at_the_tail_of_phase_one_equal_the_separate_launches(D, dt
         gf, gs = f[5].float(), s_[5].float()
         tol = gs.abs() * (1e-4 if dtype == torch.float32 else 2.0 ** -7) + gs.abs().amax(-1, keepdim=True) * 2e-6
         assert ((gf - gs).abs() <= tol).all(), ((gf - gs).abs() / tol).max()
+
+
+@pytest.mark.parametrize("dtype,V", [(torch.float32, 32000), (torch.bfloat16, 32003), (torch.bfloat16, 128256)])
+@pytest.mark.parametrize("T", [1.0, 2.0])
+def test_logits_masked_with_low_finite_values(D, dtype, V, T):
+    """A vocabulary masked with the lowest value of the type or other low finite ones instead of -inf (its first two thirds, all
+    that many threads of phase 1 have met when they choose their first bias): log-sum-exps and the composite's loss and
+    gradient are those of the -inf mask."""
+    values = [torch.finfo(dtype).min, -1e30, -2e9, -1e9, -6e4, -float("inf")]
+    N, K, b = 12, 40, 2 * V // 3
+    s, _, _, _ = _convo(N, V, K, V, dtype)
+    ti = torch.stack([torch.randperm(V - b, generator=torch.Generator().manual_seed(r))[:K] + b for r in range(N)])
+    tv = torch.log_softmax(torch.randn(N, K, generator=torch.Generator().manual_seed(3)), -1)
+    labels = ti[:N - 1, 0].clone()
+    got = []
+    for v in values:
+        x = s.clone()
+        x[:, :b] = v
+        lse, _ = D.rowstats_topk(x.to(DEV), ti.to(DEV), None, 1.0 / T)
+        np.testing.assert_allclose(lse.cpu().double().numpy(), torch.logsumexp(x.double() / T, -1).numpy(), rtol=2e-6)
+        y = (x.to(DEV) / T).requires_grad_(True)
+        res = D.calculate_divergence(y, tv.to(DEV), ti.to(DEV), labels.to(DEV), 2.0, torch.tensor([3], device=DEV))
+        res["train_loss"].backward()
+        got.append((res["train_loss"].item(), y.grad))
+    for loss, grad in got[:-1]:
+        assert np.isfinite(loss) and abs(loss - got[-1][0]) <= 1e-6 * abs(loss)
+        assert torch.isfinite(grad).all() and torch.linalg.norm(grad.double() - got[-1][1].double()) <= 1e-3 * torch.linalg.norm(got[-1][1].double())

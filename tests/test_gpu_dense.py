@@ -514,3 +514,24 @@ def test_reverse_kl_gradient_rows_off_the_grid_sum_to_nothing(D, dtype, t_dtype,
     _, rows64, grad64 = O.mean_loss_and_grad("rkl", s, T, t_logits=t, dtype=torch.float64)
     np.testing.assert_allclose(rl.cpu().double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
     assert torch.linalg.norm(g.cpu().double() - grad64 * R) <= 1e-6 * torch.linalg.norm(grad64 * R)
+
+
+@pytest.mark.parametrize("kind", ["fkl", "rkl", "jsd"])
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 128256), (torch.float32, 150000)])      # the student's row on the CU; both rows streamed
+@pytest.mark.parametrize("T", [1.0, 2.0])
+def test_streamed_rows_masked_with_low_finite_values(D, kind, dtype, V, T):
+    """Rows swept from memory choose a bias per thread from the columns it has met: where those are all masked with low finite
+    values (the first two thirds of the row), the row's loss and gradient are those of an -inf mask."""
+    values = [torch.finfo(dtype).min, -1e30, -2e9, -1e9, -6e4]
+    R = len(values)
+    s, t = _pair(R, V, dtype, V, noise=1.5, std=3.0)
+    b = 2 * V // 3
+    s[:, :b] = t[:, :b] = -float("inf")
+    rl0, g0 = D.div_dense(kind, s.to(DEV), t.to(DEV), T=T, split=False)
+    if kind != "jsd":
+        _check(D, kind, s, t, T, split=False)
+    for r, v in enumerate(values):
+        s[r, :b] = t[r, :b] = v
+    rl, g = D.div_dense(kind, s.to(DEV), t.to(DEV), T=T, split=False)
+    np.testing.assert_allclose(rl.cpu().numpy(), rl0.cpu().numpy(), rtol=1e-6)
+    assert torch.isfinite(g).all() and torch.allclose(g.float(), g0.float(), rtol=1e-2 if dtype != torch.float32 else 1e-5, atol=1e-9)

@@ -506,7 +506,8 @@ def test_probabilities_of_wide_rows_off_the_grid_are_rounded_once(D, monkeypatch
     assert (err <= 0.5 * ulp + 1e-5 * ref)[dense].all(), (err / ulp)[dense].max()
 
 
-@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 128256), (torch.bfloat16, 128251), (torch.float32, 65536), (torch.float32, 65533)])
+@pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 128256), (torch.bfloat16, 128251), (torch.float32, 65536), (torch.float32, 65533),
+                                     (torch.bfloat16, 300000), (torch.float32, 150003)])      # streamed: threads that have met masked columns only
 @pytest.mark.parametrize("T", [1.0, 2.0])
 @pytest.mark.parametrize("level", [0.0, -300.0])
 def test_a_column_part_masked_with_low_finite_values(D, dtype, V, T, level):
@@ -514,7 +515,7 @@ def test_a_column_part_masked_with_low_finite_values(D, dtype, V, T, level):
     instead of -inf: the row's loss and gradient are those of the -inf mask, which is held against the oracle; also where the
     row's other logits lie so low that 2^-(their log-sum-exp) is out of fp32's range."""
     g = torch.Generator().manual_seed(V)
-    values = [torch.finfo(dtype).min, -3.38e38, -1e30, -2e9, -1e9, -6e4]
+    values = [torch.finfo(dtype).min, -3.38e38, -1e30, -2e9, -1.3e9, -1e9, -7e8, -3e8, -1.1e8, -3.3e7, -1.7e7, -6e4]
     R, K = len(values), 64
     logits = (torch.randn(R, V, generator=g) * 3 + level).to(dtype)
     a, b = int(0.24 * V), int(0.76 * V)
