@@ -73,15 +73,15 @@ def _packed_rows(tensors) -> Tensor:
         return tensors[0].contiguous()
     live = [t for t in tensors if t.numel()]      # an empty view has no address
     first = live[0] if live else tensors[0]
-    at = first.data_ptr()
+    at, base, dim, width = first.data_ptr(), first.untyped_storage().data_ptr(), first.dim(), first.size(-1)
     for t in live or tensors:
-        if not t.is_contiguous() or t.dtype != first.dtype or t.shape[1:] != first.shape[1:] or t.data_ptr() != at or \
-                t.untyped_storage().data_ptr() != first.untyped_storage().data_ptr():
+        if not t.is_contiguous() or t.dtype != first.dtype or t.dim() != dim or (dim == 2 and t.size(-1) != width) or \
+                t.data_ptr() != at or t.untyped_storage().data_ptr() != base:
             return torch.cat(tensors, dim=0)
         at += t.numel() * t.element_size()
     rows = sum(t.shape[0] for t in tensors)
     # strides from the shape: a tensor of one row counts as contiguous whatever its own row stride is
-    return torch.as_strided(first, (rows, *first.shape[1:]), (first.shape[1], 1) if first.dim() == 2 else (1,))
+    return torch.as_strided(first, (rows, width) if dim == 2 else (rows,), (width, 1) if dim == 2 else (1,))
 
 
 def _fusable(counts, labels, alpha) -> bool:
