@@ -610,19 +610,12 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
   // Second sweep: 2^(x a - max a + bias) takes the place of x in the registers; the gradient is
   // that value times a row constant, so each element costs one exp2, not two.  (Not with KEEP_LOGITS, see above.)
   constexpr float BIAS = KEEP_LOGITS ? 0.f : C::stash_bias;
-  // A part that holds only -inf logits, or only masked ones (MASKED_BELOW; sooner where values are stashed in 16 bits, see
-  // below): every 2^(.) below is 0, not NaN.
-  if (SPLIT && mx * a < (Tag::bytes == 2 ? -0x1p27f : MASKED_BELOW)) mx = -INFINITY;
-  float mb = (mx == -INFINITY) ? 0.f : mx * a;
-  float mb_own = mb - BIAS, lift = 0.f;
-  if constexpr (SPLIT && Tag::bytes == 2) {
-    // Where the bias of a part (masked with -1e7, say) is rounded by an exponent or more, up to 2^3 of them, the stashed values
-    // keep clear of fp16's infinity by as much: the part's factor kc of 0 then makes them 0.
-    if (mb < -0x1p20f) {
-      lift = mb * -0x1p-23f;
-      mb_own = mb + lift - BIAS;
-    }
-  }
+  // A part that holds only -inf logits, or only masked ones: every 2^(.) below is 0, not NaN.  (MASKED_BELOW; for two-byte
+  // logits already where the rounding of x a - bias could carry a stashed value past fp16's infinity: they are thousands apart there.)
+  float mb = mx * a;
+  const bool masked = SPLIT ? mb < (Tag::bytes == 2 ? -0x1p20f : MASKED_BELOW) : mx == -INFINITY;
+  if (masked) { mb = 0.f; mx = -INFINITY; }
+  const float mb_own = mb - BIAS;
   float sm = ANY ? fast_exp2(fmaf(x_rest, a, -mb_own)) : 0.f;
 #pragma unroll
   for (int i = 0; i < NCH; ++i) {
@@ -638,7 +631,6 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
     forget(reg[i]);         // pins the schedule chunk by chunk: no pile-up of unpacked values
   }
   sm = block_sum<NT>(sm * __builtin_exp2f(-BIAS), s.red);      // exact: a power of two
-  if constexpr (SPLIT && Tag::bytes == 2) sm *= fast_exp2(lift);
 
   if (SPLIT) {
     // publish this part's statistics, collect the others'
@@ -672,7 +664,7 @@ __device__ __forceinline__ void fkl_topk_part(const TopkParams& p, const TopkLds
 
   if (gpart) {
     const float c = p.inv_T_s * p.grad_scale;
-    const float kc = SPLIT && mx == -INFINITY ? 0.f : fast_exp2(mb_own - b) * c;       // stashed value -> gradient (a masked part's: 0)
+    const float kc = SPLIT && masked ? 0.f : fast_exp2(mb_own - b) * c;       // stashed value -> gradient (a masked part's: 0)
     // 16 chunks of 4-byte logits leave no registers for placing the corrections during the sweep
     // (it spills): those shapes write them behind the dense stores instead.
     constexpr bool IN_REGISTERS = !(Tag::bytes == 4 && NCH == 16);
