@@ -102,8 +102,8 @@ def test_dense_16bit_rows_with_one_towering_logit(D, kind, dtype):
 @pytest.mark.parametrize("in_place", [False, True])
 def test_dense_rows_off_the_16_byte_grid(D, kind, dtype, V, pitch, offset, in_place):
     """Student and teacher rows of one dtype that do not start on 16-byte boundaries or do not end on one
-    stay in the register kernel (unaligned 16-byte accesses, the last, partly filled chunk element by
-    element), with masked rows and the gradient written over the logits."""
+    stay in the register kernel (units from the student row's first 16-byte boundary on, the columns beside
+    them one by one), with masked rows and the gradient written over the logits."""
     R = 6
     s, t = _pair(R, V, dtype, 13)
     valid = torch.ones(R, dtype=torch.bool)
@@ -158,13 +158,14 @@ def test_teacher_with_zero_mass_entries(D, kind):
 
 
 @pytest.mark.parametrize("V,dtype", [(1001, torch.float32), (70000, torch.bfloat16), (50264, torch.float32),
-                                     (128256, torch.bfloat16), (151936, torch.bfloat16), (70000, torch.float32)])
+                                     (128256, torch.bfloat16), (151936, torch.bfloat16), (70000, torch.float32), (70001, torch.bfloat16)])
 def test_dense_rows_beyond_the_register_budget(D, V, dtype):
-    # up to 131072 16-bit / 65536 fp32 columns the student row stays on the CU and the teacher row is
-    # streamed; beyond, both are streamed (multi-pass, 16-byte loads); odd vocabularies take the scalar kernel
+    # in column parts; without a workspace up to 131072 16-bit / 65536 fp32 columns the student row stays on the CU and the
+    # teacher row is streamed, beyond both are streamed (multi-pass, 16-byte loads), and odd vocabularies take the scalar kernel
     s, t = _pair(5, V, dtype, 5)
     for kind in ("fkl", "rkl", "jsd"):
-        _check(D, kind, s, t, T=1.3)
+        for split in (True, False):
+            _check(D, kind, s, t, T=1.3, split=split)
 
 
 @pytest.mark.parametrize("kind", ["fkl", "rkl", "jsd"])

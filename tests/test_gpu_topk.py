@@ -99,20 +99,17 @@ def test_streaming_path_odd_vocab_and_int64_fp32_teacher(D, V):
                                                   (torch.bfloat16, 5001, 5120, 3),          # a column slice of aligned rows: one phase for all rows
                                                   (torch.float16, 7, 7, 0),                 # rows shorter than a chunk
                                                   (torch.float32, 4099, 4104, 2),
-                                                  (torch.bfloat16, 50257, 50257, 0),        # wider than 256 x 16 chunks: two column parts
+                                                  (torch.bfloat16, 50257, 50257, 0),        # wider than 256 x 16 chunks: 512 threads x 13
                                                   (torch.float16, 151665, 151665, 0),       # five
                                                   (torch.float32, 40003, 40003, 0),         # three, of four-byte chunks
                                                   (torch.float32, 10001, 10001, 0)])        # 512 threads x 8 chunks of fp32
 @pytest.mark.parametrize("grad_mode", ["fresh", "in_place", "other_phase"])
 @pytest.mark.parametrize("kind", ["fkl", "rkl"])
 def test_rows_off_the_16_byte_grid(D, kind, dtype, V, pitch, offset, grad_mode):
-    """Rows that do not start on 16-byte boundaries or do not end on one.  Forward KL: rows of up to
-    256 x 16 chunks stay in the register kernels (unaligned 16-byte accesses, the last, partly filled chunk
-    element by element); wider ones stream, their 16-byte chunks through aligned vector accesses when
-    logits and gradient rows share their address modulo 16 (a fresh gradient of the same pitch, or the
-    gradient written over the logits), else through the unaligned register kernel as far as that holds a
-    row.  Reverse KL, which only gathers from the logits, goes by the gradient rows alone.  All against
-    the oracle."""
+    """Rows that do not start on 16-byte boundaries or do not end on one.  Forward KL: the register kernels of rows on the
+    grid, their chunks from the row's first boundary on, the columns beside them one by one, whatever the gradient row's
+    phase (a fresh gradient of the same pitch, the gradient written over the logits, another pitch).  Reverse KL, which
+    only gathers from the logits, goes by the gradient rows alone.  All against the oracle."""
     R, K = 7, min(24, V)
     logits, tv, ti = _case(R, V, K, dtype, 61, std=3.0)
     valid = torch.ones(R, dtype=torch.bool)
@@ -161,8 +158,8 @@ def test_rows_off_the_16_byte_grid(D, kind, dtype, V, pitch, offset, grad_mode):
 def test_crop_of_a_padded_vocabulary(D, dtype, V, pitch, grad_mode):
     """logits[:, :, :crop] of rows padded to a multiple of 16 bytes (classes/student/model.py:408): rows start on
     the 16-byte grid and end inside a chunk.  The register kernels take them like whole rows, one workgroup per
-    row or cut into column parts, and move only the row's last chunk element by element; nothing beyond the crop
-    is written.  A gradient buffer off the grid (other_phase) falls back to the unaligned / streaming kernels.
+    row or cut into column parts, and move only the columns behind the last whole chunk one by one; nothing beyond the crop
+    is written.  A gradient buffer off the grid (other_phase) is written by the same kernels, unaligned.
     With and without waiting for the partners: the oracle's numbers and the same bits."""
     R, K = 11, 48
     logits, tv, ti = _case(R, V, K, dtype, 71, std=3.0)
@@ -472,14 +469,14 @@ def test_columns_beside_the_chunks_of_a_part(D, dtype, V):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("V,pitch,offset", [(50304, 50312, 1),      # 512 x 13: whole chunks of columns, off the grid
-                                            (65536, 65537, 0),      # 512 x 16
-                                            (80008, 80013, 0), (100277, 100277, 0)])      # 1024 x 16: without a workspace
-@pytest.mark.parametrize("teachers", [1, 3])
+@pytest.mark.parametrize("V,pitch,offset,teachers", [(50304, 50312, 1, 1), (50304, 50312, 1, 3),      # 512 x 13: whole chunks of columns, off the grid
+                                                     (65536, 65537, 0, 1), (65536, 65537, 0, 3),      # 512 x 16
+                                                     (80008, 80013, 0, 1), (100277, 100277, 0, 1)])   # 1024 x 16: without a workspace
 def test_probabilities_of_wide_rows_off_the_grid_are_rounded_once(D, monkeypatch, dtype, V, pitch, offset, teachers):
     """Gradients of 16-bit rows that lie off the 16-byte grid and that one workgroup of 512 threads or more holds (whole chunks
-    of columns; without a workspace also wider rows of any length) are made from the logits, not from 16-bit probabilities: one rounding to the gradient's type (half a unit in the last place, and the 1e-5
-    that exponents of up to 64 leave of an fp32 exponential), also for probabilities of 2^-50 of the row's largest."""
+    of columns; without a workspace also wider rows of any length) are made from the logits, not from 16-bit probabilities: one
+    rounding to the gradient's type (half a unit in the last place, and the 1e-5 that exponents of up to 64 leave of an fp32
+    exponential), also for probabilities of 2^-50 of the row's largest."""
     R, K = 5, 16
     g = torch.Generator().manual_seed(V + pitch)
     x = torch.zeros(R, pitch + 8, dtype=dtype, device=DEV)[:, offset:offset + V] if pitch != V else torch.zeros(R, V, dtype=dtype, device=DEV)
@@ -493,8 +490,6 @@ def test_probabilities_of_wide_rows_off_the_grid_are_rounded_once(D, monkeypatch
     if teachers == 1:
         monkeypatch.setattr(D._lib.load(), "dl_div_topk_workspace_bytes", lambda *a: 0)
         _, grad = D.div_topk("fkl", x, tv.to(DEV), ti.to(DEV), grad_scale=scale)
-    elif V > 65536:
-        pytest.skip("prepared teachers always bring their workspace: column parts")
     else:
         _, grad = D.fkl_multi_teacher(x, [tv.to(DEV)] * 3, [ti.to(DEV)] * 3, [0.5, 0.25, 0.25], None, grad_scale=scale)
     ref = torch.softmax(logits.double(), -1) * scale
