@@ -105,9 +105,10 @@ class BatchIndex:
         """Cross-entropy labels per conversation from the batch's token ids [B, S]
         (classes/student/model.py:423: `batch_tokenized[i][CE_indices]`).  Raises IndexError where a label lies
         behind the sequence (a conversation cut at `seq_len` whose length says that it goes on)."""
+        if self._labels_beyond is not None and isinstance(tokens, torch.Tensor) and tokens.shape[-1] <= self.seq_len:
+            # (in the flat gather it would be the next conversation's first token, on the device an assertion)
+            raise IndexError(f"conversation {self._labels_beyond}: a label lies behind the {self.seq_len} tokens of its sequence")
         if isinstance(tokens, torch.Tensor) and tokens.shape == (self._batch, self.seq_len) and tokens.is_contiguous():
-            if self._labels_beyond is not None:      # in the flat gather it would be the next conversation's first token
-                raise IndexError(f"conversation {self._labels_beyond}: a label lies behind the {self.seq_len} tokens of its sequence")
             # one gather for the batch; the conversations' labels are views of it (a gather each costs more host time
             # than the loss's own launches on short conversations)
             return list(tokens.view(-1)[self._label_flat].split([pos.numel() for pos in self.label_pos]))

@@ -499,6 +499,9 @@ def test_probabilities_of_wide_rows_off_the_grid_are_rounded_once(D, monkeypatch
     assert dense[0].sum() > V // 2 and (dtype == torch.float16 or (dense[1] & (ref[1] < 2.0 ** -50)).any())
     err = (grad.cpu().double() - ref).abs()
     assert (err <= 0.5 * ulp + 1e-5 * ref)[dense].all(), (err / ulp)[dense].max()
+    if teachers == 1:                                        # and the same bits written over the logits
+        _, over = D.div_topk("fkl", x, tv.to(DEV), ti.to(DEV), grad_scale=scale, grad_out=x)
+        assert over.data_ptr() == x.data_ptr() and torch.equal(grad, x)
 
 
 @pytest.mark.parametrize("dtype,V", [(torch.bfloat16, 128256), (torch.bfloat16, 128251), (torch.float32, 65536), (torch.float32, 65533),
