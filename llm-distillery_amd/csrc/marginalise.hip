@@ -75,12 +75,12 @@ __device__ __forceinline__ float plan_tile_value(const float* tile, unsigned byt
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(tile) + byte_offset);
 }
 
-// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows of whole 16-byte units that start on any element (a column
-// slice, an odd pitch), for the planned form only: the same loads, unaligned.  Measured, 4000 rows x 152064
-// probabilities onto 32000 ids: 3.71 ms with LDS atomics, which run at one lane per three cycles, 0.62 ms so, as on the
-// grid; 457 x 151664 465 -> 87 us.  Rows that end inside a unit take the scalar form, plan or not (4000 x 151665: 3.70 ms):
-// with the row's last 16 bytes shifted into place on their way to LDS the last 1-3 elements came out wrong for a plan
-// of 16387 ids onto 8192, for a reason that is not known.
+// How a kernel reads the teacher's rows.  MARG_ANY: fp32 rows of at least one 16-byte unit that start on any element (a column
+// slice, an odd pitch) and may end inside a unit, for the planned form only: the same loads, unaligned; the up to three
+// probabilities behind the last whole unit travel one per thread in the first threads and join the last tile in LDS
+// behind its units, at the price of one more barrier per row.  MARG_SCALAR runs LDS atomics, one lane per three cycles: 6432
+// rows x 125857 probabilities onto 32000 ids 5.02 ms with them, 0.96 ms so; 447 x 100277 onto 10528 270 -> 54 us; 4000 x
+// 152064 (whole units off the grid) 3.71 -> 0.62 ms.  Rows shorter than a unit keep the scalar form.
 enum MargLoad : int { MARG_SCALAR = 0, MARG_VEC = 1, MARG_ANY = 2 };
 
 // Marginal of one teacher row into marg[0, Vs) (LDS, zeroed here) along a plan; `tile` is LDS
@@ -151,6 +151,9 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   const int ntiles = (int)((p.Vt + TS - 1) / TS);
   const int64_t n4 = p.Vt / 4;
   const int n_slots = (int)plan_slot_words(p.Vs, p.plan_n_extra);
+  const int rest = LOAD == MARG_ANY ? (int)(p.Vt - n4 * 4) : 0;       // probabilities behind the last whole unit
+  float p_rest = 0.f;
+  if (LOAD == MARG_ANY && tid < rest) p_rest = reinterpret_cast<const float*>(prow)[n4 * 4 + tid];
   for (int j = tid; j < n_slots; j += MARG_NT) marg[j] = 0.f;
   if (tid < PLAN_ZERO_WORDS) tile[TS + tid] = 0.f;  // the tile's stores never reach these
   // Byte offsets inside a tile are 32-bit and the tile's base is uniform: loads with a scalar base.
@@ -160,7 +163,7 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   // wait for the load right away instead of two tiles later.
   u32x4 tbuf[2][2];
   auto fetch_tile = [&](int k, u32x4 (&buf)[2]) {
-    const bool in_row = k < ntiles;
+    const bool in_row = (int64_t)k * q_tile < n4;     // (the last tile of a row that ends inside a unit may hold no whole one)
     const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
     const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;      // 16-byte units from the tile's start to the row's end
 #pragma unroll
@@ -212,6 +215,10 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
 #pragma unroll
     for (int u = 0; u < 2; ++u)
       if (u * MARG_NT + tid < q_tile) *reinterpret_cast<u32x4*>(tile + ((int64_t)u * MARG_NT + tid) * 4) = buf[u];
+    if (LOAD == MARG_ANY && rest > 0 && k == ntiles - 1) {
+      __syncthreads();                               // over what a clamped load has left in their unit
+      if (tid < rest) tile[n4 * 4 - (int64_t)k * TS + tid] = p_rest;
+    }
     __syncthreads();
     fetch_batch(next.first, next.packed, e_next);
     __builtin_amdgcn_sched_barrier(0);
@@ -828,7 +835,7 @@ static int marg_load_of(const void* probs, int p_dtype, int64_t p_stride, int64_
   using namespace dl;
   if (p_dtype != DL_F32) return MARG_SCALAR;
   if (Vt % 4 == 0 && ok16(probs, p_stride, 4) && ok16(t2s, 0, 4)) return MARG_VEC;
-  return Vt % 4 == 0 && reinterpret_cast<uintptr_t>(probs) % 4 == 0 ? MARG_ANY : MARG_SCALAR;
+  return Vt >= 4 && reinterpret_cast<uintptr_t>(probs) % 4 == 0 ? MARG_ANY : MARG_SCALAR;
 }
 
 // Fills the plan fields of `p` if a usable plan is given; returns the dynamic LDS bytes to request.
