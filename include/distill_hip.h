@@ -130,6 +130,10 @@ int dl_div_topk(int kind,
 /* Scratch size dl_div_topk can make use of for this problem (0 = none needed).  Host-only. */
 int64_t dl_div_topk_workspace_bytes(int kind, int logits_dtype, int64_t n_rows, int64_t V);
 
+/* The same for DL_RKL with a gradient, where wide rows are written by a launch of their own: K (id, value) pairs of
+ * 8 bytes per row (0: such rows take one launch; so do calls with less workspace than this). */
+int64_t dl_rkl_topk_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t V, int K);
+
 /*
  * dl_div_topk for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same

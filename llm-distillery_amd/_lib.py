@@ -33,6 +33,7 @@ _SIGNATURES = {
     "dl_div_topk": (c_int, [c_int, _P, c_int, c_int64, c_int64, c_int64, _P, _P, c_int, _P, c_int, c_int, c_int64, _P,
                             c_float, c_float, c_float, _P, _P, c_int64, _P, c_int64, c_int, _P]),
     "dl_div_topk_workspace_bytes": (c_int64, [c_int, c_int, c_int64, c_int64]),
+    "dl_rkl_topk_workspace_bytes": (c_int64, [c_int, c_int64, c_int64, c_int]),
     "dl_div_topk_static": (c_int, [c_int, _P, c_int, c_int64, c_int64, c_int64, _P, _P, c_int, _P, c_int, c_int, c_int64, _P,
                                    c_float, c_float, c_float, _P, _P, c_int64, c_int, _P]),
     "dl_div_dense": (c_int, [c_int, _P, c_int, c_int64, c_int64, c_int64, _P, _P, c_int, c_int64, c_int64,

@@ -235,27 +235,32 @@ __device__ __forceinline__ void correction_link(int* head, unsigned* own, int* n
 // 2^-40 of the largest term.  Every term is scaled by a power of two chosen from the largest
 // magnitude (an exact operation), cut to an integer and added as such; a single term comes back
 // bit for bit.
-template <class Term>
-__device__ __forceinline__ float correction_exact_sum(const int* next, const int* col, int first, int want, Term term) {
+// `each(f)` calls f(t) for every term t, in any order, the same terms each time.
+template <class Each>
+__device__ __forceinline__ float exact_sum(Each each) {
   float big = 0.f;
   bool odd = false;                                   // NaN or infinity among the terms
-  for (int k = first; k >= 0; k = next[k])
-    if (col[k] == want) {
-      const float t = term(k);
-      odd = odd || !(fabsf(t) <= 3.0e38f);
-      big = fmaxf(big, fabsf(t));
-    }
+  each([&](float t) {
+    odd = odd || !(fabsf(t) <= 3.0e38f);
+    big = fmaxf(big, fabsf(t));
+  });
   if (odd || big == 0.f) {                            // nothing to scale by: plain sum (its value is NaN, an infinity or 0)
     float sum = 0.f;
-    for (int k = first; k >= 0; k = next[k]) sum += col[k] == want ? term(k) : 0.f;
+    each([&](float t) { sum += t; });
     return sum;
   }
   int e;
   (void)frexpf(big, &e);                              // big = m * 2^e, 0.5 <= m < 1
   long long acc = 0;
-  for (int k = first; k >= 0; k = next[k])
-    if (col[k] == want) acc += (long long)ldexp((double)term(k), 40 - e);      // |.| < 2^40; up to 2048 of them: < 2^52
+  each([&](float t) { acc += (long long)ldexp((double)t, 40 - e); });      // |.| < 2^40; up to 2048 of them: < 2^52
   return (float)ldexp((double)acc, e - 40);
+}
+template <class Term>
+__device__ __forceinline__ float correction_exact_sum(const int* next, const int* col, int first, int want, Term term) {
+  return exact_sum([&](auto f) {
+    for (int k = first; k >= 0; k = next[k])
+      if (col[k] == want) f(term(k));
+  });
 }
 
 template <class Tag, int NT, int NCH = 0, class Term, class Finish>
@@ -312,6 +317,8 @@ __device__ __forceinline__ void correction_repeats(const int* head, const int* n
 __device__ __forceinline__ int64_t xcd_banded_row(unsigned b) {
   return (int64_t)(b >> 6) * 64 + (b & 7u) * 8 + ((b & 63u) >> 3);
 }
+// The other way: every XCD works on a contiguous eighth of the items (`grid` workgroups, a multiple of 8).
+__device__ __forceinline__ unsigned xcd_eighth(unsigned b, unsigned grid) { return (b & 7u) * (grid >> 3) + (b >> 3); }
 static inline unsigned xcd_banded_grid(int64_t n_rows) { return (unsigned)((n_rows + 63) / 64 * 64); }
 
 // ---- reductions: fixed order => bit-reproducible ---------------------------------

@@ -11,6 +11,11 @@ extern "C" int64_t dl_div_topk_workspace_bytes(int kind, int logits_dtype, int64
   return dl::RetryList::bytes(n_rows, nch <= 1024 * 16 ? 4 : dl::MAX_COARSE_PARTS);
 }
 
+extern "C" int64_t dl_rkl_topk_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t V, int K) {
+  if (n_rows <= 0 || V <= 0 || K <= 0) return 0;
+  return dl::rkl_workspace_bytes(logits_dtype, n_rows, V, K);
+}
+
 // Argument checks and dispatch shared by dl_div_topk and dl_div_topk_static.
 static int div_topk_checked(int kind, const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows,
                             int64_t V, const int32_t* row_map, const void* t_val, int t_val_dtype,
@@ -43,9 +48,9 @@ static int div_topk_checked(int kind, const void* logits, int logits_dtype, int6
     return logits_dtype == DL_F32 ? launch_fkl<TagF32, false>(p, workspace_bytes, st)
            : logits_dtype == DL_BF16 ? launch_fkl<TagBF16, false>(p, workspace_bytes, st)
                                      : launch_fkl<TagF16, false>(p, workspace_bytes, st);
-  const hipError_t e = logits_dtype == DL_F32 ? launch_rkl<TagF32>(p, aligned, st)
-                       : logits_dtype == DL_BF16 ? launch_rkl<TagBF16>(p, aligned, st)
-                                                 : launch_rkl<TagF16>(p, aligned, st);
+  const hipError_t e = logits_dtype == DL_F32 ? launch_rkl<TagF32>(p, workspace_bytes, aligned, st)
+                       : logits_dtype == DL_BF16 ? launch_rkl<TagBF16>(p, workspace_bytes, aligned, st)
+                                                 : launch_rkl<TagF16>(p, workspace_bytes, aligned, st);
   return e == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
 }
 

@@ -839,108 +839,255 @@ __global__ __launch_bounds__(NT) void fkl_topk_stream_kernel(const TopkParams p)
 // ---------------------------------------------------------------------------------------
 // Reverse KL on the teacher's support: K gathered logits per row, gradient = zero row + K values.
 // ---------------------------------------------------------------------------------------
-// MODE 0: element-wise stores.  MODE 1: gradient rows on the 16-byte grid, a whole number of chunks long.
-// MODE 2: any other gradient row: its 16-byte chunks by vector stores (the teacher ids counted from the
-// first of them), the columns before and behind them one by one.
-template <class Tag, int NT, int MODE>
+// The K-wide part of a row.  Returns false if the row has no usable teacher entry (then nothing else is valid); else every
+// entry k has its id (-1: none), the student's mass on it within the support in s.q and the log ratio to the teacher's in
+// s.z, and rkl is the row's divergence: the gradient at an entry's column is c * q (z - rkl).  Ends in a barrier; an
+// entry's values are written by thread k % NT.  J > 0: K <= J * NT entries in registers, all loads of a kind in flight together.
+template <class Tag, int NT, int J>
+__device__ __forceinline__ bool rkl_on_support(const TopkParams& p, const TopkLds& s, int64_t r, int64_t trow, float& rkl) {
+  if (trow < 0) return false;
+  const int tid = threadIdx.x, K = p.K;
+  const char* row = reinterpret_cast<const char*>(p.logits) + r * p.row_stride * Tag::bytes;
+  if constexpr (J > 0) {
+    const int cnt = p.t_cnt ? min(p.t_cnt[trow], K) : K;
+    int id[J];
+    float t[J], z[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int k = tid + j * NT;
+      int64_t i = -1;
+      float v = -INFINITY;
+      if (k < cnt) {
+        const int64_t at = trow * (int64_t)K + k;
+        i = load_index(p.t_idx, p.t_idx_itype, at);
+        v = load_as_float(p.t_val, p.t_val_dtype, at);
+      }
+      const bool in = i >= 0 && i < p.V;
+      t[j] = in ? v * p.inv_T_t : -INFINITY;
+      id[j] = in && t[j] > -INFINITY ? (int)i : -1;          // an entry of zero mass is no entry
+    }
+    float tmax = -INFINITY, zm = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < J; ++j) z[j] = id[j] >= 0 ? load_as_float(row, Tag::id, id[j]) : 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      tmax = fmaxf(tmax, t[j]);
+      z[j] = id[j] >= 0 ? z[j] * p.inv_T_s : -INFINITY;
+      zm = fmaxf(zm, z[j]);
+    }
+    block_max2<NT>(tmax, zm, s.red);
+    if (tmax == -INFINITY) return false;
+    float ts = 0.f, zs = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      ts += expf(t[j] - tmax);
+      zs += id[j] >= 0 ? expf(z[j] - zm) : 0.f;
+    }
+    block_sum2<NT>(ts, zs, s.red);
+    const float tlse = tmax + logf(ts), slse = zm + logf(zs);
+    float part = 0.f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int k = tid + j * NT;
+      const float sp = z[j] - slse, d = sp - (t[j] - tlse), rk = expf(sp);
+      if (id[j] >= 0) part += rk * d;
+      if (k < s.Kp) { s.idx[k] = id[j]; s.q[k] = rk; s.z[k] = d; }
+    }
+    rkl = block_sum<NT>(part, s.red);
+    return true;
+  } else {
+    if (stage_teacher<Tag, NT>(p, s, trow, row, 0, (int)p.V) == -INFINITY) return false;
+    // student renormalised over the staged ids
+    float zm = -INFINITY;
+    for (int k = tid; k < s.Kp; k += NT)
+      if (s.idx[k] >= 0) zm = fmaxf(zm, s.z[k] * p.inv_T_s);
+    zm = block_max<NT>(zm, s.red);
+    float part = 0.f;
+    for (int k = tid; k < s.Kp; k += NT)
+      if (s.idx[k] >= 0) part += expf(s.z[k] * p.inv_T_s - zm);
+    const float slse = zm + logf(block_sum<NT>(part, s.red));
+    part = 0.f;
+    for (int k = tid; k < s.Kp; k += NT) {
+      if (s.idx[k] >= 0) {
+        const float sp = s.z[k] * p.inv_T_s - slse;
+        const float d = sp - s.t[k];
+        const float rk = expf(sp);
+        part += rk * d;
+        s.q[k] = rk;      // student mass on the support
+        s.z[k] = d;       // log ratio
+      }
+    }
+    rkl = block_sum<NT>(part, s.red);     // barriers inside publish s.q / s.z
+    return true;
+  }
+}
+
+// One launch: every workgroup makes its row's values and then writes the row.
+// MODE 1: gradient rows on the 16-byte grid, a whole number of chunks long.  MODE 2: any other gradient row: its 16-byte
+// chunks by vector stores (the teacher ids counted from the first of them), the columns before and behind them one by one.
+template <class Tag, int NT, int MODE, int J>
 __global__ __launch_bounds__(NT) void rkl_topk_kernel(const TopkParams p) {
-  constexpr bool VEC = MODE != 0;
   extern __shared__ __align__(16) unsigned char smem[];
   const TopkLds s(smem, p.K, NT);
   using C = Chunk<Tag>;
   const int64_t r = xcd_banded_row(blockIdx.x);
   if (r >= p.n_rows) return;
   const int tid = threadIdx.x;
-  const int64_t V = p.V;
   char* grow = p.grad ? reinterpret_cast<char*>(p.grad) + r * p.grad_stride * Tag::bytes : nullptr;
   const int64_t trow = teacher_row(p.row_map, r, p.n_trows);
-  const char* row = reinterpret_cast<const char*>(p.logits) + r * p.row_stride * Tag::bytes;
-  const RowSplit<Tag> sp(grow, V, MODE == 2 && grow);              // the row that is written decides
+  const RowSplit<Tag> sp(grow, p.V, MODE == 2 && grow);              // the row that is written decides
   char* gbody = grow + (int64_t)sp.head * Tag::bytes;
   correction_clear<NT>(s.head, s.own);
-  float tlse = -INFINITY;
-  if (trow >= 0) tlse = stage_teacher<Tag, NT>(p, s, trow, row, 0, (int)V);
-  // Every store comes after the K logits have been gathered (stage_teacher ends in barriers), so
+  // Every store comes after the K logits have been gathered (rkl_on_support ends in a barrier), so
   // the gradient may be written over the logits.
-  if (grow && (!VEC || tlse == -INFINITY)) {
-    if (VEC) {
+  float rkl;
+  if (!rkl_on_support<Tag, NT, J>(p, s, r, trow, rkl)) {
+    if (grow) {
       zero_row<Tag, NT>(gbody, sp.nbody);
       if (MODE == 2 && tid < sp.leftovers()) store_from_float(grow, Tag::id, sp.column(tid), 0.f);
-    } else {
-      for (int64_t j = tid; j < V; j += NT) store_from_float(grow, Tag::id, j, 0.f);
     }
-  }
-  if (tlse == -INFINITY) {
     if (tid == 0 && p.row_loss) p.row_loss[r] = 0.f;
     return;
   }
-  // student renormalised over the staged ids
-  float zm = -INFINITY;
-  for (int k = tid; k < s.Kp; k += NT)
-    if (s.idx[k] >= 0) zm = fmaxf(zm, s.z[k] * p.inv_T_s);
-  zm = block_max<NT>(zm, s.red);
-  float part = 0.f;
-  for (int k = tid; k < s.Kp; k += NT)
-    if (s.idx[k] >= 0) part += expf(s.z[k] * p.inv_T_s - zm);
-  const float slse = zm + logf(block_sum<NT>(part, s.red));
-  part = 0.f;
-  for (int k = tid; k < s.Kp; k += NT) {
-    if (s.idx[k] >= 0) {
-      const float sp = s.z[k] * p.inv_T_s - slse;
-      const float d = sp - s.t[k];
-      const float rk = expf(sp);
-      part += rk * d;
-      s.q[k] = rk;      // student mass on the support
-      s.z[k] = d;       // log ratio
-    }
-  }
-  const float rkl = block_sum<NT>(part, s.red);     // barriers inside publish s.t / s.z
   if (tid == 0 && p.row_loss) p.row_loss[r] = rkl;
   if (grow) {
     const float c = p.inv_T_s * p.grad_scale;
-    __syncthreads();    // zero fill precedes the sparse values (scalar path); s.q / s.z complete
     for (int k = tid; k < s.Kp; k += NT) {
       const int id = s.idx[k];
       if (id < 0) continue;
-      if (VEC) {
-        // placed by the thread that writes the column's chunk; columns beside the body are left to the last step
-        const int64_t idb = (int64_t)id - sp.head;
-        if (idb >= 0 && idb < sp.nbody * C::N) correction_link<Tag, NT>(s.head, s.own, s.next, k, (int)idb);
-      } else {
-        float g = 0.f;
-        for (int j = 0; j < s.Kp; ++j) g += (s.idx[j] == id) ? s.q[j] * (s.z[j] - rkl) : 0.f;
-        store_from_float(grow, Tag::id, id, g * c);
-      }
+      // placed by the thread that writes the column's chunk; columns beside the body are left to the last step
+      const int64_t idb = (int64_t)id - sp.head;
+      if (idb >= 0 && idb < sp.nbody * C::N) correction_link<Tag, NT>(s.head, s.own, s.next, k, (int)idb);
     }
-    if (VEC) {
-      // the row of zeros, each chunk written once with the support's values already in place
-      __syncthreads();
-      const unsigned mine = s.own[tid];
-      const int64_t nch = sp.nbody;
-      const auto term = [&](int k) { return s.q[k] * (s.z[k] - rkl); };
-      const auto value = [&](int, float g) { return g * c; };
-      unsigned repeats = 0u;
-      int n_own = 0;
-      for (int64_t ch = tid, i = 0; ch < nch; ch += NT, ++i) {
-        float f[C::N];
+    // the row of zeros, each chunk written once with the support's values already in place
+    __syncthreads();
+    const unsigned mine = s.own[tid];
+    const int64_t nch = sp.nbody;
+    const auto term = [&](int k) { return s.q[k] * (s.z[k] - rkl); };
+    const auto value = [&](int, float g) { return g * c; };
+    unsigned repeats = 0u;
+    int n_own = 0;
+    for (int64_t ch = tid, i = 0; ch < nch; ch += NT, ++i) {
+      float f[C::N];
 #pragma unroll
-        for (int e = 0; e < C::N; ++e) f[e] = 0.f;
-        if (mine & (1u << (i & 31)))
-          if (correction_apply<Tag, NT>(s.head, s.next, s.idx, sp.head, (int)i, f, term, value)) repeats |= 1u << (i & 31);
-        store16_stream(gbody + ch * 16, C::pack(f));
-        n_own = (int)i + 1;
-      }
-      if (repeats)
-        correction_repeats<Tag, NT>(s.head, s.next, s.idx, sp.head, repeats, n_own, term, value,
-                                    [&](int column, float v) { store_from_float(grow, Tag::id, column, v); });
-      if (MODE == 2 && tid < sp.leftovers()) {
-        const int64_t j = sp.column(tid);
-        float g = 0.f;
-        for (int k = 0; k < s.Kp; ++k) g += (s.idx[k] == j) ? term(k) : 0.f;
-        store_from_float(grow, Tag::id, j, g * c);
-      }
+      for (int e = 0; e < C::N; ++e) f[e] = 0.f;
+      if (mine & (1u << (i & 31)))
+        if (correction_apply<Tag, NT>(s.head, s.next, s.idx, sp.head, (int)i, f, term, value)) repeats |= 1u << (i & 31);
+      store16_stream(gbody + ch * 16, C::pack(f));
+      n_own = (int)i + 1;
+    }
+    if (repeats)
+      correction_repeats<Tag, NT>(s.head, s.next, s.idx, sp.head, repeats, n_own, term, value,
+                                  [&](int column, float v) { store_from_float(grow, Tag::id, column, v); });
+    if (MODE == 2 && tid < sp.leftovers()) {
+      const int64_t j = sp.column(tid);
+      const float g = exact_sum([&](auto f) {
+        for (int k = 0; k < s.Kp; ++k)
+          if (s.idx[k] == j) f(term(k));
+      });
+      store_from_float(grow, Tag::id, j, g * c);
     }
   }
+}
+
+// Two launches, through a workspace of K (id, q (z - rkl)) pairs per row: the values of all rows, then nothing but the
+// stores, in the order of the gradient's addresses.  A workgroup that makes a row's values and then writes the row is a
+// chain of dependent round trips ahead of its stores, and 2048 rows are written at a time, spread over the whole buffer.
+// Bound by the stores: a bare fill of 8192 x 128256 bf16 takes 300 us at best (7.0 TB/s: 4 KiB per workgroup, every XCD in an
+// eighth of the buffer of its own), 314 with 16 KiB per workgroup, 345 with the workgroups dealt round the XCDs in
+// address order, 320-455 from persistent grids.  Measured with the row's values (K = 200): 448 us in one launch, 359 so, of
+// which 34 for the values; 384 with slabs of 16 KiB instead of 8, 420 with the correction lists of the register kernels
+// instead of a slab in LDS and the workgroups in address order.  4096 x 128256 fp32, K = 20: 434 -> 331 us.
+template <class Tag, int NT, int J>
+__global__ __launch_bounds__(NT) void rkl_values_kernel(const TopkParams p) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const TopkLds s(smem, p.K);
+  const int64_t r = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int64_t trow = teacher_row(p.row_map, r, p.n_trows);
+  uint2* out = reinterpret_cast<uint2*>(p.workspace) + r * p.K;
+  float rkl = 0.f;
+  const bool live = rkl_on_support<Tag, NT, J>(p, s, r, trow, rkl);
+  if (tid == 0 && p.row_loss) p.row_loss[r] = live ? rkl : 0.f;
+  for (int k = tid; k < p.K; k += NT)
+    out[k] = live ? uint2{(unsigned)s.idx[k], __float_as_uint(s.q[k] * (s.z[k] - rkl))} : uint2{~0u, 0u};
+}
+
+// Item b is part b % parts of row b / parts: SLAB bytes of the row's body (and with part 0 the columns beside the body:
+// MODE 2).  The part is made in LDS: zeroed, the pairs that name one of its columns (out of all K pairs of the row, from
+// L2) written into place, and stored in one piece; a bit per column tells a repeated id, whose pairs are then added up.
+constexpr int RKL_FILL_NT = 256, RKL_FILL_NCH = 2, RKL_SLAB = RKL_FILL_NT * RKL_FILL_NCH * 16;
+template <class Tag, int MODE>
+__global__ __launch_bounds__(RKL_FILL_NT) void rkl_fill_kernel(const TopkParams p, unsigned parts) {
+  using C = Chunk<Tag>;
+  constexpr int NT = RKL_FILL_NT, NCH = RKL_FILL_NCH, COLS = RKL_SLAB / Tag::bytes, WORDS = COLS / 32 + 1;
+  __shared__ __align__(16) u32x4 slab[NT * NCH];
+  __shared__ unsigned named[WORDS];                                  // a bit per column; the last word: the columns beside the body
+  __shared__ unsigned twice[WORDS];                                  // set: by more than one pair
+  __shared__ float beside[REST_HEADS];
+  __shared__ int repeats;
+  const int tid = threadIdx.x;
+  const unsigned item = xcd_eighth(blockIdx.x, gridDim.x);
+  const int64_t r = item / parts;
+  const int h = (int)(item % parts);
+  if (r >= p.n_rows) return;
+  const uint2* ent = reinterpret_cast<const uint2*>(p.workspace) + r * p.K;
+  uint2 mine = tid < p.K ? ent[tid] : uint2{~0u, 0u};
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) slab[i * NT + tid] = u32x4{0u, 0u, 0u, 0u};
+  for (int i = tid; i < WORDS; i += NT) { named[i] = 0u; twice[i] = 0u; }
+  if (tid == 0) repeats = 0;
+  if (MODE == 2 && tid < REST_HEADS) beside[tid] = 0.f;
+  char* grow = reinterpret_cast<char*>(p.grad) + r * p.grad_stride * Tag::bytes;
+  const RowSplit<Tag> sp(grow, p.V, MODE == 2);
+  const int c0 = h * NT * NCH;                                       // first chunk of the part
+  const int nch = (int)min((int64_t)NT * NCH, sp.nbody - c0);        // its chunks (behind a row's head there may be none left: <= 0)
+  const int lo = sp.head + c0 * C::N, hi = lo + max(nch, 0) * C::N;
+  const int behind = sp.head + (int)sp.nbody * C::N;
+  const float c = p.inv_T_s * p.grad_scale;
+  // place of column `id`: inside the part, behind it (>= COLS) among the columns beside the body, or -1
+  const auto place_of = [&](int id) {
+    if (id >= lo && id < hi) return id - lo;
+    if (MODE == 2 && h == 0 && id >= 0 && id < sp.head) return COLS + id;
+    if (MODE == 2 && h == 0 && id >= behind) return COLS + sp.head + (id - behind);
+    return -1;
+  };
+  const auto put = [&](int at, float g) {
+    if (MODE == 2 && at >= COLS) beside[at - COLS] = g;
+    else store_from_float(slab, Tag::id, at, g);
+  };
+  __syncthreads();
+  for (int k = tid; k < p.K; k += NT) {
+    if (k >= NT) mine = ent[k];
+    const int at = place_of((int)mine.x);
+    if (at < 0) continue;
+    const unsigned bit = 1u << (at & 31);
+    if (atomicOr(&named[at >> 5], bit) & bit) {
+      atomicOr(&twice[at >> 5], bit);
+      repeats = 1;
+    } else {
+      put(at, __uint_as_float(mine.y) * c);
+    }
+  }
+  __syncthreads();
+  if (repeats) {                                                     // every pair of a repeated id writes the same sum
+    for (int k = tid; k < p.K; k += NT) {
+      const int id = (int)ent[k].x, at = place_of(id);
+      if (at < 0 || !(twice[at >> 5] & (1u << (at & 31)))) continue;
+      put(at, exact_sum([&](auto f) {
+        for (int q = 0; q < p.K; ++q) {
+          const uint2 e = ent[q];
+          if ((int)e.x == id) f(__uint_as_float(e.y));
+        }
+      }) * c);
+    }
+    __syncthreads();
+  }
+  char* gpart = grow + (int64_t)lo * Tag::bytes;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i)
+    if (i * NT + tid < nch) store16_stream(gpart + (i * NT + tid) * 16, slab[i * NT + tid]);
+  if (MODE == 2 && h == 0 && tid < sp.leftovers()) store_from_float(grow, Tag::id, sp.column(tid), beside[tid]);
 }
 
 // clears the `ready` words of the split kernel's workspace (a template only so that it may live in a header)
@@ -1140,15 +1287,44 @@ static int launch_fkl(const TopkParams& p, int64_t ws_bytes, hipStream_t st, boo
 int launch_fkl_any(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool off_grid);
 int launch_fkl_any_multi(int logits_dtype, const TopkParams& p, int64_t ws_bytes, hipStream_t st, bool ws_cleared, bool off_grid);
 
+// Reverse KL.  Parts of a row for the two-launch form; 0: one launch.  Narrow rows give a workgroup of the one-launch form
+// little to write behind its K values, and a part of the two-launch form many pairs to look through for each of its columns
+// (8192 x 32000 bf16, K = 200: 115 us in one launch, 120 in two; 16384 x 12000: 116, 123).  From 96 KiB per row on two
+// launches pay where there is enough to write to cover the second one (2048 x 50304 bf16 49 -> 44 us, 1024 x 36696 fp32 43 ->
+// 36; 1024 x 50304 bf16 28 against 29), from 195 KiB on always: few rows leave most of the chip idle in one launch (32 x
+// 128256 bf16 32 -> 29 us, 512 rows 36 -> 29).
+static int64_t rkl_fill_parts(int logits_dtype, int64_t n_rows, int64_t V) {
+  const int64_t row_bytes = V * (logits_dtype == F32 ? 4 : 2);
+  if (row_bytes < 96 * 1024 || (row_bytes < 200000 && n_rows * row_bytes < (128LL << 20))) return 0;
+  const int64_t parts = (row_bytes / 16 + RKL_FILL_NT * RKL_FILL_NCH - 1) / (RKL_FILL_NT * RKL_FILL_NCH);
+  return n_rows * parts <= 0x7fffffffLL - 7 ? parts : 0;
+}
+static int64_t rkl_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t V, int K) {
+  return rkl_fill_parts(logits_dtype, n_rows, V) ? n_rows * K * (int64_t)sizeof(uint2) : 0;
+}
+
 template <class Tag>
-static hipError_t launch_rkl(const TopkParams& p, bool aligned, hipStream_t st) {
+static hipError_t launch_rkl(const TopkParams& p, int64_t ws_bytes, bool aligned, hipStream_t st) {
   // the logits are only gathered from; what is written decides: MODE 2 takes any gradient row
-  if (aligned)
-    hipLaunchKernelGGL((rkl_topk_kernel<Tag, 256, 1>), dim3(xcd_banded_grid(p.n_rows)), dim3(256),
-                       TopkLds::bytes(p.K, 256), st, p);
-  else
-    hipLaunchKernelGGL((rkl_topk_kernel<Tag, 256, 2>), dim3(xcd_banded_grid(p.n_rows)), dim3(256),
-                       TopkLds::bytes(p.K, 256), st, p);
+  const int64_t need = p.grad && p.workspace ? rkl_workspace_bytes(Tag::id, p.n_rows, p.V, p.K) : 0;
+  const bool two = need > 0 && ws_bytes >= need;
+  const int J = p.K <= 256 ? 1 : p.K <= 512 ? 2 : 0;
+  if (two) {
+    const dim3 rows((unsigned)p.n_rows), by(256);
+    if (J == 1) hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 1>), rows, by, TopkLds::bytes(p.K), st, p);
+    else if (J == 2) hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 2>), rows, by, TopkLds::bytes(p.K), st, p);
+    else hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 0>), rows, by, TopkLds::bytes(p.K), st, p);
+    const unsigned parts = (unsigned)rkl_fill_parts(Tag::id, p.n_rows, p.V);
+    const dim3 grid((unsigned)((p.n_rows * parts + 7) / 8 * 8)), block(RKL_FILL_NT);
+    if (aligned) hipLaunchKernelGGL((rkl_fill_kernel<Tag, 1>), grid, block, 0, st, p, parts);
+    else hipLaunchKernelGGL((rkl_fill_kernel<Tag, 2>), grid, block, 0, st, p, parts);
+    return hipGetLastError();
+  }
+#define DL_LAUNCH_RKL(MODE, J) \
+  hipLaunchKernelGGL((rkl_topk_kernel<Tag, 256, MODE, J>), dim3(xcd_banded_grid(p.n_rows)), dim3(256), TopkLds::bytes(p.K, 256), st, p)
+  if (aligned) { if (J == 1) DL_LAUNCH_RKL(1, 1); else if (J == 2) DL_LAUNCH_RKL(1, 2); else DL_LAUNCH_RKL(1, 0); }
+  else { if (J == 1) DL_LAUNCH_RKL(2, 1); else if (J == 2) DL_LAUNCH_RKL(2, 2); else DL_LAUNCH_RKL(2, 0); }
+#undef DL_LAUNCH_RKL
   return hipGetLastError();
 }
 

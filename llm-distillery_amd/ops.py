@@ -123,7 +123,10 @@ def div_topk(kind: str, logits: torch.Tensor, t_val: torch.Tensor, t_idx: torch.
     flags = (_lib.DL_TOPK_UNIQUE_IDS if unique_ids else 0) | (_lib.DL_TOPK_NO_WAIT if no_wait else 0) | \
         (_lib.DL_TOPK_FINE_PARTS if parts == 16 else parts << _lib.DL_TOPK_PARTS_SHIFT)
     lib = _lib.load()
-    ws_bytes = lib.dl_div_topk_workspace_bytes(KINDS[kind], _DT[x.dtype], R, V) if want_grad else 0
+    ws_bytes = 0
+    if want_grad:
+        ws_bytes = (lib.dl_div_topk_workspace_bytes(KINDS[kind], _DT[x.dtype], R, V) if kind == "fkl"
+                    else lib.dl_rkl_topk_workspace_bytes(_DT[x.dtype], R, V, K))
     if parts == 16 and want_grad:
         ws_bytes = R * 16 * 20 + 16
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None

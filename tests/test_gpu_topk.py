@@ -529,3 +529,38 @@ def test_a_column_part_masked_with_low_finite_values(D, dtype, V, T, level):
         rl, grad = D.div_topk("fkl", logits.to(DEV), tv.to(DEV), ti.to(DEV), T=T, no_wait=no_wait)
         np.testing.assert_allclose(rl.cpu().numpy(), rl0.cpu().numpy(), rtol=1e-6)
         assert torch.isfinite(grad).all() and torch.equal(grad, g0)
+
+
+@pytest.mark.parametrize("dtype,V,pitch,K", [(torch.bfloat16, 102400, 102400, 200),      # 25 whole parts of 8 KiB
+                                             (torch.bfloat16, 102408, 102408, 256),      # a last part of one chunk
+                                             (torch.float16, 102407, 102407, 257),       # off the 16-byte grid: columns beside the chunks
+                                             (torch.bfloat16, 106497, 106504, 513),      # a loop over the entries
+                                             (torch.float32, 51201, 51201, 40), (torch.float32, 51200, 51204, 1)])
+@pytest.mark.parametrize("grad_mode", ["fresh", "in_place", "other_phase"])
+def test_rkl_values_and_fill_match_the_one_launch_form(D, dtype, V, pitch, K, grad_mode):
+    """Wide rows: the values of all rows in one launch, the rows themselves in a second one, through a workspace;
+    dl_div_topk_static, which has none for it, keeps one launch.  The same arithmetic, bit for bit; repeated ids (their values
+    are added up), ids outside the row, entries in the first and last columns, masked rows, rows without an entry."""
+    assert D._lib.load().dl_rkl_topk_workspace_bytes(D.ops._DT[dtype], 9, V, K) == 9 * K * 8
+    R = 9
+    g = torch.Generator().manual_seed(V + K)
+    x = torch.zeros(R, pitch, dtype=dtype, device=DEV)[:, :V]
+    x.copy_((torch.randn(R, V, generator=g) * 3).to(dtype).to(DEV))
+    tv = torch.log_softmax(torch.randn(R, K, generator=g) * 2, -1).half().to(DEV)
+    ti = torch.randint(0, V, (R, K), generator=g, dtype=torch.int32).to(DEV)
+    if K > 8:
+        ti[:, 0], ti[:, 1], ti[:, 2], ti[:, 3] = 0, V - 1, V, -1
+        ti[1, 4:8] = ti[1, 8]                            # one id five times
+        ti[2, K // 2:] = ti[2, :K - K // 2].clone()      # every id twice, the ends of the row among them
+        tv[3] = float("-inf")                            # no entry at all
+    rm = torch.arange(R, dtype=torch.int32, device=DEV)
+    rm[5] = -1
+    rl, grad = torch.empty(R, device=DEV), torch.empty_like(x)
+    D.div_topk_static("rkl", x, tv, ti, rl, grad, row_map=rm, T=1.4, grad_scale=0.3)
+    out = None
+    if grad_mode == "in_place":
+        out = x
+    elif grad_mode == "other_phase":
+        out = torch.full((R * (V + 3) + 1,), float("nan"), dtype=dtype, device=DEV)[1:].view(R, V + 3)[:, :V]
+    rl2, grad2 = D.div_topk("rkl", x, tv, ti, row_map=rm, T=1.4, grad_scale=0.3, grad_out=out)
+    assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
