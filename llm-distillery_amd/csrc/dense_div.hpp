@@ -123,11 +123,25 @@ __device__ __forceinline__ float rkl_centre(float mean, const DenseStats& st, fl
   return (float)((double)mean - ((double)st.ls - bs) + ((double)st.lt - bt)) * LN2;
 }
 
-// This thread's share of the JSD sums KL(P || M), KL(Q || M) (log2), given the row's normalisers; STASH as below.
-template <bool STASH, class Rows>
+// What the JSD sums leave in registers for the gradient (see dense_stats).
+constexpr int JSD_KEEP_NOTHING = 0, JSD_KEEP_RATIO = 1, JSD_KEEP_BOTH = 2;
+// This thread's share of the JSD sums KL(P || M), KL(Q || M) (log2), given the row's normalisers.
+template <int KEEP, class Rows>
 __device__ __forceinline__ void dense_jsd_sums(Rows& rows, const DenseStats& st, float& x, float& y) {
   const float a_s = st.a_s, a_t = st.a_t;
-  if constexpr (STASH) {
+  if constexpr (KEEP == JSD_KEEP_RATIO) {
+    rows.sweep_keep([&](const float* s, const float* t, float* keep, auto n) {
+#pragma unroll
+      for (int e = 0; e < decltype(n)::value; ++e) {
+        const float lp = fmaf(s[e], a_s, -st.ls), lq = fmaf(t[e], a_t, -st.lt);
+        const float pr = fast_exp2(lp), q = fast_exp2(lq);
+        const float lm = fast_log2(0.5f * pr + 0.5f * q);
+        keep[e] = log_ratio_to_mixture(lp, lm);
+        x = fmaf(pr, keep[e], x);
+        y = fmaf(q, log_ratio_to_mixture(lq, lm), y);
+      }
+    });
+  } else if constexpr (KEEP == JSD_KEEP_BOTH) {
     rows.sweep_rewrite([&](int64_t, float* s, float* t, auto n) {
 #pragma unroll
       for (int e = 0; e < decltype(n)::value; ++e) {
@@ -162,14 +176,17 @@ __device__ __forceinline__ void dense_jsd_sums(Rows& rows, const DenseStats& st,
 // so the divergence sum rides along with the sums of exponentials.  JSD needs the normalised
 // probabilities inside a logarithm and keeps its own sweep.
 //
-// STASH (JSD on rows of fp32 pairs held in registers): the divergence sweep leaves p and
+// KEEP (JSD on rows held in registers): JSD_KEEP_BOTH, for fp32 pairs: the divergence sweep leaves p and
 // log2 p - log2 m in the registers of the logits, exactly, and the gradient
 //   g = c p / 2 ((log2 p - log2 m) ln 2 - KL(P || M))
-// takes two instructions per column (dense_jsd_grad_from_stash) instead of recomputing three
+// takes two instructions per column (dense_jsd_grad_kept) instead of recomputing three
 // transcendentals (8192 x 32000: 0.70 -> 0.67 ms).  The same for forward and reverse KL (their
 // exponentials kept) shortened the arithmetic by a third and the kernel not at all: with fp32 rows
-// those two are not bound by the vector ALU.
-template <int KIND, int NT, bool STASH = false, class Rows>
+// those two are not bound by the vector ALU.  JSD_KEEP_RATIO, for the other pairs: the log ratio alone, in fp32, which leaves
+// one exponential to the gradient (six transcendentals per column in all instead of eight); p as well would take half of a
+// CU's registers for one row.  8192 x 32000 bf16 pairs, a quarter masked: 284 -> 242 us; 2048 x 128256 bf16 469 -> 413; bf16
+// against fp32 4096 x 24000 185 -> 171, fp32 against bf16 255 -> 235.
+template <int KIND, int NT, int KEEP = JSD_KEEP_NOTHING, class Rows>
 __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, float inv_T_t, float* red) {
   DenseStats st;
   st.a_s = inv_T_s * LOG2E;
@@ -270,7 +287,7 @@ __device__ __forceinline__ DenseStats dense_stats(Rows& rows, float inv_T_s, flo
     return st;
   }
   float x = 0.f, y = 0.f;
-  dense_jsd_sums<STASH>(rows, st, x, y);
+  dense_jsd_sums<KEEP>(rows, st, x, y);
   block_sum2<NT>(x, y, red);
   st.loss = 0.5f * LN2 * (x + y);
   st.aux = x * LN2;
@@ -289,16 +306,25 @@ __device__ __forceinline__ void dense_grad_sweep(Rows& rows, const DenseStats& s
   });
 }
 
-// The JSD gradient from what dense_stats<DL_JSD, NT, true> left in the registers.
-template <class TagS, class Rows>
-__device__ __forceinline__ void dense_jsd_grad_from_stash(Rows& rows, const DenseStats& st, float c, char* grow) {
+// The JSD gradient from what dense_stats<DL_JSD, NT, KEEP> left in registers.
+template <int KEEP, class TagS, class Rows>
+__device__ __forceinline__ void dense_jsd_grad_kept(Rows& rows, const DenseStats& st, float c, char* grow) {
   const float kb = 0.5f * c * LN2, k0 = -0.5f * c * st.aux;
-  rows.sweep([&](int64_t u, const float* pr, const float* d, auto n) {
-    float g[decltype(n)::value];
+  if constexpr (KEEP == JSD_KEEP_RATIO) {
+    rows.sweep_kept([&](int64_t u, const float* s, const float* d, auto n) {
+      float g[decltype(n)::value];
 #pragma unroll
-    for (int e = 0; e < decltype(n)::value; ++e) g[e] = pr[e] * fmaf(d[e], kb, k0);
-    rows.store(grow, u, g, n);
-  });
+      for (int e = 0; e < decltype(n)::value; ++e) g[e] = fast_exp2(fmaf(s[e], st.a_s, -st.ls)) * fmaf(d[e], kb, k0);
+      rows.store(grow, u, g, n);
+    });
+  } else {
+    rows.sweep([&](int64_t u, const float* pr, const float* d, auto n) {
+      float g[decltype(n)::value];
+#pragma unroll
+      for (int e = 0; e < decltype(n)::value; ++e) g[e] = pr[e] * fmaf(d[e], kb, k0);
+      rows.store(grow, u, g, n);
+    });
+  }
 }
 
 }  // namespace dl

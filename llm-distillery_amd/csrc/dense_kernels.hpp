@@ -153,6 +153,54 @@ struct RegRows {
       if ((int)threadIdx.x < rest) f(nunits, &s_rest, &t_rest, Columns<1>{});
     }
   }
+  // JSD on the other pairs: the divergence sweep keeps a column's log ratio to the mixture, in fp32, for the gradient: in the
+  // teacher's registers where those are fp32, else in registers of its own (a 16-bit teacher's are then free).
+  static constexpr bool RATIO_STASH = !EXACT_STASH, RATIO_IN_T = TagT::bytes == 4;
+  float ratio[RATIO_STASH && !RATIO_IN_T ? NU : 1][8];
+  float ratio_rest;
+  // f(s, t, d): sets d, the values to keep (per wave, as sweep_rewrite)
+  template <class F>
+  __device__ __forceinline__ void sweep_keep(F f) {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int64_t u = (int64_t)i * NT + threadIdx.x;
+      if (__builtin_amdgcn_readfirstlane((int)((u & ~(int64_t)63) < nunits))) {
+        float a[8], b[8], d[8];
+        s[i].unpack(a);
+        t[i].unpack(b);
+        f(a, b, d, Columns<8>{});
+        if constexpr (RATIO_IN_T) t[i].repack(d);
+        else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) ratio[i][e] = d[e];
+        }
+      }
+    }
+    if constexpr (ANY) {
+      if ((int)threadIdx.x < rest) f(&s_rest, &t_rest, &ratio_rest, Columns<1>{});
+    }
+  }
+  // f(u, s, d): the kept values beside the student's
+  template <class F>
+  __device__ __forceinline__ void sweep_kept(F f) {
+#pragma unroll
+    for (int i = 0; i < NU; ++i) {
+      const int64_t u = (int64_t)i * NT + threadIdx.x;
+      if (u < nunits) {
+        float a[8], d[8];
+        s[i].unpack(a);
+        if constexpr (RATIO_IN_T) t[i].unpack(d);
+        else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) d[e] = ratio[i][e];
+        }
+        f(u, a, d, Columns<8>{});
+      }
+    }
+    if constexpr (ANY) {
+      if ((int)threadIdx.x < rest) f(nunits, &s_rest, &ratio_rest, Columns<1>{});
+    }
+  }
   // Maxima of both rows from the raw bit patterns, for two 16-bit rows: non-negative 16-bit floats
   // order like their patterns read as signed integers and every negative one reads as a negative
   // integer, so the packed integer maximum is the row's maximum whenever that is not negative (half
@@ -194,8 +242,10 @@ struct RegRows {
   }
 };
 
+// JSD: four waves per SIMD are asked for (128 registers): with the kept ratios the 16-bit pairs off the grid would take a few
+// more, one workgroup fewer per CU (8192 x 32100 bf16: 386 us against 252).
 template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY = false>
-__global__ __launch_bounds__(NT) void dense_reg_kernel(const DenseParams p) {
+__global__ __launch_bounds__(NT, KIND == DL_JSD ? 4 : 1) void dense_reg_kernel(const DenseParams p) {
   __shared__ float red[64];
   const int64_t r = xcd_banded_row(blockIdx.x);
   if (r >= p.n_rows) return;
@@ -217,12 +267,13 @@ __global__ __launch_bounds__(NT) void dense_reg_kernel(const DenseParams p) {
   const int64_t nunits = (p.V - head) / 8;
   rows.load(srow + head * TagS::bytes, tl + head * TagT::bytes, nunits, head, ANY ? (int)(p.V - head - nunits * 8) : 0);
   if (ANY && grow) grow += head * TagS::bytes;
-  if constexpr (KIND == DL_JSD && RegRows<TagS, TagT, NT, NU, ANY>::EXACT_STASH) {
-    // The divergence sweep leaves the gradient's ingredients in the rows' registers (at no cost for fp32
-    // rows, so also when no gradient is asked for: a second copy of the sweeps for that case costs registers).
-    const DenseStats st = dense_stats<KIND, NT, true>(rows, p.inv_T_s, p.inv_T_t, red);
+  if constexpr (KIND == DL_JSD) {
+    // The divergence sweep leaves the gradient's ingredients in registers (also when no gradient is asked for: a second
+    // copy of the sweeps for that case costs registers).
+    constexpr int KEEP = RegRows<TagS, TagT, NT, NU, ANY>::EXACT_STASH ? JSD_KEEP_BOTH : JSD_KEEP_RATIO;
+    const DenseStats st = dense_stats<KIND, NT, KEEP>(rows, p.inv_T_s, p.inv_T_t, red);
     if (tid == 0 && p.row_loss) p.row_loss[r] = st.loss;
-    if (grow) dense_jsd_grad_from_stash<TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+    if (grow) dense_jsd_grad_kept<KEEP, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
   } else {
     const DenseStats st = dense_stats<KIND, NT>(rows, p.inv_T_s, p.inv_T_t, red);
     if (tid == 0 && p.row_loss) p.row_loss[r] = st.loss;
@@ -435,7 +486,7 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
   st.tmax = Mt;
   if constexpr (KIND == DL_JSD) {
     float kp = 0.f, kq = 0.f;
-    dense_jsd_sums<Rows::EXACT_STASH>(rows, st, kp, kq);
+    dense_jsd_sums<Rows::EXACT_STASH ? JSD_KEEP_BOTH : JSD_KEEP_RATIO>(rows, st, kp, kq);
     block_sum2<NT>(kp, kq, red);
     DenseRecord* ws2 = x.second + r * P;
     if (RETRY == SPLIT_SECOND) {
@@ -454,7 +505,8 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
   }
   if (tid == 0 && h == 0 && p.row_loss) p.row_loss[r] = st.loss;
   if (grow) {
-    if constexpr (KIND == DL_JSD && Rows::EXACT_STASH) dense_jsd_grad_from_stash<TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+    if constexpr (KIND == DL_JSD)
+      dense_jsd_grad_kept<Rows::EXACT_STASH ? JSD_KEEP_BOTH : JSD_KEEP_RATIO, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
     else dense_grad_sweep<KIND, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
   }
 }
