@@ -138,37 +138,39 @@ __device__ __forceinline__ void plan_consume_packed(const u32x4& d, const float*
 // scheduling barriers pin.  (With the entries of the first tile issued ahead of its data, as the
 // compiler had it, every wait in the loop became a wait for all but one or none of the loads: one
 // tile in flight whatever the depth, and the entries' trip to L2 and back waited for in full.)
-template <int LOAD>
+template <int LOAD, int NT>
 __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p, const char* prow, float* marg,
                                                             float* tile) {
   const int tid = threadIdx.x, lane = tid & (WAVE - 1);
   // the wave index as a scalar: plan offsets are then fetched with scalar loads, which have their own
   // counter and do not queue behind the vector prefetches
   const int w = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  constexpr int NW = MARG_NT / WAVE;
+  constexpr int NW = MARG_NT / WAVE;                 // lists per tile
+  constexpr int LPW = MARG_NT / NT;                  // of which a wave of a smaller workgroup walks several
+  constexpr int U = 2 * LPW;                         // 16-byte loads per thread and tile
   const int TS = p.plan_tile;
-  const int q_tile = TS / 4;                        // 16-byte loads per tile: 1024 .. 2048, up to two per thread
+  const int q_tile = TS / 4;                        // 16-byte loads per tile: 1024 .. 2048, up to U per thread
   const int ntiles = (int)((p.Vt + TS - 1) / TS);
   const int64_t n4 = p.Vt / 4;
   const int n_slots = (int)plan_slot_words(p.Vs, p.plan_n_extra);
   const int rest = LOAD == MARG_ANY ? (int)(p.Vt - n4 * 4) : 0;       // probabilities behind the last whole unit
   float p_rest = 0.f;
   if (LOAD == MARG_ANY && tid < rest) p_rest = reinterpret_cast<const float*>(prow)[n4 * 4 + tid];
-  for (int j = tid; j < n_slots; j += MARG_NT) marg[j] = 0.f;
+  for (int j = tid; j < n_slots; j += NT) marg[j] = 0.f;
   if (tid < PLAN_ZERO_WORDS) tile[TS + tid] = 0.f;  // the tile's stores never reach these
   // Byte offsets inside a tile are 32-bit and the tile's base is uniform: loads with a scalar base.
   // Unconditional load from a clamped offset: with branch-free loads the compiler knows how many are
   // in flight and never has to drain the whole queue.  What a clamped load brings is never used: no
   // entry points behind the end of the row, and a select on the value here would make the thread
   // wait for the load right away instead of two tiles later.
-  u32x4 tbuf[2][2];
-  auto fetch_tile = [&](int k, u32x4 (&buf)[2]) {
+  u32x4 tbuf[2][U];
+  auto fetch_tile = [&](int k, u32x4 (&buf)[U]) {
     const bool in_row = (int64_t)k * q_tile < n4;     // (the last tile of a row that ends inside a unit may hold no whole one)
     const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
     const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;      // 16-byte units from the tile's start to the row's end
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      const int c = u * MARG_NT + tid;
+    for (int u = 0; u < U; ++u) {
+      const int c = u * NT + tid;
       const unsigned off = (c < q_tile && c < left) ? (unsigned)c * 16u : 0u;
       if constexpr (LOAD == MARG_ANY) buf[u] = load16_stream_any(base + off);
       else buf[u] = load16_stream(base + off);
@@ -181,10 +183,11 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   // Row numbers are multiples of 4; bit 0 of a list's first row number says that the list is packed.
   // Behind the last tile: the plan's first list, fetched and dropped.
   struct List { int first, end, packed; };
-  auto list_of = [&](int k) {
+  auto list_of = [&](int k, int q) {
     List l{0, 0, 0};
     if (k < ntiles) {
-      const int a = row_off[k * NW + w], b = row_off[k * NW + w + 1];
+      const int at = k * NW + q * (NT / WAVE) + w;
+      const int a = row_off[at], b = row_off[at + 1];
       l.first = a & ~3;
       l.end = b & ~3;
       l.packed = a & 1;
@@ -201,41 +204,48 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
       b.hi = *reinterpret_cast<const u32x4*>(at + (unsigned)lane * 8u + 4u);
     }
   };
-  PlanBatch e_even, e_odd;
-  List cur = list_of(0), next = list_of(1);           // the descriptors run two tiles ahead of the entries
+  PlanBatch e_even[LPW], e_odd[LPW];
+  List cur[LPW], next[LPW];                           // the descriptors run two tiles ahead of the entries
+#pragma unroll
+  for (int q = 0; q < LPW; ++q) { cur[q] = list_of(0, q); next[q] = list_of(1, q); }
   fetch_tile(0, tbuf[0]);
   __builtin_amdgcn_sched_barrier(0);
-  fetch_batch(cur.first, cur.packed, e_even);
+#pragma unroll
+  for (int q = 0; q < LPW; ++q) fetch_batch(cur[q].first, cur[q].packed, e_even[q]);
   __builtin_amdgcn_sched_barrier(0);
   fetch_tile(1, tbuf[1]);
   __builtin_amdgcn_sched_barrier(0);
   float run = 0.f;
-  auto do_tile = [&](int k, u32x4 (&buf)[2], PlanBatch& e, PlanBatch& e_next) {
+  auto do_tile = [&](int k, u32x4 (&buf)[U], PlanBatch (&e)[LPW], PlanBatch (&e_next)[LPW]) {
     __syncthreads();                                 // previous tile fully consumed (first pass: marg zeroed)
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
-      if (u * MARG_NT + tid < q_tile) *reinterpret_cast<u32x4*>(tile + ((int64_t)u * MARG_NT + tid) * 4) = buf[u];
+    for (int u = 0; u < U; ++u)
+      if (u * NT + tid < q_tile) *reinterpret_cast<u32x4*>(tile + ((int64_t)u * NT + tid) * 4) = buf[u];
     if (LOAD == MARG_ANY && rest > 0 && k == ntiles - 1) {
       __syncthreads();                               // over what a clamped load has left in their unit
       if (tid < rest) tile[n4 * 4 - (int64_t)k * TS + tid] = p_rest;
     }
     __syncthreads();
-    fetch_batch(next.first, next.packed, e_next);
+#pragma unroll
+    for (int q = 0; q < LPW; ++q) fetch_batch(next[q].first, next[q].packed, e_next[q]);
     __builtin_amdgcn_sched_barrier(0);
     fetch_tile(k + 2, buf);
     __builtin_amdgcn_sched_barrier(0);
-    const List after = list_of(k + 2);
-    if (cur.packed) {                                          // wave-uniform: the flag came by a scalar load
-      plan_consume_packed(e.lo, tile, marg);
-    } else {
-      plan_consume(e, tile, marg, run);
-      for (int r = cur.first + PLAN_EB; r < cur.end; r += PLAN_EB) {   // a list longer than one batch (rare: not enough LDS
-        fetch_batch(r, 0, e);                                          // for replicas): fetched on the spot
-        plan_consume(e, tile, marg, run);
+#pragma unroll
+    for (int q = 0; q < LPW; ++q) {
+      const List after = list_of(k + 2, q);
+      if (cur[q].packed) {                                     // wave-uniform: the flag came by a scalar load
+        plan_consume_packed(e[q].lo, tile, marg);
+      } else {
+        plan_consume(e[q], tile, marg, run);
+        for (int r = cur[q].first + PLAN_EB; r < cur[q].end; r += PLAN_EB) {   // a list longer than one batch (rare: not enough LDS
+          fetch_batch(r, 0, e[q]);                                             // for replicas): fetched on the spot
+          plan_consume(e[q], tile, marg, run);
+        }
       }
+      cur[q] = next[q];
+      next[q] = after;
     }
-    cur = next;
-    next = after;
   };
   // unrolled by two: the registers are addressed statically.  No path may enter the loop body with a
   // different set of loads in flight than the others, or every wait falls back to the worst case: an
@@ -248,7 +258,7 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   if (k < ntiles) do_tile(k, tbuf[0], e_even, e_odd);
   __syncthreads();
   // replicas into their id's slot: own slot first, then the replicas in ascending order
-  for (int f = tid; f < p.plan_n_fold; f += MARG_NT) {
+  for (int f = tid; f < p.plan_n_fold; f += NT) {
     const int sid = p.plan_fold[3 * f], first = p.plan_fold[3 * f + 1], cnt = p.plan_fold[3 * f + 2];
     float a = marg[sid];
     for (int j = 0; j < cnt; ++j) a += marg[first + j];
@@ -326,7 +336,7 @@ __global__ __launch_bounds__(MARG_NT) void marginalise_map_kernel(const MargPara
   float* out = p.marg + r * p.marg_stride;
   if (LOAD != MARG_SCALAR && p.plan_ent) {
     float* marg = acc + p.plan_tile + PLAN_ZERO_WORDS;      // the tile sits first: its addresses are then plain offsets
-    accumulate_marginal_planned<LOAD>(p, prow, marg, acc);
+    accumulate_marginal_planned<LOAD, MARG_NT>(p, prow, marg, acc);
     for (int j = threadIdx.x; j < p.Vs; j += MARG_NT) out[j] = p.out_log ? logf(marg[j]) : marg[j];
     return;
   }
@@ -386,7 +396,7 @@ __device__ __forceinline__ void gather_unit(Unit<TagS>& x, const char* srow, con
   gather_unit<TagS>(x, srow, unit_ids(cols, u));
 }
 
-template <class TagS, int NU>
+template <class TagS, int NU, int NT>
 struct StudentRow {
   Unit<TagS> s[NU];
   int64_t nunits;
@@ -394,7 +404,7 @@ struct StudentRow {
     nunits = nu;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      const int64_t u = (int64_t)i * MARG_NT + threadIdx.x;
+      const int64_t u = (int64_t)i * NT + threadIdx.x;
       if (u < nunits) s[i].load(srow, u); else s[i].fill_neg_inf();
     }
   }
@@ -404,7 +414,7 @@ struct StudentRow {
     UnitIds ids[NU];
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      const int64_t u = (int64_t)i * MARG_NT + threadIdx.x;
+      const int64_t u = (int64_t)i * NT + threadIdx.x;
       ids[i] = u < nunits ? unit_ids(cols, u) : UnitIds{int4{-1, -1, -1, -1}, int4{-1, -1, -1, -1}};
     }
 #pragma unroll
@@ -438,13 +448,13 @@ constexpr float XT_OFF = -1e30f;
 // entries above 2^103 would overflow (probabilities are at most 1).
 constexpr float MARG_LOG_SCALE = 0x1p24f, MARG_LOG_SHIFT = 24.f;
 
-template <class TagS, int NU, bool UNIT_T>
+template <class TagS, int NU, int NT, bool UNIT_T>
 __device__ __forceinline__ void rkl_sums_optimistic(Unit<TagS> (&s)[NU], int64_t nunits, float* marg, float a_s, float bs,
                                                     float inv_T_t, float& ss, float& stt, float& w) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < NU; ++i) {
-    const int64_t u = (int64_t)i * MARG_NT + tid;
+    const int64_t u = (int64_t)i * NT + tid;
     if (u < nunits) {
       float sv[8], m[8];
       s[i].unpack(sv);
@@ -477,7 +487,7 @@ __device__ __forceinline__ void rkl_sums_optimistic(Unit<TagS> (&s)[NU], int64_t
 //                                            so that xt can be had back exactly enough from any slot)
 // ss, stt (unless UNIT_T) and w come out multiplied by 2^B.
 constexpr float XS_DEAD = -256.f;
-template <class TagS, int NU, bool UNIT_T>
+template <class TagS, int NU, int NT, bool UNIT_T>
 __device__ __forceinline__ void rkl_sums_stash(Unit<TagS> (&s)[NU], int64_t nunits, float* marg, float a_s, float bs2,
                                                float inv_T_t, float& ss, float& stt, float& w) {
   constexpr float B = Chunk<TagS>::stash_bias;
@@ -485,7 +495,7 @@ __device__ __forceinline__ void rkl_sums_stash(Unit<TagS> (&s)[NU], int64_t nuni
   const float ct = UNIT_T ? B - MARG_LOG_SHIFT : B - MARG_LOG_SHIFT * inv_T_t;
 #pragma unroll
   for (int i = 0; i < NU; ++i) {
-    const int64_t u = (int64_t)i * MARG_NT + tid;
+    const int64_t u = (int64_t)i * NT + tid;
     if (u < nunits) {
       float sv[8], m[8];
       s[i].unpack(sv);
@@ -529,14 +539,14 @@ __device__ __forceinline__ void put_gradient_unit(char* grow, float* marg, int64
   }
 }
 
-template <class TagS, int NU>
+template <class TagS, int NU, int NT>
 __device__ __forceinline__ void rkl_gradient_from_stash(Unit<TagS> (&s)[NU], int64_t nunits, float* marg, float k1,
                                                         float wbar, char* grow, bool to_lds) {
   const int tid = threadIdx.x;
   const float k0 = -k1 * wbar;
 #pragma unroll
   for (int i = 0; i < NU; ++i) {
-    const int64_t u = (int64_t)i * MARG_NT + tid;
+    const int64_t u = (int64_t)i * NT + tid;
     if (u < nunits) {
       float es[8], d[8], g[8];
 #pragma unroll
@@ -551,13 +561,13 @@ __device__ __forceinline__ void rkl_gradient_from_stash(Unit<TagS> (&s)[NU], int
 }
 
 // Pass C on the stored xt (rows whose sums were redone on their maxima).
-template <class TagS, int NU>
+template <class TagS, int NU, int NT>
 __device__ __forceinline__ void rkl_gradient_pass(Unit<TagS> (&s)[NU], int64_t nunits, float* marg, float a_s, float bs,
                                                   float k1, float wbar, char* grow, bool to_lds) {
   const int tid = threadIdx.x;
 #pragma unroll
   for (int i = 0; i < NU; ++i) {
-    const int64_t u = (int64_t)i * MARG_NT + tid;
+    const int64_t u = (int64_t)i * NT + tid;
     if (u < nunits) {
       float sv[8], xt[8], g[8];
       s[i].unpack(sv);
@@ -579,7 +589,7 @@ __device__ __forceinline__ void rkl_gradient_pass(Unit<TagS> (&s)[NU], int64_t n
 // and takes the passes on its maxima like a row without a gradient.
 // Compact rows (p.Vs_full > 0): returns true when the gradient of the compact columns was left in marg for the
 // caller to expand; false when there is none to expand (no gradient asked for, or the row was zero-filled here).
-template <class TagS, int NU>
+template <class TagS, int NU, int NT>
 __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_t nunits, float* marg, float* red,
                                                      const MargParams& p, int64_t r, char* grow, const char* srow) {
   const int tid = threadIdx.x;
@@ -609,7 +619,7 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
         pm = __builtin_elementwise_max(pm, __builtin_bit_cast(i16x2, w16));
       }
     }
-    const float top = block_max<MARG_NT>((float)max((int)pm.x, (int)pm.y), red);      // exact, order-preserving
+    const float top = block_max<NT>((float)max((int)pm.x, (int)pm.y), red);      // exact, order-preserving
     if (top >= 0.f) {                                                                 // the same for every thread
       const unsigned bits = (unsigned)(int)top;
       ms = TagS::id == BF16 ? __uint_as_float(bits << 16) : (float)__builtin_bit_cast(_Float16, (unsigned short)bits);
@@ -624,7 +634,7 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
 #pragma unroll
       for (int e = 0; e < 8; ++e) ms = fmaxf(ms, sv[e]);
     }
-    ms = block_max<MARG_NT>(ms, red);
+    ms = block_max<NT>(ms, red);
   }
   float bs = ms > -INFINITY ? ms * a_s : 0.f;
   float ss = 0.f, stt = 0.f, w = 0.f;
@@ -633,9 +643,9 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
   if (TagS::bytes == 4 || grow) {
     constexpr float B = Chunk<TagS>::stash_bias;
     const float bs2 = bs - B;
-    if (unit_T) rkl_sums_stash<TagS, NU, true>(s, nunits, marg, a_s, bs2, 1.f, ss, stt, w);
-    else rkl_sums_stash<TagS, NU, false>(s, nunits, marg, a_s, bs2, p.inv_T_t, ss, stt, w);
-    block_sum3<MARG_NT>(ss, stt, w, red);
+    if (unit_T) rkl_sums_stash<TagS, NU, NT, true>(s, nunits, marg, a_s, bs2, 1.f, ss, stt, w);
+    else rkl_sums_stash<TagS, NU, NT, false>(s, nunits, marg, a_s, bs2, p.inv_T_t, ss, stt, w);
+    block_sum3<NT>(ss, stt, w, red);
     const float unscale = __uint_as_float((unsigned)(127 - (int)B) << 23);      // 2^-B
     const float ss1 = ss * unscale, stt1 = unit_T ? stt : stt * unscale;
     // 16-bit rows: the stash keeps 2^xs down to 2^-29 of the row's largest entry, on the support or off it.
@@ -645,12 +655,12 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
     if (stash_ok && in_range(ss1) && in_range(stt1)) {      // the same for every thread
       const float wbar = w / ss;
       if (tid == 0 && p.row_loss) p.row_loss[r] = (wbar - fast_log2(ss1) + fast_log2(stt1)) * LN2;
-      if (grow) rkl_gradient_from_stash<TagS, NU>(s, nunits, marg, p.inv_T_s * p.grad_scale * LN2 / ss, wbar, grow, compact);
+      if (grow) rkl_gradient_from_stash<TagS, NU, NT>(s, nunits, marg, p.inv_T_s * p.grad_scale * LN2 / ss, wbar, grow, compact);
       return compact && grow;
     }
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      const int64_t u = (int64_t)i * MARG_NT + tid;
+      const int64_t u = (int64_t)i * NT + tid;
       if (u < nunits) {
         if (compact) gather_unit<TagS>(s[i], srow, p.cols, u);
         else s[i].load(srow, u);
@@ -668,9 +678,9 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
     }
     redo = true;
   } else {
-    if (unit_T) rkl_sums_optimistic<TagS, NU, true>(s, nunits, marg, a_s, bs, 1.f, ss, stt, w);
-    else rkl_sums_optimistic<TagS, NU, false>(s, nunits, marg, a_s, bs, p.inv_T_t, ss, stt, w);
-    block_sum3<MARG_NT>(ss, stt, w, red);
+    if (unit_T) rkl_sums_optimistic<TagS, NU, NT, true>(s, nunits, marg, a_s, bs, 1.f, ss, stt, w);
+    else rkl_sums_optimistic<TagS, NU, NT, false>(s, nunits, marg, a_s, bs, p.inv_T_t, ss, stt, w);
+    block_sum3<NT>(ss, stt, w, red);
     redo = !(in_range(ss) && in_range(stt));      // the same for every thread
   }
   if (redo) {
@@ -678,7 +688,7 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
     ms = -INFINITY;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      const int64_t u = (int64_t)i * MARG_NT + tid;
+      const int64_t u = (int64_t)i * NT + tid;
       if (u < nunits) {
         float sv[8], xt[8];
         s[i].unpack(sv);
@@ -690,17 +700,17 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
         }
       }
     }
-    block_max2<MARG_NT>(tmax, ms, red);
+    block_max2<NT>(tmax, ms, red);
     if (!(tmax > 0.5f * XT_OFF)) {                    // the teacher row carried no mass at all
       if (tid == 0 && p.row_loss) p.row_loss[r] = 0.f;
-      if (grow) zero_row<TagS, MARG_NT>(grow, (compact ? p.Vs_full : p.Vs) / TagS::epc);
+      if (grow) zero_row<TagS, NT>(grow, (compact ? p.Vs_full : p.Vs) / TagS::epc);
       return false;
     }
     bs = ms * a_s;
     ss = 0.f, stt = 0.f, w = 0.f;
 #pragma unroll
     for (int i = 0; i < NU; ++i) {
-      const int64_t u = (int64_t)i * MARG_NT + tid;
+      const int64_t u = (int64_t)i * NT + tid;
       if (u < nunits) {
         float sv[8], xt[8];
         s[i].unpack(sv);
@@ -719,26 +729,26 @@ __device__ __forceinline__ bool rkl_against_marginal(Unit<TagS> (&s)[NU], int64_
         *reinterpret_cast<float4*>(marg + u * 8 + 4) = float4{xt[4], xt[5], xt[6], xt[7]};
       }
     }
-    block_sum3<MARG_NT>(ss, stt, w, red);
+    block_sum3<NT>(ss, stt, w, red);
   }
   const float wbar = w / ss;
   if (tid == 0 && p.row_loss) p.row_loss[r] = (wbar - fast_log2(ss) + fast_log2(stt)) * LN2;
-  if (grow) rkl_gradient_pass<TagS, NU>(s, nunits, marg, a_s, bs, p.inv_T_s * p.grad_scale * LN2 / ss, wbar, grow, compact);
+  if (grow) rkl_gradient_pass<TagS, NU, NT>(s, nunits, marg, a_s, bs, p.inv_T_s * p.grad_scale * LN2 / ss, wbar, grow, compact);
   return compact && grow;
 }
 
 // The gradient of a compact row (fp32 in marg, one value per compact id) into the full-width row: column j takes the
 // value of compact id col_src16[j], or 0; every chunk of the row is written once, by a 16-byte store.
-template <class TagS>
+template <class TagS, int NT>
 __device__ __forceinline__ void expand_gradient_row(const float* marg, const unsigned short* col_src16, int64_t Vs_full, char* grow) {
   using C = Chunk<TagS>;
   constexpr int U = 8;                                   // chunks in flight per thread: their table loads are issued together
   const int64_t nch = Vs_full / C::N;
-  for (int64_t c0 = threadIdx.x; c0 < nch; c0 += (int64_t)U * MARG_NT) {
+  for (int64_t c0 = threadIdx.x; c0 < nch; c0 += (int64_t)U * NT) {
     u32x4 t[U];
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-      const int64_t ch = c0 + (int64_t)j * MARG_NT;
+      const int64_t ch = c0 + (int64_t)j * NT;
       if constexpr (C::N == 8) {
         t[j] = ch < nch ? *reinterpret_cast<const u32x4*>(col_src16 + ch * 8) : u32x4{~0u, ~0u, ~0u, ~0u};
       } else {
@@ -748,7 +758,7 @@ __device__ __forceinline__ void expand_gradient_row(const float* marg, const uns
     }
 #pragma unroll
     for (int j = 0; j < U; ++j) {
-      const int64_t ch = c0 + (int64_t)j * MARG_NT;
+      const int64_t ch = c0 + (int64_t)j * NT;
       if (ch < nch) {
         float g[C::N];
 #pragma unroll
@@ -762,8 +772,8 @@ __device__ __forceinline__ void expand_gradient_row(const float* marg, const uns
   }
 }
 
-template <class TagS, int NU, int LOAD>
-__global__ __launch_bounds__(MARG_NT) void rkl_marginalised_kernel(const MargParams p) {
+template <class TagS, int NU, int LOAD, int NT>
+__global__ __launch_bounds__(NT, 4) void rkl_marginalised_kernel(const MargParams p) {
   extern __shared__ __align__(16) float acc[];
   __shared__ float red[64];
   const int64_t r = xcd_banded_row(blockIdx.x);
@@ -773,11 +783,11 @@ __global__ __launch_bounds__(MARG_NT) void rkl_marginalised_kernel(const MargPar
   const int64_t trow = teacher_row(p.row_map, r, p.n_rows);
   const bool compact = p.Vs_full > 0;
   if (trow < 0) {
-    if (grow) zero_row<TagS, MARG_NT>(grow, (compact ? p.Vs_full : p.Vs) / TagS::epc);
+    if (grow) zero_row<TagS, NT>(grow, (compact ? p.Vs_full : p.Vs) / TagS::epc);
     if (tid == 0 && p.row_loss) p.row_loss[r] = 0.f;
     return;
   }
-  StudentRow<TagS, NU> rows;
+  StudentRow<TagS, NU, NT> rows;
   const char* srow = reinterpret_cast<const char*>(p.logits) + r * p.row_stride * TagS::bytes;
   const int pb = p.p_dtype == F32 ? 4 : 2;
   const char* prow = reinterpret_cast<const char*>(p.probs) + trow * p.p_stride * pb;
@@ -786,15 +796,30 @@ __global__ __launch_bounds__(MARG_NT) void rkl_marginalised_kernel(const MargPar
   if (LOAD != MARG_SCALAR && p.plan_ent) {
     marg = acc + p.plan_tile + PLAN_ZERO_WORDS;  // the tile sits first: its addresses are then plain offsets
     if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
-    accumulate_marginal_planned<LOAD>(p, prow, marg, acc);
-  } else {
+    accumulate_marginal_planned<LOAD, NT>(p, prow, marg, acc);
+  } else if constexpr (NT == MARG_NT) {
     if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
     accumulate_marginal<LOAD>(p, prow, acc, 0, (int)p.Vs);
   }
-  if (rkl_against_marginal<TagS, NU>(rows.s, rows.nunits, marg, red, p, r, grow, srow)) {      // the same for every thread
+  if (rkl_against_marginal<TagS, NU, NT>(rows.s, rows.nunits, marg, red, p, r, grow, srow)) {      // the same for every thread
     __syncthreads();                             // the gradient of every compact column is in LDS
-    expand_gradient_row<TagS>(marg, p.col_src16, p.Vs_full, grow);
+    expand_gradient_row<TagS, NT>(marg, p.col_src16, p.Vs_full, grow);
   }
+}
+
+// Workgroups of half as many threads, each wave walking two of a tile's lists (the plan and the order of its additions are
+// the same), two to a CU where LDS and registers allow it: a row is a chain of phases with a barrier between them and no
+// memory traffic in the last, and one 1024-thread workgroup, alone on its CU, kept the vector ALU 42-44 % busy.  8192
+// rows x 152064 probabilities onto 32000 ids, 3749 / 1986 / 6687 of them in use: 1265 / 1143 / 1297 us with one workgroup per CU,
+// 1136 / 1028 / 1140 with two (5.3-5.9 TB/s); 5842 x 32000 onto 9408 298 -> 210 us.  Up to one row per CU the wider
+// workgroup is ahead (256 rows 41 against 45 us), from there on the two (260 rows 74 and 70, 600 rows 116 and 108).
+// Rows of up to 16384 ids behind the marginal (8192 of fp32 logits) fit the registers.
+constexpr int MARG_HALF_NT = 512, MARG_HALF_ROWS = 256;
+template <class TagS> constexpr int MARG_HALF_NU = TagS::bytes == 4 ? 2 : 4;
+template <class TagS>
+static bool marg_half(const MargParams& p, size_t lds) {
+  if (!p.plan_ent || p.Vs > (int64_t)MARG_HALF_NU<TagS> * 8 * MARG_HALF_NT || lds > 80 * 1024 - 512) return false;
+  return p.n_srows > MARG_HALF_ROWS;
 }
 
 static bool ok16(const void* ptr, int64_t stride, int eb) {
@@ -817,9 +842,11 @@ static void allow_large_lds() {
   allow_large_lds_for(&marginalise_map_kernel<MARG_VEC>);
   allow_large_lds_for(&marginalise_map_kernel<MARG_ANY>);
 #define DL_LARGE_RKLM(TAG)                                                      \
-  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR>);     \
-  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_VEC>);        \
-  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_ANY>)
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR, MARG_NT>);                       \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_VEC, MARG_NT>);                          \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_ANY, MARG_NT>);                          \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_HALF_NU<TAG>, MARG_VEC, MARG_HALF_NT>);           \
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_HALF_NU<TAG>, MARG_ANY, MARG_HALF_NT>)
   DL_LARGE_RKLM(TagF32);
   DL_LARGE_RKLM(TagBF16);
   DL_LARGE_RKLM(TagF16);
@@ -932,18 +959,24 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
   const size_t lds = attach_plan(p, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold, plan_n_extra, load, (size_t)Vs * 4);
   if (load == MARG_ANY && !p.plan_ent) load = MARG_SCALAR;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(xcd_banded_grid(n_rows)), block(MARG_NT);
+  const dim3 grid(xcd_banded_grid(n_rows));
   allow_large_lds();
-#define DL_LAUNCH_RKLM(TAG)                                                                                  \
-  do {                                                                                                       \
-    if (load == MARG_VEC) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_VEC>), grid, block, lds, st, p);        \
-    else if (load == MARG_ANY) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_ANY>), grid, block, lds, st, p);   \
-    else hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR>), grid, block, lds, st, p);                      \
+#define DL_LAUNCH_RKLM_NT(TAG, NU, NT)                                                                                             \
+  do {                                                                                                                            \
+    if (load == MARG_VEC) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, NU, MARG_VEC, NT>), grid, dim3(NT), lds, st, p);        \
+    else hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, NU, MARG_ANY, NT>), grid, dim3(NT), lds, st, p);                         \
+  } while (0)
+#define DL_LAUNCH_RKLM(TAG)                                                                                                        \
+  do {                                                                                                                            \
+    if (load == MARG_SCALAR) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR, MARG_NT>), grid, dim3(MARG_NT), lds, st, p); \
+    else if (marg_half<TAG>(p, lds)) DL_LAUNCH_RKLM_NT(TAG, MARG_HALF_NU<TAG>, MARG_HALF_NT);                                      \
+    else DL_LAUNCH_RKLM_NT(TAG, MARG_NU, MARG_NT);                                                                                 \
   } while (0)
   if (logits_dtype == DL_F32) DL_LAUNCH_RKLM(TagF32);
   else if (logits_dtype == DL_BF16) DL_LAUNCH_RKLM(TagBF16);
   else DL_LAUNCH_RKLM(TagF16);
 #undef DL_LAUNCH_RKLM
+#undef DL_LAUNCH_RKLM_NT
   return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
 }
 

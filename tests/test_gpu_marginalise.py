@@ -450,3 +450,37 @@ def test_a_plan_with_teacher_rows_that_end_inside_a_unit(D, Vt, Vs, shift):
         bound = O.marginal_rkl_gradient_tolerance(grad64, logits, t_logits, rows64, 1.3, 1.3, 1.0 / R, torch.float32, 1e-4)
         err = (grad.cpu().double() - grad64).abs()
         assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("Vt,Vs,used", [(1027, 1000, 300), (8192, 2048, 2048), (24581, 4096, 700), (40000, 16384, 9000)])
+def test_more_rows_than_cus_take_two_workgroups_per_cu(D, Vt, Vs, used, dtype):
+    """More than 256 rows: workgroups of 512 threads that walk two lists per wave and tile (one tile, odd numbers of tiles, a
+    row that ends inside a unit, ids enough for several units per thread), masked rows, the gradient over the logits."""
+    R = 259
+    rng = np.random.default_rng(Vt)
+    ids = rng.permutation(Vs)[:used]
+    t2s = ids[rng.integers(0, used, Vt)].astype(np.int32)
+    t2s[rng.random(Vt) < 0.05] = -1
+    t2s[-1] = ids[0]
+    g = torch.Generator().manual_seed(Vt)
+    probs = torch.softmax(torch.randn(R - 2, Vt, generator=g) * 2, -1)
+    logits = (torch.randn(R, Vs, generator=g) * 2).to(dtype)
+    rm = torch.full((R,), -1, dtype=torch.int32)
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[[0, 200]] = False
+    rm[valid] = torch.arange(R - 2, dtype=torch.int32)
+    ref = O.marginalise_map(probs.numpy(), t2s, Vs)
+    with np.errstate(divide="ignore"):
+        t_logits = O.marginal_to_teacher_logits(torch.tensor(ref))
+    _, rows64, grad64 = O.mean_loss_and_grad("rkl", logits[valid], 1.3, t_logits=t_logits, dtype=torch.float64)
+    x = logits.to(DEV)
+    plan = _map_in_the_form(D, "auto", t2s, Vs)
+    rl, grad = D.vocab_utils.rkl_marginalised(x, probs.to(DEV), plan, row_map=rm.to(DEV), T=1.3, grad_scale=1.0 / (R - 2), grad_out=x)
+    rl, grad = rl.cpu(), grad.cpu()
+    assert torch.count_nonzero(rl[~valid]) == 0 and torch.count_nonzero(grad[~valid]) == 0
+    np.testing.assert_allclose(rl[valid].double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+    bound = O.marginal_rkl_gradient_tolerance(grad64, logits[valid], t_logits, rows64, 1.3, 1.3, 1.0 / (R - 2), dtype,
+                                              1e-4 if dtype == torch.float32 else 2e-3)
+    err = (grad[valid].double() - grad64).abs()
+    assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
