@@ -280,6 +280,16 @@ int dl_composite_forward_fused(const void* logits, int logits_dtype, int64_t row
                                int n_convos, float alpha, float* lse, float* zk, void* row_records,
                                void* row_coef, float* out, void* stream);
 
+/* The same, with the conversations' train_loss (out[c][0]) written a second time to train [n_convos] (may be NULL): a
+ * buffer of their own for callers that hand them on apart from the logged values, without a copy behind the launch. */
+int dl_composite_forward_train(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t V,
+                               const int32_t* row_map, int64_t n_teacher_rows, float inv_T, const void* t_val,
+                               int t_val_dtype, float inv_T_teacher, const void* t_idx, int t_idx_itype, int K,
+                               const int64_t* labels, const void* avoid, int avoid_itype, const int32_t* row_off,
+                               const int32_t* label_off, const int32_t* avoid_off, int offsets_on_host,
+                               int n_convos, float alpha, float* lse, float* zk, void* row_records,
+                               void* row_coef, float* out, float* train, void* stream);
+
 /*
  * Backward of dl_composite_forward for upstream gradients g_train [n_convos] on each conversation's
  * train_loss: g_lse [n_rows] = dL/dlse and g_zk [n_rows, K] = dL/dzk, the inputs of

@@ -70,6 +70,8 @@ _SIGNATURES = {
                                       _P, _P]),
     "dl_composite_forward_fused": (c_int, [_P, c_int, c_int64, c_int64, c_int64, _P, c_int64, c_float, _P, c_int, c_float, _P, c_int, c_int,
                                            _P, _P, c_int, _P, _P, _P, c_int, c_int, c_float, _P, _P, _P, _P, _P, _P]),
+    "dl_composite_forward_train": (c_int, [_P, c_int, c_int64, c_int64, c_int64, _P, c_int64, c_float, _P, c_int, c_float, _P, c_int, c_int,
+                                           _P, _P, c_int, _P, _P, _P, c_int, c_int, c_float, _P, _P, _P, _P, _P, _P, _P]),
     "dl_composite_backward_fused": (c_int, [_P, c_int, c_int64, c_int64, c_int64, _P, c_int64, c_float, _P, c_int, c_float, _P, c_int, c_int,
                                             _P, c_int, c_int, _P, _P, _P, _P, _P, _P, c_int64, _P]),
     "dl_teacher_topk": (c_int, [_P, c_int, c_int64, c_int64, c_int64, _P, c_int64, c_int, _P, c_int, _P, c_int, _P, c_int64, _P]),

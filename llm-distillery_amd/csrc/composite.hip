@@ -84,6 +84,7 @@ __global__ __launch_bounds__(CONVO_NT) void composite_convo_kernel(const Composi
   float* out = p.out + (int64_t)c * 9;
   if (n <= 0) {
     if (tid < 9) out[tid] = NAN;
+    if (tid == 0 && p.train) p.train[c] = NAN;
     return;
   }
   const float alpha = p.alpha;
@@ -146,6 +147,7 @@ __global__ __launch_bounds__(CONVO_NT) void composite_convo_kernel(const Composi
     const float wkl = (float)(a_wkl / n), wrkl = (float)(a_wrkl / n);
     const float total = (wkl + wrkl) * 0.5f;
     out[0] = total;                         // train_loss
+    if (p.train) p.train[c] = total;
     out[1] = total;                         // custom loss
     out[2] = (float)(a_ces / m);            // CE loss
     out[3] = (float)(a_kl / n);             // kl_div

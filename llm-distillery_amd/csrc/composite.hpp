@@ -31,6 +31,7 @@ struct CompositeParams {
   ConvoOffsets off;
   int n_convos; int64_t n_rows; float alpha;
   RowRec* rec; RowCoef* coef; float* out;         // out [C, 9]
+  float* train;                                   // [C], or NULL: out[c][0] once more
   const float* g_train; float* g_lse; float* g_zk;
 };
 

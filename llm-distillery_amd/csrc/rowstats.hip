@@ -581,13 +581,13 @@ extern "C" int dl_rowstats_topk(const void* logits, int logits_dtype, int64_t ro
   return e == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
 }
 
-extern "C" int dl_composite_forward_fused(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t V,
+extern "C" int dl_composite_forward_train(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t V,
                                           const int32_t* row_map, int64_t n_teacher_rows, float inv_T, const void* t_val,
                                           int t_val_dtype, float inv_T_teacher, const void* t_idx, int t_idx_itype, int K,
                                           const int64_t* labels, const void* avoid, int avoid_itype, const int32_t* row_off,
                                           const int32_t* label_off, const int32_t* avoid_off, int offsets_on_host,
                                           int n_convos, float alpha, float* lse, float* zk, void* row_records,
-                                          void* row_coef, float* out, void* stream) {
+                                          void* row_coef, float* out, float* train, void* stream) {
   using namespace dl;
   const int rc = check_common(logits, logits_dtype, row_stride, n_rows, V, t_idx, t_idx_itype, K, n_teacher_rows);
   if (rc != DL_OK) return rc;
@@ -597,6 +597,7 @@ extern "C" int dl_composite_forward_fused(const void* logits, int logits_dtype, 
                                            avoid_itype, row_off, label_off, avoid_off, offsets_on_host, n_convos,
                                            n_teacher_rows, alpha, row_records, row_coef, out);
   if (st0 != DL_OK) return st0;
+  cp.train = train;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int eb = logits_dtype == DL_F32 ? 4 : 2;
   if (n_rows > 0) {
@@ -623,6 +624,19 @@ extern "C" int dl_composite_forward_fused(const void* logits, int logits_dtype, 
   }
   launch_composite_convo(cp, st);
   return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
+}
+
+extern "C" int dl_composite_forward_fused(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t V,
+                                          const int32_t* row_map, int64_t n_teacher_rows, float inv_T, const void* t_val,
+                                          int t_val_dtype, float inv_T_teacher, const void* t_idx, int t_idx_itype, int K,
+                                          const int64_t* labels, const void* avoid, int avoid_itype, const int32_t* row_off,
+                                          const int32_t* label_off, const int32_t* avoid_off, int offsets_on_host,
+                                          int n_convos, float alpha, float* lse, float* zk, void* row_records,
+                                          void* row_coef, float* out, void* stream) {
+  return dl_composite_forward_train(logits, logits_dtype, row_stride, n_rows, V, row_map, n_teacher_rows, inv_T, t_val,
+                                    t_val_dtype, inv_T_teacher, t_idx, t_idx_itype, K, labels, avoid, avoid_itype, row_off,
+                                    label_off, avoid_off, offsets_on_host, n_convos, alpha, lse, zk, row_records, row_coef,
+                                    out, nullptr, stream);
 }
 
 extern "C" int dl_rowcoef_grad_topk(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows,

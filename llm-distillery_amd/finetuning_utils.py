@@ -84,6 +84,11 @@ def _packed_rows(tensors) -> Tensor:
     return torch.as_strided(first, (rows, width) if dim == 2 else (rows,), (width, 1) if dim == 2 else (1,))
 
 
+def _first(t: Tensor, n: int) -> Tensor:
+    """t[:n] without a view where that is all of t."""
+    return t if t.size(0) <= n else t[:n]
+
+
 def _fusable(counts, labels, alpha) -> bool:
     """The fused epilogue covers what the reference's code can run: a Python-number alpha and, per
     conversation, exactly one label fewer than rows (anything else raises inside the reference's
@@ -112,13 +117,16 @@ def _fused_dicts(x: Tensor, row_map, inv_T: float, crop: int, counts, t_vals, t_
         avoid_cat = _packed_rows([a.to(torch.int64) for a in avoids])
     else:
         avoid_cat = avoids[0] if avoids[0].dtype in ops._IT else avoids[0].to(torch.int64)
+    one = {"single": True} if C == 1 else {}
     train, nine = ops.composite_loss(x, _packed_rows(t_vals), _packed_rows(t_idxs), lab_cat, avoid_cat.contiguous(), offs,
-                                     row_map, inv_T, inv_T_teacher, alpha, crop)
+                                     row_map, inv_T, inv_T_teacher, alpha, crop, **one)
     out = []
     for c in range(C):
         row = nine[c]
         d = LossDict(zip(LOSS_KEYS, row.unbind(0)))
-        d["train_loss"] = d["custom loss"] = train[c]      # one tensor under both keys, with its graph, as in the reference
+        # one tensor under both keys, with its graph, as in the reference; a conversation by itself is the node's own output
+        # (a select of it would add a fill and a copy to the backward)
+        d["train_loss"] = d["custom loss"] = train if C == 1 else train[c]
         d.packed, d.keys_packed = row, LOSS_KEYS
         d.batch = (train, nine, c, d["train_loss"], row)
         out.append(d)
@@ -145,16 +153,16 @@ def calculate_divergence(student_logits: Tensor, teacher_logits: Tensor, indices
         raise TypeError("calculate_divergence needs top-K indices: the dense-teacher form of the reference "
                         "composite is not executable (use dense_divergence for dense teachers)")
     n = min(student_logits.size(0), teacher_logits.size(0), indices.size(0))
-    idx = indices[:n]
+    idx = _first(indices, n)
     # Rows beyond n are masked through the row map instead of sliced away: the backward of a slice
     # would zero-fill a second [N, V] buffer and copy the gradient into it.
     row_map = None
     if n < student_logits.size(0):
         row_map = torch.full((student_logits.size(0),), -1, dtype=torch.int32, device=student_logits.device)
         row_map[:n] = torch.arange(n, dtype=torch.int32, device=student_logits.device)
-    labels = convo_CE_tokens[:n]
+    labels = _first(convo_CE_tokens, n)
     if _fusable([n], [labels], alpha) and teacher_logits.dtype in ops._DT:
-        return _fused_dicts(student_logits, row_map, 1.0, 0, [n], [teacher_logits[:n]], [idx], [labels], [avoid_indices], 1.0,
+        return _fused_dicts(student_logits, row_map, 1.0, 0, [n], [_first(teacher_logits, n)], [idx], [labels], [avoid_indices], 1.0,
                             alpha)[0]
     lse, zk = ops.rowstats_topk(student_logits, idx, row_map, 1.0)
     s_sup = zk - lse.unsqueeze(-1)                       # log_softmax over V, gathered at the ids

@@ -172,7 +172,9 @@ class Losses:
         if self._packed is not None:
             if self._train is None:
                 raise KeyError("train_loss")                  # a second backward: the key is gone, as in the reference
-            loss, self._train = self._train / divisor, None
+            loss, self._train = self._train, None
+            if type(divisor) is not int or divisor != 1:
+                loss = loss / divisor
         else:
             loss = self._dict.pop("train_loss") / divisor
         loss.backward()

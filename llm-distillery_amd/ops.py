@@ -3,6 +3,7 @@ stream; all arithmetic happens in the HIP kernels.  No fallbacks: a CPU tensor o
 a missing library raises."""
 from __future__ import annotations
 
+import contextlib
 import ctypes
 from typing import Optional, Tuple
 
@@ -15,8 +16,17 @@ _IT = {torch.int32: _lib.DL_I32, torch.int64: _lib.DL_I64}
 KINDS = {"fkl": _lib.DL_FKL, "rkl": _lib.DL_RKL, "jsd": _lib.DL_JSD}
 
 
+_HERE = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    """`torch.cuda.device(dev)` where that changes anything: entering and leaving it costs a microsecond a launch."""
+    return _HERE if dev.index == torch.cuda.current_device() else torch.cuda.device(dev)
+
+
 def _stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The handle of torch's current stream on `dev` (without the Stream object around it: 0.1 us instead of 1.9)."""
+    return torch._C._cuda_getCurrentRawStream(dev.index)
 
 
 def _dev(t: torch.Tensor, name: str, dev: torch.device | None = None) -> None:
@@ -130,7 +140,7 @@ def div_topk(kind: str, logits: torch.Tensor, t_val: torch.Tensor, t_idx: torch.
     if parts == 16 and want_grad:
         ws_bytes = R * 16 * 20 + 16
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = lib.dl_div_topk(KINDS[kind], x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr,
                              t_val.data_ptr(), _DT[t_val.dtype], t_idx.data_ptr(), _IT[t_idx.dtype], K, N,
                              cnt_ptr, 1.0 / T, 1.0 / (T if teacher_T is None else teacher_T), grad_scale,
@@ -177,7 +187,7 @@ def div_topk_static(kind: str, logits: torch.Tensor, t_val: torch.Tensor, t_idx:
         g_ptr, g_stride = g.data_ptr(), g.stride(0)
     flags = (_lib.DL_TOPK_UNIQUE_IDS if unique_ids else 0) | (_lib.DL_TOPK_NO_WAIT if no_wait else 0) | \
         (parts << _lib.DL_TOPK_PARTS_SHIFT)
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _lib.load().dl_div_topk_static(KINDS[kind], x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr,
                                             t_val.data_ptr(), _DT[t_val.dtype], t_idx.data_ptr(), _IT[t_idx.dtype], K, N,
                                             cnt_ptr, 1.0 / T, 1.0 / (T if teacher_T is None else teacher_T), grad_scale,
@@ -217,7 +227,7 @@ def div_dense(kind: str, logits: torch.Tensor, t_logits: torch.Tensor, *, row_ma
     lib = _lib.load()
     ws_bytes = lib.dl_div_dense_workspace_bytes(KINDS[kind], _DT[x.dtype], _DT[t.dtype], R, V) if split else 0
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = lib.dl_div_dense_ws(KINDS[kind], x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr,
                                  t.data_ptr(), _DT[t.dtype], t.stride(0), N, 1.0 / T,
                                  1.0 / (T if teacher_T is None else teacher_T), grad_scale,
@@ -248,7 +258,7 @@ def _rowstats_raw(x: torch.Tensor, t_idx: torch.Tensor, row_map, inv_T: float):
     make = torch.empty if row_map is None and N == R else torch.zeros
     lse = make(N, dtype=torch.float32, device=x.device)
     zk = make((N, K), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _lib.load().dl_rowstats_topk(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, t_idx.data_ptr(),
                                           _IT[t_idx.dtype], K, N, inv_T, lse.data_ptr(), zk.data_ptr(),
                                           _stream_ptr(x.device))
@@ -268,7 +278,7 @@ def _rowcoef_grad_raw(x: torch.Tensor, t_idx: torch.Tensor, row_map, inv_T: floa
     for name, t in (("t_idx", t_idx), ("lse", lse), ("g_lse", g_lse), ("g_zk", g_zk)):
         _dev(t, name, x.device)
     grad = _grad_target(grad_out, R, V, x.dtype, x.device, like=x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _lib.load().dl_rowcoef_grad_topk(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, t_idx.data_ptr(),
                                               _IT[t_idx.dtype], K, N, inv_T, lse.data_ptr(), g_lse.data_ptr(),
                                               g_zk.data_ptr(), grad.data_ptr(), grad.stride(0),
@@ -349,14 +359,17 @@ def _offsets_arg(offsets):
     return (arr(*offsets[0]), arr(*offsets[1]), arr(*offsets[2])), 1, C
 
 
+def _convos(offsets) -> int:
+    return offsets.shape[1] - 1 if isinstance(offsets, torch.Tensor) else len(offsets[0]) - 1
+
+
 # True: phase 1 and the K-wide epilogue of the composite loss as the two entry points a caller with launches of its own
 # uses (dl_rowstats_topk, dl_composite_forward) instead of the one call that stands for them; the tests compare the two.
 SEPARATE_COMPOSITE_FORWARD = False
 
 
-def _composite_forward_raw(logits, t_val, t_idx, labels, avoid, offsets, row_map, inv_T, inv_T_teacher, alpha, crop, need_grad):
-    """Phase 1 over the logits + the K-wide epilogue: (nine values [C, 9], lse, zk, rec, coef or None)."""
-    x = _cropped(logits, crop)
+def _composite_launch(x, row_map, t_val, t_idx, labels, avoid, offsets, inv_T, inv_T_teacher, alpha, lse, zk, rec, coef, out, train):
+    """The launches of phase 1 and the K-wide epilogue; lse .. coef, train: device addresses (coef, train: or 0)."""
     dev = x.device
     R, V = x.shape
     N, K = t_idx.shape
@@ -365,33 +378,47 @@ def _composite_forward_raw(logits, t_val, t_idx, labels, avoid, offsets, row_map
     if not on_host:      # with offsets on the device the library cannot see that a list is empty and wants both pointers
         labels = labels if labels.numel() else torch.zeros(1, dtype=torch.int64, device=dev)
         avoid = avoid if avoid.numel() else torch.zeros(1, dtype=avoid.dtype, device=dev)
-    # every teacher row is written by phase 1 unless a row map leaves some out or teacher rows outnumber the logits rows
-    make = torch.empty if row_map is None and N == R else torch.zeros
+    rm_ptr = row_map.data_ptr() if row_map is not None else 0
+    stream = _stream_ptr(dev)
+    with _on(dev):
+        if SEPARATE_COMPOSITE_FORWARD:
+            st = lib.dl_rowstats_topk(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, t_idx.data_ptr(), _IT[t_idx.dtype],
+                                      K, N, inv_T, lse, zk, stream)
+            _lib.check(st, "dl_rowstats_topk")
+            st = lib.dl_composite_forward(
+                lse, zk, t_val.data_ptr(), _DT[t_val.dtype], inv_T_teacher, t_idx.data_ptr(),
+                _IT[t_idx.dtype], K, labels.data_ptr() if labels.numel() else 0, avoid.data_ptr() if avoid.numel() else 0,
+                _IT[avoid.dtype], offs[0], offs[1], offs[2], on_host, C, N, alpha, rec, coef, out.data_ptr(), stream)
+            _lib.check(st, "dl_composite_forward")
+            if train is not None:
+                train.copy_(out[:, 0].view(train.shape))
+        else:
+            st = lib.dl_composite_forward_train(
+                x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, N, inv_T, t_val.data_ptr(), _DT[t_val.dtype],
+                inv_T_teacher, t_idx.data_ptr(), _IT[t_idx.dtype], K, labels.data_ptr() if labels.numel() else 0,
+                avoid.data_ptr() if avoid.numel() else 0, _IT[avoid.dtype], offs[0], offs[1], offs[2], on_host, C, alpha,
+                lse, zk, rec, coef, out.data_ptr(), train.data_ptr() if train is not None else 0, stream)
+            _lib.check(st, "dl_composite_forward_train")
+
+
+def _all_rows_written(x, t_idx, row_map) -> bool:
+    """Every teacher row is written by phase 1 unless a row map leaves some out or teacher rows outnumber the logits rows."""
+    return row_map is None and t_idx.shape[0] == x.shape[0]
+
+
+def _composite_forward_raw(logits, t_val, t_idx, labels, avoid, offsets, row_map, inv_T, inv_T_teacher, alpha, crop, need_grad):
+    """Phase 1 over the logits + the K-wide epilogue: (nine values [C, 9], lse, zk, rec, coef or None)."""
+    x = _cropped(logits, crop)
+    dev = x.device
+    N, K = t_idx.shape
+    make = torch.empty if _all_rows_written(x, t_idx, row_map) else torch.zeros
     lse = make(N, dtype=torch.float32, device=dev)
     zk = make((N, K), dtype=torch.float32, device=dev)
     rec = torch.empty((N, 8), dtype=torch.float32, device=dev)
     coef = torch.empty((N, 4), dtype=torch.float32, device=dev) if need_grad else None
-    out = torch.empty((C, 9), dtype=torch.float32, device=dev)
-    rm_ptr = row_map.data_ptr() if row_map is not None else 0
-    stream = _stream_ptr(dev)
-    with torch.cuda.device(dev):
-        if SEPARATE_COMPOSITE_FORWARD:
-            st = lib.dl_rowstats_topk(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, t_idx.data_ptr(), _IT[t_idx.dtype],
-                                      K, N, inv_T, lse.data_ptr(), zk.data_ptr(), stream)
-            _lib.check(st, "dl_rowstats_topk")
-            st = lib.dl_composite_forward(
-                lse.data_ptr(), zk.data_ptr(), t_val.data_ptr(), _DT[t_val.dtype], inv_T_teacher, t_idx.data_ptr(),
-                _IT[t_idx.dtype], K, labels.data_ptr() if labels.numel() else 0, avoid.data_ptr() if avoid.numel() else 0,
-                _IT[avoid.dtype], offs[0], offs[1], offs[2], on_host, C, N, alpha, rec.data_ptr(),
-                coef.data_ptr() if need_grad else 0, out.data_ptr(), stream)
-            _lib.check(st, "dl_composite_forward")
-        else:
-            st = lib.dl_composite_forward_fused(
-                x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, N, inv_T, t_val.data_ptr(), _DT[t_val.dtype],
-                inv_T_teacher, t_idx.data_ptr(), _IT[t_idx.dtype], K, labels.data_ptr() if labels.numel() else 0,
-                avoid.data_ptr() if avoid.numel() else 0, _IT[avoid.dtype], offs[0], offs[1], offs[2], on_host, C, alpha,
-                lse.data_ptr(), zk.data_ptr(), rec.data_ptr(), coef.data_ptr() if need_grad else 0, out.data_ptr(), stream)
-            _lib.check(st, "dl_composite_forward_fused")
+    out = torch.empty((_convos(offsets), 9), dtype=torch.float32, device=dev)
+    _composite_launch(x, row_map, t_val, t_idx, labels, avoid, offsets, inv_T, inv_T_teacher, alpha, lse.data_ptr(), zk.data_ptr(),
+                      rec.data_ptr(), coef.data_ptr() if need_grad else 0, out, None)
     return out, lse, zk, rec, coef
 
 
@@ -401,7 +428,8 @@ FORCE_COMPOSITE_BACKWARD = None
 
 
 def _composite_backward_raw(logits, t_val, t_idx, lse, zk, rec, coef, g_train, offsets, row_map, inv_T, inv_T_teacher, crop):
-    """The epilogue's backward + phase 2: d(sum_c g_train[c] * train_loss[c]) / d logits, full width."""
+    """The epilogue's backward + phase 2: d(sum_c g_train[c] * train_loss[c]) / d logits, full width; lse .. coef: device
+    addresses of what the forward left."""
     x = _cropped(logits, crop)
     dev = x.device
     R, V = x.shape
@@ -419,25 +447,25 @@ def _composite_backward_raw(logits, t_val, t_idx, lse, zk, rec, coef, g_train, o
     # fp32 rows, K = 400) and costs beyond (4.01 against 3.95 ms on 32768 x 128256 bf16 rows, K = 200: eight parts)
     fused = V * x.element_size() <= 4 * 32768 if FORCE_COMPOSITE_BACKWARD is None else FORCE_COMPOSITE_BACKWARD == "fused"
     if fused:
-        with torch.cuda.device(dev):
+        with _on(dev):
             st = lib.dl_composite_backward_fused(
                 x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, row_map.data_ptr() if row_map is not None else 0, N, inv_T,
                 t_val.data_ptr(), _DT[t_val.dtype], inv_T_teacher,
-                t_idx.data_ptr(), _IT[t_idx.dtype], K, offs[0], on_host, C, lse.data_ptr(), zk.data_ptr(), rec.data_ptr(),
-                coef.data_ptr(), g.data_ptr(), gx.data_ptr(), gx.stride(0), stream)
+                t_idx.data_ptr(), _IT[t_idx.dtype], K, offs[0], on_host, C, lse, zk, rec,
+                coef, g.data_ptr(), gx.data_ptr(), gx.stride(0), stream)
             _lib.check(st, "dl_composite_backward_fused")
         return grad
-    g_lse = torch.empty_like(lse)
-    g_zk = torch.empty_like(zk)
-    with torch.cuda.device(dev):
+    g_state = torch.empty(N * (K + 1), dtype=torch.float32, device=dev)
+    g_zk = g_state.data_ptr()
+    g_lse = g_zk + 4 * N * K
+    with _on(dev):
         st = lib.dl_composite_backward(
-            lse.data_ptr(), zk.data_ptr(), t_val.data_ptr(), _DT[t_val.dtype], inv_T_teacher, t_idx.data_ptr(),
-            _IT[t_idx.dtype], K, offs[0], on_host, C, N, rec.data_ptr(), coef.data_ptr(), g.data_ptr(),
-            g_lse.data_ptr(), g_zk.data_ptr(), stream)
+            lse, zk, t_val.data_ptr(), _DT[t_val.dtype], inv_T_teacher, t_idx.data_ptr(),
+            _IT[t_idx.dtype], K, offs[0], on_host, C, N, rec, coef, g.data_ptr(), g_lse, g_zk, stream)
         _lib.check(st, "dl_composite_backward")
         st = lib.dl_rowcoef_grad_topk(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V,
                                       row_map.data_ptr() if row_map is not None else 0, t_idx.data_ptr(),
-                                      _IT[t_idx.dtype], K, N, inv_T, lse.data_ptr(), g_lse.data_ptr(), g_zk.data_ptr(),
+                                      _IT[t_idx.dtype], K, N, inv_T, lse, g_lse, g_zk,
                                       gx.data_ptr(), gx.stride(0), stream)
         _lib.check(st, "dl_rowcoef_grad_topk")
     return grad
@@ -455,31 +483,47 @@ class _CompositeLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, logits, t_val, t_idx, labels, avoid, offsets, row_map, inv_T: float, inv_T_teacher: float,
-                alpha: float, crop: int):
+                alpha: float, crop: int, single: bool = False):
         need_grad = ctx.needs_input_grad[0]          # False under torch.no_grad() (the validation loop) and for detached logits
-        out, lse, zk, rec, coef = _composite_forward_raw(logits, t_val, t_idx, labels, avoid, offsets, row_map, inv_T,
-                                                         inv_T_teacher, alpha, crop, need_grad)
+        x = _cropped(logits, crop)
+        dev = x.device
+        N, K = t_idx.shape
+        C = _convos(offsets)
+        # one buffer for what the rows leave behind: records [N, 8], coefficients [N, 4], zk [N, K], lse [N]
+        make = torch.empty if _all_rows_written(x, t_idx, row_map) else torch.zeros
+        state = make(N * (K + 13), dtype=torch.float32, device=dev)
+        out = torch.empty((C, 9), dtype=torch.float32, device=dev)
+        # its own storage: the differentiable output must not alias the logged one; `single`: 0-dim, one conversation
+        train = torch.empty(() if single else (C,), dtype=torch.float32, device=dev)
+        lse, zk, rec, coef = _state_addresses(state, N, K)
+        _composite_launch(x, row_map, t_val, t_idx, labels, avoid, offsets, inv_T, inv_T_teacher, alpha, lse, zk, rec,
+                          coef if need_grad else 0, out, train)
         if need_grad:
             on_host = not isinstance(offsets, torch.Tensor)
-            ctx.save_for_backward(logits, t_val, t_idx, lse, zk, rec, coef, *([row_map] if row_map is not None else []),
+            ctx.save_for_backward(logits, t_val, t_idx, state, *([row_map] if row_map is not None else []),
                                   *([] if on_host else [offsets]))
             ctx.host_offsets = offsets if on_host else None
             ctx.has_map = row_map is not None
             ctx.scalars = (inv_T, inv_T_teacher, crop)
-        train = out[:, 0].clone()      # its own storage: the differentiable output must not alias the logged one
         ctx.mark_non_differentiable(out)
         return train, out
 
     @staticmethod
     def backward(ctx, g_train, _g_logged):
         saved = ctx.saved_tensors
-        logits, t_val, t_idx, lse, zk, rec, coef = saved[:7]
-        row_map = saved[7] if ctx.has_map else None
+        logits, t_val, t_idx, state = saved[:4]
+        row_map = saved[4] if ctx.has_map else None
         offsets = ctx.host_offsets if ctx.host_offsets is not None else saved[-1]
         inv_T, inv_T_teacher, crop = ctx.scalars
-        grad = _composite_backward_raw(logits, t_val, t_idx, lse, zk, rec, coef, g_train, offsets, row_map, inv_T,
-                                       inv_T_teacher, crop)
-        return (grad,) + (None,) * 10
+        grad = _composite_backward_raw(logits, t_val, t_idx, *_state_addresses(state, *t_idx.shape), g_train, offsets, row_map,
+                                       inv_T, inv_T_teacher, crop)
+        return (grad,) + (None,) * 11
+
+
+def _state_addresses(state, N, K):
+    """(lse, zk, rec, coef) inside the buffer of _CompositeLoss.forward."""
+    rec = state.data_ptr()
+    return rec + 4 * N * (12 + K), rec + 48 * N, rec, rec + 32 * N
 
 
 # The same two halves as registered operators (torch.library): visible to torch.compile, FakeTensor tracing and
@@ -508,7 +552,8 @@ def _(logits, t_val, t_idx, labels, avoid, offsets, row_map, inv_T, inv_T_teache
 def composite_backward_op(logits: torch.Tensor, t_val: torch.Tensor, t_idx: torch.Tensor, lse: torch.Tensor, zk: torch.Tensor,
                           rec: torch.Tensor, coef: torch.Tensor, g_train: torch.Tensor, offsets: torch.Tensor,
                           row_map: Optional[torch.Tensor], inv_T: float, inv_T_teacher: float, crop: int = 0) -> torch.Tensor:
-    return _composite_backward_raw(logits, t_val, t_idx, lse, zk, rec, coef, g_train, offsets, row_map, inv_T, inv_T_teacher, crop)
+    return _composite_backward_raw(logits, t_val, t_idx, lse.data_ptr(), zk.data_ptr(), rec.data_ptr(), coef.data_ptr(), g_train,
+                                   offsets, row_map, inv_T, inv_T_teacher, crop)
 
 
 @composite_backward_op.register_fake
@@ -540,8 +585,8 @@ composite_forward_op.register_autograd(_composite_op_backward, setup_context=_co
 
 def composite_loss(logits: torch.Tensor, t_val: torch.Tensor, t_idx: torch.Tensor, labels: torch.Tensor,
                    avoid: torch.Tensor, offsets, row_map: Optional[torch.Tensor], inv_T: float, inv_T_teacher: float,
-                   alpha: float, crop: int = 0) -> Tuple[torch.Tensor, torch.Tensor]:
-    """(train_loss [C], nine values [C, 9]) of C conversations straight from the logits [rows, V]:
+                   alpha: float, crop: int = 0, single: bool = False) -> Tuple[torch.Tensor, torch.Tensor]:
+    """(train_loss [C] -- `single`: of the one conversation, 0-dim --, nine values [C, 9]) of C conversations straight from the logits [rows, V]:
     `t_val` / `t_idx` [N, K] the stored teacher rows of all conversations back to back, `labels` int64
     and `avoid` int32 / int64 concatenated, `offsets` = three host lists (first row, first label,
     first ignore entry of every conversation, C + 1 entries each; C <= DL_MAX_HOST_CONVOS) or a device
@@ -573,19 +618,19 @@ def composite_loss(logits: torch.Tensor, t_val: torch.Tensor, t_idx: torch.Tenso
             offsets = torch.tensor(offsets, dtype=torch.int32, device=dev)
         res = composite_forward_op(logits, t_val, t_idx, labels, avoid, offsets, row_map, float(inv_T), float(inv_T_teacher),
                                    float(alpha), int(crop))
-        return res[0], res[1].detach()
+        return res[0][0] if single else res[0], res[1].detach()
     return _CompositeLoss.apply(logits, t_val, t_idx, labels, avoid, offsets, row_map, float(inv_T), float(inv_T_teacher),
-                                float(alpha), int(crop))
+                                float(alpha), int(crop), single)
 
 
 def reduce_sum(values: torch.Tensor, scale: float = 1.0) -> torch.Tensor:
     """Deterministic sum(values) * scale as a 0-d fp32 tensor."""
     _dev(values, "values")
-    v = values.contiguous().view(-1)
+    v = values if values.dim() == 1 and values.is_contiguous() else values.contiguous().view(-1)
     if v.dtype != torch.float32:
         raise RuntimeError("reduce_sum takes fp32 values")
     out = torch.empty((), dtype=torch.float32, device=v.device)
-    with torch.cuda.device(v.device):
+    with _on(v.device):
         st = _lib.load().dl_reduce_sum(v.data_ptr(), v.numel(), scale, out.data_ptr(), _stream_ptr(v.device))
     _lib.check(st, "dl_reduce_sum")
     return out
@@ -597,7 +642,7 @@ def copy16(src: torch.Tensor, dst: torch.Tensor) -> None:
     n = src.numel() * src.element_size()
     if not (src.is_contiguous() and dst.is_contiguous()) or dst.numel() * dst.element_size() != n:
         raise RuntimeError("copy16 needs two contiguous buffers of the same byte size")
-    with torch.cuda.device(src.device):
+    with _on(src.device):
         st = _lib.load().dl_copy16(src.data_ptr(), dst.data_ptr(), n, _stream_ptr(src.device))
     _lib.check(st, "dl_copy16")
 
@@ -614,7 +659,7 @@ def copy_rows(src: torch.Tensor, dst: torch.Tensor, threads: int, chunks: int, p
     if not 0 <= int(lds_kb) <= 64:
         raise ValueError("lds_kb must be 0..64")
     flags = (1 if parts_on_one_xcd else 0) | (2 if wave_major else 0) | (int(lds_kb) << 8)
-    with torch.cuda.device(src.device):
+    with _on(src.device):
         st = _lib.load().dl_copy_rows(src.data_ptr(), dst.data_ptr(), src.shape[0], src.shape[1] * src.element_size(), int(threads),
                                       int(chunks), flags, _stream_ptr(src.device))
     _lib.check(st, "dl_copy_rows")

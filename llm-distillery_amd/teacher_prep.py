@@ -9,7 +9,7 @@ from typing import Sequence
 import torch
 
 from . import _lib, ops
-from .ops import _DT, _IT, _dev, _stream_ptr
+from .ops import _DT, _IT, _dev, _on, _stream_ptr
 
 
 def _ptr_array(tensors: Sequence[torch.Tensor]):
@@ -52,7 +52,7 @@ def merge_remap_topk(vals: Sequence[torch.Tensor], idxs: Sequence[torch.Tensor],
     out_lm = torch.empty((N, E), dtype=torch.float32, device=dev)
     out_cnt = torch.empty((N,), dtype=torch.int32, device=dev)
     w = (ctypes.c_float * n)(*[float(x) for x in weights])
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _lib.load().dl_merge_remap_topk(n, _ptr_array(vals), _ptr_array(idxs), _DT[vals[0].dtype],
                                              _IT[idxs[0].dtype], K, w, N,
                                              id_map.data_ptr() if id_map is not None else 0,
@@ -78,7 +78,7 @@ def merge_topk_pair(disk_val: torch.Tensor, disk_idx: torch.Tensor, new_val: tor
     dev = disk_val.device
     out_lm = torch.empty((n, K), dtype=torch.float32, device=dev)
     out_idx = torch.empty((n, K), dtype=torch.int64, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _lib.load().dl_merge_topk_pair(disk_val.data_ptr(), disk_idx.data_ptr(), disk_val.shape[0],
                                             new_val.data_ptr(), new_idx.data_ptr(), new_val.shape[0],
                                             _DT[disk_val.dtype], _IT[disk_idx.dtype], K, int(vocab),
@@ -161,7 +161,7 @@ def _fkl_multi_fused(logits, vals, idxs, weights, id_map, row_map, T, grad_scale
         flags |= _lib.DL_TOPK_ANY_ROWS
     ws_bytes = lib.dl_fkl_multi_teacher_workspace_bytes(_DT[x.dtype], R, V, n, K, N, flags)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = lib.dl_fkl_multi_teacher(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rm_ptr, n, _ptr_array(vals),
                                       _ptr_array(idxs), _DT[vals[0].dtype], _IT[idxs[0].dtype], K, N, w, map_ptr,
                                       id_map.numel() if id_map is not None else 0, 1.0 / T, grad_scale,
@@ -195,7 +195,7 @@ def teacher_topk(logits: torch.Tensor, K: int, *, crop_to_size: int | None = Non
     out_i = torch.empty((n_out, K), dtype=idx_dtype, device=dev)
     lib = _lib.load()
     ws = torch.empty((max(16, lib.dl_teacher_topk_workspace_bytes(_DT[x.dtype], n_out, V, K)),), dtype=torch.uint8, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = lib.dl_teacher_topk(x.data_ptr(), _DT[x.dtype], x.stride(0), R, V, rl_ptr, n_out, K,
                                  out_v.data_ptr(), _DT[val_dtype], out_i.data_ptr(), _IT[idx_dtype],
                                  ws.data_ptr(), ws.numel(), _stream_ptr(dev))

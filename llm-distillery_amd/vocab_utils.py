@@ -16,7 +16,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .ops import _DT, _dev, _grad_target, _opt_i32, _rows_2d, _stream_ptr
+from .ops import _DT, _dev, _grad_target, _opt_i32, _rows_2d, _on, _stream_ptr
 
 
 def _pack(vocab: Sequence[bytes]):
@@ -180,7 +180,7 @@ def marginalise(probs: torch.Tensor, *, t2s: torch.Tensor | None = None, csr=Non
         raise ValueError("marginalise needs one of plan=, t2s= or csr=")
     out = torch.empty((R, n_student), dtype=torch.float32, device=x.device)
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         if csr is not None:
             off, ind = csr
             _dev(off, "offsets", x.device), _dev(ind, "indices", x.device)
@@ -217,7 +217,7 @@ def gather_columns(x: torch.Tensor, cols: torch.Tensor) -> torch.Tensor:
     R, V = x.shape
     out = torch.empty((R, cols.numel()), dtype=x.dtype, device=x.device)
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         for a in range(0, R, 65535):
             n = min(65535, R - a)
             st = lib.dl_gather_columns(x[a:].data_ptr(), _DT[x.dtype], x.stride(0), n, V, cols.data_ptr(), cols.numel(),
@@ -232,7 +232,7 @@ def expand_columns(xc: torch.Tensor, col_src: torch.Tensor, V: int, out: torch.T
     if out is None:
         out = torch.empty((R, V), dtype=xc.dtype, device=xc.device)
     lib = _lib.load()
-    with torch.cuda.device(xc.device):
+    with _on(xc.device):
         for a in range(0, R, 65535):
             m = min(65535, R - a)
             st = lib.dl_expand_columns(xc[a:].data_ptr(), _DT[xc.dtype], xc.stride(0), m, n, col_src.data_ptr(), V,
@@ -270,7 +270,7 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
             if want_grad:
                 grad = _grad_target(grad_out, R, Vs, x.dtype, dev)
                 g_ptr, g_stride = grad.data_ptr(), grad.stride(0)
-            with torch.cuda.device(dev):
+            with _on(dev):
                 st = _lib.load().dl_rkl_marginalised_compact(
                     x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, plan.cols.data_ptr(), plan.col_src16.data_ptr(),
                     plan.n_compact, rm_ptr, tp.data_ptr(), _DT[tp.dtype], tp.stride(0), N, Vt, plan.t2c.data_ptr(),
@@ -294,7 +294,7 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
     if want_grad:
         grad = _grad_target(grad_out, R, Vs, x.dtype, dev)
         g_ptr, g_stride = grad.data_ptr(), grad.stride(0)
-    with torch.cuda.device(dev):
+    with _on(dev):
         st = _lib.load().dl_rkl_marginalised(x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, rm_ptr, tp.data_ptr(),
                                              _DT[tp.dtype], tp.stride(0), N, Vt, t2s.data_ptr(), *plan_args, 1.0 / T,
                                              1.0 / (T if teacher_T is None else teacher_T), grad_scale,
