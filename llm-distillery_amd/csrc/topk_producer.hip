@@ -901,8 +901,8 @@ __host__ __device__ inline int producer_select_cands(int K) {
 __host__ __device__ inline int producer_select_groups(int K) { return 2 * K > 512 ? 2 * K : 512; }
 // Dynamic LDS of topk_select_kernel: the group maxima of all parts, later the candidate words; the selected
 // words; the list of groups to open.
-__host__ __device__ inline size_t producer_select_lds(int K, int parts, int key_bytes, int G) {
-  const size_t maxima = (size_t)parts * G * PROD_NT * key_bytes, cands = (size_t)producer_select_cands(K) * 8;
+__host__ __device__ inline size_t producer_select_lds(int K, int parts, int key_bytes, int G, bool maxima_in_lds = true) {
+  const size_t maxima = maxima_in_lds ? (size_t)parts * G * PROD_NT * key_bytes : 0, cands = (size_t)producer_select_cands(K) * 8;
   return ((maxima > cands ? maxima : cands) + 15) / 16 * 16 + (size_t)producer_sel_cap(K) * 8 + (size_t)producer_select_groups(K) * 4;
 }
 
@@ -913,7 +913,9 @@ __host__ __device__ inline size_t producer_select_lds(int K, int parts, int key_
 // Against thresholds per part this opens a quarter of the groups when a row has four parts, and the part kernel,
 // bound by vector-ALU issue, sheds its collection stage (a third of its instructions) for 20 % more bytes fetched.
 // MAXR > 0: the group maxima stay in the threads' registers (MAXR rounds of 16 bytes per thread: every pass over them
-// then costs no LDS access and no address arithmetic); MAXR == 0: any number of them, in LDS.
+// then costs no LDS access and no address arithmetic, and the LDS holds more workgroups per CU); MAXR == 0: any number of
+// them, in LDS.  Eight rounds serve the four-byte rows of 4097 to 8192 groups: 5734 x 131072 fp32, K = 357, 743 -> 643 us
+// for the whole call, 10707 x 100277, K = 114, 873 -> 789, 4096 x 128256, K = 200, 471 -> 429.
 template <class Tag, int G, bool ALIGNED, int MAXR>
 __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -930,7 +932,8 @@ __global__ __launch_bounds__(256) void topk_select_kernel(const ProducerParams p
   const int P = p.parts, K = p.K;
   const int n_g = P * GPP;
   const int acap = producer_select_cands(K), qcap = producer_select_groups(K), sel_cap = producer_sel_cap(K);
-  const size_t region = (((size_t)n_g * sizeof(KS) > (size_t)acap * 8 ? (size_t)n_g * sizeof(KS) : (size_t)acap * 8) + 15) / 16 * 16;
+  const size_t maxima = MAXR > 0 ? 0 : (size_t)n_g * sizeof(KS);      // as producer_select_lds lays it out
+  const size_t region = ((maxima > (size_t)acap * 8 ? maxima : (size_t)acap * 8) + 15) / 16 * 16;
   KS* gmax = reinterpret_cast<KS*>(smem_raw);
   u64* all = reinterpret_cast<u64*>(smem_raw);                      // takes the place of the maxima
   unsigned* all32 = reinterpret_cast<unsigned*>(smem_raw);          // the same list in narrow words
@@ -1243,9 +1246,13 @@ static void launch_producer_shape(const ProducerParams& p, bool select, hipStrea
     return;
   }
   hipLaunchKernelGGL((topk_part_kernel<Tag, G, ALIGNED, PART_LIGHT>), grid, dim3(PROD_NT), 0, st, p);
-  // the maxima of a row in the selection's registers where four rounds of 16 bytes per thread hold them
-  if ((size_t)p.parts * G * PROD_NT * sizeof(typename Keys<Tag>::Stored) <= (size_t)4 * 256 * 16)
-    hipLaunchKernelGGL((topk_select_kernel<Tag, G, ALIGNED, 4>), dim3((unsigned)p.n_out), dim3(256), lds_select, st, p);
+  // the maxima of a row in the selection's registers where four (eight) rounds of 16 bytes per thread hold them
+  const size_t maxima = (size_t)p.parts * G * PROD_NT * sizeof(typename Keys<Tag>::Stored);
+  const size_t lds_regs = producer_select_lds(p.K, p.parts, Tag::bytes == 4 ? 4 : 2, G, false);
+  if (maxima <= (size_t)4 * 256 * 16)
+    hipLaunchKernelGGL((topk_select_kernel<Tag, G, ALIGNED, 4>), dim3((unsigned)p.n_out), dim3(256), lds_regs, st, p);
+  else if (Tag::bytes == 4 && maxima <= (size_t)8 * 256 * 16)
+    hipLaunchKernelGGL((topk_select_kernel<Tag, G, ALIGNED, Tag::bytes == 4 ? 8 : 4>), dim3((unsigned)p.n_out), dim3(256), lds_regs, st, p);
   else
     hipLaunchKernelGGL((topk_select_kernel<Tag, G, ALIGNED, 0>), dim3((unsigned)p.n_out), dim3(256), lds_select, st, p);
   // the rows handed back (none, as a rule: the workgroups then leave at once)

@@ -229,3 +229,9 @@ def test_producer_limits(D):
         D.teacher_topk(torch.zeros(2, 4096, device=DEV), 2000)
     with pytest.raises(RuntimeError):
         D.teacher_topk(torch.zeros(2, 100, device=DEV), 101)              # K > V
+
+
+@pytest.mark.parametrize("V,pitch,K", [(65537, 65540, 100), (81920, 81920, 357), (131071, 131071, 200), (131072, 131072, 512)])
+def test_four_byte_rows_of_five_to_eight_parts(D, V, pitch, K):
+    """More chunk groups than four rounds of the selection's registers hold (5 parts: 5120, 8 parts: 8192 of 8192)."""
+    test_borders_of_the_rules_for_groups_and_rows_off_the_grid(D, torch.float32, V, pitch, K)
