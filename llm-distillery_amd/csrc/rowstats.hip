@@ -498,31 +498,56 @@ static bool same_phase16(const void* a, int64_t stride_a, const void* b, int64_t
   return reinterpret_cast<uintptr_t>(a) % 16 == reinterpret_cast<uintptr_t>(b) % 16 && ((stride_a - stride_b) * eb) % 16 == 0;
 }
 
+// Threads per row in phase 1.  256 of them keep 16 KiB of a row in flight, eight rows to a CU, and their 64 rounds hold
+// 16384 chunks.  Rows wider than that take 1024, whose rounds hold them: no gathers, no launch for the rows' records, and a
+// longer share of the row in flight (phase 1 and records: 2048 x 75487 fp32 112 -> 105 us, 2048 x 151665 fp32 216 -> 198, 4084 x
+// 151665 bf16, half of them content rows, 152 -> 143; 512 threads measure the same on the first and 209 / 148 on the others).
+// Up to two rows per CU the chip is better filled by 512 threads each (131 x 32000 fp32 14.9 -> 11.7 us, 434 rows 18.1 ->
+// 16.4; 700 rows 20.7 -> 22.0).
+static int stats_threads(int64_t n_rows, int64_t V, int epc) {
+  const int64_t chunks = (V + epc - 1) / epc;
+  if (chunks > (int64_t)STASH_ROUNDS * 256 && chunks <= (int64_t)STASH_ROUNDS * 1024) return 1024;
+  return n_rows <= 512 ? 512 : 256;
+}
+// the logits at the teacher's ids out of the sweep where the row's chunks fit the threads' 64 rounds (the bound holds
+// for every row: a peeled head only shortens the body)
+static bool stash_fits(int mode, int K, int64_t V, int epc, int64_t n_rows) {
+  return mode != 0 && K <= STASH_MAX_K && (V + epc - 1) / epc <= (int64_t)STASH_ROUNDS * stats_threads(n_rows, V, epc);
+}
 // phase 1 with the rows' records of the composite loss made at its tail (the caller has checked stash_fits)
-static bool stash_fits(int mode, int K, int64_t V, int epc) {
-  return mode != 0 && K <= STASH_MAX_K && (V + epc - 1) / epc <= (int64_t)STASH_ROUNDS * 256;
+template <class Tag, int NT>
+static void launch_stats_record_nt(const StatsParams& p, int mode, const CompositeParams& cp, hipStream_t st) {
+  const size_t lds = (size_t)p.K * 16;
+  const dim3 grid((unsigned)p.n_rows), block(NT);
+  if (mode == 1) hipLaunchKernelGGL((rowstats_record_kernel<Tag, NT, 1>), grid, block, lds, st, p, cp);
+  else hipLaunchKernelGGL((rowstats_record_kernel<Tag, NT, 2>), grid, block, lds, st, p, cp);
 }
 template <class Tag>
 static hipError_t launch_stats_record(const StatsParams& p, int mode, const CompositeParams& cp, hipStream_t st) {
-  const size_t lds = (size_t)p.K * 16;
-  const dim3 grid((unsigned)p.n_rows), block(256);
-  if (mode == 1) hipLaunchKernelGGL((rowstats_record_kernel<Tag, 256, 1>), grid, block, lds, st, p, cp);
-  else hipLaunchKernelGGL((rowstats_record_kernel<Tag, 256, 2>), grid, block, lds, st, p, cp);
+  const int nt = stats_threads(p.n_rows, p.V, Tag::epc);
+  if (nt == 1024) launch_stats_record_nt<Tag, 1024>(p, mode, cp, st);
+  else if (nt == 512) launch_stats_record_nt<Tag, 512>(p, mode, cp, st);
+  else launch_stats_record_nt<Tag, 256>(p, mode, cp, st);
   return hipGetLastError();
 }
 
+template <class Tag, int NT>
+static void launch_stats_nt(const StatsParams& p, int mode, hipStream_t st) {
+  const bool stash = stash_fits(mode, p.K, p.V, Tag::epc, p.n_rows);
+  const size_t lds = stash ? (size_t)p.K * 16 : 0;
+  const dim3 grid((unsigned)p.n_rows), block(NT);
+  if (mode == 1 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 1, true>), grid, block, lds, st, p);
+  else if (mode == 2 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 2, true>), grid, block, lds, st, p);
+  else if (mode == 1) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 1, false>), grid, block, 0, st, p);
+  else if (mode == 2) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 2, false>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 0, false>), grid, block, 0, st, p);
+}
 template <class Tag>
 static hipError_t launch_stats(const StatsParams& p, int mode, hipStream_t st) {
-  // the logits at the teacher's ids out of the sweep where the row's chunks fit the threads' 64 rounds (the bound holds
-  // for every row: a peeled head only shortens the body)
-  const bool stash = stash_fits(mode, p.K, p.V, Tag::epc);
-  const size_t lds = stash ? (size_t)p.K * 16 : 0;
-  const dim3 grid((unsigned)p.n_rows), block(256);
-  if (mode == 1 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, 256, 1, true>), grid, block, lds, st, p);
-  else if (mode == 2 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, 256, 2, true>), grid, block, lds, st, p);
-  else if (mode == 1) hipLaunchKernelGGL((rowstats_kernel<Tag, 256, 1, false>), grid, block, 0, st, p);
-  else if (mode == 2) hipLaunchKernelGGL((rowstats_kernel<Tag, 256, 2, false>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((rowstats_kernel<Tag, 256, 0, false>), grid, block, 0, st, p);
+  const int nt = stats_threads(p.n_rows, p.V, Tag::epc);
+  if (nt == 1024) launch_stats_nt<Tag, 1024>(p, mode, st);
+  else if (nt == 512) launch_stats_nt<Tag, 512>(p, mode, st);
+  else launch_stats_nt<Tag, 256>(p, mode, st);
   return hipGetLastError();
 }
 
@@ -607,7 +632,7 @@ extern "C" int dl_composite_forward_train(const void* logits, int logits_dtype, 
                   nullptr, nullptr, nullptr, 0};
     // every teacher row has its logits row (no map, as many of the one as of the other): the rows' records at the
     // tail of phase 1; else teacher rows without a logits row need records too: the launch of their own
-    if (!row_map && n_teacher_rows == n_rows && stash_fits(vec, K, V, 16 / eb)) {
+    if (!row_map && n_teacher_rows == n_rows && stash_fits(vec, K, V, 16 / eb, n_rows)) {
       const hipError_t e = logits_dtype == DL_F32 ? launch_stats_record<TagF32>(p, vec, cp, st)
                            : logits_dtype == DL_BF16 ? launch_stats_record<TagBF16>(p, vec, cp, st)
                                                      : launch_stats_record<TagF16>(p, vec, cp, st);

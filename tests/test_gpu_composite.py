@@ -604,3 +604,19 @@ def test_logits_masked_with_low_finite_values(D, dtype, V, T):
     for loss, grad in got[:-1]:
         assert np.isfinite(loss) and abs(loss - got[-1][0]) <= 1e-6 * abs(loss)
         assert torch.isfinite(grad).all() and torch.linalg.norm(grad.double() - got[-1][1].double()) <= 1e-3 * torch.linalg.norm(got[-1][1].double())
+
+
+@pytest.mark.parametrize("dtype,V,pitch,K,lens", [
+    (torch.float32, 65540, 65540, 100, [7, 6]),                 # one chunk more than 64 rounds of 256 threads: 1024
+    (torch.bfloat16, 151665, 151936, 200, [9]),
+    (torch.float32, 75487, 75487, 64, [5, 4]),                  # the same off the 16-byte grid
+    (torch.float16, 524288, 524288, 40, [4]),                   # 64 rounds of 1024 threads,
+    (torch.float16, 524296, 524296, 40, [4]),                   # and one chunk more: no launch takes the ids out of the sweep
+    (torch.float32, 2048, 2048, 300, [513]), (torch.float32, 2048, 2048, 300, [300, 212])])      # 256 threads from 513 rows on, 512 below
+def test_threads_of_phase_one_by_rows_and_width(D, dtype, V, pitch, K, lens):
+    test_records_made_at_the_tail_of_phase_one_equal_the_separate_launches(D, dtype, V, pitch, K, lens, True)
+
+
+@pytest.mark.parametrize("V,dtype", [(65540, torch.float32), (131080, torch.bfloat16), (524296, torch.bfloat16)])
+def test_phase_one_on_rows_wider_than_256_threads_hold_rounds_for(D, V, dtype):
+    test_phase_one_ids_out_of_the_sweep_or_gathered(D, dtype, V, 64)
