@@ -539,6 +539,31 @@ int dl_rkl_marginalised_compact(const void* logits, int logits_dtype, int64_t ro
                                 float inv_T_student, float inv_T_teacher, float grad_scale,
                                 float* row_loss, void* grad, int64_t grad_stride, void* stream);
 
+/* The two above with a workspace (16-byte aligned, contents irrelevant on entry and return, not shared by launches that may
+ * overlap in time): a call of up to 128 rows against a wide teacher then deals each row's tiles to several workgroups, whose
+ * partial marginals meet in it, and runs the passes behind the marginal in a second launch.  Without it, or with
+ * less than dl_rkl_marginalised_workspace_bytes(...) (n_columns: Vs, or n_compact; 0: one launch), as above. */
+int64_t dl_rkl_marginalised_workspace_bytes(int64_t n_rows, int64_t Vt, int64_t n_columns, int plan_tile);
+int dl_rkl_marginalised_ws(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t Vs,
+                           const int32_t* row_map,
+                           const void* t_probs, int p_dtype, int64_t p_stride, int64_t n_teacher_rows, int64_t Vt,
+                           const int32_t* t2s,
+                           const int32_t* plan_row_off, const uint32_t* plan_ent, int plan_tile,
+                           const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
+                           float inv_T_student, float inv_T_teacher, float grad_scale,
+                           float* row_loss, void* grad, int64_t grad_stride,
+                           void* workspace, int64_t workspace_bytes, void* stream);
+int dl_rkl_marginalised_compact_ws(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t Vs_full,
+                                   const int32_t* cols, const uint16_t* col_src16, int64_t n_compact,
+                                   const int32_t* row_map,
+                                   const void* t_probs, int p_dtype, int64_t p_stride, int64_t n_teacher_rows, int64_t Vt,
+                                   const int32_t* t2c,
+                                   const int32_t* plan_row_off, const uint32_t* plan_ent, int plan_tile,
+                                   const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
+                                   float inv_T_student, float inv_T_teacher, float grad_scale,
+                                   float* row_loss, void* grad, int64_t grad_stride,
+                                   void* workspace, int64_t workspace_bytes, void* stream);
+
 
 /*
  * Deterministic sum of n fp32 values times `scale` into out[0] (fixed reduction tree,

@@ -21,6 +21,7 @@
 //   * fused reverse KL: the marginal never leaves LDS; its logarithm is the teacher row of the
 //     dense-divergence sweeps, the student row sits in registers.
 #include "dense_div.hpp"
+#include <algorithm>
 
 namespace dl {
 
@@ -71,6 +72,8 @@ constexpr int PLAN_ZERO_WORDS = 4;   // LDS words behind the tile that stay 0
 
 struct PlanBatch { u32x4 lo, hi; };
 
+__host__ __device__ inline int plan_tiles(const MargParams& p) { return (int)((p.Vt + p.plan_tile - 1) / p.plan_tile); }
+
 __device__ __forceinline__ float plan_tile_value(const float* tile, unsigned byte_offset) {
   return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(tile) + byte_offset);
 }
@@ -83,7 +86,7 @@ __device__ __forceinline__ float plan_tile_value(const float* tile, unsigned byt
 // 152064 (whole units off the grid) 3.71 -> 0.62 ms.  Rows shorter than a unit keep the scalar form.
 enum MargLoad : int { MARG_SCALAR = 0, MARG_VEC = 1, MARG_ANY = 2 };
 
-// Marginal of one teacher row into marg[0, Vs) (LDS, zeroed here) along a plan; `tile` is LDS
+// Marginal of one teacher row, its tiles [k0, k1), into marg[0, Vs) (LDS, zeroed here) along a plan; `tile` is LDS
 // scratch of plan_tile floats.  fp32 probabilities; LOAD = MARG_VEC: 16-byte aligned rows of whole units.
 //
 // The hot loop is straight-line code: per entry a read of the tile, a read of the entry's slot, the
@@ -140,7 +143,7 @@ __device__ __forceinline__ void plan_consume_packed(const u32x4& d, const float*
 // tile in flight whatever the depth, and the entries' trip to L2 and back waited for in full.)
 template <int LOAD, int NT>
 __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p, const char* prow, float* marg,
-                                                            float* tile) {
+                                                            float* tile, int k0, int k1) {
   const int tid = threadIdx.x, lane = tid & (WAVE - 1);
   // the wave index as a scalar: plan offsets are then fetched with scalar loads, which have their own
   // counter and do not queue behind the vector prefetches
@@ -150,7 +153,7 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   constexpr int U = 2 * LPW;                         // 16-byte loads per thread and tile
   const int TS = p.plan_tile;
   const int q_tile = TS / 4;                        // 16-byte loads per tile: 1024 .. 2048, up to U per thread
-  const int ntiles = (int)((p.Vt + TS - 1) / TS);
+  const int ntiles = plan_tiles(p);
   const int64_t n4 = p.Vt / 4;
   const int n_slots = (int)plan_slot_words(p.Vs, p.plan_n_extra);
   const int rest = LOAD == MARG_ANY ? (int)(p.Vt - n4 * 4) : 0;       // probabilities behind the last whole unit
@@ -165,7 +168,7 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   // wait for the load right away instead of two tiles later.
   u32x4 tbuf[2][U];
   auto fetch_tile = [&](int k, u32x4 (&buf)[U]) {
-    const bool in_row = (int64_t)k * q_tile < n4;     // (the last tile of a row that ends inside a unit may hold no whole one)
+    const bool in_row = k < k1 && (int64_t)k * q_tile < n4;     // (the last tile of a row that ends inside a unit may hold no whole one)
     const char* base = prow + (in_row ? (int64_t)k * TS * 4 : 0);
     const int left = in_row ? (int)(n4 - (int64_t)k * q_tile) : 0;      // 16-byte units from the tile's start to the row's end
 #pragma unroll
@@ -185,7 +188,7 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   struct List { int first, end, packed; };
   auto list_of = [&](int k, int q) {
     List l{0, 0, 0};
-    if (k < ntiles) {
+    if (k < k1) {
       const int at = k * NW + q * (NT / WAVE) + w;
       const int a = row_off[at], b = row_off[at + 1];
       l.first = a & ~3;
@@ -207,13 +210,13 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   PlanBatch e_even[LPW], e_odd[LPW];
   List cur[LPW], next[LPW];                           // the descriptors run two tiles ahead of the entries
 #pragma unroll
-  for (int q = 0; q < LPW; ++q) { cur[q] = list_of(0, q); next[q] = list_of(1, q); }
-  fetch_tile(0, tbuf[0]);
+  for (int q = 0; q < LPW; ++q) { cur[q] = list_of(k0, q); next[q] = list_of(k0 + 1, q); }
+  fetch_tile(k0, tbuf[0]);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < LPW; ++q) fetch_batch(cur[q].first, cur[q].packed, e_even[q]);
   __builtin_amdgcn_sched_barrier(0);
-  fetch_tile(1, tbuf[1]);
+  fetch_tile(k0 + 1, tbuf[1]);
   __builtin_amdgcn_sched_barrier(0);
   float run = 0.f;
   auto do_tile = [&](int k, u32x4 (&buf)[U], PlanBatch (&e)[LPW], PlanBatch (&e_next)[LPW]) {
@@ -250,12 +253,12 @@ __device__ __forceinline__ void accumulate_marginal_planned(const MargParams& p,
   // unrolled by two: the registers are addressed statically.  No path may enter the loop body with a
   // different set of loads in flight than the others, or every wait falls back to the worst case: an
   // odd last tile is therefore a third copy behind the loop, not a skipped second half.
-  int k = 0;
-  for (; k + 1 < ntiles; k += 2) {
+  int k = k0;
+  for (; k + 1 < k1; k += 2) {
     do_tile(k, tbuf[0], e_even, e_odd);
     do_tile(k + 1, tbuf[1], e_odd, e_even);
   }
-  if (k < ntiles) do_tile(k, tbuf[0], e_even, e_odd);
+  if (k < k1) do_tile(k, tbuf[0], e_even, e_odd);
   __syncthreads();
   // replicas into their id's slot: own slot first, then the replicas in ascending order
   for (int f = tid; f < p.plan_n_fold; f += NT) {
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(MARG_NT) void marginalise_map_kernel(const MargPara
   float* out = p.marg + r * p.marg_stride;
   if (LOAD != MARG_SCALAR && p.plan_ent) {
     float* marg = acc + p.plan_tile + PLAN_ZERO_WORDS;      // the tile sits first: its addresses are then plain offsets
-    accumulate_marginal_planned<LOAD, MARG_NT>(p, prow, marg, acc);
+    accumulate_marginal_planned<LOAD, MARG_NT>(p, prow, marg, acc, 0, plan_tiles(p));
     for (int j = threadIdx.x; j < p.Vs; j += MARG_NT) out[j] = p.out_log ? logf(marg[j]) : marg[j];
     return;
   }
@@ -796,7 +799,7 @@ __global__ __launch_bounds__(NT, 4) void rkl_marginalised_kernel(const MargParam
   if (LOAD != MARG_SCALAR && p.plan_ent) {
     marg = acc + p.plan_tile + PLAN_ZERO_WORDS;  // the tile sits first: its addresses are then plain offsets
     if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
-    accumulate_marginal_planned<LOAD, NT>(p, prow, marg, acc);
+    accumulate_marginal_planned<LOAD, NT>(p, prow, marg, acc, 0, plan_tiles(p));
   } else if constexpr (NT == MARG_NT) {
     if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
     accumulate_marginal<LOAD>(p, prow, acc, 0, (int)p.Vs);
@@ -805,6 +808,65 @@ __global__ __launch_bounds__(NT, 4) void rkl_marginalised_kernel(const MargParam
     __syncthreads();                             // the gradient of every compact column is in LDS
     expand_gradient_row<TagS, NT>(marg, p.col_src16, p.Vs_full, grow);
   }
+}
+
+// Few rows leave most CUs idle while a wide teacher row's tiles are walked one after the other (1.2 us each).  Two launches
+// then: the tiles of a row dealt to `parts` workgroups, whose partial marginals (fp32) go to a workspace, and the passes behind
+// the marginal on their sum, taken in part order.  64 rows x
+// 152064 onto 32000 ids 37.0 -> 23.7 us for the call (four workgroups a row), 54 x 170432 41.0 -> 26.5, 27 x 151680 onto 21352
+// 37.1 -> 23.4, 128 x 152064 (two a row) 37.3 -> 32.2; rows of less than eight tiles have too little to share (90 x 50304 22 us).
+template <int LOAD>
+__global__ __launch_bounds__(MARG_NT) void marginal_parts_kernel(const MargParams p, float* out, int parts) {
+  extern __shared__ __align__(16) float acc[];
+  const int64_t r = blockIdx.x / (unsigned)parts;
+  const int h = (int)(blockIdx.x % (unsigned)parts);
+  const int64_t trow = teacher_row(p.row_map, r, p.n_rows);
+  if (trow < 0) return;
+  const char* prow = reinterpret_cast<const char*>(p.probs) + trow * p.p_stride * 4;
+  float* marg = acc + p.plan_tile + PLAN_ZERO_WORDS;
+  const int ntiles = plan_tiles(p);
+  accumulate_marginal_planned<LOAD, MARG_NT>(p, prow, marg, acc, h * ntiles / parts, (h + 1) * ntiles / parts);
+  float* o = out + (r * parts + h) * p.Vs;
+  for (int j = threadIdx.x * 4; j < p.Vs; j += MARG_NT * 4) *reinterpret_cast<float4*>(o + j) = *reinterpret_cast<const float4*>(marg + j);
+}
+
+template <class TagS, int NU>
+__global__ __launch_bounds__(MARG_NT) void rkl_marginal_parts_kernel(const MargParams p, const float* in, int parts) {
+  extern __shared__ __align__(16) float acc[];
+  __shared__ float red[64];
+  const int64_t r = blockIdx.x;
+  const int tid = threadIdx.x;
+  char* grow = p.grad ? reinterpret_cast<char*>(p.grad) + r * p.grad_stride * TagS::bytes : nullptr;
+  const bool compact = p.Vs_full > 0;
+  if (teacher_row(p.row_map, r, p.n_rows) < 0) {
+    if (grow) zero_row<TagS, MARG_NT>(grow, (compact ? p.Vs_full : p.Vs) / TagS::epc);
+    if (tid == 0 && p.row_loss) p.row_loss[r] = 0.f;
+    return;
+  }
+  StudentRow<TagS, NU, MARG_NT> rows;
+  const char* srow = reinterpret_cast<const char*>(p.logits) + r * p.row_stride * TagS::bytes;
+  if (compact) rows.load_gathered(srow, p.cols, p.Vs / 8); else rows.load(srow, p.Vs / 8);
+  const float* part0 = in + r * parts * p.Vs;
+  for (int j = tid * 4; j < p.Vs; j += MARG_NT * 4) {
+    float4 m = *reinterpret_cast<const float4*>(part0 + j);
+    for (int h = 1; h < parts; ++h) {
+      const float4 v = *reinterpret_cast<const float4*>(part0 + h * p.Vs + j);
+      m.x += v.x; m.y += v.y; m.z += v.z; m.w += v.w;
+    }
+    *reinterpret_cast<float4*>(acc + j) = m;
+  }
+  __syncthreads();
+  if (rkl_against_marginal<TagS, NU, MARG_NT>(rows.s, rows.nunits, acc, red, p, r, grow, srow)) {      // the same for every thread
+    __syncthreads();
+    expand_gradient_row<TagS, MARG_NT>(acc, p.col_src16, p.Vs_full, grow);
+  }
+}
+
+// Workgroups that share a row's tiles: as many as there are CUs for, at least four tiles each (1: one launch).
+static int marg_parts(int64_t n_rows, int64_t Vt, int plan_tile) {
+  if (n_rows <= 0 || n_rows > 128 || plan_tile < 4096) return 1;
+  const int64_t ntiles = (Vt + plan_tile - 1) / plan_tile;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / n_rows, ntiles / 4, 8}));
 }
 
 // Workgroups of half as many threads, each wave walking two of a tile's lists (the plan and the order of its additions are
@@ -841,12 +903,15 @@ static void allow_large_lds() {
   allow_large_lds_for(&marginalise_map_kernel<MARG_SCALAR>);
   allow_large_lds_for(&marginalise_map_kernel<MARG_VEC>);
   allow_large_lds_for(&marginalise_map_kernel<MARG_ANY>);
+  allow_large_lds_for(&marginal_parts_kernel<MARG_VEC>);
+  allow_large_lds_for(&marginal_parts_kernel<MARG_ANY>);
 #define DL_LARGE_RKLM(TAG)                                                      \
   allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_SCALAR, MARG_NT>);                       \
   allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_VEC, MARG_NT>);                          \
   allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_NU, MARG_ANY, MARG_NT>);                          \
   allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_HALF_NU<TAG>, MARG_VEC, MARG_HALF_NT>);           \
-  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_HALF_NU<TAG>, MARG_ANY, MARG_HALF_NT>)
+  allow_large_lds_for(&rkl_marginalised_kernel<TAG, MARG_HALF_NU<TAG>, MARG_ANY, MARG_HALF_NT>);           \
+  allow_large_lds_for(&rkl_marginal_parts_kernel<TAG, MARG_NU>)
   DL_LARGE_RKLM(TagF32);
   DL_LARGE_RKLM(TagBF16);
   DL_LARGE_RKLM(TagF16);
@@ -933,7 +998,7 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
                                    const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
                                    float inv_T_student, float inv_T_teacher, float grad_scale, float* row_loss,
                                    void* grad, int64_t grad_stride, const int32_t* cols, const unsigned short* col_src16,
-                                   int64_t Vs_full, void* stream) {
+                                   int64_t Vs_full, void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace dl;
   if (!logits || !t_probs || !t2s) return DL_ERR_NULL;
   if (logits_dtype < DL_F32 || logits_dtype > DL_F16 || p_dtype < DL_F32 || p_dtype > DL_F16) return DL_ERR_DTYPE;
@@ -961,6 +1026,19 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid(xcd_banded_grid(n_rows));
   allow_large_lds();
+  const int parts = p.plan_ent ? marg_parts(n_rows, Vt, plan_tile) : 1;
+  if (parts > 1 && workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= n_rows * parts * Vs * 4) {
+    float* buf = reinterpret_cast<float*>(workspace);
+    const dim3 by(MARG_NT);
+    if (load == MARG_VEC) hipLaunchKernelGGL((marginal_parts_kernel<MARG_VEC>), dim3((unsigned)(n_rows * parts)), by, lds, st, p, buf, parts);
+    else hipLaunchKernelGGL((marginal_parts_kernel<MARG_ANY>), dim3((unsigned)(n_rows * parts)), by, lds, st, p, buf, parts);
+    const dim3 rows((unsigned)n_rows);
+    const size_t lds_marg = (size_t)Vs * 4;
+    if (logits_dtype == DL_F32) hipLaunchKernelGGL((rkl_marginal_parts_kernel<TagF32, MARG_NU>), rows, by, lds_marg, st, p, buf, parts);
+    else if (logits_dtype == DL_BF16) hipLaunchKernelGGL((rkl_marginal_parts_kernel<TagBF16, MARG_NU>), rows, by, lds_marg, st, p, buf, parts);
+    else hipLaunchKernelGGL((rkl_marginal_parts_kernel<TagF16, MARG_NU>), rows, by, lds_marg, st, p, buf, parts);
+    return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
+  }
 #define DL_LAUNCH_RKLM_NT(TAG, NU, NT)                                                                                             \
   do {                                                                                                                            \
     if (load == MARG_VEC) hipLaunchKernelGGL((rkl_marginalised_kernel<TAG, NU, MARG_VEC, NT>), grid, dim3(NT), lds, st, p);        \
@@ -980,6 +1058,25 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
   return hipGetLastError() == hipSuccess ? DL_OK : DL_ERR_LAUNCH;
 }
 
+extern "C" int64_t dl_rkl_marginalised_workspace_bytes(int64_t n_rows, int64_t Vt, int64_t n_columns, int plan_tile) {
+  if (Vt <= 0 || n_columns <= 0) return 0;
+  const int parts = dl::marg_parts(n_rows, Vt, plan_tile);
+  return parts > 1 ? n_rows * parts * n_columns * 4 : 0;
+}
+
+extern "C" int dl_rkl_marginalised_ws(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t Vs,
+                                      const int32_t* row_map, const void* t_probs, int p_dtype, int64_t p_stride,
+                                      int64_t n_teacher_rows, int64_t Vt, const int32_t* t2s,
+                                      const int32_t* plan_row_off, const uint32_t* plan_ent, int plan_tile,
+                                      const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
+                                      float inv_T_student, float inv_T_teacher, float grad_scale, float* row_loss,
+                                      void* grad, int64_t grad_stride, void* workspace, int64_t workspace_bytes, void* stream) {
+  return rkl_marginalised_launch(logits, logits_dtype, row_stride, n_rows, Vs, row_map, t_probs, p_dtype, p_stride,
+                                 n_teacher_rows, Vt, t2s, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold,
+                                 plan_n_extra, inv_T_student, inv_T_teacher, grad_scale, row_loss, grad, grad_stride, nullptr,
+                                 nullptr, 0, workspace, workspace_bytes, stream);
+}
+
 extern "C" int dl_rkl_marginalised(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows, int64_t Vs,
                                    const int32_t* row_map, const void* t_probs, int p_dtype, int64_t p_stride,
                                    int64_t n_teacher_rows, int64_t Vt, const int32_t* t2s,
@@ -987,10 +1084,26 @@ extern "C" int dl_rkl_marginalised(const void* logits, int logits_dtype, int64_t
                                    const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
                                    float inv_T_student, float inv_T_teacher, float grad_scale, float* row_loss,
                                    void* grad, int64_t grad_stride, void* stream) {
-  return rkl_marginalised_launch(logits, logits_dtype, row_stride, n_rows, Vs, row_map, t_probs, p_dtype, p_stride,
-                                 n_teacher_rows, Vt, t2s, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold,
-                                 plan_n_extra, inv_T_student, inv_T_teacher, grad_scale, row_loss, grad, grad_stride, nullptr,
-                                 nullptr, 0, stream);
+  return dl_rkl_marginalised_ws(logits, logits_dtype, row_stride, n_rows, Vs, row_map, t_probs, p_dtype, p_stride,
+                                n_teacher_rows, Vt, t2s, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold,
+                                plan_n_extra, inv_T_student, inv_T_teacher, grad_scale, row_loss, grad, grad_stride, nullptr, 0,
+                                stream);
+}
+
+extern "C" int dl_rkl_marginalised_compact_ws(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows,
+                                              int64_t Vs_full, const int32_t* cols, const uint16_t* col_src16, int64_t n_compact,
+                                              const int32_t* row_map, const void* t_probs, int p_dtype, int64_t p_stride,
+                                              int64_t n_teacher_rows, int64_t Vt, const int32_t* t2c,
+                                              const int32_t* plan_row_off, const uint32_t* plan_ent, int plan_tile,
+                                              const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
+                                              float inv_T_student, float inv_T_teacher, float grad_scale, float* row_loss,
+                                              void* grad, int64_t grad_stride, void* workspace, int64_t workspace_bytes,
+                                              void* stream) {
+  if (!cols || !col_src16) return DL_ERR_NULL;
+  return rkl_marginalised_launch(logits, logits_dtype, row_stride, n_rows, n_compact, row_map, t_probs, p_dtype, p_stride,
+                                 n_teacher_rows, Vt, t2c, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold,
+                                 plan_n_extra, inv_T_student, inv_T_teacher, grad_scale, row_loss, grad, grad_stride, cols,
+                                 reinterpret_cast<const unsigned short*>(col_src16), Vs_full, workspace, workspace_bytes, stream);
 }
 
 extern "C" int dl_rkl_marginalised_compact(const void* logits, int logits_dtype, int64_t row_stride, int64_t n_rows,
@@ -1001,9 +1114,8 @@ extern "C" int dl_rkl_marginalised_compact(const void* logits, int logits_dtype,
                                            const int32_t* plan_fold, int plan_n_fold, int plan_n_extra,
                                            float inv_T_student, float inv_T_teacher, float grad_scale, float* row_loss,
                                            void* grad, int64_t grad_stride, void* stream) {
-  if (!cols || !col_src16) return DL_ERR_NULL;
-  return rkl_marginalised_launch(logits, logits_dtype, row_stride, n_rows, n_compact, row_map, t_probs, p_dtype, p_stride,
-                                 n_teacher_rows, Vt, t2c, plan_row_off, plan_ent, plan_tile, plan_fold, plan_n_fold,
-                                 plan_n_extra, inv_T_student, inv_T_teacher, grad_scale, row_loss, grad, grad_stride, cols,
-                                 reinterpret_cast<const unsigned short*>(col_src16), Vs_full, stream);
+  return dl_rkl_marginalised_compact_ws(logits, logits_dtype, row_stride, n_rows, Vs_full, cols, col_src16, n_compact, row_map,
+                                        t_probs, p_dtype, p_stride, n_teacher_rows, Vt, t2c, plan_row_off, plan_ent, plan_tile,
+                                        plan_fold, plan_n_fold, plan_n_extra, inv_T_student, inv_T_teacher, grad_scale, row_loss,
+                                        grad, grad_stride, nullptr, 0, stream);
 }

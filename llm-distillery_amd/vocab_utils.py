@@ -241,6 +241,12 @@ def expand_columns(xc: torch.Tensor, col_src: torch.Tensor, V: int, out: torch.T
     return out
 
 
+def _parts_workspace(rows: int, n_teacher: int, n_columns: int, tile: int, dev):
+    """(tensor or None, bytes): room for the partial marginals of a call with few rows."""
+    n = _lib.load().dl_rkl_marginalised_workspace_bytes(rows, n_teacher, n_columns, tile)
+    return (torch.empty(n, dtype=torch.uint8, device=dev) if n else None), n
+
+
 def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "torch.Tensor | MarginalPlan", *,
                      row_map: torch.Tensor | None = None, T: float = 1.0, teacher_T: float | None = None,
                      grad_scale: float = 1.0, want_grad: bool = True, grad_out: torch.Tensor | None = None):
@@ -270,12 +276,13 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
             if want_grad:
                 grad = _grad_target(grad_out, R, Vs, x.dtype, dev)
                 g_ptr, g_stride = grad.data_ptr(), grad.stride(0)
+            ws, ws_bytes = _parts_workspace(R, Vt, plan.n_compact, plan.compact.tile, dev)
             with _on(dev):
-                st = _lib.load().dl_rkl_marginalised_compact(
+                st = _lib.load().dl_rkl_marginalised_compact_ws(
                     x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, plan.cols.data_ptr(), plan.col_src16.data_ptr(),
                     plan.n_compact, rm_ptr, tp.data_ptr(), _DT[tp.dtype], tp.stride(0), N, Vt, plan.t2c.data_ptr(),
                     *plan.compact.args(), 1.0 / T, 1.0 / (T if teacher_T is None else teacher_T), grad_scale,
-                    row_loss.data_ptr(), g_ptr, g_stride, _stream_ptr(dev))
+                    row_loss.data_ptr(), g_ptr, g_stride, ws.data_ptr() if ws is not None else 0, ws_bytes, _stream_ptr(dev))
             _lib.check(st, "dl_rkl_marginalised_compact")
             if grad is not None and logits.dim() != 2 and grad_out is None:
                 grad = grad.view(logits.shape)
@@ -294,10 +301,12 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
     if want_grad:
         grad = _grad_target(grad_out, R, Vs, x.dtype, dev)
         g_ptr, g_stride = grad.data_ptr(), grad.stride(0)
+    ws, ws_bytes = _parts_workspace(R, Vt, Vs, plan_args[2], dev)
     with _on(dev):
-        st = _lib.load().dl_rkl_marginalised(x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, rm_ptr, tp.data_ptr(),
-                                             _DT[tp.dtype], tp.stride(0), N, Vt, t2s.data_ptr(), *plan_args, 1.0 / T,
-                                             1.0 / (T if teacher_T is None else teacher_T), grad_scale,
-                                             row_loss.data_ptr(), g_ptr, g_stride, _stream_ptr(dev))
+        st = _lib.load().dl_rkl_marginalised_ws(x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, rm_ptr, tp.data_ptr(),
+                                                _DT[tp.dtype], tp.stride(0), N, Vt, t2s.data_ptr(), *plan_args, 1.0 / T,
+                                                1.0 / (T if teacher_T is None else teacher_T), grad_scale,
+                                                row_loss.data_ptr(), g_ptr, g_stride, ws.data_ptr() if ws is not None else 0,
+                                                ws_bytes, _stream_ptr(dev))
     _lib.check(st, "dl_rkl_marginalised")
     return row_loss, grad

@@ -484,3 +484,43 @@ def test_more_rows_than_cus_take_two_workgroups_per_cu(D, Vt, Vs, used, dtype):
                                               1e-4 if dtype == torch.float32 else 2e-3)
     err = (grad[valid].double() - grad64).abs()
     assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+
+
+@pytest.mark.parametrize("R,Vt,Vs,used,dtype", [(3, 70001, 2048, 500, torch.bfloat16),      # tiles dealt to several workgroups, a ragged end
+                                                (2, 200064, 16384, 16384, torch.float16),    # the full plan, eight parts
+                                                (128, 70000, 2048, 700, torch.float32), (129, 70000, 2048, 700, torch.float32)])
+def test_few_rows_against_a_wide_teacher(D, R, Vt, Vs, used, dtype):
+    """Up to 128 rows a row's tiles are shared by several workgroups through a workspace, and the passes take a launch of their
+    own; masked rows, the gradient over the logits; the same within rounding as one launch (dl_rkl_marginalised without one)."""
+    rng = np.random.default_rng(Vt + R)
+    ids = rng.permutation(Vs)[:used]
+    t2s = ids[rng.integers(0, used, Vt)].astype(np.int32)
+    t2s[rng.random(Vt) < 0.05] = -1
+    t2s[-1] = ids[0]
+    plan = _map_in_the_form(D, "auto", t2s, Vs)
+    tile = (plan.compact or plan.full).tile
+    n = plan.n_compact if plan.compact is not None else Vs
+    ws = D._lib.load().dl_rkl_marginalised_workspace_bytes(R, Vt, n, tile)
+    assert (ws == 0) == (R > 128 or 256 // R < 2 or -(-Vt // tile) < 8)
+    g = torch.Generator().manual_seed(Vt)
+    probs = torch.softmax(torch.randn(R, Vt, generator=g) * 2, -1)
+    logits = (torch.randn(R, Vs, generator=g) * 2).to(dtype)
+    rm = torch.arange(R, dtype=torch.int32)
+    valid = torch.ones(R, dtype=torch.bool)
+    rm[1], valid[1] = -1, False
+    ref = O.marginalise_map(probs[valid].numpy(), t2s, Vs)
+    with np.errstate(divide="ignore"):
+        t_logits = O.marginal_to_teacher_logits(torch.tensor(ref))
+    _, rows64, grad64 = O.mean_loss_and_grad("rkl", logits[valid], 1.3, t_logits=t_logits, dtype=torch.float64)
+    nv = int(valid.sum())
+    for in_place in (False, True):
+        x = logits.to(DEV)
+        rl, grad = D.vocab_utils.rkl_marginalised(x, probs.to(DEV), plan, row_map=rm.to(DEV), T=1.3, grad_scale=1.0 / nv,
+                                                  grad_out=x if in_place else None)
+        rl, grad = rl.cpu(), grad.cpu()
+        assert torch.count_nonzero(rl[~valid]) == 0 and torch.count_nonzero(grad[~valid]) == 0
+        np.testing.assert_allclose(rl[valid].double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+        bound = O.marginal_rkl_gradient_tolerance(grad64, logits[valid], t_logits, rows64, 1.3, 1.3, 1.0 / nv, dtype,
+                                                  1e-4 if dtype == torch.float32 else 2e-3)
+        err = (grad[valid].double() - grad64).abs()
+        assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
