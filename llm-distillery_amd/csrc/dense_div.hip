@@ -279,11 +279,11 @@ static int dense_split_units(int s_dtype, int t_dtype) {
 //     the CUs busy by itself below that, and has no partners to wait for).
 //   * JSD, whose parts meet twice and have one more launch behind them: a pair that 1024 threads hold stays whole below
 //     1536 rows of 16-bit pairs and 3072 rows of others; a pair that they do not hold is always cut.  At the lines, whole
-//     and cut: 16-bit pairs, 1536 rows of 33000 / 40960 / 50257 / 65536 columns 110 / 126 / 157 / 205 and 106 / 117 / 146 /
-//     169 us (1024 rows: 78 / 85 / 104 / 133 and 80 / 86 / 104 / 119); 3072 rows of 16392 / 24000 / 32768 columns, bf16
-//     against fp32 130 / 175 / 222 and 114 / 143 / 212, fp32 149 / 193 / 245 and 152 / 187 / 225, fp32 against bf16 154 /
-//     200 / 261 and 146 / 180 / 227.  (Mixed pairs gain up to 19 % from 2048 rows on, fp32 pairs up to 7 %, but not at every
-//     width: 2048 x 28000 bf16 against fp32 129 and 132.)
+//     and cut: 16-bit pairs, 1536 rows of 33000 / 40960 / 50257 / 65536 columns 103 / 117 / 150 / 184 and 94 / 103 / 131 /
+//     147 us (1024 rows: 69 / 81 / 103 / 125 and 71 / 78 / 94 / 104); 3072 rows of 16392 / 24000 / 32768 columns, bf16
+//     against fp32 119 / 162 / 205 and 103 / 129 / 199, fp32 148 / 193 / 244 and 152 / 190 / 228, fp32 against bf16 141 /
+//     183 / 242 and 150 / 181 / 224.  (bf16 against fp32 gains from 2048 rows on, but not at every width: 24000 / 28000 /
+//     32768 columns 105 / 118 / 138 and 91 / 123 / 134.)
 // `forced_nt` (256 / 512 / 1024, a tuning hook) fixes the thread count and cuts wherever two parts or more come out.
 struct DenseCut { int nt, parts; };
 static DenseCut dense_split_cut(int kind, int s_dtype, int t_dtype, int64_t n_rows, int64_t V, int forced_nt = 0) {
