@@ -564,3 +564,23 @@ def test_rkl_values_and_fill_match_the_one_launch_form(D, dtype, V, pitch, K, gr
         out = torch.full((R * (V + 3) + 1,), float("nan"), dtype=dtype, device=DEV)[1:].view(R, V + 3)[:, :V]
     rl2, grad2 = D.div_topk("rkl", x, tv, ti, row_map=rm, T=1.4, grad_scale=0.3, grad_out=out)
     assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
+
+
+@pytest.mark.parametrize("dtype,V,std", [(torch.bfloat16, 4104, 4.0), (torch.float32, 4104, 15.0), (torch.float16, 102400, 4.0)])
+@pytest.mark.parametrize("K", [1, 200, 256, 257, 512])
+def test_rkl_entries_in_registers_match_the_general_form(D, dtype, V, std, K):
+    """Up to 512 stored entries a row are held in registers, more pass through LDS.  The same rows with 528 stored entries
+    of which `t_cnt` leaves K take the second way: the same roundings, bit for bit.  In particular the logits are scaled by
+    1 / T (which is not exact here) inside a fused multiply-add in both: a product rounded by itself costs precision where
+    logits are large."""
+    R, KW = 24, 528
+    g = torch.Generator().manual_seed(V + K)
+    x = (torch.randn(R, V, generator=g) * std + 15).to(dtype).to(DEV)
+    tv = torch.log_softmax(torch.randn(R, KW, generator=g) * 2, -1).half().to(DEV)
+    ti = torch.stack([torch.randperm(V, generator=g)[:KW] for _ in range(R)]).int().to(DEV)
+    ti[2, 0] = -1                                                    # an entry that does not count
+    cnt = torch.full((R,), K, dtype=torch.int32, device=DEV)
+    kw = dict(T=1.4, teacher_T=1.3, grad_scale=0.3)
+    rl, grad = D.div_topk("rkl", x, tv[:, :K], ti[:, :K], **kw)
+    rl2, grad2 = D.div_topk("rkl", x, tv, ti, t_cnt=cnt, **kw)
+    assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
