@@ -1299,7 +1299,8 @@ static int64_t rkl_fill_parts(int logits_dtype, int64_t n_rows, int64_t V) {
   const int64_t row_bytes = V * (logits_dtype == F32 ? 4 : 2);
   if (row_bytes < 96 * 1024 || (row_bytes < 200000 && n_rows * row_bytes < (128LL << 20))) return 0;
   const int64_t parts = (row_bytes / 16 + RKL_FILL_NT * RKL_FILL_NCH - 1) / (RKL_FILL_NT * RKL_FILL_NCH);
-  return n_rows * parts <= 0x7fffffffLL - 7 ? parts : 0;
+  // a launch takes fewer than 2^32 threads; one workgroup per row has no such limit here, as rows are this wide
+  return (n_rows * parts + 7) / 8 * 8 * RKL_FILL_NT < (1LL << 32) ? parts : 0;
 }
 static int64_t rkl_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t V, int K) {
   return rkl_fill_parts(logits_dtype, n_rows, V) ? n_rows * K * (int64_t)sizeof(uint2) : 0;

@@ -376,3 +376,16 @@ def test_rows_that_one_workgroup_holds_need_no_workspace():
         assert all(size(torch.float32, rows, V) == 0 for V in (5, 16385, 32767, 32768)) and size(torch.bfloat16, rows, 128256, 1) == 0
         assert all(size(dt, rows, V) > 16 * rows for dt, V in ((torch.bfloat16, 65537), (torch.bfloat16, 262144), (torch.float32, 32769)))
     assert size(torch.bfloat16, 1 << 20, 262145) == 0      # too wide to be cut
+
+
+@pytest.mark.parametrize("dtype,V,threads_per_row", [(0, 65536, 32 * 256), (1, 128256, 32 * 256), (2, 102408, 26 * 256)])
+def test_reverse_kl_rows_in_two_launches_stay_below_the_threads_of_a_launch(dtype, V, threads_per_row):
+    """A launch takes fewer than 2^32 threads.  Reverse KL on wide rows has a workgroup of 256 threads for every 8 KiB of a
+    gradient row; calls with more of them (gradients of 128 GiB) get no workspace, which leaves them one workgroup per row."""
+    lib = D._lib.load()
+    most = 2 ** 32 // threads_per_row
+    while (most * threads_per_row // 256 + 7) // 8 * 8 * 256 >= 2 ** 32:      # the grid is a multiple of 8
+        most -= 1
+    assert lib.dl_rkl_topk_workspace_bytes(dtype, most, V, 16) == most * 16 * 8
+    assert lib.dl_rkl_topk_workspace_bytes(dtype, most + 1, V, 16) == 0
+    assert lib.dl_rkl_topk_workspace_bytes(dtype, 2 ** 31 - 1, V, 16) == 0
