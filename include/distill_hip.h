@@ -131,7 +131,8 @@ int dl_div_topk(int kind,
 int64_t dl_div_topk_workspace_bytes(int kind, int logits_dtype, int64_t n_rows, int64_t V);
 
 /* The same for DL_RKL with a gradient, where wide rows are written by a launch of their own: K (id, value) pairs of
- * 8 bytes per row (0: such rows take one launch; so do calls with less workspace than this). */
+ * 8 bytes per row, up to 16 MiB, with which more rows are taken in turns (0: the rows take one launch; so do calls with
+ * less workspace than this). */
 int64_t dl_rkl_topk_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t V, int K);
 
 /*

@@ -993,8 +993,8 @@ __global__ __launch_bounds__(NT) void rkl_topk_kernel(const TopkParams p) {
   }
 }
 
-// Two launches, through a workspace of K (id, q (z - rkl)) pairs per row: the values of all rows, then nothing but the
-// stores, in the order of the gradient's addresses.  A workgroup that makes a row's values and then writes the row is a
+// Two launches, through a workspace of K (id, q (z - rkl)) pairs per row: the values of the rows, then nothing but the
+// stores, in the order of the gradient's addresses (many rows: several turns of the two, see rkl_fill_rows).  A workgroup that makes a row's values and then writes the row is a
 // chain of dependent round trips ahead of its stores, and 2048 rows are written at a time, spread over the whole buffer.
 // Bound by the stores: a bare fill of 8192 x 128256 bf16 takes 300 us at best (7.0 TB/s: 4 KiB per workgroup, every XCD in an
 // eighth of the buffer of its own), 314 with 16 KiB per workgroup, 345 with the workgroups dealt round the XCDs in
@@ -1002,13 +1002,13 @@ __global__ __launch_bounds__(NT) void rkl_topk_kernel(const TopkParams p) {
 // which 34 for the values; 384 with slabs of 16 KiB instead of 8, 420 with the correction lists of the register kernels
 // instead of a slab in LDS and the workgroups in address order.  4096 x 128256 fp32, K = 20: 434 -> 331 us.
 template <class Tag, int NT, int J>
-__global__ __launch_bounds__(NT) void rkl_values_kernel(const TopkParams p) {
+__global__ __launch_bounds__(NT) void rkl_values_kernel(const TopkParams p, int64_t row0) {
   extern __shared__ __align__(16) unsigned char smem[];
   const TopkLds s(smem, p.K);
-  const int64_t r = blockIdx.x;
+  const int64_t r = row0 + blockIdx.x;
   const int tid = threadIdx.x;
   const int64_t trow = teacher_row(p.row_map, r, p.n_trows);
-  uint2* out = reinterpret_cast<uint2*>(p.workspace) + r * p.K;
+  uint2* out = reinterpret_cast<uint2*>(p.workspace) + (int64_t)blockIdx.x * p.K;
   float rkl = 0.f;
   const bool live = rkl_on_support<Tag, NT, J>(p, s, r, trow, rkl);
   if (tid == 0 && p.row_loss) p.row_loss[r] = live ? rkl : 0.f;
@@ -1016,12 +1016,12 @@ __global__ __launch_bounds__(NT) void rkl_values_kernel(const TopkParams p) {
     out[k] = live ? uint2{(unsigned)s.idx[k], __float_as_uint(s.q[k] * (s.z[k] - rkl))} : uint2{~0u, 0u};
 }
 
-// Item b is part b % parts of row b / parts: SLAB bytes of the row's body (and with part 0 the columns beside the body:
+// Item b is part b % parts of row row0 + b / parts: SLAB bytes of the row's body (and with part 0 the columns beside the body:
 // MODE 2).  The part is made in LDS: zeroed, the pairs that name one of its columns (out of all K pairs of the row, from
 // L2) written into place, and stored in one piece; a bit per column tells a repeated id, whose pairs are then added up.
 constexpr int RKL_FILL_NT = 256, RKL_FILL_NCH = 2, RKL_SLAB = RKL_FILL_NT * RKL_FILL_NCH * 16;
 template <class Tag, int MODE>
-__global__ __launch_bounds__(RKL_FILL_NT) void rkl_fill_kernel(const TopkParams p, unsigned parts) {
+__global__ __launch_bounds__(RKL_FILL_NT) void rkl_fill_kernel(const TopkParams p, int64_t row0, int64_t rows, unsigned parts) {
   using C = Chunk<Tag>;
   constexpr int NT = RKL_FILL_NT, NCH = RKL_FILL_NCH, COLS = RKL_SLAB / Tag::bytes, WORDS = COLS / 32 + 1;
   __shared__ __align__(16) u32x4 slab[NT * NCH];
@@ -1031,10 +1031,10 @@ __global__ __launch_bounds__(RKL_FILL_NT) void rkl_fill_kernel(const TopkParams 
   __shared__ int repeats;
   const int tid = threadIdx.x;
   const unsigned item = xcd_eighth(blockIdx.x, gridDim.x);
-  const int64_t r = item / parts;
+  const int64_t at = item / parts, r = row0 + at;
   const int h = (int)(item % parts);
-  if (r >= p.n_rows) return;
-  const uint2* ent = reinterpret_cast<const uint2*>(p.workspace) + r * p.K;
+  if (at >= rows) return;
+  const uint2* ent = reinterpret_cast<const uint2*>(p.workspace) + at * p.K;
   uint2 mine = tid < p.K ? ent[tid] : uint2{~0u, 0u};
 #pragma unroll
   for (int i = 0; i < NCH; ++i) slab[i * NT + tid] = u32x4{0u, 0u, 0u, 0u};
@@ -1295,16 +1295,35 @@ int launch_fkl_any_multi(int logits_dtype, const TopkParams& p, int64_t ws_bytes
 // (8192 x 32000 bf16, K = 200: 115 us in one launch, 120 in two; 16384 x 12000: 116, 123).  From 96 KiB per row on two
 // launches pay where there is enough to write to cover the second one (2048 x 50304 bf16 49 -> 44 us, 1024 x 36696 fp32 43 ->
 // 36; 1024 x 50304 bf16 28 against 29), from 195 KiB on always: few rows leave most of the chip idle in one launch (32 x
-// 128256 bf16 32 -> 29 us, 512 rows 36 -> 29).
-static int64_t rkl_fill_parts(int logits_dtype, int64_t n_rows, int64_t V) {
+// 128256 bf16 32 -> 29 us, 512 rows 36 -> 29).  Below 160 KB, many rows of some thousand entries stay in one launch: each
+// part of 8 KiB looks through all of them, and the values' launch holds up to 512 in registers only (16384 x 50304 bf16, K =
+// 768 / 1000 / 1025 / 1300: 577 / 608 / 656 / 825 us in one launch, 577 / 657 / 734 / 816 in two; 16384 x 99000, K = 1000 1161
+// and 1026).  At K = 2048 one launch has LDS for two workgroups per CU only: 32768 x 65536 bf16 2978 against 2416.
+static int64_t rkl_fill_parts(int logits_dtype, int64_t n_rows, int64_t V, int K) {
   const int64_t row_bytes = V * (logits_dtype == F32 ? 4 : 2);
-  if (row_bytes < 96 * 1024 || (row_bytes < 200000 && n_rows * row_bytes < (128LL << 20))) return 0;
-  const int64_t parts = (row_bytes / 16 + RKL_FILL_NT * RKL_FILL_NCH - 1) / (RKL_FILL_NT * RKL_FILL_NCH);
-  // a launch takes fewer than 2^32 threads; one workgroup per row has no such limit here, as rows are this wide
-  return (n_rows * parts + 7) / 8 * 8 * RKL_FILL_NT < (1LL << 32) ? parts : 0;
+  if (row_bytes < 96 * 1024) return 0;
+  if (row_bytes < 200000 && n_rows * row_bytes < (128LL << 20)) return 0;
+  if (row_bytes < 160000 && n_rows > 2048 && K > 768 && K <= 1792) return 0;
+  return (row_bytes / 16 + RKL_FILL_NT * RKL_FILL_NCH - 1) / (RKL_FILL_NT * RKL_FILL_NCH);
+}
+// The pairs of all rows at once would be read from beyond L2 once there are more than about 24 MB of them, in the middle of
+// the stores (fill alone, 8192 x 128256 bf16: 320 us at K = 100 to 300, 500 at 400, 576 at 500, 762 at 1000).  The rows are
+// therefore taken a few thousand at a time, values and stores in turn, over the same 16 MiB.  Inputs that no cache holds, one
+// launch / all rows at once / by 16 MiB: 32768 x 128256 bf16, K = 200 1765 / 1954 / 1413 us, K = 500 1976 / 2579 / 1637; 8192
+// rows, K = 500 513 / 660 / 413; 16384 x 128256 fp32, K = 300 1778 / 2022 / 1319.  4 and 8 MiB measure 1-30 % more than 16, 24
+// MiB up to 20 % more.
+constexpr int64_t RKL_WORKSPACE_MOST = 16LL << 20;
+// Rows per turn (0: one launch for all rows)
+static int64_t rkl_fill_rows(int logits_dtype, int64_t n_rows, int64_t V, int K) {
+  const int64_t parts = rkl_fill_parts(logits_dtype, n_rows, V, K);
+  if (!parts) return 0;
+  const int64_t threads = ((1LL << 32) / RKL_FILL_NT - 8) / parts;      // a launch takes fewer than 2^32 threads
+  const int64_t most = std::min(threads, RKL_WORKSPACE_MOST / (K * (int64_t)sizeof(uint2)));
+  const int64_t turns = (n_rows + most - 1) / most;
+  return (n_rows + turns - 1) / turns;
 }
 static int64_t rkl_workspace_bytes(int logits_dtype, int64_t n_rows, int64_t V, int K) {
-  return rkl_fill_parts(logits_dtype, n_rows, V) ? n_rows * K * (int64_t)sizeof(uint2) : 0;
+  return rkl_fill_rows(logits_dtype, n_rows, V, K) * K * (int64_t)sizeof(uint2);
 }
 
 template <class Tag>
@@ -1314,14 +1333,18 @@ static hipError_t launch_rkl(const TopkParams& p, int64_t ws_bytes, bool aligned
   const bool two = need > 0 && ws_bytes >= need;
   const int J = p.K <= 256 ? 1 : p.K <= 512 ? 2 : 0;
   if (two) {
-    const dim3 rows((unsigned)p.n_rows), by(256);
-    if (J == 1) hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 1>), rows, by, TopkLds::bytes(p.K), st, p);
-    else if (J == 2) hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 2>), rows, by, TopkLds::bytes(p.K), st, p);
-    else hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 0>), rows, by, TopkLds::bytes(p.K), st, p);
-    const unsigned parts = (unsigned)rkl_fill_parts(Tag::id, p.n_rows, p.V);
-    const dim3 grid((unsigned)((p.n_rows * parts + 7) / 8 * 8)), block(RKL_FILL_NT);
-    if (aligned) hipLaunchKernelGGL((rkl_fill_kernel<Tag, 1>), grid, block, 0, st, p, parts);
-    else hipLaunchKernelGGL((rkl_fill_kernel<Tag, 2>), grid, block, 0, st, p, parts);
+    const int64_t step = rkl_fill_rows(Tag::id, p.n_rows, p.V, p.K);
+    const unsigned parts = (unsigned)rkl_fill_parts(Tag::id, p.n_rows, p.V, p.K);
+    for (int64_t row0 = 0; row0 < p.n_rows; row0 += step) {
+      const int64_t n = std::min(step, p.n_rows - row0);
+      const dim3 rows((unsigned)n), by(256);
+      if (J == 1) hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 1>), rows, by, TopkLds::bytes(p.K), st, p, row0);
+      else if (J == 2) hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 2>), rows, by, TopkLds::bytes(p.K), st, p, row0);
+      else hipLaunchKernelGGL((rkl_values_kernel<Tag, 256, 0>), rows, by, TopkLds::bytes(p.K), st, p, row0);
+      const dim3 grid((unsigned)((n * parts + 7) / 8 * 8)), block(RKL_FILL_NT);
+      if (aligned) hipLaunchKernelGGL((rkl_fill_kernel<Tag, 1>), grid, block, 0, st, p, row0, n, parts);
+      else hipLaunchKernelGGL((rkl_fill_kernel<Tag, 2>), grid, block, 0, st, p, row0, n, parts);
+    }
     return hipGetLastError();
   }
 #define DL_LAUNCH_RKL(MODE, J) \

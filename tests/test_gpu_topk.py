@@ -584,3 +584,24 @@ def test_rkl_entries_in_registers_match_the_general_form(D, dtype, V, std, K):
     rl, grad = D.div_topk("rkl", x, tv[:, :K], ti[:, :K], **kw)
     rl2, grad2 = D.div_topk("rkl", x, tv, ti, t_cnt=cnt, **kw)
     assert torch.equal(rl, rl2) and torch.equal(grad, grad2)
+
+
+@pytest.mark.parametrize("R,K", [(1025, 2048), (2051, 2048), (8200, 257)])      # 2, 3 and 2 turns of at most 16 MiB of pairs
+@pytest.mark.parametrize("in_place", [False, True])
+def test_rkl_on_many_rows_takes_them_in_turns(D, R, K, in_place):
+    """More rows than the workspace of the two launches holds: values and stores of a share of the rows, then of the next one.
+    Bit for bit what one launch writes, masked rows and rows mapped onto others' teachers among them."""
+    V = 100004                                                       # rows off the 16-byte grid in turn
+    per_turn, rest = divmod(D._lib.load().dl_rkl_topk_workspace_bytes(D.ops._DT[torch.bfloat16], R, V, K), 8 * K)
+    assert rest == 0 and 0 < per_turn < R
+    g = torch.Generator(device=DEV).manual_seed(R)
+    x = torch.randn(R, V, generator=g, device=DEV, dtype=torch.bfloat16) * 3
+    tv = torch.log_softmax(torch.randn(R, K, generator=g, device=DEV) * 2, -1).half()
+    ti = torch.randint(0, V, (R, K), generator=g, device=DEV, dtype=torch.int32)
+    rm = torch.arange(R, dtype=torch.int32, device=DEV).flip(0)
+    rm[::17] = -1
+    rm[per_turn] = -1
+    rl, grad = torch.empty(R, device=DEV), torch.empty_like(x)
+    D.div_topk_static("rkl", x, tv, ti, rl, grad, row_map=rm, T=1.4, grad_scale=0.3)
+    rl2, grad2 = D.div_topk("rkl", x, tv, ti, row_map=rm, T=1.4, grad_scale=0.3, grad_out=x if in_place else None)
+    assert torch.equal(rl, rl2) and torch.equal(grad, grad2)

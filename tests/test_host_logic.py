@@ -378,14 +378,14 @@ def test_rows_that_one_workgroup_holds_need_no_workspace():
     assert size(torch.bfloat16, 1 << 20, 262145) == 0      # too wide to be cut
 
 
-@pytest.mark.parametrize("dtype,V,threads_per_row", [(0, 65536, 32 * 256), (1, 128256, 32 * 256), (2, 102408, 26 * 256)])
-def test_reverse_kl_rows_in_two_launches_stay_below_the_threads_of_a_launch(dtype, V, threads_per_row):
-    """A launch takes fewer than 2^32 threads.  Reverse KL on wide rows has a workgroup of 256 threads for every 8 KiB of a
-    gradient row; calls with more of them (gradients of 128 GiB) get no workspace, which leaves them one workgroup per row."""
+@pytest.mark.parametrize("dtype,V,parts", [(0, 65536, 32), (1, 128256, 32), (2, 102408, 26), (1, 6 << 20, 1536)])
+@pytest.mark.parametrize("K", [1, 16, 500, 2048])
+def test_reverse_kl_in_two_launches_takes_many_rows_in_turns(dtype, V, parts, K):
+    """The pairs of ids and values between the two launches take no more than 16 MiB however many rows there are, and neither
+    launch reaches 2^32 threads (a workgroup of 256 threads for every 8 KiB of a gradient row), the most that one takes."""
     lib = D._lib.load()
-    most = 2 ** 32 // threads_per_row
-    while (most * threads_per_row // 256 + 7) // 8 * 8 * 256 >= 2 ** 32:      # the grid is a multiple of 8
-        most -= 1
-    assert lib.dl_rkl_topk_workspace_bytes(dtype, most, V, 16) == most * 16 * 8
-    assert lib.dl_rkl_topk_workspace_bytes(dtype, most + 1, V, 16) == 0
-    assert lib.dl_rkl_topk_workspace_bytes(dtype, 2 ** 31 - 1, V, 16) == 0
+    for rows in (1, 100, 4096, 32768, 524287, 524288, 2 ** 24, 2 ** 31 - 1):
+        per_turn, rest = divmod(lib.dl_rkl_topk_workspace_bytes(dtype, rows, V, K), 8 * K)
+        assert rest == 0 and 0 < per_turn <= rows and per_turn * K * 8 <= 16 << 20
+        assert (per_turn * parts + 7) // 8 * 8 * 256 < 2 ** 32
+        assert per_turn == rows or 2 * per_turn * max(K * 8 / 2 ** 24, parts * 256 / 2 ** 32) > 0.99      # no more turns than that asks for
