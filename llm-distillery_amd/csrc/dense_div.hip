@@ -220,9 +220,9 @@ static bool launch_dense_kind(const DenseParams& p, hipStream_t st) {
   const int64_t units = p.V / 8;
   constexpr int NUS = 256 / (16 * Unit<TagS>::NC);      // the student row alone: 256 bytes of registers per thread
   const dim3 grid(xcd_banded_grid(p.n_rows));
-  if (units <= 256 * NU) hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, 256, NU>), grid, dim3(256), 0, st, p);
-  else if (units <= 512 * NU) hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, 512, NU>), grid, dim3(512), 0, st, p);
-  else if (units <= 1024 * NU) hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, 1024, NU>), grid, dim3(1024), 0, st, p);
+  if (units <= 256 * NU) launch_dense_reg_nt<KIND, TagS, TagT, 256, NU, false>(p, st);
+  else if (units <= 512 * NU) launch_dense_reg_nt<KIND, TagS, TagT, 512, NU, false>(p, st);
+  else if (units <= 1024 * NU) launch_dense_reg_nt<KIND, TagS, TagT, 1024, NU, false>(p, st);
   else if (units <= 1024 * NUS) {
     // more than 64 KiB of dynamic LDS has to be requested per kernel, once per device (the call is slow)
     constexpr size_t lds = StudentRegRows<TagS, TagT, 1024, NUS>::LDS_BYTES;

@@ -6,10 +6,9 @@ namespace dl {
 template <int KIND, class TagS, class TagT, int NU>
 static bool launch_any_kind(const DenseParams& p, hipStream_t st) {
   const int64_t units = p.V / 8;      // the columns behind them ride along whatever the shape
-  const dim3 grid(xcd_banded_grid(p.n_rows));
-  if (units <= 256 * NU) hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, 256, NU, true>), grid, dim3(256), 0, st, p);
-  else if (units <= 512 * NU) hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, 512, NU, true>), grid, dim3(512), 0, st, p);
-  else if (units <= 1024 * NU) hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, 1024, NU, true>), grid, dim3(1024), 0, st, p);
+  if (units <= 256 * NU) launch_dense_reg_nt<KIND, TagS, TagT, 256, NU, true>(p, st);
+  else if (units <= 512 * NU) launch_dense_reg_nt<KIND, TagS, TagT, 512, NU, true>(p, st);
+  else if (units <= 1024 * NU) launch_dense_reg_nt<KIND, TagS, TagT, 1024, NU, true>(p, st);
   else return false;
   return true;
 }

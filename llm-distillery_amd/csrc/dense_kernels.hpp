@@ -242,10 +242,15 @@ struct RegRows {
   }
 };
 
-// JSD: four waves per SIMD are asked for (128 registers): with the kept ratios the 16-bit pairs off the grid would take a few
-// more, one workgroup fewer per CU (8192 x 32100 bf16: 386 us against 252).
-template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY = false>
-__global__ __launch_bounds__(NT, KIND == DL_JSD ? 4 : 1) void dense_reg_kernel(const DenseParams p) {
+// What JSD keeps of its divergence sweep for the gradient (see dense_stats).
+template <class Rows, bool GRAD>
+constexpr int JSD_KEEP = Rows::EXACT_STASH ? JSD_KEEP_BOTH : GRAD ? JSD_KEEP_RATIO : JSD_KEEP_NOTHING;
+
+// JSD with a gradient: four waves per SIMD are asked for (128 registers): with the kept ratios the 16-bit pairs off the grid
+// would take a few more, one workgroup fewer per CU (8192 x 32100 bf16: 386 us against 252).  GRAD = false: a call without a
+// gradient, for which nothing is kept (JSD only: what a call's gradient costs the other kinds is a branch).
+template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY = false, bool GRAD = true>
+__global__ __launch_bounds__(NT, KIND == DL_JSD && GRAD ? 4 : 1) void dense_reg_kernel(const DenseParams p) {
   __shared__ float red[64];
   const int64_t r = xcd_banded_row(blockIdx.x);
   if (r >= p.n_rows) return;
@@ -268,17 +273,29 @@ __global__ __launch_bounds__(NT, KIND == DL_JSD ? 4 : 1) void dense_reg_kernel(c
   rows.load(srow + head * TagS::bytes, tl + head * TagT::bytes, nunits, head, ANY ? (int)(p.V - head - nunits * 8) : 0);
   if (ANY && grow) grow += head * TagS::bytes;
   if constexpr (KIND == DL_JSD) {
-    // The divergence sweep leaves the gradient's ingredients in registers (also when no gradient is asked for: a second
-    // copy of the sweeps for that case costs registers).
-    constexpr int KEEP = RegRows<TagS, TagT, NT, NU, ANY>::EXACT_STASH ? JSD_KEEP_BOTH : JSD_KEEP_RATIO;
+    constexpr int KEEP = JSD_KEEP<RegRows<TagS, TagT, NT, NU, ANY>, GRAD>;
     const DenseStats st = dense_stats<KIND, NT, KEEP>(rows, p.inv_T_s, p.inv_T_t, red);
     if (tid == 0 && p.row_loss) p.row_loss[r] = st.loss;
-    if (grow) dense_jsd_grad_kept<KEEP, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+    if (GRAD && grow) dense_jsd_grad_kept<KEEP, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
   } else {
     const DenseStats st = dense_stats<KIND, NT>(rows, p.inv_T_s, p.inv_T_t, red);
     if (tid == 0 && p.row_loss) p.row_loss[r] = st.loss;
     if (grow) dense_grad_sweep<KIND, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
   }
+}
+
+// One launch over rows that NT threads hold whole.  JSD of pairs that keep the log ratio: without a gradient the kernel that
+// keeps nothing (2048 x 12000 fp32 against bf16 32.5 us with the ratios kept, 29.2 without; 512 x 50257 bf16 42.5, 40.5).
+template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY>
+static void launch_dense_reg_nt(const DenseParams& p, hipStream_t st) {
+  const dim3 grid(xcd_banded_grid(p.n_rows)), block(NT);
+  if constexpr (KIND == DL_JSD && RegRows<TagS, TagT, NT, NU, ANY>::RATIO_STASH) {
+    if (!p.grad) {
+      hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, NT, NU, ANY, false>), grid, block, 0, st, p);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((dense_reg_kernel<KIND, TagS, TagT, NT, NU, ANY>), grid, block, 0, st, p);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -296,6 +313,9 @@ __global__ __launch_bounds__(NT, KIND == DL_JSD ? 4 : 1) void dense_reg_kernel(c
 // JSD needs the row's normalisers inside a logarithm, and the divergence again in its gradient: its parts meet a second
 // time, over (KL(P || M), KL(Q || M)) of their columns, in a second record each.  A part that gave up at either meeting is
 // finished by two launches: the first makes the second records of all listed parts, the second finds every record complete.
+// Those two keep nothing for the gradient: their body is a real call, and with the ratios its stack grew from 192 to 268
+// bytes a lane.  The runtime gives a queue scratch for the largest it has met, and every launch that uses any then waits
+// longer: with them in a process, all calls that cut rows, of any pair, took 4 us more (64 x 50257 fp32 26.3 -> 30.2).
 // Against streaming such rows from memory (four scalar passes off the 16-byte grid): 4013 x 98922 bf16 against fp32
 // 3600 -> 897 us, 327 x 125715 fp32 against bf16 428 -> 143 us, 4096 x 128256 bf16 1064 -> 916 us.
 // ---------------------------------------------------------------------------------------
@@ -386,7 +406,7 @@ __device__ __forceinline__ bool dense_exchange(const DenseSplit& x, DenseRecord*
 // (JSD) over the listed ones before that, up to their second record.
 constexpr int SPLIT_FIRST = 0, SPLIT_FINISH = 1, SPLIT_SECOND = 2;
 
-template <int KIND, class TagS, class TagT, int NT, int NU, int RETRY, bool ANY>
+template <int KIND, class TagS, class TagT, int NT, int NU, int RETRY, bool ANY, bool GRAD>
 __device__ __forceinline__ void dense_split_part(const DenseParams& p, const DenseSplit& x, int64_t r, int h, float* red,
                                                  float (*xch)[DENSE_MAX_PARTS], int* xok) {
   const int tid = threadIdx.x;
@@ -410,6 +430,7 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
     return;
   }
   using Rows = RegRows<TagS, TagT, NT, NU, ANY>;
+  constexpr int KEEP = JSD_KEEP<Rows, GRAD && RETRY == SPLIT_FIRST>;
   Rows rows;
   rows.load(srow + first * TagS::bytes, reinterpret_cast<const char*>(p.t_logits) + (trow * p.t_stride + first) * TagT::bytes, nu,
             head, tail);
@@ -486,7 +507,7 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
   st.tmax = Mt;
   if constexpr (KIND == DL_JSD) {
     float kp = 0.f, kq = 0.f;
-    dense_jsd_sums<Rows::EXACT_STASH ? JSD_KEEP_BOTH : JSD_KEEP_RATIO>(rows, st, kp, kq);
+    dense_jsd_sums<KEEP>(rows, st, kp, kq);
     block_sum2<NT>(kp, kq, red);
     DenseRecord* ws2 = x.second + r * P;
     if (RETRY == SPLIT_SECOND) {
@@ -504,14 +525,13 @@ __device__ __forceinline__ void dense_split_part(const DenseParams& p, const Den
     st.aux = KIND == DL_RKL && Rows::CENTRED ? rkl_centre(W / S, st, Ms * a_s, Mt * a_t) : st.loss;
   }
   if (tid == 0 && h == 0 && p.row_loss) p.row_loss[r] = st.loss;
-  if (grow) {
-    if constexpr (KIND == DL_JSD)
-      dense_jsd_grad_kept<Rows::EXACT_STASH ? JSD_KEEP_BOTH : JSD_KEEP_RATIO, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
+  if (GRAD && grow) {
+    if constexpr (KIND == DL_JSD && KEEP != JSD_KEEP_NOTHING) dense_jsd_grad_kept<KEEP, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
     else dense_grad_sweep<KIND, TagS>(rows, st, p.inv_T_s * p.grad_scale, grow);
   }
 }
 
-template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY>
+template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY, bool GRAD = true>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void dense_split_kernel(const DenseParams p, const DenseSplit x) {
   __shared__ float red[64];
@@ -521,14 +541,14 @@ void dense_split_kernel(const DenseParams p, const DenseSplit x) {
   const unsigned grp = blockIdx.x / (8u * P), t_in = blockIdx.x % (8u * P);
   const int64_t r = (int64_t)grp * 8 + (t_in & 7u);
   if (r >= p.n_rows) return;
-  dense_split_part<KIND, TagS, TagT, NT, NU, SPLIT_FIRST, ANY>(p, x, r, (int)(t_in >> 3), red, xch, xok);
+  dense_split_part<KIND, TagS, TagT, NT, NU, SPLIT_FIRST, ANY, GRAD>(p, x, r, (int)(t_in >> 3), red, xch, xok);
 }
 
 // One listed part, as a real call: the loop around it then costs the body no registers.
 template <int KIND, class TagS, class TagT, int NT, int NU, int RETRY, bool ANY>
 __device__ __attribute__((noinline)) void dense_split_part_again(const DenseParams& p, const DenseSplit& x, unsigned at, float* red,
                                                                  float (*xch)[DENSE_MAX_PARTS], int* xok) {
-  dense_split_part<KIND, TagS, TagT, NT, NU, RETRY, ANY>(p, x, (int64_t)(at / (unsigned)x.parts), (int)(at % (unsigned)x.parts), red, xch, xok);
+  dense_split_part<KIND, TagS, TagT, NT, NU, RETRY, ANY, true>(p, x, (int64_t)(at / (unsigned)x.parts), (int)(at % (unsigned)x.parts), red, xch, xok);
 }
 
 // The parts that gave up waiting, a fixed grid striding over their list (normally empty).
@@ -557,8 +577,10 @@ static void launch_dense_split_kind(const DenseParams& p, const DenseSplit& x, h
   const int64_t n16 = DenseSplit::n_records(KIND, p.n_rows, x.parts) * 2 + 1;      // records, then the retry counter
   hipLaunchKernelGGL((dense_clear_kernel<256>), dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st,
                      reinterpret_cast<u32x4*>(x.records), n16);
-  hipLaunchKernelGGL((dense_split_kernel<KIND, TagS, TagT, NT, NU, ANY>), dim3((unsigned)((p.n_rows + 7) / 8 * 8 * x.parts)),
-                     dim3(NT), 0, st, p, x);
+  const dim3 grid((unsigned)((p.n_rows + 7) / 8 * 8 * x.parts));
+  constexpr bool KEEPS = KIND == DL_JSD && RegRows<TagS, TagT, NT, NU, ANY>::RATIO_STASH;      // see launch_dense_reg_nt
+  if (KEEPS && !p.grad) hipLaunchKernelGGL((dense_split_kernel<KIND, TagS, TagT, NT, NU, ANY, !KEEPS>), grid, dim3(NT), 0, st, p, x);
+  else hipLaunchKernelGGL((dense_split_kernel<KIND, TagS, TagT, NT, NU, ANY>), grid, dim3(NT), 0, st, p, x);
   const dim3 again((unsigned)std::min<int64_t>(p.n_rows * x.parts, 256));
   if constexpr (KIND == DL_JSD)
     hipLaunchKernelGGL((dense_split_retry_kernel<KIND, TagS, TagT, NT, NU, SPLIT_SECOND, ANY>), again, dim3(NT), 0, st, p, x);
