@@ -425,8 +425,8 @@ def test_planned_forms_on_teacher_rows_off_the_16_byte_grid(D, Vt, shift):
                                    (24577, 2048)])
 @pytest.mark.parametrize("shift", [0, 3])
 def test_a_plan_with_teacher_rows_that_end_inside_a_unit(D, Vt, Vs, shift):
-    """Teacher vocabularies that are no multiple of four ids: the last 1-3 probabilities of every row count, also where the last
-    tile of the attached plan holds nothing but those.  The rows end where the buffer ends."""
+    """Teacher vocabularies that are no multiple of four ids: the last 1-3 probabilities of every row count.  The rows end where
+    the buffer ends."""
     R = 5
     rng = np.random.default_rng(Vt)
     t2s = rng.integers(-1, 700, Vt).astype(np.int32)
@@ -456,7 +456,7 @@ def test_a_plan_with_teacher_rows_that_end_inside_a_unit(D, Vt, Vs, shift):
 @pytest.mark.parametrize("Vt,Vs,used", [(1027, 1000, 300), (8192, 2048, 2048), (24581, 4096, 700), (40000, 16384, 9000)])
 def test_more_rows_than_cus_take_two_workgroups_per_cu(D, Vt, Vs, used, dtype):
     """More than 256 rows: workgroups of 512 threads that walk two lists per wave and tile (one tile, odd numbers of tiles, a
-    row that ends inside a unit, ids enough for several units per thread), masked rows, the gradient over the logits."""
+    row that ends inside a unit; the last map is too wide for two workgroups per CU), masked rows, the gradient over the logits."""
     R = 259
     rng = np.random.default_rng(Vt)
     ids = rng.permutation(Vs)[:used]
@@ -487,11 +487,11 @@ def test_more_rows_than_cus_take_two_workgroups_per_cu(D, Vt, Vs, used, dtype):
 
 
 @pytest.mark.parametrize("R,Vt,Vs,used,dtype", [(3, 70001, 2048, 500, torch.bfloat16),      # tiles dealt to several workgroups, a ragged end
-                                                (2, 200064, 16384, 16384, torch.float16),    # the full plan, eight parts
+                                                (2, 200064, 16384, 16384, torch.float16),    # the full plan, six parts
                                                 (128, 70000, 2048, 700, torch.float32), (129, 70000, 2048, 700, torch.float32)])
 def test_few_rows_against_a_wide_teacher(D, R, Vt, Vs, used, dtype):
     """Up to 128 rows a row's tiles are shared by several workgroups through a workspace, and the passes take a launch of their
-    own; masked rows, the gradient over the logits; the same within rounding as one launch (dl_rkl_marginalised without one)."""
+    own; masked rows, the gradient over the logits."""
     rng = np.random.default_rng(Vt + R)
     ids = rng.permutation(Vs)[:used]
     t2s = ids[rng.integers(0, used, Vt)].astype(np.int32)
@@ -524,3 +524,139 @@ def test_few_rows_against_a_wide_teacher(D, R, Vt, Vs, used, dtype):
                                                   1e-4 if dtype == torch.float32 else 2e-3)
         err = (grad[valid].double() - grad64).abs()
         assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+
+
+def _map_onto(Vt, Vs, used, dropped=0.05):
+    """Teacher ids onto `used` of the student ids, every one of them named; some teacher ids onto none."""
+    rng = np.random.default_rng(Vt + used)
+    ids = rng.permutation(Vs)[:used]
+    t2s = ids[rng.integers(0, used, Vt)].astype(np.int32)
+    t2s[rng.random(Vt) < dropped] = -1
+    t2s[rng.permutation(Vt)[:used]] = ids
+    t2s[-3:] = ids[:3]                               # the last three count
+    t2s[:3] = ids[-3:]
+    t2s[5] = t2s[6] = -1
+    missing = np.setdiff1d(ids, t2s)
+    t2s[np.nonzero(t2s < 0)[0][:missing.size]] = missing
+    return t2s
+
+
+def _check_against_marginal(rl, grad, logits, probs, t2s, T, scale, dtype, rows=None):
+    """Row losses and gradients of `rows` (all: None) against float64."""
+    sel = torch.arange(logits.shape[0]) if rows is None else rows
+    marg = torch.tensor(O.marginalise_map(probs[sel].double().numpy(), t2s, logits.shape[1]))
+    with np.errstate(divide="ignore"):
+        t_logits = O.marginal_to_teacher_logits(marg)
+    _, rows64, grad64 = O.mean_loss_and_grad("rkl", logits[sel], T, t_logits=t_logits, dtype=torch.float64)
+    grad64 = grad64 * (len(sel) * scale)
+    np.testing.assert_allclose(rl[sel].cpu().double().numpy(), rows64.numpy(), rtol=3e-5, atol=3e-6)
+    bound = O.marginal_rkl_gradient_tolerance(grad64, logits[sel], t_logits, rows64, T, T, scale, dtype,
+                                              1e-4 if dtype == torch.float32 else 2e-3)
+    err = (grad[sel].cpu().double() - grad64).abs()
+    assert (err <= bound).all(), f"worst ratio {(err / bound).max():.2f}"
+    assert torch.count_nonzero(grad[sel].cpu()[marg == 0]) == 0
+
+
+@pytest.mark.parametrize("R", [3, 130, 259])         # several workgroups per row; one of 1024 threads; of 512
+@pytest.mark.parametrize("Vt,Vs,used,tile", [(61441, 2048, 700, 6144), (61442, 2048, 700, 6144), (86019, 2048, 300, 7168),
+                                             (131075, 8192, 8192, 8192)])
+def test_a_last_tile_without_a_whole_unit(D, R, Vt, Vs, used, tile):
+    """One to three probabilities are all that the last tile of the plan holds: no whole 16-byte unit of it is fetched.  The rows
+    end where the buffer ends, and start on any element."""
+    t2s = _map_onto(Vt, Vs, used)
+    plan = _map_in_the_form(D, "auto", t2s, Vs)
+    assert (plan.compact or plan.full).tile == plan.full.tile == tile and Vt % tile in (1, 2, 3) and (t2s[-(Vt % tile):] >= 0).all()
+    g = torch.Generator().manual_seed(Vt)
+    probs = torch.softmax(torch.randn(R, Vt, generator=g) * 2, -1)
+    probs[:, -(Vt % tile):] += 0.05                  # what the last tile brings is no rounding
+    logits = torch.randn(R, Vs, generator=g) * 2
+    buf = torch.zeros(1 + R * Vt, device=DEV)
+    on_gpu = buf[1:].view(R, Vt)
+    on_gpu.copy_(probs)
+    few = torch.arange(min(R, 40))
+    got = D.vocab_utils.marginalise(on_gpu, plan=plan, n_student=Vs).cpu().numpy()[few]
+    ref = O.marginalise_map(probs[few].numpy(), t2s, Vs)
+    np.testing.assert_allclose(got, ref, rtol=2e-6, atol=1e-9)
+    assert np.array_equal(got == 0, ref == 0)
+    rl, grad = D.vocab_utils.rkl_marginalised(logits.to(DEV), on_gpu, plan, T=1.3, grad_scale=0.25)
+    _check_against_marginal(rl, grad, logits, probs, t2s, 1.3, 0.25, torch.float32, few)
+
+
+@pytest.mark.parametrize("Vt,Vs,used,dtype,half", [
+    (40000, 32000, 6704, torch.bfloat16, True),      # 838 units of 8 ids for 512 threads: two each
+    (40000, 32000, 6704, torch.float32, True),
+    (40000, 18000, 8192, torch.float32, True),       # as many fp32 ids as two units per thread hold,
+    (40000, 18000, 8200, torch.float32, False),      # and a unit more
+    (40001, 32000, 12088, torch.float16, True),      # as many as the LDS of two workgroups per CU holds (three units each),
+    (40001, 32000, 12096, torch.float16, False)])    # and a unit more
+def test_widths_that_two_workgroups_per_cu_hold(D, Vt, Vs, used, dtype, half):
+    """The passes behind the marginal with several units per thread of a 512-thread workgroup, and the borders of its rule, among
+    them rows whose sums leave the range and are redone on their maxima, a row without mass, a masked row."""
+    R = 259
+    t2s = _map_onto(Vt, Vs, used)
+    plan = _map_in_the_form(D, "auto", t2s, Vs)
+    c = plan.compact
+    assert plan.n_compact == used and c.tile == 8192 and c.n_extra == 0
+    lds = 4 * (used + 64 + c.tile + 4)               # the marginal, the lanes' spare slots, the tile and its zeros
+    assert half == (used <= (8192 if dtype == torch.float32 else 16384) and lds <= 80 * 1024 - 512)
+    g = torch.Generator().manual_seed(Vt)
+    probs = torch.softmax(torch.randn(R, Vt, generator=g) * 2, -1)
+    logits = torch.randn(R, Vs, generator=g) * 2
+    probs[7] *= 1e-25
+    probs[8] *= 1e25
+    off = int(t2s[20])
+    probs[9, torch.tensor(t2s == off)] = 0.0         # the student's mass on a column that is off row 9's support
+    logits[9, off] = 300.0
+    probs[10] = 0.0
+    logits = logits.to(dtype)
+    rm = torch.arange(R, dtype=torch.int32)
+    rm[11] = -1
+    x = logits.to(DEV)
+    rl, grad = D.vocab_utils.rkl_marginalised(x, probs.to(DEV), plan, row_map=rm.to(DEV), T=1.3, grad_scale=0.25, grad_out=x)
+    assert torch.count_nonzero(rl[10:12]) == 0 and torch.count_nonzero(grad[10:12]) == 0
+    _check_against_marginal(rl, grad, logits, probs, t2s, 1.3, 0.25, dtype, torch.tensor([0, 1, 7, 8, 9, 12, 100, 255, 256, 258]))
+
+
+@pytest.mark.parametrize("R,Vt,Vs,used,dtype,parts", [
+    (2, 270000, 16384, 16384, torch.float16, 8),     # the full plan, 33 tiles of 8192: as many parts as there ever are
+    (3, 70001, 2048, 500, torch.bfloat16, 3),        # a ragged end
+    (85, 100000, 8192, 8192, torch.float32, 3),      # 256 / 85
+    (128, 131075, 8192, 8192, torch.float32, 2)])    # the last of 17 tiles holds three probabilities
+def test_partial_marginals_against_one_launch(D, R, Vt, Vs, used, dtype, parts):
+    """With a workspace the tiles of few rows are dealt to `parts` workgroups each: the same within rounding as one launch.  A
+    workspace that is too small, off the 16-byte grid or absent is one launch, bit for bit."""
+    lib = D._lib.load()
+    t2s = _map_onto(Vt, Vs, used)
+    plan = _map_in_the_form(D, "full", t2s, Vs)
+    assert lib.dl_rkl_marginalised_workspace_bytes(R, Vt, Vs, plan.full.tile) == R * parts * Vs * 4
+    g = torch.Generator(device=DEV).manual_seed(Vt)
+    probs = torch.softmax(torch.randn(R, Vt, generator=g, device=DEV) * 2, -1)
+    logits = (torch.randn(R, Vs, generator=g, device=DEV) * 2).to(dtype)
+    rm = torch.arange(R, dtype=torch.int32, device=DEV)
+    rm[1] = -1
+    ws = torch.full((R * parts * Vs + 4,), float("nan"), device=DEV)
+    assert ws.data_ptr() % 16 == 0
+
+    def run(workspace):
+        rl, grad = torch.empty(R, device=DEV), torch.empty_like(logits)
+        args = [logits.data_ptr(), D.ops._DT[dtype], Vs, R, Vs, rm.data_ptr(), probs.data_ptr(), D.ops._DT[torch.float32], Vt, R, Vt,
+                plan.t2s.data_ptr(), *plan.full.args(), 1 / 1.3, 1 / 1.3, 0.25, rl.data_ptr(), grad.data_ptr(), Vs]
+        stream = torch.cuda.current_stream().cuda_stream
+        if workspace is None:
+            D._lib.check(lib.dl_rkl_marginalised(*args, stream), "dl_rkl_marginalised")
+        else:
+            D._lib.check(lib.dl_rkl_marginalised_ws(*args, *workspace, stream), "dl_rkl_marginalised_ws")
+        return rl, grad
+
+    n = R * parts * Vs * 4
+    one = run(None)
+    for short in ((ws.data_ptr(), n - 1), (ws.data_ptr() + 4, n), (0, 0)):
+        assert all(torch.equal(a, b) for a, b in zip(one, run(short)))
+    assert torch.isnan(ws).all()
+    rl, grad = run((ws.data_ptr(), n))
+    assert not torch.isnan(ws[:Vs]).any()
+    torch.testing.assert_close(rl, one[0], rtol=3e-5, atol=3e-6)
+    live = [r for r in range(min(R, 40)) if r != 1]
+    for got in (one, (rl, grad)):
+        assert got[0][1] == 0 and torch.count_nonzero(got[1][1]) == 0
+        _check_against_marginal(*got, logits.cpu(), probs.cpu(), t2s, 1.3, 0.25, dtype, torch.tensor(live))
