@@ -18,9 +18,8 @@ struct StatsParams {
 };
 
 // ---- phase 1: lse_r = logsumexp_j(x_rj * inv_T),  zk_rk = x[r, idx_rk] * inv_T ------------------
-// MODE 0: element-wise loads (rows that are not even element-aligned never get here; kept for reference
-// and for rows shorter than a chunk).  MODE 1: rows on the 16-byte grid, a whole number of chunks long.
-// MODE 2: any other row: its 16-byte chunks by vector loads, the elements before and behind them one by one.
+// MODE 1: rows on the 16-byte grid, a whole number of chunks long.  MODE 2: any other row: its 16-byte chunks (a row
+// shorter than a chunk has none) by vector loads, the elements before and behind them one by one.
 //
 // STASH: the logits at the teacher's ids are not fetched by loads of their own (K random reads of cold lines per
 // row, which the sweep then fetches a second time: a quarter more traffic and 9 of the kernel's 50 us on 2048
@@ -75,193 +74,184 @@ __device__ __forceinline__ void rowstats_row(const StatsParams& p, const Composi
       p.zk[trow * p.K + k] = (id >= 0 && id < p.V) ? load_as_float(row, Tag::id, id) * p.inv_T : 0.f;
     }
   }
-  if (MODE != 0) {
-    const RowSplit<Tag> sp(row, p.V, MODE == 2);
-    const char* body = row + (int64_t)sp.head * Tag::bytes;
-    const int64_t nch = sp.nbody;
-    u32x4* stash = reinterpret_cast<u32x4*>(smem);
-    unsigned long long mybits = 0;
-    int slot = 0;
-    int64_t idv[RECORD ? E : 1];      // RECORD: the thread's teacher ids, its row's label and whether that counts: known
-    bool want = false;                // before the sweep, so that the record behind it waits for no load
-    int64_t label = -1;
-    if constexpr (STASH) {
-      s_bits[tid] = 0;
-      __syncthreads();
-      const auto mark = [&](int64_t id) {
-        const int64_t rel = id - sp.head;
-        if (rel >= 0 && rel < nch * C::N) {
-          const int ch = (int)(rel / C::N);
-          atomicOr(&s_bits[ch % NT], 1ull << (ch / NT));
-        }
-      };
-      if constexpr (RECORD) {
-#pragma unroll
-        for (int j = 0; j < E; ++j) {
-          const int k = tid + j * NT;
-          idv[j] = load_index(p.t_idx, p.t_idx_itype, trow * p.K + (k < p.K ? k : 0));
-        }
-        const int c = convo_of_row(cp->off, cp->n_convos, trow);
-        const int li = (int)(trow - cp->off.row(c));
-        want = li < cp->off.label(c + 1) - cp->off.label(c);
-        if (want) {
-          label = cp->labels[cp->off.label(c) + li];
-          for (int av = cp->off.avoid(c); av < cp->off.avoid(c + 1); ++av) want = want && (load_index(cp->avoid, cp->avoid_itype, av) != li);
-        }
-#pragma unroll
-        for (int j = 0; j < E; ++j) {
-          if (tid + j * NT < p.K) mark(idv[j]);
-          else idv[j] = -1;
-        }
-      } else {
-        for (int k = tid; k < p.K; k += NT) mark(load_index(p.t_idx, p.t_idx_itype, trow * p.K + k));
+  const RowSplit<Tag> sp(row, p.V, MODE == 2);
+  const char* body = row + (int64_t)sp.head * Tag::bytes;
+  const int64_t nch = sp.nbody;
+  u32x4* stash = reinterpret_cast<u32x4*>(smem);
+  unsigned long long mybits = 0;
+  int slot = 0;
+  int64_t idv[RECORD ? E : 1];      // RECORD: the thread's teacher ids, its row's label and whether that counts: known
+  bool want = false;                // before the sweep, so that the record behind it waits for no load
+  int64_t label = -1;
+  if constexpr (STASH) {
+    s_bits[tid] = 0;
+    __syncthreads();
+    const auto mark = [&](int64_t id) {
+      const int64_t rel = id - sp.head;
+      if (rel >= 0 && rel < nch * C::N) {
+        const int ch = (int)(rel / C::N);
+        atomicOr(&s_bits[ch % NT], 1ull << (ch / NT));
       }
-      __syncthreads();
-      mybits = s_bits[tid];
-      const int cnt = __popcll(mybits);
-      int inc = cnt;                                         // inclusive scan over the wave, then over the waves
+    };
+    if constexpr (RECORD) {
 #pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(inc, d, 64);
-        if ((tid & 63) >= d) inc += up;
+      for (int j = 0; j < E; ++j) {
+        const int k = tid + j * NT;
+        idv[j] = load_index(p.t_idx, p.t_idx_itype, trow * p.K + (k < p.K ? k : 0));
       }
-      if ((tid & 63) == 63) s_wave[tid >> 6] = inc;
-      __syncthreads();
-      int before = 0;
+      const int c = convo_of_row(cp->off, cp->n_convos, trow);
+      const int li = (int)(trow - cp->off.row(c));
+      want = li < cp->off.label(c + 1) - cp->off.label(c);
+      if (want) {
+        label = cp->labels[cp->off.label(c) + li];
+        for (int av = cp->off.avoid(c); av < cp->off.avoid(c + 1); ++av) want = want && (load_index(cp->avoid, cp->avoid_itype, av) != li);
+      }
 #pragma unroll
-      for (int w = 0; w < NT / 64; ++w) before += (w < (tid >> 6)) ? s_wave[w] : 0;
-      slot = before + inc - cnt;
-      s_pre[tid] = slot;
+      for (int j = 0; j < E; ++j) {
+        if (tid + j * NT < p.K) mark(idv[j]);
+        else idv[j] = -1;
+      }
+    } else {
+      for (int k = tid; k < p.K; k += NT) mark(load_index(p.t_idx, p.t_idx_itype, trow * p.K + k));
     }
-    for (int64_t c0 = 0; c0 < nch; c0 += 4 * NT) {          // four 16-byte loads in flight per thread
-      u32x4 v[4];
+    __syncthreads();
+    mybits = s_bits[tid];
+    const int cnt = __popcll(mybits);
+    int inc = cnt;                                         // inclusive scan over the wave, then over the waves
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t ch = c0 + (int64_t)u * NT + tid;
-        // streamed, not cached: with cached loads the kernel is slower, whether or not gathers follow that could hit
-        v[u] = ch < nch ? load16_stream(body + ch * 16) : C::neg_inf();
-      }
-      float cm = -INFINITY;
-      float f[4][C::N];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        C::unpack(v[u], f[u]);
-#pragma unroll
-        for (int e = 0; e < C::N; ++e) cm = fmaxf(cm, f[u][e]);
-      }
-      if constexpr (STASH) {
-        const unsigned four = (unsigned)(mybits >> (c0 / NT)) & 15u;
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-          if (four >> u & 1) stash[slot++] = v[u];
-      }
-      if (cm > m) { sm *= fast_exp2((m - cm) * a); m = cm; }
-      const float mb = m * a;
-      if (mb > MASKED_BELOW) {      // nothing but masked columns so far: no bias to sum on
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int e = 0; e < C::N; ++e) sm += fast_exp2(fmaf(f[u][e], a, -mb));
-      }
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(inc, d, 64);
+      if ((tid & 63) >= d) inc += up;
     }
-    if (MODE == 2 && tid < sp.leftovers()) one(load_as_float(row, Tag::id, sp.column(tid)));
-    const float mx = block_max<NT>(m, red);
-    sm = (m == -INFINITY) ? 0.f : sm * fast_exp2((m - mx) * a);
-    sm = block_sum<NT>(sm, red);
-    const float lse = (mx * a + fast_log2(sm)) * LN2;
-    if (tid == 0) p.lse[trow] = lse;
-    if constexpr (STASH) {
-      __syncthreads();
-      // the logit at teacher entry k out of its chunk's slot (the few columns before and behind the body: from memory)
-      const auto logit_at = [&](int64_t id) {
-        const int64_t rel = id - sp.head;
-        float z = 0.f;
-        if (rel >= 0 && rel < nch * C::N) {
-          const int ch = (int)(rel / C::N), t = ch % NT, j = ch / NT;
-          const int at = s_pre[t] + __popcll(s_bits[t] & ((1ull << j) - 1ull));
-          const int e = at * C::N + (int)(rel % C::N);
-          if constexpr (Tag::bytes == 4) z = reinterpret_cast<const float*>(smem)[e];
-          else z = load_as_float(reinterpret_cast<const unsigned short*>(smem) + e, Tag::id, 0);
-        } else if (id >= 0 && id < p.V) {
-          z = load_as_float(row, Tag::id, id);
-        }
-        return z * p.inv_T;
-      };
-      if constexpr (!RECORD) {
-        for (int k = tid; k < p.K; k += NT) p.zk[trow * p.K + k] = logit_at(load_index(p.t_idx, p.t_idx_itype, trow * p.K + k));
-      } else {
-        const int K = p.K;
-        float tv[E], zv[E];
+    if ((tid & 63) == 63) s_wave[tid >> 6] = inc;
+    __syncthreads();
+    int before = 0;
 #pragma unroll
-        for (int j = 0; j < E; ++j) {
-          const int k = tid + j * NT;
-          tv[j] = zv[j] = -INFINITY;
-          if (j * NT >= K) continue;
-          if (k < K) {
-            zv[j] = logit_at(idv[j]);
-            p.zk[trow * K + k] = zv[j];
-            const float t = cp->t_val_dtype == F32 ? __uint_as_float(traw[j])
-                            : cp->t_val_dtype == BF16 ? __uint_as_float(traw[j] << 16)
-                                                      : (float)__builtin_bit_cast(_Float16, (unsigned short)traw[j]);
-            tv[j] = t * cp->inv_T_t;
-          }
-        }
-        // the arithmetic of composite_row_record, entry for entry, with the reductions over the workgroup
-        float tmax = -INFINITY, zmax = -INFINITY;
-#pragma unroll
-        for (int j = 0; j < E; ++j) { tmax = fmaxf(tmax, tv[j]); zmax = fmaxf(zmax, zv[j]); }
-        block_max2<NT>(tmax, zmax, red);
-        // (rounds j that hold no entry at all are skipped by the whole workgroup; exponentials and logarithms by the
-        // hardware's base-2 instructions: a few units in the last place, against a record that is good to 1e-6)
-        const auto ex = [](float v) { return fast_exp2(v * LOG2E); };
-        float tsum = 0.f, zsum = 0.f;
-#pragma unroll
-        for (int j = 0; j < E; ++j)
-          if (j * NT < K) { tsum += ex(tv[j] - tmax); zsum += ex(zv[j] - zmax); }      // exp(-inf) = 0 beyond K
-        block_sum2<NT>(tsum, zsum, red);
-        const float t_lse = tmax + fast_log2(tsum) * LN2;
-        const float z_lse = zmax + fast_log2(zsum) * LN2;
-        const float s_lse = z_lse - lse;
-        float kl = 0.f, rkl = 0.f, found = -INFINITY;      // found: minus the first entry that carries the label
-#pragma unroll
-        for (int j = 0; j < E; ++j) {
-          const int k = tid + j * NT;
-          if (j * NT >= K) continue;
-          if (k < K) {
-            const float t = tv[j] - t_lse;
-            const float sk = zv[j] - lse;
-            const float s2 = sk - s_lse;
-            kl += ex(t) * (t - sk);
-            rkl += ex(s2) * (s2 - t);
-            if (want && idv[j] == label) found = fmaxf(found, -(float)k);
-          }
-        }
-        block_sum2<NT>(kl, rkl, red);
-        found = block_max<NT>(found, red);
-        const int kstar = found == -INFINITY ? -1 : (int)(-found);
-#pragma unroll
-        for (int j = 0; j < E; ++j)
-          if (kstar >= 0 && tid + j * NT == kstar) { red[0] = zv[j] - lse; red[1] = tv[j] - t_lse; }
-        __syncthreads();
-        if (tid == 0) {
-          RowRec rr;
-          rr.kl = kl; rr.rkl = rkl; rr.t_lse = t_lse; rr.s_lse = s_lse;
-          rr.valid = kstar >= 0 ? 1 : 0;
-          rr.kstar = kstar;
-          rr.own_s = kstar >= 0 ? red[0] : 0.f;
-          rr.own_t = kstar >= 0 ? red[1] : 0.f;
-          cp->rec[trow] = rr;
-        }
-      }
-    }
-    return;
-  } else {
-    for (int64_t j = tid; j < p.V; j += NT) one(load_as_float(row, Tag::id, j));
+    for (int w = 0; w < NT / 64; ++w) before += (w < (tid >> 6)) ? s_wave[w] : 0;
+    slot = before + inc - cnt;
+    s_pre[tid] = slot;
   }
+  for (int64_t c0 = 0; c0 < nch; c0 += 4 * NT) {          // four 16-byte loads in flight per thread
+    u32x4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t ch = c0 + (int64_t)u * NT + tid;
+      // streamed, not cached: with cached loads the kernel is slower, whether or not gathers follow that could hit
+      v[u] = ch < nch ? load16_stream(body + ch * 16) : C::neg_inf();
+    }
+    float cm = -INFINITY;
+    float f[4][C::N];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      C::unpack(v[u], f[u]);
+#pragma unroll
+      for (int e = 0; e < C::N; ++e) cm = fmaxf(cm, f[u][e]);
+    }
+    if constexpr (STASH) {
+      const unsigned four = (unsigned)(mybits >> (c0 / NT)) & 15u;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (four >> u & 1) stash[slot++] = v[u];
+    }
+    if (cm > m) { sm *= fast_exp2((m - cm) * a); m = cm; }
+    const float mb = m * a;
+    if (mb > MASKED_BELOW) {      // nothing but masked columns so far: no bias to sum on
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < C::N; ++e) sm += fast_exp2(fmaf(f[u][e], a, -mb));
+    }
+  }
+  if (MODE == 2 && tid < sp.leftovers()) one(load_as_float(row, Tag::id, sp.column(tid)));
   const float mx = block_max<NT>(m, red);
   sm = (m == -INFINITY) ? 0.f : sm * fast_exp2((m - mx) * a);
   sm = block_sum<NT>(sm, red);
-  if (tid == 0) p.lse[trow] = (mx * a + fast_log2(sm)) * LN2;
+  const float lse = (mx * a + fast_log2(sm)) * LN2;
+  if (tid == 0) p.lse[trow] = lse;
+  if constexpr (STASH) {
+    __syncthreads();
+    // the logit at teacher entry k out of its chunk's slot (the few columns before and behind the body: from memory)
+    const auto logit_at = [&](int64_t id) {
+      const int64_t rel = id - sp.head;
+      float z = 0.f;
+      if (rel >= 0 && rel < nch * C::N) {
+        const int ch = (int)(rel / C::N), t = ch % NT, j = ch / NT;
+        const int at = s_pre[t] + __popcll(s_bits[t] & ((1ull << j) - 1ull));
+        const int e = at * C::N + (int)(rel % C::N);
+        if constexpr (Tag::bytes == 4) z = reinterpret_cast<const float*>(smem)[e];
+        else z = load_as_float(reinterpret_cast<const unsigned short*>(smem) + e, Tag::id, 0);
+      } else if (id >= 0 && id < p.V) {
+        z = load_as_float(row, Tag::id, id);
+      }
+      return z * p.inv_T;
+    };
+    if constexpr (!RECORD) {
+      for (int k = tid; k < p.K; k += NT) p.zk[trow * p.K + k] = logit_at(load_index(p.t_idx, p.t_idx_itype, trow * p.K + k));
+    } else {
+      const int K = p.K;
+      float tv[E], zv[E];
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        const int k = tid + j * NT;
+        tv[j] = zv[j] = -INFINITY;
+        if (j * NT >= K) continue;
+        if (k < K) {
+          zv[j] = logit_at(idv[j]);
+          p.zk[trow * K + k] = zv[j];
+          const float t = cp->t_val_dtype == F32 ? __uint_as_float(traw[j])
+                          : cp->t_val_dtype == BF16 ? __uint_as_float(traw[j] << 16)
+                                                    : (float)__builtin_bit_cast(_Float16, (unsigned short)traw[j]);
+          tv[j] = t * cp->inv_T_t;
+        }
+      }
+      // the arithmetic of composite_row_record, entry for entry, with the reductions over the workgroup
+      float tmax = -INFINITY, zmax = -INFINITY;
+#pragma unroll
+      for (int j = 0; j < E; ++j) { tmax = fmaxf(tmax, tv[j]); zmax = fmaxf(zmax, zv[j]); }
+      block_max2<NT>(tmax, zmax, red);
+      // (rounds j that hold no entry at all are skipped by the whole workgroup; exponentials and logarithms by the
+      // hardware's base-2 instructions: a few units in the last place, against a record that is good to 1e-6)
+      const auto ex = [](float v) { return fast_exp2(v * LOG2E); };
+      float tsum = 0.f, zsum = 0.f;
+#pragma unroll
+      for (int j = 0; j < E; ++j)
+        if (j * NT < K) { tsum += ex(tv[j] - tmax); zsum += ex(zv[j] - zmax); }      // exp(-inf) = 0 beyond K
+      block_sum2<NT>(tsum, zsum, red);
+      const float t_lse = tmax + fast_log2(tsum) * LN2;
+      const float z_lse = zmax + fast_log2(zsum) * LN2;
+      const float s_lse = z_lse - lse;
+      float kl = 0.f, rkl = 0.f, found = -INFINITY;      // found: minus the first entry that carries the label
+#pragma unroll
+      for (int j = 0; j < E; ++j) {
+        const int k = tid + j * NT;
+        if (j * NT >= K) continue;
+        if (k < K) {
+          const float t = tv[j] - t_lse;
+          const float sk = zv[j] - lse;
+          const float s2 = sk - s_lse;
+          kl += ex(t) * (t - sk);
+          rkl += ex(s2) * (s2 - t);
+          if (want && idv[j] == label) found = fmaxf(found, -(float)k);
+        }
+      }
+      block_sum2<NT>(kl, rkl, red);
+      found = block_max<NT>(found, red);
+      const int kstar = found == -INFINITY ? -1 : (int)(-found);
+#pragma unroll
+      for (int j = 0; j < E; ++j)
+        if (kstar >= 0 && tid + j * NT == kstar) { red[0] = zv[j] - lse; red[1] = tv[j] - t_lse; }
+      __syncthreads();
+      if (tid == 0) {
+        RowRec rr;
+        rr.kl = kl; rr.rkl = rkl; rr.t_lse = t_lse; rr.s_lse = s_lse;
+        rr.valid = kstar >= 0 ? 1 : 0;
+        rr.kstar = kstar;
+        rr.own_s = kstar >= 0 ? red[0] : 0.f;
+        rr.own_t = kstar >= 0 ? red[1] : 0.f;
+        cp->rec[trow] = rr;
+      }
+    }
+  }
 }
 
 template <class Tag, int NT, int MODE, bool STASH>
@@ -314,8 +304,8 @@ __device__ __forceinline__ bool correction_add(const int* head, const int* next,
   return again != 0u;
 }
 
-// MODE as for phase 1.  MODE 2 needs the gradient row to sit on the 16-byte grid exactly as the logits row does
-// (same address modulo 16): the kernel then works on the rows' bodies, with the teacher ids counted
+// MODE 1 as for phase 1.  MODE 0: element-wise.  MODE 2 needs the gradient row to sit on the 16-byte grid exactly as the
+// logits row does (same address modulo 16; pairs that do not take MODE 0): the kernel then works on the rows' bodies, with the teacher ids counted
 // from the body's first column, and part 0 adds the few columns before and behind the body one by one.
 // MODE 3: logits and gradient rows on the 16-byte grid that end inside a chunk (logits[:, :, :crop] of padded
 // rows): the ragged chunk is loaded and converted like the others -- its 16 bytes start inside the row and,
@@ -511,8 +501,8 @@ static int stats_threads(int64_t n_rows, int64_t V, int epc) {
 }
 // the logits at the teacher's ids out of the sweep where the row's chunks fit the threads' 64 rounds (the bound holds
 // for every row: a peeled head only shortens the body)
-static bool stash_fits(int mode, int K, int64_t V, int epc, int64_t n_rows) {
-  return mode != 0 && K <= STASH_MAX_K && (V + epc - 1) / epc <= (int64_t)STASH_ROUNDS * stats_threads(n_rows, V, epc);
+static bool stash_fits(int K, int64_t V, int epc, int64_t n_rows) {
+  return K <= STASH_MAX_K && (V + epc - 1) / epc <= (int64_t)STASH_ROUNDS * stats_threads(n_rows, V, epc);
 }
 // phase 1 with the rows' records of the composite loss made at its tail (the caller has checked stash_fits)
 template <class Tag, int NT>
@@ -533,14 +523,13 @@ static hipError_t launch_stats_record(const StatsParams& p, int mode, const Comp
 
 template <class Tag, int NT>
 static void launch_stats_nt(const StatsParams& p, int mode, hipStream_t st) {
-  const bool stash = stash_fits(mode, p.K, p.V, Tag::epc, p.n_rows);
+  const bool stash = stash_fits(p.K, p.V, Tag::epc, p.n_rows);
   const size_t lds = stash ? (size_t)p.K * 16 : 0;
   const dim3 grid((unsigned)p.n_rows), block(NT);
   if (mode == 1 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 1, true>), grid, block, lds, st, p);
-  else if (mode == 2 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 2, true>), grid, block, lds, st, p);
+  else if (stash) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 2, true>), grid, block, lds, st, p);
   else if (mode == 1) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 1, false>), grid, block, 0, st, p);
-  else if (mode == 2) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 2, false>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 0, false>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 2, false>), grid, block, 0, st, p);
 }
 template <class Tag>
 static hipError_t launch_stats(const StatsParams& p, int mode, hipStream_t st) {
@@ -632,7 +621,7 @@ extern "C" int dl_composite_forward_train(const void* logits, int logits_dtype, 
                   nullptr, nullptr, nullptr, 0};
     // every teacher row has its logits row (no map, as many of the one as of the other): the rows' records at the
     // tail of phase 1; else teacher rows without a logits row need records too: the launch of their own
-    if (!row_map && n_teacher_rows == n_rows && stash_fits(vec, K, V, 16 / eb, n_rows)) {
+    if (!row_map && n_teacher_rows == n_rows && stash_fits(K, V, 16 / eb, n_rows)) {
       const hipError_t e = logits_dtype == DL_F32 ? launch_stats_record<TagF32>(p, vec, cp, st)
                            : logits_dtype == DL_BF16 ? launch_stats_record<TagBF16>(p, vec, cp, st)
                                                      : launch_stats_record<TagF16>(p, vec, cp, st);
