@@ -18,8 +18,10 @@
 //     tile at random (LDS), and adds runs of equal slot into LDS words only it touches in that
 //     tile, so no atomics, and the order of additions is fixed: bit-reproducible.  Replicas are
 //     folded into their id's slot after the last tile.
-//   * fused reverse KL: the marginal never leaves LDS; its logarithm is the teacher row of the
-//     dense-divergence sweeps, the student row sits in registers.
+//   * fused reverse KL: the marginal stays in LDS; its logarithm is the teacher row of the
+//     dense-divergence sweeps, the student row sits in registers.  (Up to 128 rows against a wide
+//     teacher, along a plan: partial marginals of a row by several workgroups, summed by the one that
+//     runs the sweeps in a second launch.)
 #include "dense_div.hpp"
 #include <algorithm>
 

@@ -241,9 +241,10 @@ def expand_columns(xc: torch.Tensor, col_src: torch.Tensor, V: int, out: torch.T
     return out
 
 
-def _parts_workspace(rows: int, n_teacher: int, n_columns: int, tile: int, dev):
-    """(tensor or None, bytes): room for the partial marginals of a call with few rows."""
-    n = _lib.load().dl_rkl_marginalised_workspace_bytes(rows, n_teacher, n_columns, tile)
+def _parts_workspace(rows: int, n_teacher: int, p_dtype: torch.dtype, n_columns: int, tile: int, dev):
+    """(tensor or None, bytes): room for the partial marginals of a call with few rows (none for probabilities of 16 bits,
+    which go without a plan)."""
+    n = _lib.load().dl_rkl_marginalised_workspace_bytes(rows, n_teacher, n_columns, tile) if p_dtype == torch.float32 else 0
     return (torch.empty(n, dtype=torch.uint8, device=dev) if n else None), n
 
 
@@ -252,7 +253,8 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
                      grad_scale: float = 1.0, want_grad: bool = True, grad_out: torch.Tensor | None = None):
     """Reverse KL of the student (logits [rows, Vs]) against the teacher's distribution
     (teacher_probs [N, Vt]) marginalised into the student vocabulary along `t2s`, loss and gradient
-    in one launch; the marginal stays in LDS.  `t2s` is the int32 [Vt] map on the GPU or, better, a
+    in one launch, the marginal in LDS; with a plan, up to 128 rows against a wide fp32 teacher take two, and
+    partial marginals pass through a workspace.  `t2s` is the int32 [Vt] map on the GPU or, better, a
     MarginalPlan built from it.  Returns (row_loss fp32 [rows], grad or None)."""
     _dev(logits, "logits")
     x, tp = _rows_2d(logits), _rows_2d(teacher_probs)
@@ -276,7 +278,7 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
             if want_grad:
                 grad = _grad_target(grad_out, R, Vs, x.dtype, dev)
                 g_ptr, g_stride = grad.data_ptr(), grad.stride(0)
-            ws, ws_bytes = _parts_workspace(R, Vt, plan.n_compact, plan.compact.tile, dev)
+            ws, ws_bytes = _parts_workspace(R, Vt, tp.dtype, plan.n_compact, plan.compact.tile, dev)
             with _on(dev):
                 st = _lib.load().dl_rkl_marginalised_compact_ws(
                     x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, plan.cols.data_ptr(), plan.col_src16.data_ptr(),
@@ -301,7 +303,7 @@ def rkl_marginalised(logits: torch.Tensor, teacher_probs: torch.Tensor, t2s: "to
     if want_grad:
         grad = _grad_target(grad_out, R, Vs, x.dtype, dev)
         g_ptr, g_stride = grad.data_ptr(), grad.stride(0)
-    ws, ws_bytes = _parts_workspace(R, Vt, Vs, plan_args[2], dev)
+    ws, ws_bytes = _parts_workspace(R, Vt, tp.dtype, Vs, plan_args[2], dev)
     with _on(dev):
         st = _lib.load().dl_rkl_marginalised_ws(x.data_ptr(), _DT[x.dtype], x.stride(0), R, Vs, rm_ptr, tp.data_ptr(),
                                                 _DT[tp.dtype], tp.stride(0), N, Vt, t2s.data_ptr(), *plan_args, 1.0 / T,

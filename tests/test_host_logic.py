@@ -389,3 +389,13 @@ def test_reverse_kl_in_two_launches_takes_many_rows_in_turns(dtype, V, parts, K)
         assert rest == 0 and 0 < per_turn <= rows and per_turn * K * 8 <= 16 << 20
         assert (per_turn * parts + 7) // 8 * 8 * 256 < 2 ** 32
         assert per_turn == rows or 2 * per_turn * max(K * 8 / 2 ** 24, parts * 256 / 2 ** 32) > 0.99      # no more turns than that asks for
+
+
+def test_partial_marginals_take_a_workspace_for_fp32_probabilities_only():
+    """Probabilities of 16 bits go without a plan, in one launch: no room for partial marginals is taken for them."""
+    from llm_distillery_amd.vocab_utils import _parts_workspace
+    ws, n = _parts_workspace(16, 152064, torch.float32, 2048, 8192, "cpu")
+    assert n == ws.numel() == 16 * 4 * 2048 * 4
+    for dtype in (torch.bfloat16, torch.float16):
+        assert _parts_workspace(16, 152064, dtype, 2048, 8192, "cpu") == (None, 0)
+    assert _parts_workspace(129, 152064, torch.float32, 2048, 8192, "cpu") == (None, 0)
