@@ -815,7 +815,7 @@ __global__ __launch_bounds__(NT, 4) void rkl_marginalised_kernel(const MargParam
 // Few rows leave most CUs idle while a wide teacher row's tiles are walked one after the other (1.2 us each).  Two launches
 // then: the tiles of a row dealt to `parts` workgroups, whose partial marginals (fp32) go to a workspace, and the passes behind
 // the marginal on their sum, taken in part order.  64 rows x
-// 152064 onto 32000 ids 37.0 -> 23.7 us for the call (four workgroups a row), 54 x 170432 41.0 -> 26.5, 27 x 151680 onto 21352
+// 152064 onto 32000 ids, 3749 in use, 37.0 -> 23.7 us for the call (four workgroups a row), 54 x 170432 41.0 -> 26.5, 27 x 151680 onto 21352
 // 37.1 -> 23.4, 128 x 152064 (two a row) 37.3 -> 32.2; rows of less than eight tiles have too little to share (90 x 50304 22 us).
 template <int LOAD>
 __global__ __launch_bounds__(MARG_NT) void marginal_parts_kernel(const MargParams p, float* out, int parts) {
@@ -864,11 +864,22 @@ __global__ __launch_bounds__(MARG_NT) void rkl_marginal_parts_kernel(const MargP
   }
 }
 
-// Workgroups that share a row's tiles: as many as there are CUs for, at least four tiles each (1: one launch).
-static int marg_parts(int64_t n_rows, int64_t Vt, int plan_tile) {
+// Workgroups that share a row's tiles: as many as there are CUs for, at least four tiles each (1: one launch), and only
+// where the tiles that a row's longest walk is spared (730 ns and 75 per 1024 ids each) outweigh the second launch and what the
+// partial marginals cost on their way: 3.6 us, 11 ns per KB of one row's, which one workgroup reads, 0.43 ns per KB of all rows',
+// 0.31 beyond 16 MB.  (Fitted to 360 shapes, one to eight parts, 1 to 128 rows, 50304 to 262144 onto 700 to 36000 columns;
+// rms 1.6 us.)  One launch and with parts: 128 x 70000 onto 700 / 9000 / 15000 / 32000 columns 19.8 and 17.8 / 27.5 and 29.4 /
+// 29.2 and 35.5 / 27.6 and 41.1 us, 27 rows onto 32000 26.4 and 29.8; 64 x 152064 onto 9000 / 24576 / 32000 39.6 and 30.8 / 39.5
+// and 39.1 / 41.2 and 43.7, 128 x 262144 onto 36000 86 and 73.
+static int marg_parts(int64_t n_rows, int64_t Vt, int64_t n_columns, int plan_tile) {
   if (n_rows <= 0 || n_rows > 128 || plan_tile < 4096) return 1;
   const int64_t ntiles = (Vt + plan_tile - 1) / plan_tile;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / n_rows, ntiles / 4, 8}));
+  const int64_t parts = std::min<int64_t>({256 / n_rows, ntiles / 4, 8});
+  if (parts < 2) return 1;
+  const int64_t row_kb = parts * n_columns * 4 / 1000, all_kb = n_rows * parts * n_columns * 4 / 1000;
+  const int64_t spared = (ntiles - (ntiles + parts - 1) / parts) * (730 + 75 * (int64_t)plan_tile / 1024);
+  const int64_t cost = 3600 + 11 * row_kb + (43 * std::min<int64_t>(all_kb, 16000) + 31 * std::max<int64_t>(all_kb - 16000, 0)) / 100;
+  return spared > cost ? (int)parts : 1;
 }
 
 // Workgroups of half as many threads, each wave walking two of a tile's lists (the plan and the order of its additions are
@@ -1028,7 +1039,7 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const dim3 grid(xcd_banded_grid(n_rows));
   allow_large_lds();
-  const int parts = p.plan_ent ? marg_parts(n_rows, Vt, plan_tile) : 1;
+  const int parts = p.plan_ent ? marg_parts(n_rows, Vt, Vs, plan_tile) : 1;
   if (parts > 1 && workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= n_rows * parts * Vs * 4) {
     float* buf = reinterpret_cast<float*>(workspace);
     const dim3 by(MARG_NT);
@@ -1062,7 +1073,7 @@ static int rkl_marginalised_launch(const void* logits, int logits_dtype, int64_t
 
 extern "C" int64_t dl_rkl_marginalised_workspace_bytes(int64_t n_rows, int64_t Vt, int64_t n_columns, int plan_tile) {
   if (Vt <= 0 || n_columns <= 0) return 0;
-  const int parts = dl::marg_parts(n_rows, Vt, plan_tile);
+  const int parts = dl::marg_parts(n_rows, Vt, n_columns, plan_tile);
   return parts > 1 ? n_rows * parts * n_columns * 4 : 0;
 }
 

@@ -399,3 +399,15 @@ def test_partial_marginals_take_a_workspace_for_fp32_probabilities_only():
     for dtype in (torch.bfloat16, torch.float16):
         assert _parts_workspace(16, 152064, dtype, 2048, 8192, "cpu") == (None, 0)
     assert _parts_workspace(129, 152064, torch.float32, 2048, 8192, "cpu") == (None, 0)
+
+
+@pytest.mark.parametrize("rows,Vt,columns,tile,parts", [
+    (64, 152064, 3752, 8192, 4), (128, 152064, 3752, 8192, 2), (1, 270000, 16384, 8192, 8), (27, 152064, 16384, 8192, 4),      # narrow marginals, many tiles
+    (128, 70000, 704, 7168, 2), (128, 70000, 9000, 8192, 1), (64, 70000, 15000, 8192, 1),      # few tiles: up to a width
+    (27, 70000, 32000, 8192, 1), (128, 100000, 36000, 4096, 1), (128, 152064, 32000, 8192, 1), (128, 262144, 36000, 4096, 2),
+    (129, 262144, 704, 8192, 1), (0, 262144, 704, 8192, 1), (64, 262144, 704, 0, 1)])
+def test_partial_marginals_are_taken_where_the_tiles_spared_outweigh_them(rows, Vt, columns, tile, parts):
+    """Several workgroups to a row write and read partial marginals as wide as the columns: more than a call gains where a wide
+    marginal meets few tiles."""
+    n = D._lib.load().dl_rkl_marginalised_workspace_bytes(rows, Vt, columns, tile)
+    assert n == (rows * parts * columns * 4 if parts > 1 else 0)
