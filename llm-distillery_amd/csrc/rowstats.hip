@@ -489,20 +489,28 @@ static bool same_phase16(const void* a, int64_t stride_a, const void* b, int64_t
 }
 
 // Threads per row in phase 1.  256 of them keep 16 KiB of a row in flight, eight rows to a CU, and their 64 rounds hold
-// 16384 chunks.  Rows wider than that take 1024, whose rounds hold them: no gathers, no launch for the rows' records, and a
-// longer share of the row in flight (phase 1 and records: 2048 x 75487 fp32 112 -> 105 us, 2048 x 151665 fp32 216 -> 198, 4084 x
-// 151665 bf16, half of them content rows, 152 -> 143; 512 threads measure the same on the first and 209 / 148 on the others).
-// Up to two rows per CU the chip is better filled by 512 threads each (131 x 32000 fp32 14.9 -> 11.7 us, 434 rows 18.1 ->
-// 16.4; 700 rows 20.7 -> 22.0).
-static int stats_threads(int64_t n_rows, int64_t V, int epc) {
-  const int64_t chunks = (V + epc - 1) / epc;
-  if (chunks > (int64_t)STASH_ROUNDS * 256 && chunks <= (int64_t)STASH_ROUNDS * 1024) return 1024;
-  return n_rows <= 512 ? 512 : 256;
+// 16384 chunks.
+// Up to 512 rows, two per CU, the chip is better filled by 512 threads each where those take half the sweeps of four chunks a
+// thread (131 x 32000 fp32 11.0 -> 8.1 us, 400 x 32000 13.6 -> 12.0, 512 x 32000 bf16 10.6 -> 9.6).  A row that 256 threads take
+// in one such sweep keeps them (512 x 4096 bf16 5.1 against 5.6 us); so does, beyond 256 rows, one of three, where 512 would
+// take two with the second half empty (2100 to 3072 chunks: 2-6 % slower; at 64 rows 4-8 % faster).
+// Rows wider than 16384 chunks take 1024, whose rounds hold them: no gathers, no launch for the rows' records, and a
+// longer share of the row in flight (phase 1 alone: 64 x 151665 fp32 36.5 -> 19.2 us, 2048 x 75487 107 -> 97, 2048 x 151665 bf16
+// 102 -> 97; with records 500 x 151665 bf16 59 -> 42).  They run two rows per CU, and where there are few gathers and no
+// launch of records to save (`record`: there is one; that and the gathers outweigh it from an entry per 64 chunks on), 401 to 768 rows are
+// better off with 256 threads, all rows at once and none in a second round (600 x 131080 bf16, K = 64: 31.2
+// against 34.9 us, 600 x 262144, K = 500: 53.9 against 57.0; 512 x 131072 fp32 40 against 46; with records, K = 50, 200 and
+// 400: 600 x 151665 bf16 45.1, 46.5 and 49.9 against 47.9, 48.2 and 48.8); to 1024 rows from 32768 chunks on (1024 x 262144 bf16 82 against 86).
+static int stats_threads(int64_t n_rows, int64_t V, int epc, int K, bool record) {
+  const int64_t chunks = (V + epc - 1) / epc, sweeps = (V / epc + 1023) / 1024;
+  if (chunks > (int64_t)STASH_ROUNDS * 256 && chunks <= (int64_t)STASH_ROUNDS * 1024)
+    return (record && K * 64LL >= chunks) || n_rows <= 400 || n_rows > (chunks < 32768 ? 768 : 1024) ? 1024 : 256;
+  return n_rows > 512 || sweeps <= 1 || (n_rows > 256 && sweeps == 3) ? 256 : 512;
 }
 // the logits at the teacher's ids out of the sweep where the row's chunks fit the threads' 64 rounds (the bound holds
 // for every row: a peeled head only shortens the body)
-static bool stash_fits(int K, int64_t V, int epc, int64_t n_rows) {
-  return K <= STASH_MAX_K && (V + epc - 1) / epc <= (int64_t)STASH_ROUNDS * stats_threads(n_rows, V, epc);
+static bool stash_fits(int K, int64_t V, int epc, int64_t n_rows, bool record) {
+  return K <= STASH_MAX_K && (V + epc - 1) / epc <= (int64_t)STASH_ROUNDS * stats_threads(n_rows, V, epc, K, record);
 }
 // phase 1 with the rows' records of the composite loss made at its tail (the caller has checked stash_fits)
 template <class Tag, int NT>
@@ -514,7 +522,7 @@ static void launch_stats_record_nt(const StatsParams& p, int mode, const Composi
 }
 template <class Tag>
 static hipError_t launch_stats_record(const StatsParams& p, int mode, const CompositeParams& cp, hipStream_t st) {
-  const int nt = stats_threads(p.n_rows, p.V, Tag::epc);
+  const int nt = stats_threads(p.n_rows, p.V, Tag::epc, p.K, true);
   if (nt == 1024) launch_stats_record_nt<Tag, 1024>(p, mode, cp, st);
   else if (nt == 512) launch_stats_record_nt<Tag, 512>(p, mode, cp, st);
   else launch_stats_record_nt<Tag, 256>(p, mode, cp, st);
@@ -523,7 +531,7 @@ static hipError_t launch_stats_record(const StatsParams& p, int mode, const Comp
 
 template <class Tag, int NT>
 static void launch_stats_nt(const StatsParams& p, int mode, hipStream_t st) {
-  const bool stash = stash_fits(p.K, p.V, Tag::epc, p.n_rows);
+  const bool stash = stash_fits(p.K, p.V, Tag::epc, p.n_rows, false);
   const size_t lds = stash ? (size_t)p.K * 16 : 0;
   const dim3 grid((unsigned)p.n_rows), block(NT);
   if (mode == 1 && stash) hipLaunchKernelGGL((rowstats_kernel<Tag, NT, 1, true>), grid, block, lds, st, p);
@@ -533,7 +541,7 @@ static void launch_stats_nt(const StatsParams& p, int mode, hipStream_t st) {
 }
 template <class Tag>
 static hipError_t launch_stats(const StatsParams& p, int mode, hipStream_t st) {
-  const int nt = stats_threads(p.n_rows, p.V, Tag::epc);
+  const int nt = stats_threads(p.n_rows, p.V, Tag::epc, p.K, false);
   if (nt == 1024) launch_stats_nt<Tag, 1024>(p, mode, st);
   else if (nt == 512) launch_stats_nt<Tag, 512>(p, mode, st);
   else launch_stats_nt<Tag, 256>(p, mode, st);
@@ -621,7 +629,7 @@ extern "C" int dl_composite_forward_train(const void* logits, int logits_dtype, 
                   nullptr, nullptr, nullptr, 0};
     // every teacher row has its logits row (no map, as many of the one as of the other): the rows' records at the
     // tail of phase 1; else teacher rows without a logits row need records too: the launch of their own
-    if (!row_map && n_teacher_rows == n_rows && stash_fits(K, V, 16 / eb, n_rows)) {
+    if (!row_map && n_teacher_rows == n_rows && stash_fits(K, V, 16 / eb, n_rows, true)) {
       const hipError_t e = logits_dtype == DL_F32 ? launch_stats_record<TagF32>(p, vec, cp, st)
                            : logits_dtype == DL_BF16 ? launch_stats_record<TagBF16>(p, vec, cp, st)
                                                      : launch_stats_record<TagF16>(p, vec, cp, st);

@@ -612,7 +612,7 @@ def test_logits_masked_with_low_finite_values(D, dtype, V, T):
     (torch.float32, 75487, 75487, 64, [5, 4]),                  # the same off the 16-byte grid
     (torch.float16, 524288, 524288, 40, [4]),                   # 64 rounds of 1024 threads,
     (torch.float16, 524296, 524296, 40, [4]),                   # and one chunk more: no launch takes the ids out of the sweep
-    (torch.float32, 2048, 2048, 300, [513]), (torch.float32, 2048, 2048, 300, [300, 212])])      # 256 threads from 513 rows on, 512 below
+    (torch.float32, 2048, 2048, 300, [513]), (torch.float32, 2048, 2048, 300, [300, 212])])      # either side of 512 rows
 def test_threads_of_phase_one_by_rows_and_width(D, dtype, V, pitch, K, lens):
     test_records_made_at_the_tail_of_phase_one_equal_the_separate_launches(D, dtype, V, pitch, K, lens, True)
 
@@ -620,3 +620,36 @@ def test_threads_of_phase_one_by_rows_and_width(D, dtype, V, pitch, K, lens):
 @pytest.mark.parametrize("V,dtype", [(65540, torch.float32), (131080, torch.bfloat16), (524296, torch.bfloat16)])
 def test_phase_one_on_rows_wider_than_256_threads_hold_rounds_for(D, V, dtype):
     test_phase_one_ids_out_of_the_sweep_or_gathered(D, dtype, V, 64)
+
+
+@pytest.mark.parametrize("dtype,V,rows,K", [
+    (torch.float32, 4099, 512, 64), (torch.float32, 4100, 512, 64), (torch.float32, 4100, 513, 64),      # one sweep of 256 threads; 512
+    (torch.bfloat16, 24576, 256, 64), (torch.bfloat16, 24576, 257, 64), (torch.bfloat16, 24592, 257, 64),      # three sweeps; four
+    (torch.float32, 65540, 400, 64), (torch.float32, 65540, 401, 256), (torch.float32, 65540, 401, 257),      # too wide for 256 threads' rounds:
+    (torch.float32, 65540, 768, 64), (torch.float32, 65540, 769, 64), (torch.bfloat16, 131081, 768, 64),      # all the same from 401 to 768 rows,
+    (torch.bfloat16, 262144, 769, 64), (torch.bfloat16, 262143, 769, 64)])                                    # or 1024, where few ids are gathered
+def test_phase_one_at_the_borders_of_its_thread_rule(D, dtype, V, rows, K):
+    """Log-sum-exps and the logits at the teacher's ids at the rows and widths where the number of threads changes, by themselves
+    and with the records of the composite loss at their tail; the loss with its launches apart is the same within rounding."""
+    from llm_distillery_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(V + rows)
+    x = torch.randn(rows, V, generator=g, device=DEV, dtype=dtype) * 2
+    first = torch.randint(0, V, (rows, 1), generator=g, device=DEV)
+    ti = (first + torch.arange(K, device=DEV) * (V // K)) % V                        # distinct ids over the whole row,
+    ti[:, :2] = torch.tensor([0, V - 1], device=DEV)                                 # its ends among them
+    tv = torch.log_softmax(torch.randn(rows, K, generator=g, device=DEV) * 2, -1)
+    # 2e-6 of a log-sum-exp of 10 and more: the rounding of its fp32 value and of a sum of up to 262144 terms taken by threads, waves and rows
+    ref = torch.logsumexp(x.double() / 1.3, -1)
+    zk64 = x.gather(1, ti).float() * torch.tensor(1.0 / 1.3, device=DEV)
+    offsets = [[0, rows], [0, rows - 1], [0, 1]]
+    args = (tv, ti, ti[:rows - 1, K // 3].contiguous(), torch.tensor([5], device=DEV), offsets, None, 1.0 / 1.3, 1.0, 2.0, 0, True)
+    out, lse, zk, _, _ = ops._composite_forward_raw(x, *args)
+    ops.SEPARATE_COMPOSITE_FORWARD = True
+    try:
+        out2, lse2, zk2, _, _ = ops._composite_forward_raw(x, *args)
+    finally:
+        ops.SEPARATE_COMPOSITE_FORWARD = False
+    for a, b in ((lse, zk), (lse2, zk2)):
+        assert ((a.double() - ref).abs() <= 2e-6 * ref.abs()).all()
+        assert torch.equal(b, zk64)
+    np.testing.assert_allclose(out.cpu().numpy(), out2.cpu().numpy(), rtol=2e-5, atol=2e-6)
