@@ -278,12 +278,14 @@ static int dense_split_units(int s_dtype, int t_dtype) {
 //   * on fewer than 1024 rows the cut pays only from 256 KiB of row pair upwards (one workgroup per row keeps
 //     the CUs busy by itself below that, and has no partners to wait for).
 //   * JSD, whose parts meet twice and have one more launch behind them: a pair that 1024 threads hold stays whole below
-//     1536 rows of 16-bit pairs and 3072 rows of others; a pair that they do not hold is always cut.  At the lines, whole
-//     and cut: 16-bit pairs, 1536 rows of 33000 / 40960 / 50257 / 65536 columns 103 / 117 / 150 / 184 and 94 / 103 / 131 /
-//     147 us (1024 rows: 69 / 81 / 103 / 125 and 71 / 78 / 94 / 104); 3072 rows of 16392 / 24000 / 32768 columns, bf16
-//     against fp32 119 / 162 / 205 and 103 / 129 / 199, fp32 148 / 193 / 244 and 152 / 190 / 228, fp32 against bf16 141 /
-//     183 / 242 and 150 / 181 / 224.  (bf16 against fp32 gains from 2048 rows on, but not at every width: 24000 / 28000 /
-//     32768 columns 105 / 118 / 138 and 91 / 123 / 134.)
+//     1536 rows of 16-bit pairs and 3072 rows of others; a pair that they do not hold is always cut.  From these lines on the
+//     cut was ahead at every width when both forms made the log ratios twice.  Now that they are kept, the two meet elsewhere,
+//     earlier for wide rows (whole and cut, us): 16-bit pairs of 33000 / 40960 / 50257 / 65536 columns, 512 rows 37 / 41 / 54 / 70 and
+//     46 / 49 / 57 / 62, 1024 rows 70 / 81 / 102 / 126 and 71 / 77 / 94 / 106, 1536 rows 103 / 118 / 149 / 182 and 96 / 107 / 132 / 147;
+//     16392 / 24000 / 32768 columns, fp32 2048 rows 100 / 130 / 169 and 108 / 132 / 161, 3072 rows 148 / 186 / 240 and 148 / 186 /
+//     230; bf16 against fp32 1536 rows 62 / 85 / 103 and 60 / 76 / 103 (28000: 98 and 101), 3072 rows 120 / 161 / 203 and 102 / 132 /
+//     197; fp32 against bf16 1536 rows 77 / 102 / 135 and 86 / 102 / 126, 3072 rows 140 / 186 / 237 and 146 / 178 / 219 (16392
+//     columns of this pair are ahead whole to 4096 rows: 178 and 185).
 // `forced_nt` (256 / 512 / 1024, a tuning hook) fixes the thread count and cuts wherever two parts or more come out.
 struct DenseCut { int nt, parts; };
 static DenseCut dense_split_cut(int kind, int s_dtype, int t_dtype, int64_t n_rows, int64_t V, int forced_nt = 0) {

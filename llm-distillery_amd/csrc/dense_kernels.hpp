@@ -247,7 +247,10 @@ template <class Rows, bool GRAD>
 constexpr int JSD_KEEP = Rows::EXACT_STASH ? JSD_KEEP_BOTH : GRAD ? JSD_KEEP_RATIO : JSD_KEEP_NOTHING;
 
 // JSD with a gradient: four waves per SIMD are asked for (128 registers): with the kept ratios the 16-bit pairs off the grid
-// would take a few more, one workgroup fewer per CU (8192 x 32100 bf16: 386 us against 252).  GRAD = false: a call without a
+// would take a few more, one workgroup fewer per CU (8192 x 32100 bf16: 386 us against 252).  The instances of 1024 threads
+// for 16-bit pairs spill 5 to 7 registers so, those of 512 off the grid and the column parts of 512 one or two (8 to 32 bytes
+// a lane); with the ratios made again they took 108 and none, and 8 to 15 % longer (128 x 50257 bf16 25.4 -> 23.4 us, 512 x
+// 40960 45.7 -> 43.8, 4096 x 65536 411 -> 354).  GRAD = false: a call without a
 // gradient, for which nothing is kept (JSD only: what a call's gradient costs the other kinds is a branch).
 template <int KIND, class TagS, class TagT, int NT, int NU, bool ANY = false, bool GRAD = true>
 __global__ __launch_bounds__(NT, KIND == DL_JSD && GRAD ? 4 : 1) void dense_reg_kernel(const DenseParams p) {

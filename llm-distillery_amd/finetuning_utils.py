@@ -117,9 +117,8 @@ def _fused_dicts(x: Tensor, row_map, inv_T: float, crop: int, counts, t_vals, t_
         avoid_cat = _packed_rows([a.to(torch.int64) for a in avoids])
     else:
         avoid_cat = avoids[0] if avoids[0].dtype in ops._IT else avoids[0].to(torch.int64)
-    one = {"single": True} if C == 1 else {}
     train, nine = ops.composite_loss(x, _packed_rows(t_vals), _packed_rows(t_idxs), lab_cat, avoid_cat.contiguous(), offs,
-                                     row_map, inv_T, inv_T_teacher, alpha, crop, **one)
+                                     row_map, inv_T, inv_T_teacher, alpha, crop, C == 1)
     out = []
     for c in range(C):
         row = nine[c]
