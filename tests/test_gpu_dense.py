@@ -463,6 +463,32 @@ def test_jsd_rows_cut_into_column_parts(D, dtype, t_dtype, V, threads):
         assert g4.data_ptr() == y.data_ptr() and torch.equal(rl, rl4) and torch.equal(g, y)
 
 
+@pytest.mark.parametrize("dtype,t_dtype", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.bfloat16, torch.float32),
+                                           (torch.float32, torch.float16), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("V,threads", [(8192, 0), (8195, 0), (12000, 0), (20000, 0), (20005, 0),      # rows held whole, on the grid and off it
+                                       (40960, 256), (40963, 256), (40960, 512), (66001, 512)])      # rows in column parts
+def test_jsd_without_a_gradient(D, dtype, t_dtype, V, threads):
+    """Calls without a gradient run instances of their own, which keep nothing for it: the row losses are those of float64, and of the
+    call with a gradient, also where every part is finished by the later launches; masked rows, a masked student column."""
+    R = 7
+    g = torch.Generator().manual_seed(V + threads)
+    s, t = (torch.randn(R, V, generator=g) * 3).to(dtype), (torch.randn(R, V, generator=g) * 3).to(t_dtype)
+    s[2, :V // 2] = float("-inf")
+    valid = torch.ones(R, dtype=torch.bool)
+    valid[4] = False
+    rm = torch.full((R,), -1, dtype=torch.int32)
+    rm[valid] = torch.arange(R - 1, dtype=torch.int32)
+    ref = O.jsd_dense_rows(s[valid].double() / 1.3, t[valid].double())
+    xs, xt = s.to(DEV), t[valid].to(DEV)
+    for no_wait in (False, True):
+        kw = dict(row_map=rm.to(DEV), T=1.3, teacher_T=1.0, part_threads=threads, no_wait=no_wait)
+        rl, none = D.div_dense("jsd", xs, xt, want_grad=False, **kw)
+        assert none is None and rl[4] == 0
+        np.testing.assert_allclose(rl.cpu()[valid].double().numpy(), ref.numpy(), rtol=3e-5, atol=3e-6)      # as _check
+        with_grad, _ = D.div_dense("jsd", xs, xt, **kw)
+        torch.testing.assert_close(rl, with_grad, rtol=3e-5, atol=3e-6)
+
+
 @pytest.mark.parametrize("kind", ["fkl", "rkl", "jsd"])
 @pytest.mark.parametrize("dtype,t_dtype,V,threads", [(torch.bfloat16, torch.bfloat16, 40000, 256), (torch.bfloat16, torch.bfloat16, 40003, 256),
                                                      (torch.float32, torch.float32, 33000, 256), (torch.float32, torch.float32, 33001, 256),
